@@ -311,6 +311,32 @@ int sbnet_sparse_scatter_functor_ws(const float* x, int N, int H, int W, int C, 
                                     int add, int transpose, int atomic,
                                     void* workspace, size_t workspace_bytes, void* stream);
 
+/* ------------------------------------------------------------------------------------------
+ * Convolution over the active blocks (inference)
+ * ------------------------------------------------------------------------------------------
+ * What the reference's layers compose from sparse_gather, batch norm, ReLU and library convolutions
+ * (benchmark/sparse_conv_lib.py:536-587, 677-824), without the block stacks in between; fp32 products and sums.
+ * Block positions, list and count are those of sparse_gather; bin_counts_device may be NULL, else num_active is the
+ * list's capacity and only the blocks before the count are computed.  Kernels are [kh, kw, in, out] with stride 1,
+ * applied to each block without padding; w_dims holds four ints per kernel.  Sizes whose byte offsets exceed 32 bits
+ * are refused with SBNET_EINVAL_ARG.
+ *
+ * sbnet_block_conv: q [num_active, bsize - k + 1, out] (NHWC stack) = convolution of the gathered blocks.
+ *
+ * sbnet_block_bottleneck: three convolutions (weights[3]), each behind an inference batch norm and a ReLU.
+ * batch_norms[12]: gamma, beta, mean, variance in front of each; the first four NULL for no batch norm and no ReLU in
+ * front of the first kernel.  The result goes to q (NHWC stack), or is added to y [x_dims] at pixels
+ * (bh * out_bstride[0], bw * out_bstride[1]) of each block's image; y may be x.  Exactly one of q and y is given. */
+int sbnet_block_conv(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
+                     const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,
+                     const int32_t* boffset, const float* w, const int32_t* w_dims, float* q, void* stream);
+size_t sbnet_block_bottleneck_workspace_bytes(int32_t num_active, const int32_t* bsize, const int32_t* w_dims);
+int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
+                           const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,
+                           const int32_t* boffset, const float* const* weights, const int32_t* w_dims,
+                           const float* const* batch_norms, float bn_eps, float* q, float* y,
+                           const int32_t* out_bstride, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Library-managed device scratch for callers that have no allocator at hand (the functor level of the reference
    passes none down, sparse_gather.h:45-66): returns a buffer of at least `bytes` bytes on the current device.  One
    grow-only buffer is kept per (device, stream); calls on one stream run in order, so consecutive calls of ONE

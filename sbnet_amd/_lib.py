@@ -61,6 +61,10 @@ SIGNATURES = {
                                                      _i32p, _int, _int, _int, _int, _vp, _sz, _vp]),
     "sbnet_sparse_scatter_functor_ws": (_int, [_vp, _int, _int, _int, _int, _vp] + [_int] * 7 + [_vp, _int, _int,
                                                                                                  _int, _vp, _sz, _vp]),
+    "sbnet_block_conv": (_int, [_vp, _i64p, _i32, _vp, _vp, _i32p, _i32p, _i32p, _vp, _i32p, _vp, _vp]),
+    "sbnet_block_bottleneck_workspace_bytes": (_sz, [_i32, _i32p, _i32p]),
+    "sbnet_block_bottleneck": (_int, [_vp, _i64p, _i32, _vp, _vp, _i32p, _i32p, _i32p, _vp, _i32p, _vp, _f, _vp, _vp,
+                                      _i32p, _vp, _sz, _vp]),
     "sbnet_scratch_acquire": (_vp, [_sz, _vp]),
     "sbnet_shutdown": (_int, []),
     "sbnet_copy_tensor": (_int, [_vp, _vp, _sz, _vp]),

@@ -14,6 +14,7 @@
 #include <mutex>
 #include <vector>
 
+#include "sbnet_conv.h"
 #include "sbnet_launch.h"
 
 namespace {
@@ -578,6 +579,127 @@ int sbnet_sparse_gather_grad(const float* dy, int32_t num_active, const int16_t*
     SBNET_HIP(sbnet::launch_zero(dx, (size_t)x_dims[0] * x_dims[1] * x_dims[2] * x_dims[3], s));
     return scatter_impl(dy, num_active, nullptr, active_block_indices, dx, x_dims, bsize, bstride, boffset, 1, 1, transpose,
                         workspace, workspace_bytes, s);
+}
+
+// The input side of a block convolution: checks, and the geometry of [N,H,W,C] read at the listed blocks.
+static int conv_input(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
+                      const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,
+                      const int32_t* boffset, sbnet::ConvArgs& c)
+{
+    if (!x || !x_dims || !active_block_indices || !bsize || !bstride || !boffset || num_active < 0 || !dims_fit_int(x_dims))
+        return SBNET_EINVAL_ARG;
+    if (!geom_ok((int)x_dims[0], (int)x_dims[1], (int)x_dims[2], (int)x_dims[3], bsize, bstride)) return SBNET_EINVAL_ARG;
+    c = sbnet::ConvArgs();
+    c.a = x;
+    c.idx = active_block_indices;
+    c.N = (int)x_dims[0]; c.H = (int)x_dims[1]; c.W = (int)x_dims[2]; c.C = (int)x_dims[3];
+    c.U = bstride[0]; c.V = bstride[1]; c.oh = boffset[0]; c.ow = boffset[1];
+    c.M = num_active;
+    c.countDev = bin_counts_device;
+    return SBNET_OK;
+}
+
+// The kernel side: w [kh,kw,C,K] on blocks of R x S pixels, false where they do not fit together.
+static bool conv_kernel(sbnet::ConvArgs& c, const float* w, const int32_t* w_dims, int R, int S)
+{
+    if (!w || w_dims[0] <= 0 || w_dims[1] <= 0 || w_dims[2] != c.C || w_dims[3] <= 0) return false;
+    c.w = w;
+    c.kh = w_dims[0]; c.kw = w_dims[1]; c.K = w_dims[3];
+    c.Ro = R - c.kh + 1; c.So = S - c.kw + 1;
+    return c.Ro > 0 && c.So > 0;
+}
+
+int sbnet_block_conv(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
+                     const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,
+                     const int32_t* boffset, const float* w, const int32_t* w_dims, float* q, void* stream)
+{
+    sbnet::ConvArgs c;
+    const int st = conv_input(x, x_dims, num_active, bin_counts_device, active_block_indices, bsize, bstride, boffset, c);
+    if (st != SBNET_OK) return st;
+    if (!q || !w_dims || !conv_kernel(c, w, w_dims, bsize[0], bsize[1]) || !sbnet::conv_fits(c)) return SBNET_EINVAL_ARG;
+    c.y = q;
+    SBNET_HIP(sbnet::launch_block_conv(c, static_cast<hipStream_t>(stream)));
+    return SBNET_OK;
+}
+
+// The three convolutions of a bottleneck; the result of each is the block stack the next one reads.
+static int bottleneck_args(sbnet::ConvArgs (&c)[3], const float* const* weights, const int32_t* w_dims,
+                           const float* const* batch_norms, float eps, const int32_t* bsize)
+{
+    int R = bsize[0], S = bsize[1];
+    sbnet::BnArgs bn[3];
+    for (int i = 0; i < 3; ++i) {
+        const float* const* b = batch_norms + 4 * i;
+        if (i > 0 && (!b[0] || !b[1] || !b[2] || !b[3])) return SBNET_EINVAL_ARG;
+        if (i == 0 && b[0] && (!b[1] || !b[2] || !b[3])) return SBNET_EINVAL_ARG;
+        bn[i] = sbnet::BnArgs{b[0], b[1], b[2], b[3], eps};
+    }
+    for (int i = 0; i < 3; ++i) {
+        if (i > 0) {
+            c[i] = sbnet::ConvArgs();
+            c[i].N = c[i].M = c[0].M;
+            c[i].H = R; c[i].W = S; c[i].C = c[i - 1].K;
+            c[i].countDev = c[0].countDev;
+        }
+        if (!conv_kernel(c[i], weights[i], w_dims + 4 * i, R, S)) return SBNET_EINVAL_ARG;
+        R = c[i].Ro; S = c[i].So;
+        c[i].post = i < 2 ? bn[i + 1] : sbnet::BnArgs();
+    }
+    c[0].pre = bn[0];
+    for (int i = 0; i < 3; ++i)
+        if (!sbnet::conv_fits(c[i])) return SBNET_EINVAL_ARG;
+    return SBNET_OK;
+}
+
+size_t sbnet_block_bottleneck_workspace_bytes(int32_t num_active, const int32_t* bsize, const int32_t* w_dims)
+{
+    if (num_active <= 0 || !bsize || !w_dims) return 0;
+    size_t total = 0;
+    int64_t R = bsize[0], S = bsize[1];
+    for (int i = 0; i < 2; ++i) {
+        R -= w_dims[4 * i] - 1;
+        S -= w_dims[4 * i + 1] - 1;
+        if (R <= 0 || S <= 0 || w_dims[4 * i + 3] <= 0) return 0;
+        total += ((size_t)num_active * R * S * w_dims[4 * i + 3] * sizeof(float) + 255) & ~(size_t)255;
+    }
+    return total;
+}
+
+int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
+                           const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,
+                           const int32_t* boffset, const float* const* weights, const int32_t* w_dims,
+                           const float* const* batch_norms, float bn_eps, float* q, float* y,
+                           const int32_t* out_bstride, void* workspace, size_t workspace_bytes, void* stream)
+{
+    sbnet::ConvArgs c[3];
+    const int st = conv_input(x, x_dims, num_active, bin_counts_device, active_block_indices, bsize, bstride, boffset, c[0]);
+    if (st != SBNET_OK) return st;
+    if (!weights || !w_dims || !batch_norms || (q != nullptr) == (y != nullptr)) return SBNET_EINVAL_ARG;
+    if (num_active == 0) return SBNET_OK;
+    const int st2 = bottleneck_args(c, weights, w_dims, batch_norms, bn_eps, bsize);
+    if (st2 != SBNET_OK) return st2;
+    const size_t need = sbnet_block_bottleneck_workspace_bytes(num_active, bsize, w_dims);
+    if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15)) return SBNET_EINVAL_ARG;
+    float* const h1 = static_cast<float*>(workspace);
+    float* const h2 = h1 + (((size_t)num_active * c[0].Ro * c[0].So * c[0].K * sizeof(float) + 255) & ~(size_t)255) / sizeof(float);
+    c[0].y = h1;
+    c[1].a = h1;
+    c[1].y = h2;
+    c[2].a = h2;
+    if (y) {
+        // added at the blocks' positions: their results must not meet, and the image has the last kernel's channels
+        if (!out_bstride || out_bstride[0] < c[2].Ro || out_bstride[1] < c[2].So || c[2].K != c[0].C) return SBNET_EINVAL_ARG;
+        c[2].y = y;
+        c[2].oidx = active_block_indices;
+        c[2].oN = c[0].N; c[2].oH = c[0].H; c[2].oW = c[0].W;
+        c[2].oU = out_bstride[0]; c[2].oV = out_bstride[1];
+        c[2].add = 1;
+        if (!sbnet::conv_fits(c[2])) return SBNET_EINVAL_ARG;
+    } else {
+        c[2].y = q;
+    }
+    for (int i = 0; i < 3; ++i) SBNET_HIP(sbnet::launch_block_conv(c[i], static_cast<hipStream_t>(stream)));
+    return SBNET_OK;
 }
 
 int sbnet_sparse_scatter_functor(const float* x, int N, int H, int W, int C, float* y, int bOffsH0,

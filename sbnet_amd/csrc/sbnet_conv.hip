@@ -1,0 +1,311 @@
+// Convolution over the active blocks on the fp32 matrix cores of gfx950: gather, the batch norm and ReLU in front
+// of a convolution, the convolution itself, and the paste or add of its result, without a block stack in between.
+//
+// Replaces, for the layers of sparse_conv.py in inference, the chain sparse_gather -> batch norm -> ReLU -> library
+// convolution (-> batch norm -> ReLU -> ...) -> sparse_scatter (sbnet_tensorflow/benchmark/sparse_conv_lib.py:536-587,
+// 677-723, 751-824).
+#include "sbnet_device.h"
+#include "sbnet_conv.h"
+
+namespace sbnet {
+
+// ---------------------------------------------------------------------------------------------
+// k_block_conv: out[p, n] = sum over k = (tap, c) of in[p + tap, c] * w[k, n]
+// ---------------------------------------------------------------------------------------------
+//
+// Rows p are the output pixels of all listed blocks, one after the other; k runs over the kernel's taps and the input
+// channels of each, in the memory order of w [kh, kw, C, K], so w is the right-hand matrix as it stands and channel
+// counts need no padding to a tap.  The input is an NHWC image read at the blocks' positions (pixels outside it are
+// zeros, as sparse_gather has them) or a block stack [M, R, S, C].
+//
+// A wave computes 16*FP pixels x 16*FN channels with v_mfma_f32_16x16x4_f32 (full fp32 products and sums: the precision
+// of the convolution it replaces).  Channels are the rows of the matrix instruction and pixels its columns, so that a
+// lane ends with four consecutive channels of one pixel: 16-byte stores into NHWC memory.  Both operands go from memory
+// straight to registers: with the instruction's k index spread as (lane / 16) * 4 + step, a lane's four pixel values
+// are one 16-byte load, and 4 lanes read the 64 bytes of a pixel that 16 k need.  The fp32 matrix rate is low enough
+// (a 2x2 wave tile multiplies for 512 cycles per 16 k, for which it reads 4 KB) that L1 feeds it, and without LDS
+// tiles there are no barriers: the problems are small (a few thousand pixels) and their time is a chain of latencies.
+// CONV_DEPTH sets of operands are in flight per wave.
+//
+// Measured (MI355X, kernel trace): 85 blocks of 17x17x48, 3x3 to 48 channels (19 000 pixels, 0.8 GFLOP): 27 us; the library
+// convolution took 21 us behind 5 us of layout copies, and up to 800 us the first time a block count occurred.  A whole
+// bottleneck block of 200 17x17x96 blocks: 50 us in three launches against about 300 us in 17.
+//
+// WK > 1: the WK waves of a workgroup split k among them and add up through LDS.  For launches whose tiles alone would
+// leave most of the 1024 SIMDs idle.
+//
+// Batch norm of the input (pre) applies to values after the load, out-of-image zeros included, with scale and shift
+// computed once per workgroup into LDS; batch norm of the result (post), for the convolution that follows, at the end.
+
+typedef float acc_t __attribute__((ext_vector_type(4)));
+
+constexpr int CONV_DEPTH = 3;   // operand sets in flight per wave
+
+struct ConvKernelArgs {
+    ConvArgs c;
+    FastDiv dC, dKw, dP, dSo;
+    uint32_t kTot, kSteps;      // taps * C, ceil(kTot / 16)
+    uint32_t rows, P;           // output pixels in all, per block
+    uint32_t tilesP, tilesN;
+    uint32_t aBytes, wBytes, yBytes;
+};
+
+__device__ __forceinline__ float relu_keep_nan(float v) { return v < 0.f ? 0.f : v; }
+
+// scale and shift of an inference batch norm, y = x * scale + shift
+__device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& scale, float& shift)
+{
+    scale = bn.gamma[c] * (1.f / sqrtf(bn.var[c] + bn.eps));
+    shift = bn.beta[c] - bn.mean[c] * scale;
+}
+
+template <int FP, int FN, int WK, int VEC>
+__global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKernelArgs a)
+{
+    constexpr int WAVES = WK > 4 ? WK : 4, WP = WAVES / WK;
+    constexpr int TP = 16 * FP * WP, TN = 16 * FN;
+    extern __shared__ float lds[];
+    const uint32_t cPad = a.c.pre.gamma ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
+    float* const preScale = lds;
+    float* const preShift = lds + cPad;
+    float* const postScale = lds + 2 * cPad;
+    float* const postShift = postScale + TN;
+    float* const red = postScale + 2 * TN;   // [WP][WK][FP * FN][64] x 4, WK > 1 only
+
+    // Eight consecutive workgroups go to eight XCDs; the tiles of one pixel range that differ in channels only follow
+    // each other on one XCD, whose L2 then holds the pixels once.
+    const uint32_t g = blockIdx.x >> 3;
+    const uint32_t tn = g % a.tilesN, tp = (g / a.tilesN) * 8u + (blockIdx.x & 7u);
+    uint32_t rows = a.rows;
+    if (a.c.countDev) rows = min(rows, (uint32_t)max(*a.c.countDev, 0) * a.P);
+    if (tp * TP >= rows) return;   // (the whole workgroup)
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
+    const uint32_t wave = tid >> 6, wk = wave % WK, wp = wave / WK;
+    const uint32_t n0 = tn * TN;
+    const bool pre = a.c.pre.gamma != nullptr, post = a.c.post.gamma != nullptr;
+
+    // The wave's pixels: one per lane and fragment, the same for the four quads.
+    int h[FP], w[FP];
+    uint32_t base[FP];   // byte offset of channel 0 of the pixel under tap (0, 0)
+    bool rowOk[FP];
+#pragma unroll
+    for (int f = 0; f < FP; ++f) {
+        const uint32_t row = tp * TP + (wp * FP + f) * 16 + l16;
+        rowOk[f] = row < rows;
+        const uint32_t ib = fdiv(rowOk[f] ? row : 0u, a.dP), p = (rowOk[f] ? row : 0u) - ib * a.P;
+        const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
+        int n = (int)ib;
+        h[f] = (int)r;
+        w[f] = (int)s;
+        if (a.c.idx) {
+            const int16_t* t = a.c.idx + (size_t)ib * 3;
+            n = t[0];
+            h[f] += a.c.oh + t[1] * a.c.U;
+            w[f] += a.c.ow + t[2] * a.c.V;
+            rowOk[f] = rowOk[f] && (unsigned)n < (unsigned)a.c.N;
+        }
+        base[f] = (((uint32_t)n * (uint32_t)a.c.H + (uint32_t)h[f]) * (uint32_t)a.c.W + (uint32_t)w[f]) * (uint32_t)a.c.C * 4u;
+    }
+
+    const rsrc_t ra = make_rsrc(a.c.a, a.aBytes), rw = make_rsrc(a.c.w, a.wBytes);
+    const uint32_t per = (a.kSteps + WK - 1) / WK;
+    const uint32_t sBeg = wk * per, sEnd = min(sBeg + per, a.kSteps);
+    const uint32_t kEnd = min(sEnd * 16u, a.kTot);
+    const uint32_t K = (uint32_t)a.c.K;
+
+    struct Operands {
+        acc_t px[FP];
+        float wv[FN][4];
+        uint32_t c[VEC == 4 ? 1 : 4];   // input channel of the lane's k (its first, where four share a tap)
+    };
+
+    // Loads of a step: out-of-range k, channels, rows and pixels get an offset outside the descriptor and read as 0.
+    auto load = [&](uint32_t step, Operands& o) {
+        const uint32_t k = step * 16u + quad * 4u;
+#pragma unroll
+        for (int j = 0; j < (VEC == 4 ? 1 : 4); ++j) {
+            const uint32_t kj = k + j;
+            const bool live = kj < kEnd;
+            const uint32_t tap = fdiv(kj, a.dC), c = kj - tap * (uint32_t)a.c.C;
+            const int dr = (int)fdiv(tap, a.dKw), ds = (int)tap - dr * a.c.kw;
+            o.c[j] = c;
+            const uint32_t toff = (((uint32_t)dr * (uint32_t)a.c.W + (uint32_t)ds) * (uint32_t)a.c.C + c) * 4u;
+#pragma unroll
+            for (int f = 0; f < FP; ++f) {
+                const bool ok = live && rowOk[f] && (unsigned)(h[f] + dr) < (unsigned)a.c.H &&
+                                (unsigned)(w[f] + ds) < (unsigned)a.c.W;
+                const uint32_t off = ok ? base[f] + toff : BUF_OOB;
+                if constexpr (VEC == 4) o.px[f] = buf_load<4>(ra, off);
+                else o.px[f][j] = buf_load<1>(ra, off);
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < FN; ++f) {
+            const uint32_t n = n0 + f * 16 + l16;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o.wv[f][j] = buf_load<1>(rw, k + j < kEnd && n < K ? ((k + j) * K + n) * 4u : BUF_OOB);
+        }
+    };
+
+    acc_t acc[FN][FP];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int f = 0; f < FP; ++f) acc[i][f] = (acc_t)(0.f);
+
+    Operands ops[CONV_DEPTH];
+#pragma unroll
+    for (int d = 0; d < CONV_DEPTH; ++d) load(sBeg + d, ops[d]);
+
+    if (pre)
+        for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_fold(a.c.pre, c, preScale[c], preShift[c]);
+    if (post)
+        for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES)
+            if (n0 + i < K) bn_fold(a.c.post, n0 + i, postScale[i], postShift[i]);
+    if (pre || post) lds_barrier();
+
+    for (uint32_t step = sBeg; step < sEnd; step += CONV_DEPTH) {
+#pragma unroll
+        for (int d = 0; d < CONV_DEPTH; ++d) {
+            Operands& o = ops[d];
+            if (pre) {
+                acc_t sc, sh;
+                if constexpr (VEC == 4) {
+                    sc = lds_read4(preScale + o.c[0]);
+                    sh = lds_read4(preShift + o.c[0]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        sc[j] = preScale[o.c[j]];
+                        sh[j] = preShift[o.c[j]];
+                    }
+                }
+#pragma unroll
+                for (int f = 0; f < FP; ++f)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o.px[f][j] = relu_keep_nan(o.px[f][j] * sc[j] + sh[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < FN; ++i)
+#pragma unroll
+                    for (int f = 0; f < FP; ++f)
+                        acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.wv[i][j], o.px[f][j], acc[i][f], 0, 0, 0);
+            load(step + d + CONV_DEPTH, o);   // past the wave's last step: all out of range, no traffic
+        }
+    }
+
+    const rsrc_t ry = make_rsrc(a.c.y, a.yBytes);
+    auto finish = [&](int i, int f, acc_t v) {
+        const uint32_t nl = i * 16 + quad * 4, n = n0 + nl;
+        if (post) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan(v[j] * postScale[nl + j] + postShift[nl + j]);
+        }
+        const uint32_t row = tp * TP + (wp * FP + f) * 16 + l16;
+        bool ok = row < rows;
+        uint32_t pix = row;
+        if (a.c.oidx) {
+            const uint32_t ib = fdiv(ok ? row : 0u, a.dP), p = (ok ? row : 0u) - ib * a.P;
+            const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
+            const int16_t* t = a.c.oidx + (size_t)ib * 3;
+            const int on = t[0], oh = t[1] * a.c.oU + (int)r, ow = t[2] * a.c.oV + (int)s;
+            ok = ok && (unsigned)on < (unsigned)a.c.oN && (unsigned)oh < (unsigned)a.c.oH && (unsigned)ow < (unsigned)a.c.oW;
+            pix = ((uint32_t)on * (uint32_t)a.c.oH + (uint32_t)oh) * (uint32_t)a.c.oW + (uint32_t)ow;
+        }
+        const uint32_t off = (pix * K + n) * 4u;
+        if constexpr (VEC == 4) {
+            const uint32_t o = ok && n < K ? off : BUF_OOB;   // K is a multiple of 4 here
+            if (a.c.add) v += buf_load<4>(ry, o);
+            buf_store<0>(ry, o, (f4)v);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t o = ok && n + j < K ? off + 4u * j : BUF_OOB;
+                float t = v[j];
+                if (a.c.add) t += buf_load<1>(ry, o);
+                buf_store<0>(ry, o, t);
+            }
+        }
+    };
+
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int f = 0; f < FP; ++f) finish(i, f, acc[i][f]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+            for (int f = 0; f < FP; ++f)
+                *reinterpret_cast<acc_t*>(red + (((wp * WK + wk) * (FP * FN) + i * FP + f) * 64 + lane) * 4) = acc[i][f];
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < FP * FN; ++q) {
+            if (q % WK != (int)wk) continue;   // (wave-uniform)
+            acc_t v = (acc_t)(0.f);
+#pragma unroll
+            for (int k = 0; k < WK; ++k)
+                v += (acc_t)lds_read4(red + (((wp * WK + k) * (FP * FN) + q) * 64 + lane) * 4);
+            finish(q / FP, q % FP, v);
+        }
+    }
+}
+
+template <int FP, int FN, int WK, int VEC>
+static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
+{
+    constexpr int WAVES = WK > 4 ? WK : 4, TP = 16 * FP * (WAVES / WK), TN = 16 * FN;
+    a.tilesP = (a.rows + TP - 1) / TP;
+    a.tilesN = ((uint32_t)a.c.K + TN - 1) / TN;
+    const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
+    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + 2 * TN + (WK > 1 ? (size_t)WAVES * FP * FN * 256 : 0));
+    if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
+    return hipGetLastError();
+}
+
+bool conv_fits(const ConvArgs& c)
+{
+    // 32-bit byte offsets in the input, the weights and the output; scale and shift of the input's channels in LDS
+    const uint64_t most = 1ull << 30;
+    const uint64_t a = (uint64_t)c.N * c.H * c.W * c.C, w = (uint64_t)c.kh * c.kw * c.C * c.K;
+    const uint64_t rows = (uint64_t)c.M * c.Ro * c.So;
+    const uint64_t y = (c.oidx ? (uint64_t)c.oN * c.oH * c.oW : rows) * c.K;
+    return a < most && w < most && y < most && rows < (1ull << 28) && c.C <= 4096 && c.Ro > 0 && c.So > 0;
+}
+
+hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
+{
+    if (c.M <= 0) return hipSuccess;
+    if (!conv_fits(c)) return hipErrorInvalidValue;
+    ConvKernelArgs a;
+    a.c = c;
+    a.dC = make_fastdiv((uint32_t)c.C);
+    a.dKw = make_fastdiv((uint32_t)c.kw);
+    a.P = (uint32_t)(c.Ro * c.So);
+    a.dP = make_fastdiv(a.P);
+    a.dSo = make_fastdiv((uint32_t)c.So);
+    a.kTot = (uint32_t)(c.kh * c.kw * c.C);
+    a.kSteps = (a.kTot + 15) / 16;
+    a.rows = (uint32_t)c.M * a.P;
+    a.aBytes = (uint32_t)((uint64_t)c.N * c.H * c.W * c.C * 4);
+    a.wBytes = a.kTot * (uint32_t)c.K * 4u;
+    a.yBytes = (uint32_t)((c.oidx ? (uint64_t)c.oN * c.oH * c.oW : (uint64_t)a.rows) * c.K * 4);
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(c.a) | reinterpret_cast<uintptr_t>(c.y);
+    const bool vec = c.C % 4 == 0 && c.K % 4 == 0 && (bits & 15) == 0;
+#ifdef SBNET_CONV_SWEEP
+    SBNET_CONV_SWEEP
+#endif
+    const uint32_t nFrag = ((uint32_t)c.K + 15) / 16;
+    const uint64_t fragments = (uint64_t)((a.rows + 31) / 32) * nFrag;
+    if (!vec) return fragments < 2048 && a.kSteps >= 8 ? launch_conv_one<2, 1, 4, 1>(a, stream) : launch_conv_one<2, 1, 1, 1>(a, stream);
+    if (nFrag == 1) return fragments < 2048 && a.kSteps >= 8 ? launch_conv_one<2, 1, 4, 4>(a, stream) : launch_conv_one<2, 1, 1, 4>(a, stream);
+    return fragments < 4096 && a.kSteps >= 8 ? launch_conv_one<2, 2, 4, 4>(a, stream) : launch_conv_one<2, 2, 1, 4>(a, stream);
+}
+
+}  // namespace sbnet

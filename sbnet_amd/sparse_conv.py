@@ -15,8 +15,14 @@ Conventions follow the reference: activations are NHWC tensors, kernels are [kh,
 transposed ([M, C, bh, bw]) so that the convolutions run on planar data without a separate
 transpose.  Everything is differentiable through torch.autograd (the block ops through
 sbnet_amd.autograd).
+
+Where no gradient is asked for, `sparse_conv2d_custom` and `sparse_res_block_bottleneck` (in inference) run this
+package's own convolution kernels instead (sbnet_amd/csrc/sbnet_conv.hip), which read the active blocks straight from x
+and keep what lies between two convolutions of a residual block in NHWC stacks; the stack's layout is then nobody's to
+see, and `transpose` / `data_format` select nothing.
 """
 import collections
+import ctypes
 
 import torch
 import torch.nn.functional as F
@@ -46,6 +52,61 @@ def _conv_blocks(p, w, stride, transpose):
     return q.permute(0, 2, 3, 1).contiguous()
 
 
+def _plain(*tensors):
+    """Contiguous float32 tensors on one GPU of which none asks for a gradient: what the block convolutions take."""
+    grad = torch.is_grad_enabled()
+    return all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and
+               t.device == tensors[0].device and not (grad and t.requires_grad) for t in tensors)
+
+
+def _fits(*sizes):
+    """Element counts whose byte offsets the block convolutions hold in 32 bits."""
+    return all(0 < n < 1 << 30 for n in sizes)
+
+
+def _numel(*dims):
+    n = 1
+    for d in dims:
+        n *= int(d)
+    return n
+
+
+class _Blocks(object):
+    """The block list and geometry of a layer call as the C ABI takes them; `fits` is False for what it would refuse."""
+
+    def __init__(self, x, indices, block_params):
+        self.idx = ops._idx_i16(indices.active_block_indices)
+        self.count = ops._device_count(indices.bin_counts)
+        self.M = int(self.idx.shape[0]) if self.count is not None else ops._count(indices.bin_counts)
+        ops._check_count(self.M, self.idx)
+        self.pairs = [ops._pair(v) for v in (block_params.bsize, block_params.bstrides, block_params.boffset)]
+        self.bsize = self.pairs[0][0]
+        self.fits = x.dim() == 4 and all(p[2] == 2 for p in self.pairs) and bool((self.pairs[1][0] > 0).all())
+
+    def args(self, x):
+        self.dims = ops._dims(x)[0]
+        return (x.data_ptr(), self.dims, self.M, self.count.data_ptr() if self.count is not None else None,
+                self.idx.data_ptr(), *(p[1] for p in self.pairs))
+
+
+def _block_conv(x, w, indices, block_params):
+    """VALID convolution (stride 1) of the active blocks as an NHWC stack, or None where only the composed path applies."""
+    if not _plain(x, w) or w.dim() != 4:
+        return None
+    b = _Blocks(x, indices, block_params)
+    kh, kw, cin, cout = (int(d) for d in w.shape)
+    if not b.fits or x.shape[3] != cin or cin > 4096 or b.bsize[0] < kh or b.bsize[1] < kw:
+        return None
+    shape = (b.M, int(b.bsize[0]) - kh + 1, int(b.bsize[1]) - kw + 1, cout)
+    if not _fits(x.numel(), w.numel(), _numel(*shape)) or _numel(*shape[:3]) >= 1 << 28:
+        return None
+    with torch.cuda.device(x.device):
+        q = torch.empty(shape, dtype=torch.float32, device=x.device)
+        ops._check(_lib.load().sbnet_block_conv(*b.args(x), w.data_ptr(), (ctypes.c_int32 * 4)(kh, kw, cin, cout),
+                                                q.data_ptr(), ops._stream()))
+    return q
+
+
 def sparse_conv2d_custom(x, w, indices, block_params, strides, use_var=False, transpose=False, atomic=False):
     """sparse_conv_lib.py:536-587: gather blocks, VALID-convolve them, write the results over x.
 
@@ -53,9 +114,13 @@ def sparse_conv2d_custom(x, w, indices, block_params, strides, use_var=False, tr
     active block's output region replaced by the convolution result.  With use_var the paste happens in
     place on x (which must not require grad), otherwise on a copy."""
     assert strides[1] == strides[2] == 1, "Only accept strides=1"
-    p = ops.sparse_gather(x, indices.bin_counts, indices.active_block_indices, block_params.bsize,
-                          block_params.bstrides, block_params.boffset, transpose=transpose)
-    q = _conv_blocks(p, w, 1, transpose)
+    q = _block_conv(x, w, indices, block_params)
+    if q is not None:
+        transpose = False
+    else:
+        p = ops.sparse_gather(x, indices.bin_counts, indices.active_block_indices, block_params.bsize,
+                              block_params.bstrides, block_params.boffset, transpose=transpose)
+        q = _conv_blocks(p, w, 1, transpose)
     # The reference passes bstrides as the scatter stride in the in-place flavour and bsize_out in the copying
     # one (sparse_conv_lib.py:569-571, 581-583); with the stride-1 convolutions accepted here the two are equal.
     if use_var:
@@ -311,6 +376,41 @@ def res_block_bottleneck(x, params, strides, is_training, data_format="NHWC", w_
     return x_ + _bottleneck_residual(x, params, strides, "SAME", is_training, data_format, no_activation)
 
 
+def _block_bottleneck(x, params, indices, block_params, no_activation, in_place):
+    """The residual function of the active blocks in inference: added to x (returns x) or as an NHWC stack; None where
+    only the composed path applies."""
+    bn = [t for b in params.bn for t in b]
+    if len(params.w) != 3 or len(bn) != 12 or not _plain(x, *params.w, *bn) or any(w.dim() != 4 for w in params.w):
+        return None
+    b = _Blocks(x, indices, block_params)
+    if not b.fits:
+        return None
+    R, S, C = int(b.bsize[0]), int(b.bsize[1]), int(x.shape[3])
+    sizes = [x.numel()]
+    for w, norm in zip(params.w, params.bn):
+        kh, kw, cin, cout = (int(d) for d in w.shape)
+        R, S = R - kh + 1, S - kw + 1
+        if cin != C or cin > 4096 or R <= 0 or S <= 0 or any(t.numel() != cin for t in norm) or _numel(b.M, R, S) >= 1 << 28:
+            return None
+        C = cout
+        sizes += [w.numel(), _numel(b.M, R, S, C)]
+    out_stride = ops._pair(block_params.bsize_out)
+    if not _fits(*sizes) or (in_place and (C != x.shape[3] or out_stride[2] != 2 or out_stride[0][0] != R or out_stride[0][1] != S)):
+        return None
+    lib = _lib.load()
+    pointer = ctypes.c_void_p
+    weights = (pointer * 3)(*(w.data_ptr() for w in params.w))
+    w_dims = (ctypes.c_int32 * 12)(*(int(d) for w in params.w for d in w.shape))
+    norms = (pointer * 12)(*(None if no_activation and i < 4 else t.data_ptr() for i, t in enumerate(bn)))
+    with torch.cuda.device(x.device):
+        ws = ops._workspace(x.device, lib.sbnet_block_bottleneck_workspace_bytes(b.M, b.pairs[0][1], w_dims))
+        q = None if in_place else torch.empty((b.M, R, S, C), dtype=torch.float32, device=x.device)
+        ops._check(lib.sbnet_block_bottleneck(*b.args(x), weights, w_dims, norms, BN_EPS, None if in_place else q.data_ptr(),
+                                              x.data_ptr() if in_place else None, out_stride[1], ws.data_ptr(), ws.numel(),
+                                              ops._stream()))
+    return x if in_place else q
+
+
 def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_training, data_format="NHWC",
                                 w_project=None, no_activation=False, use_var=False):
     """sparse_conv_lib.py:751-824: y = x + F(x) evaluated on the active blocks only.
@@ -318,6 +418,11 @@ def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_tr
     x is NHWC in either data format (as in the reference, `data_format` only selects the layout of the block
     stack: 'NCHW' gathers with transpose=True).  The residual function runs with VALID convolutions on the
     gathered blocks and its output is scatter-added onto x (in place with use_var)."""
+    if not is_training and w_project is None and strides[1] == strides[2] == 1:
+        q = _block_bottleneck(x, params, indices, block_params, no_activation, use_var)
+        if q is not None:
+            return q if use_var else ops.sparse_scatter(q, indices.bin_counts, indices.active_block_indices, x,
+                                                        block_params.bsize_out, block_params.bsize_out, [0, 0], add=True)
     transpose = data_format == "NCHW"
     p = ops.sparse_gather(x, indices.bin_counts, indices.active_block_indices, block_params.bsize,
                           block_params.bstrides, block_params.boffset, transpose=transpose)
@@ -337,7 +442,6 @@ def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_tr
 def hip_timer_start_op():
     """sparse_conv_lib.py:527-529 (CudaTimerStart, sparse_gather.cc:390-428): records an event on the current
     stream and returns the handle to pass to hip_timer_end_op."""
-    import ctypes
     lib = _lib.load()
     handle = ctypes.c_int64(0)
     ops._check(lib.sbnet_timer_start(ops._stream(), ctypes.byref(handle)))
@@ -347,7 +451,6 @@ def hip_timer_start_op():
 def hip_timer_end_op(start_timer):
     """sparse_conv_lib.py:532-533 (CudaTimerEnd, sparse_gather.cc:430-469): records a second event, waits for
     it and returns the elapsed device time in milliseconds.  The handle is consumed."""
-    import ctypes
     lib = _lib.load()
     dt = ctypes.c_float(0.0)
     ops._check(lib.sbnet_timer_end(ctypes.c_int64(start_timer), ops._stream(), ctypes.byref(dt)))

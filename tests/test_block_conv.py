@@ -1,0 +1,126 @@
+"""The block convolutions (sbnet_amd/csrc/sbnet_conv.hip) against float64 convolutions of the gathered blocks.
+
+The bound on a float32 sum of n products in any order is n * 2^-24 * sum |a| * |w| (plus rounding of the operands,
+none here); through batch norm and ReLU the same argument runs with the folded scale, so the tests compare with that
+bound evaluated per element on the absolute values, in float64.
+"""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import sbnet_amd
+from sbnet_amd import sparse_conv as sc
+from sbnet_amd.block_params import BlockParams
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+U = 2.0 ** -24
+
+
+def blocks64(x, idx, bsize, bstride, boffset):
+    """Gathered blocks [M,C,R,S] in float64 on the CPU, zeros outside the image."""
+    R, S = bsize
+    xp = F.pad(x.double().permute(0, 3, 1, 2), (64, 64, 64, 64))
+    out = [xp[n, :, 64 + boffset[0] + bh * bstride[0]:, 64 + boffset[1] + bw * bstride[1]:][:, :R, :S] for n, bh, bw in idx.tolist()]
+    return torch.stack(out)
+
+
+def make_blocks(rng, N, H, W, bsize, bstride, boffset, M):
+    """M distinct blocks, borders included, in random order."""
+    bc = [1 + (H - boffset[0] - 1) // bstride[0], 1 + (W - boffset[1] - 1) // bstride[1]]
+    T = N * bc[0] * bc[1]
+    pick = rng.permutation(T)[:M]
+    idx = np.stack([pick // (bc[0] * bc[1]), pick // bc[1] % bc[0], pick % bc[1]], 1).astype(np.int16)
+    return torch.from_numpy(idx)
+
+
+CONVS = [
+    # N, H, W, C, K, kh, kw, bsize, M      what the size is for
+    (1, 20, 24, 1, 1, 1, 1, (5, 5), 6),     # one channel, one k
+    (2, 31, 29, 3, 5, 3, 3, (6, 9), 9),     # no vector width
+    (1, 40, 40, 8, 2, 3, 3, (7, 7), 11),    # four-wide input, narrow output
+    (1, 33, 50, 10, 10, 5, 3, (9, 11), 7),  # k not a multiple of 16, unequal kernel sides
+    (1, 40, 60, 4, 4, 3, 3, (10, 10), 8),   # four taps share a step
+    (1, 64, 64, 12, 20, 1, 1, (8, 8), 20),  # last step three quarters full, second channel fragment a quarter full
+    (1, 64, 48, 24, 24, 3, 3, (17, 17), 5),
+    (3, 40, 40, 48, 48, 3, 3, (8, 8), 30),
+    (1, 50, 50, 130, 36, 3, 3, (9, 9), 6),  # channels no multiple of four
+    (1, 60, 60, 132, 68, 1, 1, (6, 6), 40),
+    (1, 300, 300, 16, 64, 3, 3, (12, 12), 700),   # enough tiles that k is not split
+    (1, 300, 300, 7, 33, 3, 3, (12, 12), 700),
+]
+
+
+@pytest.mark.parametrize("device_count", [False, True])
+@pytest.mark.parametrize("case", CONVS, ids=lambda c: "x".join(str(v) for v in c[:7]))
+def test_block_conv(case, device_count):
+    N, H, W, C, K, kh, kw, bsize, M = case
+    rng = np.random.default_rng(C * 100 + K)
+    bstride, boffset = (bsize[0] - kh + 1, bsize[1] - kw + 1), (-(kh // 2), -(kw // 2))
+    idx = make_blocks(rng, N, H, W, bsize, bstride, boffset, M)
+    M = idx.shape[0]
+    x = torch.from_numpy(rng.standard_normal((N, H, W, C)).astype(np.float32))
+    w = torch.from_numpy(rng.standard_normal((kh, kw, C, K)).astype(np.float32))
+    listed = torch.cat([idx, torch.full((3, 3), 77, dtype=torch.int16)]) if device_count else idx
+    count = torch.tensor([M], dtype=torch.int32)
+    bp = BlockParams(bsize=list(bsize), bsize_out=list(bstride), boffset=list(boffset), bcount=None, bstrides=list(bstride))
+    q = sc._block_conv(x.to(DEV), w.to(DEV), sbnet_amd.ReduceMaskResult(listed.to(DEV), count.to(DEV) if device_count else count), bp)
+    assert q is not None and q.shape[1:] == (bstride[0], bstride[1], K)
+    p = blocks64(x, idx, bsize, bstride, boffset)
+    w64 = w.double().permute(3, 2, 0, 1)
+    want = F.conv2d(p, w64).permute(0, 2, 3, 1)
+    bound = kh * kw * C * U * F.conv2d(p.abs(), w64.abs()).permute(0, 2, 3, 1)
+    err = (q[:M].cpu().double() - want).abs()
+    assert bool((err <= bound + 1e-30).all()), float((err / (bound + 1e-30)).max())
+
+
+def bottleneck64(p, params, no_activation):
+    """Residual function in float64 and, beside it, the accumulated rounding bound: each stage adds its own sum's bound and
+    passes on the one it received through the absolute values of its scales and weights."""
+    err = torch.zeros_like(p)
+    for i, (w, bn) in enumerate(zip(params.w, params.bn)):
+        if i or not no_activation:
+            g, b, m, v = (t.detach().cpu().double().view(1, -1, 1, 1) for t in bn)
+            scale = g / (v + sc.BN_EPS).sqrt()
+            err = scale.abs() * err + 8 * U * ((p * scale).abs() + (m * scale).abs() + b.abs())
+            p = torch.relu(p * scale + b - m * scale)
+        w64 = w.detach().cpu().double().permute(3, 2, 0, 1)
+        n = w64[0].numel()
+        err = F.conv2d(err + n * U * p.abs(), w64.abs())
+        p = F.conv2d(p, w64)
+    return p.permute(0, 2, 3, 1), err.permute(0, 2, 3, 1)
+
+
+@pytest.mark.parametrize("use_var", [False, True])
+@pytest.mark.parametrize("no_activation", [False, True])
+@pytest.mark.parametrize("C,mid,bsize,shape", [(6, 3, 5, (2, 23, 31)), (24, 8, 9, (1, 40, 52)), (96, 24, 17, (1, 70, 64)),
+                                               (260, 64, 7, (1, 30, 30)), (16, 16, 24, (1, 220, 220))])
+def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
+    rng = np.random.default_rng(C)
+    ksizes = [[1, 1, C, mid], [3, 3, mid, mid], [1, 1, mid, C]]
+    bp = sbnet_amd.calc_block_params_res_block([shape[0], shape[1], shape[2], C], [1, bsize, bsize, 1], ksizes, [1, 1, 1, 1], "SAME")
+    mask = torch.from_numpy((rng.random((*shape, 1)) < 0.02).astype(np.float32)).to(DEV)
+    ind = sc.convert_mask_to_indices_custom(mask, bp, 0.0)
+    M = int(ind.bin_counts[0])
+    params = sc.BottleneckParams(ksizes, DEV, seed=C)
+    with torch.no_grad():
+        for bn in params.bn:
+            for t, (lo, hi) in zip(bn, ((0.5, 1.5), (-0.3, 0.3), (-0.3, 0.3), (0.5, 1.5))):
+                t.copy_(torch.from_numpy(rng.uniform(lo, hi, t.shape).astype(np.float32)))
+    x = torch.from_numpy(rng.standard_normal((*shape, C)).astype(np.float32))
+    xd = x.to(DEV)
+    with torch.no_grad():
+        assert sc._block_bottleneck(xd, params, ind, bp, no_activation, False) is not None
+        y = sc.sparse_res_block_bottleneck(xd, params, ind, bp, [1, 1, 1, 1], False, no_activation=no_activation, use_var=use_var)
+    assert (y.data_ptr() == xd.data_ptr()) == use_var
+    idx = ind.active_block_indices[:M].cpu()
+    q, bound = bottleneck64(blocks64(x, idx, bp.bsize, bp.bstrides, bp.boffset), params, no_activation)
+    want, most = x.double().clone(), torch.zeros(x.shape, dtype=torch.float64)
+    Ro, So = bp.bsize_out
+    for i, (n, bh, bw) in enumerate(idx.tolist()):
+        part = want[n, bh * Ro:(bh + 1) * Ro, bw * So:(bw + 1) * So]
+        part += q[i, :part.shape[0], :part.shape[1]]
+        most[n, bh * Ro:(bh + 1) * Ro, bw * So:(bw + 1) * So] = bound[i, :part.shape[0], :part.shape[1]] + U * part.abs()
+    err = (y.cpu().double() - want).abs()
+    assert bool((err <= most + 1e-30).all()), float((err / (most + 1e-30)).max())
