@@ -27,9 +27,10 @@ namespace sbnet {
 // tiles there are no barriers: the problems are small (a few thousand pixels) and their time is a chain of latencies.
 // CONV_DEPTH sets of operands are in flight per wave.
 //
-// Measured (MI355X, kernel trace): 85 blocks of 17x17x48, 3x3 to 48 channels (19 000 pixels, 0.8 GFLOP): 27 us; the library
-// convolution took 21 us behind 5 us of layout copies, and up to 800 us the first time a block count occurred.  A whole
-// bottleneck block of 200 17x17x96 blocks: 50 us in three launches against about 300 us in 17.
+// Measured (MI355X, kernel trace): 85 blocks of 17x17x48, 3x3 to 48 channels (19 000 pixels, 0.8 GFLOP; 5.2 us at the
+// rate of a large fp32 product): 19 us, 27 us while the loads of a step sat behind branches; the library convolution
+// took 21 us behind 5 us of layout copies, and up to 800 us the first time a block count occurred.  A bottleneck block of
+// 200 17x17x96 blocks: 39 us in three launches against about 300 us in 17.
 //
 // WK > 1: the WK waves of a workgroup split k among them and add up through LDS.  For launches whose tiles alone would
 // leave most of the 1024 SIMDs idle.
@@ -40,6 +41,7 @@ namespace sbnet {
 typedef float acc_t __attribute__((ext_vector_type(4)));
 
 constexpr int CONV_DEPTH = 3;   // operand sets in flight per wave
+constexpr uint32_t W_OOB = 0x40000000u;   // beyond any kernel (conv_fits), alone and added to itself
 
 struct ConvKernelArgs {
     ConvArgs c;
@@ -59,13 +61,13 @@ __device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& sca
     shift = bn.beta[c] - bn.mean[c] * scale;
 }
 
-template <int FP, int FN, int WK, int VEC>
+template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS>
 __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKernelArgs a)
 {
     constexpr int WAVES = WK > 4 ? WK : 4, WP = WAVES / WK;
     constexpr int TP = 16 * FP * WP, TN = 16 * FN;
     extern __shared__ float lds[];
-    const uint32_t cPad = a.c.pre.gamma ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
+    const uint32_t cPad = PRE ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
     float* const preScale = lds;
     float* const preShift = lds + cPad;
     float* const postScale = lds + 2 * cPad;
@@ -83,17 +85,16 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
     const uint32_t wave = tid >> 6, wk = wave % WK, wp = wave / WK;
     const uint32_t n0 = tn * TN;
-    const bool pre = a.c.pre.gamma != nullptr, post = a.c.post.gamma != nullptr;
+    const bool post = a.c.post.gamma != nullptr;
 
     // The wave's pixels: one per lane and fragment, the same for the four quads.
     int h[FP], w[FP];
     uint32_t base[FP];   // byte offset of channel 0 of the pixel under tap (0, 0)
-    bool rowOk[FP];
 #pragma unroll
     for (int f = 0; f < FP; ++f) {
         const uint32_t row = tp * TP + (wp * FP + f) * 16 + l16;
-        rowOk[f] = row < rows;
-        const uint32_t ib = fdiv(rowOk[f] ? row : 0u, a.dP), p = (rowOk[f] ? row : 0u) - ib * a.P;
+        bool ok = row < rows;
+        const uint32_t ib = fdiv(ok ? row : 0u, a.dP), p = (ok ? row : 0u) - ib * a.P;
         const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
         int n = (int)ib;
         h[f] = (int)r;
@@ -103,9 +104,10 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
             n = t[0];
             h[f] += a.c.oh + t[1] * a.c.U;
             w[f] += a.c.ow + t[2] * a.c.V;
-            rowOk[f] = rowOk[f] && (unsigned)n < (unsigned)a.c.N;
+            ok = ok && (unsigned)n < (unsigned)a.c.N;
         }
         base[f] = (((uint32_t)n * (uint32_t)a.c.H + (uint32_t)h[f]) * (uint32_t)a.c.W + (uint32_t)w[f]) * (uint32_t)a.c.C * 4u;
+        if (!ok) h[f] = -0x40000000;   // outside the image under every tap
     }
 
     const rsrc_t ra = make_rsrc(a.c.a, a.aBytes), rw = make_rsrc(a.c.w, a.wBytes);
@@ -113,6 +115,9 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     const uint32_t sBeg = wk * per, sEnd = min(sBeg + per, a.kSteps);
     const uint32_t kEnd = min(sEnd * 16u, a.kTot);
     const uint32_t K = (uint32_t)a.c.K;
+    uint32_t wCol[FN];
+#pragma unroll
+    for (int f = 0; f < FN; ++f) wCol[f] = n0 + f * 16 + l16 < K ? (n0 + f * 16 + l16) * 4u : W_OOB;
 
     struct Operands {
         acc_t px[FP];
@@ -121,31 +126,38 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     };
 
     // Loads of a step: out-of-range k, channels, rows and pixels get an offset outside the descriptor and read as 0.
+    // All by selects: written with && the compiler branches around each load and waits inside the branch.
     auto load = [&](uint32_t step, Operands& o) {
         const uint32_t k = step * 16u + quad * 4u;
 #pragma unroll
         for (int j = 0; j < (VEC == 4 ? 1 : 4); ++j) {
             const uint32_t kj = k + j;
-            const bool live = kj < kEnd;
-            const uint32_t tap = fdiv(kj, a.dC), c = kj - tap * (uint32_t)a.c.C;
-            const int dr = (int)fdiv(tap, a.dKw), ds = (int)tap - dr * a.c.kw;
+            uint32_t c = kj;
+            int dr = 0, ds = 0;
+            if constexpr (TAPS) {
+                const uint32_t tap = fdiv(kj, a.dC);
+                c = kj - tap * (uint32_t)a.c.C;
+                dr = (int)fdiv(tap, a.dKw);
+                ds = (int)tap - dr * a.c.kw;
+            } else {
+                c = min(c, (uint32_t)a.c.C - (VEC == 4 ? 4u : 1u));   // (a channel to look scale and shift up for, past the end)
+            }
             o.c[j] = c;
             const uint32_t toff = (((uint32_t)dr * (uint32_t)a.c.W + (uint32_t)ds) * (uint32_t)a.c.C + c) * 4u;
 #pragma unroll
             for (int f = 0; f < FP; ++f) {
-                const bool ok = live && rowOk[f] && (unsigned)(h[f] + dr) < (unsigned)a.c.H &&
-                                (unsigned)(w[f] + ds) < (unsigned)a.c.W;
-                const uint32_t off = ok ? base[f] + toff : BUF_OOB;
+                const uint32_t bad = (uint32_t)((unsigned)(h[f] + dr) >= (unsigned)a.c.H) |
+                                     (uint32_t)((unsigned)(w[f] + ds) >= (unsigned)a.c.W) | (uint32_t)(kj >= kEnd);
+                const uint32_t off = (base[f] + toff) | (0u - bad);
                 if constexpr (VEC == 4) o.px[f] = buf_load<4>(ra, off);
                 else o.px[f][j] = buf_load<1>(ra, off);
             }
         }
 #pragma unroll
-        for (int f = 0; f < FN; ++f) {
-            const uint32_t n = n0 + f * 16 + l16;
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t row = (k + j < kEnd) ? (k + j) * K * 4u : W_OOB;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o.wv[f][j] = buf_load<1>(rw, k + j < kEnd && n < K ? ((k + j) * K + n) * 4u : BUF_OOB);
+            for (int f = 0; f < FN; ++f) o.wv[f][j] = buf_load<1>(rw, row + wCol[f]);
         }
     };
 
@@ -159,18 +171,19 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
 #pragma unroll
     for (int d = 0; d < CONV_DEPTH; ++d) load(sBeg + d, ops[d]);
 
-    if (pre)
+    if (PRE)
         for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_fold(a.c.pre, c, preScale[c], preShift[c]);
     if (post)
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES)
             if (n0 + i < K) bn_fold(a.c.post, n0 + i, postScale[i], postShift[i]);
-    if (pre || post) lds_barrier();
+    if (PRE || post) lds_barrier();
 
     for (uint32_t step = sBeg; step < sEnd; step += CONV_DEPTH) {
 #pragma unroll
         for (int d = 0; d < CONV_DEPTH; ++d) {
+            if (d && step + d >= sEnd) break;   // (wave-uniform; a round of multiplying zeros would cost as much as a full one)
             Operands& o = ops[d];
-            if (pre) {
+            if constexpr (PRE) {
                 acc_t sc, sh;
                 if constexpr (VEC == 4) {
                     sc = lds_read4(preScale + o.c[0]);
@@ -256,8 +269,8 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     }
 }
 
-template <int FP, int FN, int WK, int VEC>
-static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
+template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS>
+static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
 {
     constexpr int WAVES = WK > 4 ? WK : 4, TP = 16 * FP * (WAVES / WK), TN = 16 * FN;
     a.tilesP = (a.rows + TP - 1) / TP;
@@ -265,8 +278,16 @@ static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
     const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + 2 * TN + (WK > 1 ? (size_t)WAVES * FP * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
+    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC, PRE, TAPS>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();
+}
+
+template <int FP, int FN, int WK, int VEC>
+static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
+{
+    const bool taps = a.c.kh * a.c.kw > 1;
+    if (a.c.pre.gamma) return taps ? launch_conv_as<FP, FN, WK, VEC, true, true>(a, stream) : launch_conv_as<FP, FN, WK, VEC, true, false>(a, stream);
+    return taps ? launch_conv_as<FP, FN, WK, VEC, false, true>(a, stream) : launch_conv_as<FP, FN, WK, VEC, false, false>(a, stream);
 }
 
 bool conv_fits(const ConvArgs& c)
@@ -276,14 +297,11 @@ bool conv_fits(const ConvArgs& c)
     const uint64_t a = (uint64_t)c.N * c.H * c.W * c.C, w = (uint64_t)c.kh * c.kw * c.C * c.K;
     const uint64_t rows = (uint64_t)c.M * c.Ro * c.So;
     const uint64_t y = (c.oidx ? (uint64_t)c.oN * c.oH * c.oW : rows) * c.K;
-    return a < most && w < most && y < most && rows < (1ull << 28) && c.C <= 4096 && c.Ro > 0 && c.So > 0;
+    return a < most && w < (1ull << 28) && y < most && rows < (1ull << 28) && c.C <= 4096 && c.Ro > 0 && c.So > 0;
 }
 
-hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
+static bool make_conv_args(const ConvArgs& c, ConvKernelArgs& a)
 {
-    if (c.M <= 0) return hipSuccess;
-    if (!conv_fits(c)) return hipErrorInvalidValue;
-    ConvKernelArgs a;
     a.c = c;
     a.dC = make_fastdiv((uint32_t)c.C);
     a.dKw = make_fastdiv((uint32_t)c.kw);
@@ -297,15 +315,40 @@ hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
     a.wBytes = a.kTot * (uint32_t)c.K * 4u;
     a.yBytes = (uint32_t)((c.oidx ? (uint64_t)c.oN * c.oH * c.oW : (uint64_t)a.rows) * c.K * 4);
     const uintptr_t bits = reinterpret_cast<uintptr_t>(c.a) | reinterpret_cast<uintptr_t>(c.y);
-    const bool vec = c.C % 4 == 0 && c.K % 4 == 0 && (bits & 15) == 0;
-#ifdef SBNET_CONV_SWEEP
-    SBNET_CONV_SWEEP
-#endif
+    return c.C % 4 == 0 && c.K % 4 == 0 && (bits & 15) == 0;   // 16-byte accesses on both sides
+}
+
+hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
+{
+    if (c.M <= 0) return hipSuccess;
+    if (!conv_fits(c)) return hipErrorInvalidValue;
+    ConvKernelArgs a;
+    const bool vec = make_conv_args(c, a);
+    // Narrow wave tiles (16 pixels x 32 channels; 48 where that leaves no channel over, 16 where there are no more) and as
+    // many waves per tile as it takes to occupy the SIMDs: a launch of fewer than about 1500 waves is four times shorter
+    // with k split four ways than its occupancy would suggest, and one with few steps per wave has nothing to split.
+    // Wider tiles read less and wait more: 32x32 is 10-40 % slower on all but the narrowest and largest problems (us for
+    // 16x32 / 32x32, best split: 2450 pixels, k 1152, 128 channels 16.4 / 19.0; 4860, 576, 64: 10.3 / 12.0; 45 000, 216, 24:
+    // 13.2 / 12.6; 38 400, 600, 24: 24.7 / 22.7).
     const uint32_t nFrag = ((uint32_t)c.K + 15) / 16;
-    const uint64_t fragments = (uint64_t)((a.rows + 31) / 32) * nFrag;
-    if (!vec) return fragments < 2048 && a.kSteps >= 8 ? launch_conv_one<2, 1, 4, 1>(a, stream) : launch_conv_one<2, 1, 1, 1>(a, stream);
-    if (nFrag == 1) return fragments < 2048 && a.kSteps >= 8 ? launch_conv_one<2, 1, 4, 4>(a, stream) : launch_conv_one<2, 1, 1, 4>(a, stream);
-    return fragments < 4096 && a.kSteps >= 8 ? launch_conv_one<2, 2, 4, 4>(a, stream) : launch_conv_one<2, 2, 1, 4>(a, stream);
+    const int fn = nFrag == 1 ? 1 : (vec && nFrag % 3 == 0 && nFrag % 2 == 1 ? 3 : 2);
+    const uint64_t waves = (uint64_t)((a.rows + 15) / 16) * ((nFrag + fn - 1) / fn);
+    const int wk = a.kSteps < 8 ? 1 : (waves < 1536 ? 4 : (waves < 3072 && a.kSteps >= 16 ? 2 : 1));
+    if (!vec) {
+        if (fn == 1) return wk > 1 ? launch_conv_one<1, 1, 4, 1>(a, stream) : launch_conv_one<1, 1, 1, 1>(a, stream);
+        return wk > 1 ? launch_conv_one<1, 2, 4, 1>(a, stream) : launch_conv_one<1, 2, 1, 1>(a, stream);
+    }
+    switch (fn * 8 + wk) {
+    case 8 + 1: return launch_conv_one<1, 1, 1, 4>(a, stream);
+    case 8 + 2: return launch_conv_one<1, 1, 2, 4>(a, stream);
+    case 8 + 4: return launch_conv_one<1, 1, 4, 4>(a, stream);
+    case 16 + 1: return launch_conv_one<1, 2, 1, 4>(a, stream);
+    case 16 + 2: return launch_conv_one<1, 2, 2, 4>(a, stream);
+    case 16 + 4: return launch_conv_one<1, 2, 4, 4>(a, stream);
+    case 24 + 1: return launch_conv_one<1, 3, 1, 4>(a, stream);
+    case 24 + 2: return launch_conv_one<1, 3, 2, 4>(a, stream);
+    default: return launch_conv_one<1, 3, 4, 4>(a, stream);
+    }
 }
 
 }  // namespace sbnet
