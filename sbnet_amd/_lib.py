@@ -73,6 +73,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 def load():
@@ -90,3 +91,16 @@ def load():
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def native():
+    """The extension module with the op wrappers' common case (sbnet_torch.cpp); like the library, it has no fallback."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError("sbnet_amd._native is not built (%s); run `make -C sbnet_amd/csrc`." % e)
+        _native = module
+    return _native

@@ -1,0 +1,477 @@
+// The op wrappers' common case in native code (Python module sbnet_amd._native): plain arguments in, one C-ABI call, the
+// result out.  Everything else (parameters that are no pair of ints, tensors that need a copy or a cast, sizes and types
+// that are an error) is left to the Python wrappers of ops.py, which these functions tell by returning None before
+// anything has been allocated or enqueued.
+//
+// A call through ctypes costs 25-35 us of host time for argument conversion, two numpy round trips per parameter pair,
+// the device context manager and the call itself: the three ops of a step took 114 us from Python on a [1,64,64,16] map
+// whose kernels take 20.  Through this module the step takes 34 us, what the same calls take from a C++ loop.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <map>
+#include <utility>
+
+#include "../../include/sbnet_amd.h"
+
+namespace {
+
+PyObject* g_check = nullptr;   // ops._check: raises the exception of a status
+
+struct Pair {
+    int32_t v[2];
+};
+
+bool int_of(PyObject* o, int32_t* out)
+{
+    if (!PyLong_CheckExact(o)) return false;
+    int overflow = 0;
+    const long v = PyLong_AsLongAndOverflow(o, &overflow);
+    if (overflow || v < INT32_MIN || v > INT32_MAX) return false;
+    *out = (int32_t)v;
+    return true;
+}
+
+// A list or tuple of exactly two ints.
+bool pair_of(PyObject* o, Pair& p)
+{
+    if (PyList_CheckExact(o))
+        return PyList_GET_SIZE(o) == 2 && int_of(PyList_GET_ITEM(o, 0), &p.v[0]) && int_of(PyList_GET_ITEM(o, 1), &p.v[1]);
+    if (PyTuple_CheckExact(o))
+        return PyTuple_GET_SIZE(o) == 2 && int_of(PyTuple_GET_ITEM(o, 0), &p.v[0]) && int_of(PyTuple_GET_ITEM(o, 1), &p.v[1]);
+    return false;
+}
+
+// A contiguous tensor of the type on the GPU.
+const at::Tensor* dev_tensor(PyObject* o, at::ScalarType type)
+{
+    if (!THPVariable_Check(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.defined() || !t.is_cuda() || t.scalar_type() != type || t.layout() != at::kStrided || !t.is_contiguous()) return nullptr;
+    return &t;
+}
+
+const at::Tensor* dev_f32(PyObject* o) { return dev_tensor(o, at::kFloat); }
+
+// The block list with its count: on the host (M) or on the device (count, M then the list's capacity).
+struct Blocks {
+    const at::Tensor* idx;
+    int32_t M;
+    const int32_t* count;
+};
+
+bool blocks_of(PyObject* counts, PyObject* list, Blocks& b)
+{
+    b.idx = dev_tensor(list, at::kShort);
+    if (!b.idx || b.idx->dim() != 2 || b.idx->size(1) != 3 || b.idx->size(0) > INT32_MAX) return false;
+    b.count = nullptr;
+    if (THPVariable_Check(counts)) {
+        const at::Tensor& c = THPVariable_Unpack(counts);
+        if (!c.defined() || c.scalar_type() != at::kInt || c.layout() != at::kStrided || c.numel() < 1) return false;
+        if (c.is_cuda()) {
+            if (c.device() != b.idx->device()) return false;
+            b.count = static_cast<const int32_t*>(c.data_ptr());
+            b.M = (int32_t)b.idx->size(0);
+            return true;
+        }
+        if (!c.is_cpu()) return false;
+        b.M = *static_cast<const int32_t*>(c.data_ptr());
+    } else if (PyList_CheckExact(counts) && PyList_GET_SIZE(counts) >= 1) {
+        if (!int_of(PyList_GET_ITEM(counts, 0), &b.M)) return false;
+    } else {
+        return false;
+    }
+    return b.M >= 0 && b.M <= b.idx->size(0);
+}
+
+bool is_stack(const at::Tensor& t, int32_t M, int64_t C, const Pair& bsize, bool planar)
+{
+    return t.dim() == 4 && t.size(0) >= M && t.size(1) == (planar ? C : bsize.v[0]) &&
+           t.size(2) == (planar ? bsize.v[0] : bsize.v[1]) && t.size(3) == (planar ? bsize.v[1] : C);
+}
+
+at::Tensor empty_f32(at::IntArrayRef size, const at::Tensor& like)
+{
+    return at::detail::empty_cuda(size, at::kFloat, like.device(), c10::nullopt);
+}
+
+at::Tensor empty_stack(int32_t M, int64_t C, const Pair& bsize, bool planar, const at::Tensor& like)
+{
+    return planar ? empty_f32({M, C, bsize.v[0], bsize.v[1]}, like) : empty_f32({M, bsize.v[0], bsize.v[1], C}, like);
+}
+
+void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// Scratch of the calls of one stream, which run in order: one buffer per (device, stream) that only grows.  The GIL
+// guards the table.  A buffer that a call still holds when another thread grows it stays alive until that call's
+// work has been enqueued, and torch's allocator hands its memory on in the order of the stream.
+std::map<std::pair<int, void*>, at::Tensor>* g_workspaces = nullptr;
+
+at::Tensor workspace(const at::Device& device, int64_t bytes)
+{
+    void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+    if (!g_workspaces) g_workspaces = new std::map<std::pair<int, void*>, at::Tensor>();
+    at::Tensor& ws = (*g_workspaces)[std::make_pair((int)device.index(), stream)];
+    if (!ws.defined() || ws.numel() < bytes)
+        ws = at::detail::empty_cuda({bytes < (1 << 16) ? (1 << 16) : bytes}, at::kByte, device, c10::nullopt);
+    return ws;
+}
+
+// Runs a library call without the GIL, as ctypes does; raises on a status other than SBNET_OK.
+template <typename F>
+bool call(F f)
+{
+    int status;
+    Py_BEGIN_ALLOW_THREADS
+    status = f();
+    Py_END_ALLOW_THREADS
+    if (status == SBNET_OK) return true;
+    PyObject* r = PyObject_CallFunction(g_check, "i", status);
+    if (r) {
+        Py_DECREF(r);
+        PyErr_SetString(PyExc_RuntimeError, "sbnet status was not raised");
+    }
+    return false;
+}
+
+template <typename F>
+PyObject* guarded(F f)
+{
+    try {
+        return f();
+    } catch (...) {
+        torch::translate_exception_to_python(std::current_exception());
+    }
+    return nullptr;
+}
+
+bool expect(Py_ssize_t n, Py_ssize_t want)
+{
+    if (n == want) return true;
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
+    return false;
+}
+
+// reduce_mask(mask, bcount, bsize, bstride, boffset, tol, avgpool, sync) -> (active_block_indices, bin_counts)
+PyObject* reduce_mask(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 8)) return nullptr;
+    const at::Tensor* mask = dev_f32(a[0]);
+    Pair bc, bs, bt, bo;
+    if (!mask || !pair_of(a[1], bc) || !pair_of(a[2], bs) || !pair_of(a[3], bt) || !pair_of(a[4], bo)) Py_RETURN_NONE;
+    if (!(mask->dim() == 3 || (mask->dim() == 4 && mask->size(3) == 1)) || !PyFloat_CheckExact(a[5])) Py_RETURN_NONE;
+    for (int i = 0; i < 3; ++i)
+        if (mask->size(i) <= 0 || mask->size(i) > INT32_MAX) Py_RETURN_NONE;
+    const int N = (int)mask->size(0), H = (int)mask->size(1), W = (int)mask->size(2);
+    if (bc.v[0] <= 0 || bc.v[1] <= 0 || N > 32768 || bc.v[0] > 32768 || bc.v[1] > 32768) Py_RETURN_NONE;
+    const int64_t T = (int64_t)N * bc.v[0] * bc.v[1];
+    if (T > INT32_MAX) Py_RETURN_NONE;
+    const float tol = (float)PyFloat_AS_DOUBLE(a[5]);
+    const int avgpool = PyObject_IsTrue(a[6]), sync = PyObject_IsTrue(a[7]);
+    if (avgpool < 0 || sync < 0) return nullptr;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(mask->device());
+        at::Tensor idx = at::detail::empty_cuda({T, 3}, at::kShort, mask->device(), c10::nullopt);
+        at::Tensor count = sync ? at::empty({1}, at::kInt) : at::detail::empty_cuda({1}, at::kInt, mask->device(), c10::nullopt);
+        int32_t* const cp = static_cast<int32_t*>(count.data_ptr());
+        at::Tensor ws = workspace(mask->device(), (int64_t)sbnet_reduce_mask_workspace_bytes(N, bc.v, 2));
+        void* const stream = stream_of(*mask);
+        if (!call([&] {
+                return sbnet_reduce_mask(static_cast<const float*>(mask->data_ptr()), N, H, W, bc.v, 2, bs.v, 2, bt.v, 2, bo.v,
+                                         2, tol, avgpool, static_cast<int16_t*>(idx.data_ptr()), sync ? cp : nullptr,
+                                         sync ? nullptr : cp, ws.data_ptr(), (size_t)ws.numel(), stream);
+            }))
+            return nullptr;
+        PyObject* pi = THPVariable_Wrap(std::move(idx));
+        PyObject* pc = THPVariable_Wrap(std::move(count));
+        PyObject* t = pi && pc ? PyTuple_Pack(2, pi, pc) : nullptr;
+        Py_XDECREF(pi);
+        Py_XDECREF(pc);
+        return t;
+    });
+}
+
+// gather(x, bin_counts, active_block_indices, bsize, bstride, boffset, transpose, out) -> stack
+PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 8)) return nullptr;
+    const at::Tensor* x = dev_f32(a[0]);
+    Blocks b;
+    Pair bs, bt, bo;
+    if (!x || x->dim() != 4 || !blocks_of(a[1], a[2], b) || b.idx->device() != x->device() || !pair_of(a[3], bs) ||
+        !pair_of(a[4], bt) || !pair_of(a[5], bo) || bs.v[0] <= 0 || bs.v[1] <= 0)
+        Py_RETURN_NONE;
+    const int transpose = PyObject_IsTrue(a[6]);
+    if (transpose < 0) return nullptr;
+    const at::Tensor* out = nullptr;
+    if (a[7] != Py_None) {
+        out = dev_f32(a[7]);
+        if (!out || out->device() != x->device() || !is_stack(*out, b.M, x->size(3), bs, transpose)) Py_RETURN_NONE;
+    }
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(x->device());
+        at::Tensor y = out ? *out : empty_stack(b.M, x->size(3), bs, transpose, *x);
+        const float* const xp = static_cast<const float*>(x->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const yp = static_cast<float*>(y.data_ptr());
+        const int64_t* const dims = x->sizes().data();
+        void* const stream = stream_of(*x);
+        if (!call([&] {
+                return b.count ? sbnet_sparse_gather_device_count(xp, dims, 4, b.count, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2,
+                                                                  transpose, yp, stream)
+                               : sbnet_sparse_gather(xp, dims, 4, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2, transpose, yp, stream);
+            }))
+            return nullptr;
+        return THPVariable_Wrap(std::move(y));
+    });
+}
+
+// gather_grad(grad, bin_counts, active_block_indices, x_shape, bsize, bstride, boffset, transpose) -> dx
+PyObject* gather_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 8)) return nullptr;
+    const at::Tensor* g = dev_f32(a[0]);
+    Blocks b;
+    Pair bs, bt, bo;
+    if (!g || !blocks_of(a[1], a[2], b) || b.count || b.idx->device() != g->device() || !PyTuple_Check(a[3]) ||
+        PyTuple_GET_SIZE(a[3]) != 4 || !pair_of(a[4], bs) || !pair_of(a[5], bt) || !pair_of(a[6], bo))
+        Py_RETURN_NONE;
+    int64_t dims[4];
+    for (int i = 0; i < 4; ++i) {
+        int32_t d;
+        if (!int_of(PyTuple_GET_ITEM(a[3], i), &d) || d <= 0) Py_RETURN_NONE;
+        dims[i] = d;
+    }
+    const int transpose = PyObject_IsTrue(a[7]);
+    if (transpose < 0) return nullptr;
+    if (!is_stack(*g, b.M, dims[3], bs, transpose)) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(g->device());
+        at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, *g);
+        const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
+        at::Tensor ws = need ? workspace(g->device(), need) : at::Tensor();
+        const float* const gp = static_cast<const float*>(g->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const dp = static_cast<float*>(dx.data_ptr());
+        void* const stream = stream_of(*g);
+        if (!call([&] {
+                return sbnet_sparse_gather_grad(gp, b.M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
+                                                need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
+            }))
+            return nullptr;
+        return THPVariable_Wrap(std::move(dx));
+    });
+}
+
+// scatter(x, bin_counts, active_block_indices, ybase, bsize, bstride, boffset, add, atomic, transpose, use_var) -> y
+PyObject* scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 11)) return nullptr;
+    const at::Tensor *x = dev_f32(a[0]), *base = dev_f32(a[3]);
+    Blocks b;
+    Pair bs, bt, bo;
+    if (!x || !base || base->dim() != 4 || !blocks_of(a[1], a[2], b) || b.idx->device() != base->device() ||
+        x->device() != base->device() || !pair_of(a[4], bs) || !pair_of(a[5], bt) || !pair_of(a[6], bo))
+        Py_RETURN_NONE;
+    const int add = PyObject_IsTrue(a[7]), atomic = PyObject_IsTrue(a[8]), transpose = PyObject_IsTrue(a[9]),
+              in_place = PyObject_IsTrue(a[10]);
+    if (add < 0 || atomic < 0 || transpose < 0 || in_place < 0) return nullptr;
+    if (b.count && x->dim() > 0 && x->size(0) < b.M) b.M = (int32_t)x->size(0);
+    if (!is_stack(*x, b.M, base->size(3), bs, transpose)) Py_RETURN_NONE;
+    const bool overlap = bt.v[0] < bs.v[0] || bt.v[1] < bs.v[1];
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(base->device());
+        const int64_t* const dims = base->sizes().data();
+        const bool scratch = (add && atomic) || !in_place || (!add && overlap);
+        const int64_t need = scratch ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
+        at::Tensor ws = need ? workspace(base->device(), need) : at::Tensor();
+        void* const wp = need ? ws.data_ptr() : nullptr;
+        const size_t wn = need ? (size_t)ws.numel() : 0;
+        at::Tensor y = in_place ? *base : empty_f32(base->sizes(), *base);
+        const float *const xp = static_cast<const float*>(x->data_ptr()), *const bp = static_cast<const float*>(base->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const yp = static_cast<float*>(y.data_ptr());
+        void* const stream = stream_of(*base);
+        if (!call([&] {
+                if (in_place)
+                    return b.count ? sbnet_sparse_scatter_var_device_count(xp, b.count, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2,
+                                                                           bo.v, 2, add, atomic, transpose, wp, wn, stream)
+                                   : sbnet_sparse_scatter_var(xp, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
+                                                              transpose, wp, wn, stream);
+                return b.count ? sbnet_sparse_scatter_device_count(xp, b.count, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2,
+                                                                   add, atomic, transpose, yp, wp, wn, stream)
+                               : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
+                                                      transpose, yp, wp, wn, stream);
+            }))
+            return nullptr;
+        if (in_place) {
+            Py_INCREF(a[3]);   // the caller's own tensor object, as the Python wrapper returns it
+            return a[3];
+        }
+        return THPVariable_Wrap(std::move(y));
+    });
+}
+
+// Contiguous, on the GPU, float32, with no gradient asked for.
+const at::Tensor* plain_f32(PyObject* o)
+{
+    const at::Tensor* t = dev_f32(o);
+    return t && !(t->requires_grad() && at::GradMode::is_enabled()) ? t : nullptr;
+}
+
+constexpr int64_t CONV_MOST = 1ll << 28, ROWS_MOST = 1ll << 28;   // elements, output pixels: inside what the kernels take
+
+// Kernel dimensions as int32, false where an input of C channels and R x S pixels does not take it.
+bool kernel_of(const at::Tensor& w, int64_t C, int64_t R, int64_t S, int32_t* dims)
+{
+    if (w.dim() != 4 || w.size(2) != C || C > 4096 || w.size(0) > R || w.size(1) > S || w.numel() <= 0 || w.numel() >= CONV_MOST) return false;
+    for (int i = 0; i < 4; ++i) dims[i] = (int32_t)w.size(i);
+    return true;
+}
+
+bool positive(const Pair& p) { return p.v[0] > 0 && p.v[1] > 0; }
+
+// block_conv(x, w, bin_counts, active_block_indices, bsize, bstride, boffset) -> NHWC stack
+PyObject* block_conv(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 7)) return nullptr;
+    const at::Tensor *x = plain_f32(a[0]), *w = plain_f32(a[1]);
+    Blocks b;
+    Pair bs, bt, bo;
+    int32_t wd[4];
+    if (!x || !w || x->dim() != 4 || x->numel() <= 0 || x->numel() >= 2 * CONV_MOST || w->device() != x->device() ||
+        !blocks_of(a[2], a[3], b) || b.idx->device() != x->device() || !pair_of(a[4], bs) || !pair_of(a[5], bt) ||
+        !pair_of(a[6], bo) || !positive(bs) || !positive(bt) || !kernel_of(*w, x->size(3), bs.v[0], bs.v[1], wd))
+        Py_RETURN_NONE;
+    const int64_t R = bs.v[0] - wd[0] + 1, S = bs.v[1] - wd[1] + 1;
+    if (R * S >= ROWS_MOST || b.M * R * S >= ROWS_MOST || b.M * R * S * wd[3] >= 2 * CONV_MOST) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(x->device());
+        at::Tensor q = empty_f32({b.M, R, S, wd[3]}, *x);
+        const float *const xp = static_cast<const float*>(x->data_ptr()), *const kp = static_cast<const float*>(w->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const qp = static_cast<float*>(q.data_ptr());
+        const int64_t* const dims = x->sizes().data();
+        void* const stream = stream_of(*x);
+        if (b.M && !call([&] { return sbnet_block_conv(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, kp, wd, qp, stream); }))
+            return nullptr;
+        return THPVariable_Wrap(std::move(q));
+    });
+}
+
+// block_bottleneck(x, [w1, w2, w3], [gamma, beta, mean, var] * 3, bin_counts, active_block_indices, bsize, bstride,
+//                  boffset, out_stride, eps, no_activation, in_place) -> NHWC stack, or x with the result added
+PyObject* block_bottleneck(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 12)) return nullptr;
+    const at::Tensor* x = plain_f32(a[0]);
+    Blocks b;
+    Pair bs, bt, bo, os;
+    if (!x || x->dim() != 4 || x->numel() <= 0 || x->numel() >= 2 * CONV_MOST || !PyList_CheckExact(a[1]) ||
+        PyList_GET_SIZE(a[1]) != 3 || !PyList_CheckExact(a[2]) || PyList_GET_SIZE(a[2]) != 12 || !blocks_of(a[3], a[4], b) ||
+        b.idx->device() != x->device() || !pair_of(a[5], bs) || !pair_of(a[6], bt) || !pair_of(a[7], bo) ||
+        !pair_of(a[8], os) || !positive(bs) || !positive(bt) || !PyFloat_CheckExact(a[9]))
+        Py_RETURN_NONE;
+    const int no_activation = PyObject_IsTrue(a[10]), in_place = PyObject_IsTrue(a[11]);
+    if (no_activation < 0 || in_place < 0) return nullptr;
+    const float *weights[3], *norms[12];
+    int32_t wd[12];
+    int64_t R = bs.v[0], S = bs.v[1], C = x->size(3);
+    for (int i = 0; i < 3; ++i) {
+        const at::Tensor* w = plain_f32(PyList_GET_ITEM(a[1], i));
+        if (!w || w->device() != x->device() || !kernel_of(*w, C, R, S, wd + 4 * i)) Py_RETURN_NONE;
+        weights[i] = static_cast<const float*>(w->data_ptr());
+        for (int j = 0; j < 4; ++j) {
+            const at::Tensor* t = plain_f32(PyList_GET_ITEM(a[2], 4 * i + j));
+            if (!t || t->device() != x->device() || t->numel() != C) Py_RETURN_NONE;
+            norms[4 * i + j] = i == 0 && no_activation ? nullptr : static_cast<const float*>(t->data_ptr());
+        }
+        R -= wd[4 * i] - 1;
+        S -= wd[4 * i + 1] - 1;
+        C = wd[4 * i + 3];
+        if (R * S >= ROWS_MOST || b.M * R * S >= ROWS_MOST || b.M * R * S * C >= 2 * CONV_MOST) Py_RETURN_NONE;
+    }
+    if (in_place && (C != x->size(3) || os.v[0] != R || os.v[1] != S)) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(x->device());
+        at::Tensor q = in_place ? *x : empty_f32({b.M, R, S, C}, *x);
+        at::Tensor ws = workspace(x->device(), (int64_t)sbnet_block_bottleneck_workspace_bytes(b.M, bs.v, wd));
+        const float* const xp = static_cast<const float*>(x->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const qp = static_cast<float*>(q.data_ptr());
+        const int64_t* const dims = x->sizes().data();
+        const float eps = (float)PyFloat_AS_DOUBLE(a[9]);
+        void* const stream = stream_of(*x);
+        if (b.M && !call([&] {
+                return sbnet_block_bottleneck(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, weights, wd, norms, eps,
+                                              in_place ? nullptr : qp, in_place ? qp : nullptr, os.v, ws.data_ptr(),
+                                              (size_t)ws.numel(), stream);
+            }))
+            return nullptr;
+        if (in_place) {
+            Py_INCREF(a[0]);
+            return a[0];
+        }
+        return THPVariable_Wrap(std::move(q));
+    });
+}
+
+// workspace(device index, bytes) -> uint8 tensor: the scratch of the current stream, for the wrappers in Python
+PyObject* workspace_py(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 2)) return nullptr;
+    const long dev = PyLong_AsLong(a[0]);
+    const long long bytes = PyLong_AsLongLong(a[1]);
+    if (PyErr_Occurred()) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const at::Device device(at::kCUDA, (c10::DeviceIndex)dev);
+        c10::DeviceGuard guard(device);
+        return THPVariable_Wrap(workspace(device, bytes));
+    });
+}
+
+PyObject* release_workspaces(PyObject*, PyObject*)
+{
+    if (g_workspaces) g_workspaces->clear();
+    Py_RETURN_NONE;
+}
+
+PyObject* has_workspaces(PyObject*, PyObject*) { return PyBool_FromLong(g_workspaces && !g_workspaces->empty()); }
+
+PyObject* set_check(PyObject*, PyObject* f)
+{
+    Py_INCREF(f);
+    Py_XSETREF(g_check, f);
+    Py_RETURN_NONE;
+}
+
+template <typename F>
+PyCFunction fast(F f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)); }
+
+PyMethodDef methods[] = {
+    {"reduce_mask", fast(reduce_mask), METH_FASTCALL, nullptr},
+    {"gather", fast(gather), METH_FASTCALL, nullptr},
+    {"gather_grad", fast(gather_grad), METH_FASTCALL, nullptr},
+    {"scatter", fast(scatter), METH_FASTCALL, nullptr},
+    {"block_conv", fast(block_conv), METH_FASTCALL, nullptr},
+    {"block_bottleneck", fast(block_bottleneck), METH_FASTCALL, nullptr},
+    {"workspace", fast(workspace_py), METH_FASTCALL, nullptr},
+    {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
+    {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},
+    {"set_check", set_check, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module_def); }

@@ -37,6 +37,20 @@ def _check(status):
     raise InvalidArgument(text)
 
 
+# The extension module with the ops' common case, once loaded.  Its functions take plain arguments (contiguous tensors,
+# pairs of ints) and return None, with nothing allocated or enqueued, for anything else; the wrappers below then go the
+# general way, which converts what can be converted and raises for the rest.
+_native = None
+
+
+def _load_native():
+    global _native
+    module = _lib.native()
+    module.set_check(_check)
+    _native = module
+    return module
+
+
 def _pair(v):
     """Host int32 parameter vector as (keepalive array, pointer, length); length is checked by the library."""
     if isinstance(v, torch.Tensor):
@@ -100,24 +114,19 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-_workspaces = {}
-
-
 def _workspace(device, nbytes):
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    """Scratch of the current stream: one uint8 tensor per (device, stream) that is kept and only grows."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return (_native or _load_native()).workspace(index, nbytes)
 
 
 def release_workspaces():
     """Drops the scratch buffers the op wrappers keep per (device, stream) between calls (they only ever grow) and
     the library's own (sbnet_shutdown).  Waits for the device; the ops can be used again afterwards."""
-    if _workspaces:
+    native = _native or _load_native()
+    if native.has_workspaces():
         torch.cuda.synchronize()
-    _workspaces.clear()
+    native.release_workspaces()
     _check(_lib.load().sbnet_shutdown())
 
 
@@ -142,12 +151,16 @@ def reduce_mask(mask, dynamic_bcount=None, dynamic_bsize=None, dynamic_bstride=N
     in (n, bh, bw) lexicographic order, and an int32 tensor [1] in host memory.  With sync=False the
     count is left on the device (bin_counts is then a GPU tensor) and the call does not wait.
     """
-    lib = _lib.load()
     dynamic_bcount, dynamic_bsize = _param(dynamic_bcount, bcount, "bcount"), _param(dynamic_bsize, bsize, "bsize")
     dynamic_bstride = _param(dynamic_bstride, bstride, "bstride")
     dynamic_boffset = _param(dynamic_boffset, boffset, "boffset")
     if tol is None:
         raise TypeError("reduce_mask: tol is required (the op attribute has no default, reduce_mask.cc:102)")
+    r = (_native or _load_native()).reduce_mask(mask, dynamic_bcount, dynamic_bsize, dynamic_bstride, dynamic_boffset, tol,
+                                                avgpool, sync)
+    if r is not None:
+        return ReduceMaskResult(*r)
+    lib = _lib.load()
     mask = _dev_f32(mask, "mask")
     if mask.dim() not in (3, 4) or (mask.dim() == 4 and mask.shape[3] != 1):
         raise InvalidArgument("mask must be [N,H,W,1] (or [N,H,W]), got %s" % (tuple(mask.shape),))
@@ -216,6 +229,10 @@ def sparse_gather(x, bin_counts, active_block_indices, dynamic_bsize=None, dynam
 def gather_forward(x, bin_counts, active_block_indices, dynamic_bsize, dynamic_bstride, dynamic_boffset,
                    transpose=False, out=None):
     """The gather without autograd bookkeeping (what SparseGatherFunction.forward and the gradients call)."""
+    y = (_native or _load_native()).gather(x, bin_counts, active_block_indices, dynamic_bsize, dynamic_bstride, dynamic_boffset,
+                                           transpose, out)
+    if y is not None:
+        return y
     lib = _lib.load()
     x = _dev_f32(x, "x")
     idx = _idx_i16(active_block_indices)
@@ -255,6 +272,10 @@ def gather_backward(grad, bin_counts, active_block_indices, x_shape, dynamic_bsi
     """Gradient of sparse_gather with respect to x (sparse_conv_lib.py:80-107: the reference scatters grad onto
     zeros_like(x) with add=True, atomic=True): a tensor of shape x_shape that is zero where no block lies and holds
     the sum of the blocks of `grad` elsewhere, built without clearing the tensor first."""
+    dx = (_native or _load_native()).gather_grad(grad, bin_counts, active_block_indices, x_shape, dynamic_bsize, dynamic_bstride,
+                                                 dynamic_boffset, transpose)
+    if dx is not None:
+        return dx
     lib = _lib.load()
     grad = _dev_f32(grad, "grad")
     idx = _idx_i16(active_block_indices)
@@ -285,6 +306,11 @@ def scatter_forward(x, bin_counts, active_block_indices, ybase, dynamic_bsize, d
     """The scatter without autograd bookkeeping.  scratch=False passes no workspace to the library (hardware
     atomics for overlapping adds, unordered overlapping plain writes, copy-then-scatter): what a caller of the
     C ABI gets who brings none."""
+    if scratch:
+        y = (_native or _load_native()).scatter(x, bin_counts, active_block_indices, ybase, dynamic_bsize, dynamic_bstride,
+                                                dynamic_boffset, add, atomic, transpose, use_var)
+        if y is not None:
+            return y
     lib = _lib.load()
     x = _dev_f32(x, "x")
     idx = _idx_i16(active_block_indices)

@@ -52,59 +52,11 @@ def _conv_blocks(p, w, stride, transpose):
     return q.permute(0, 2, 3, 1).contiguous()
 
 
-def _plain(*tensors):
-    """Contiguous float32 tensors on one GPU of which none asks for a gradient: what the block convolutions take."""
-    grad = torch.is_grad_enabled()
-    return all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and
-               t.device == tensors[0].device and not (grad and t.requires_grad) for t in tensors)
-
-
-def _fits(*sizes):
-    """Element counts whose byte offsets the block convolutions hold in 32 bits."""
-    return all(0 < n < 1 << 30 for n in sizes)
-
-
-def _numel(*dims):
-    n = 1
-    for d in dims:
-        n *= int(d)
-    return n
-
-
-class _Blocks(object):
-    """The block list and geometry of a layer call as the C ABI takes them; `fits` is False for what it would refuse."""
-
-    def __init__(self, x, indices, block_params):
-        self.idx = ops._idx_i16(indices.active_block_indices)
-        self.count = ops._device_count(indices.bin_counts)
-        self.M = int(self.idx.shape[0]) if self.count is not None else ops._count(indices.bin_counts)
-        ops._check_count(self.M, self.idx)
-        self.pairs = [ops._pair(v) for v in (block_params.bsize, block_params.bstrides, block_params.boffset)]
-        self.bsize = self.pairs[0][0]
-        self.fits = x.dim() == 4 and all(p[2] == 2 for p in self.pairs) and bool((self.pairs[1][0] > 0).all())
-
-    def args(self, x):
-        self.dims = ops._dims(x)[0]
-        return (x.data_ptr(), self.dims, self.M, self.count.data_ptr() if self.count is not None else None,
-                self.idx.data_ptr(), *(p[1] for p in self.pairs))
-
-
 def _block_conv(x, w, indices, block_params):
-    """VALID convolution (stride 1) of the active blocks as an NHWC stack, or None where only the composed path applies."""
-    if not _plain(x, w) or w.dim() != 4:
-        return None
-    b = _Blocks(x, indices, block_params)
-    kh, kw, cin, cout = (int(d) for d in w.shape)
-    if not b.fits or x.shape[3] != cin or cin > 4096 or b.bsize[0] < kh or b.bsize[1] < kw:
-        return None
-    shape = (b.M, int(b.bsize[0]) - kh + 1, int(b.bsize[1]) - kw + 1, cout)
-    if not _fits(x.numel(), w.numel(), _numel(*shape)) or _numel(*shape[:3]) >= 1 << 28:
-        return None
-    with torch.cuda.device(x.device):
-        q = torch.empty(shape, dtype=torch.float32, device=x.device)
-        ops._check(_lib.load().sbnet_block_conv(*b.args(x), w.data_ptr(), (ctypes.c_int32 * 4)(kh, kw, cin, cout),
-                                                q.data_ptr(), ops._stream()))
-    return q
+    """VALID convolution (stride 1) of the active blocks as an NHWC stack, or None where only the composed path applies
+    (a gradient is asked for, tensors that are not contiguous float32, sizes beyond 32-bit byte offsets)."""
+    return (ops._native or ops._load_native()).block_conv(x, w, indices.bin_counts, indices.active_block_indices,
+                                                          block_params.bsize, block_params.bstrides, block_params.boffset)
 
 
 def sparse_conv2d_custom(x, w, indices, block_params, strides, use_var=False, transpose=False, atomic=False):
@@ -379,36 +331,9 @@ def res_block_bottleneck(x, params, strides, is_training, data_format="NHWC", w_
 def _block_bottleneck(x, params, indices, block_params, no_activation, in_place):
     """The residual function of the active blocks in inference: added to x (returns x) or as an NHWC stack; None where
     only the composed path applies."""
-    bn = [t for b in params.bn for t in b]
-    if len(params.w) != 3 or len(bn) != 12 or not _plain(x, *params.w, *bn) or any(w.dim() != 4 for w in params.w):
-        return None
-    b = _Blocks(x, indices, block_params)
-    if not b.fits:
-        return None
-    R, S, C = int(b.bsize[0]), int(b.bsize[1]), int(x.shape[3])
-    sizes = [x.numel()]
-    for w, norm in zip(params.w, params.bn):
-        kh, kw, cin, cout = (int(d) for d in w.shape)
-        R, S = R - kh + 1, S - kw + 1
-        if cin != C or cin > 4096 or R <= 0 or S <= 0 or any(t.numel() != cin for t in norm) or _numel(b.M, R, S) >= 1 << 28:
-            return None
-        C = cout
-        sizes += [w.numel(), _numel(b.M, R, S, C)]
-    out_stride = ops._pair(block_params.bsize_out)
-    if not _fits(*sizes) or (in_place and (C != x.shape[3] or out_stride[2] != 2 or out_stride[0][0] != R or out_stride[0][1] != S)):
-        return None
-    lib = _lib.load()
-    pointer = ctypes.c_void_p
-    weights = (pointer * 3)(*(w.data_ptr() for w in params.w))
-    w_dims = (ctypes.c_int32 * 12)(*(int(d) for w in params.w for d in w.shape))
-    norms = (pointer * 12)(*(None if no_activation and i < 4 else t.data_ptr() for i, t in enumerate(bn)))
-    with torch.cuda.device(x.device):
-        ws = ops._workspace(x.device, lib.sbnet_block_bottleneck_workspace_bytes(b.M, b.pairs[0][1], w_dims))
-        q = None if in_place else torch.empty((b.M, R, S, C), dtype=torch.float32, device=x.device)
-        ops._check(lib.sbnet_block_bottleneck(*b.args(x), weights, w_dims, norms, BN_EPS, None if in_place else q.data_ptr(),
-                                              x.data_ptr() if in_place else None, out_stride[1], ws.data_ptr(), ws.numel(),
-                                              ops._stream()))
-    return x if in_place else q
+    return (ops._native or ops._load_native()).block_bottleneck(
+        x, params.w, [t for b in params.bn for t in b], indices.bin_counts, indices.active_block_indices, block_params.bsize,
+        block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
 def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_training, data_format="NHWC",

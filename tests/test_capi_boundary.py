@@ -245,6 +245,24 @@ def test_python_mirror_checks_sizes_before_any_launch():
             ops._check_stack(torch.zeros(shape), 5, 8, 3, 4, transpose, "x")
 
 
+def test_native_wrappers_leave_what_they_do_not_take():
+    """The extension module returns None, before any device work, for arguments that are not its common case: tensors that
+    are not on a GPU here; the general wrappers then raise."""
+    import torch
+    from sbnet_amd import ops
+
+    native = ops._load_native()
+    x, idx = torch.zeros((1, 8, 8, 4)), torch.zeros((4, 3), dtype=torch.int16)
+    pair = [4, 4]
+    assert native.reduce_mask(x[..., :1], [2, 2], pair, pair, [0, 0], 0.5, False, True) is None
+    assert native.gather(x, [1], idx, pair, pair, [0, 0], False, None) is None
+    assert native.gather_grad(x, [1], idx, (1, 8, 8, 4), pair, pair, [0, 0], False) is None
+    assert native.scatter(x, [1], idx, x, pair, pair, [0, 0], False, False, False, True) is None
+    assert native.block_conv(x, x, [1], idx, pair, pair, [0, 0]) is None
+    with pytest.raises(TypeError, match="float32 tensor on the GPU"):
+        ops.sparse_gather(x, [1], idx, pair, pair, [0, 0])
+
+
 @pytest.mark.gpu
 def test_scratch_provider_keeps_outgrown_buffers_until_shutdown():
     """sbnet_scratch_acquire hands one grow-only buffer per stream to callers without an allocator.  A pointer it
