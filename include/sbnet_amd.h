@@ -337,6 +337,20 @@ int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_ac
                            const float* const* batch_norms, float bn_eps, float* q, float* y,
                            const int32_t* out_bstride, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Gradient of the same bottleneck's residual function on planar block stacks in training, batch norms with the statistics
+   of the stack (replaces the backward of the layers of sparse_conv_lib.py:677-723 with is_training).  For i = 0, 1, 2:
+   z[i] [num_blocks, C, R, S] in front of batch norm i (z[0] is the gathered stack), act[i] behind its ReLU, mean[i] and
+   inv[i] = 1 / sqrt(variance + eps) of the batch, gamma[i]; weights[i] [K,C,kh,kw], w_dims[4 * i ...] = kh, kw, C, K.
+   dq: the gradient of the third convolution's result -> dp that of z[0], both planar; dw[i] [kh,kw,C,K]; dgamma, dbeta.
+   Channels in multiples of four; dw and workspace 16-byte aligned; at least two pixels per channel everywhere.
+   workspace: sbnet_bottleneck_grad_workspace_bytes() bytes (0: the sizes are not taken), any contents. */
+size_t sbnet_bottleneck_grad_workspace_bytes(int32_t num_blocks, const int32_t* bsize, const int32_t* w_dims);
+int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bsize, const float* const* z,
+                          const float* const* act, const float* const* mean, const float* const* inv,
+                          const float* const* gamma, const float* const* weights, const int32_t* w_dims, float* dp,
+                          float* const* dw, float* const* dgamma, float* const* dbeta, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* Library-managed device scratch for callers that have no allocator at hand (the functor level of the reference
    passes none down, sparse_gather.h:45-66): returns a buffer of at least `bytes` bytes on the current device.  One
    grow-only buffer is kept per (device, stream); calls on one stream run in order, so consecutive calls of ONE

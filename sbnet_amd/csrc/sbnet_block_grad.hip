@@ -1,0 +1,386 @@
+// The gradient of a bottleneck's residual function beside its convolutions (sbnet_conv.hip): the backward of the batch
+// norms, the gradients of the kernels, and block stacks from planar to NHWC and back.
+//
+// Replaces the library's backward passes behind the reference's layer functions (sbnet_tensorflow/benchmark/
+// sparse_conv_lib.py:590-723 under tf.gradients).
+#include "sbnet_conv.h"
+#include "sbnet_device.h"
+
+namespace sbnet {
+
+typedef float acc_t __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------------------------------------
+// k_norm_grad: dz = gamma / sigma * (g - mean(g) - xhat * mean(g * xhat)), xhat = (z - mean) / sigma
+// ---------------------------------------------------------------------------------------------
+//
+// Four channels per thread, `cols` threads side by side, `tall` rows at a time; a workgroup takes as many rows as leave
+// about 512 workgroups.  Two tensors in, one out, once each.
+
+struct ChannelArgs {
+    uint32_t rows, C;
+    uint32_t cols, tall, rowsPerWg;
+};
+
+static ChannelArgs channel_args(uint32_t rows, int C, dim3& grid)
+{
+    ChannelArgs a;
+    a.rows = rows;
+    a.C = (uint32_t)C;
+    a.cols = min((uint32_t)C / 4u, 64u);
+    a.tall = 256u / a.cols;
+    const uint32_t chunks = (a.C / 4u + a.cols - 1) / a.cols;
+    const uint32_t steps = ((uint64_t)rows * chunks + a.tall * 512ull - 1) / (a.tall * 512ull);
+    a.rowsPerWg = a.tall * max(steps, 4u);
+    grid = dim3((rows + a.rowsPerWg - 1) / a.rowsPerWg, chunks);
+    return a;
+}
+
+__global__ __launch_bounds__(256) void k_norm_grad(float* __restrict__ g, NormGradArgs norm, ChannelArgs a,
+                                                   float* __restrict__ dgamma, float* __restrict__ dbeta)
+{
+    const uint32_t tid = threadIdx.x, ty = tid / a.cols, tx = tid - ty * a.cols;
+    const uint32_t c = (blockIdx.y * a.cols + tx) * 4u;
+    if (ty >= a.tall || c >= a.C) return;
+    float mean[4], scale[4], c1[4], c2[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int i = 0; i < GRAD_SLOTS; ++i) {
+            const double2 t = *reinterpret_cast<const double2*>(norm.sums + ((size_t)i * a.C + c + j) * 2);
+            s1 += t.x;
+            s2 += t.y;
+        }
+        const float inv = norm.inv[c + j];
+        mean[j] = norm.mean[c + j];
+        scale[j] = inv * norm.gamma[c + j];
+        c1[j] = (float)(s1 / a.rows);
+        c2[j] = (float)(s2 / a.rows * inv);
+        if (blockIdx.x == 0 && ty == 0) {
+            dgamma[c + j] = (float)s2;
+            dbeta[c + j] = (float)s1;
+        }
+    }
+    const float* const z = norm.z;
+    const uint32_t end = min((blockIdx.x + 1) * a.rowsPerWg, a.rows);
+#pragma unroll 4
+    for (uint32_t r = blockIdx.x * a.rowsPerWg + ty; r < end; r += a.tall) {
+        const size_t at = (size_t)r * a.C + c;
+        const f4 x = *reinterpret_cast<const f4*>(z + at);
+        f4 v = *reinterpret_cast<const f4*>(g + at);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = scale[j] * (v[j] - c1[j] - (x[j] - mean[j]) * c2[j]);
+        *reinterpret_cast<f4*>(g + at) = v;
+    }
+}
+
+hipError_t launch_norm_grad(float* g, const NormGradArgs& norm, uint32_t rows, int C, float* dgamma, float* dbeta,
+                            hipStream_t stream)
+{
+    dim3 grid;
+    const ChannelArgs a = channel_args(rows, C, grid);
+    hipLaunchKernelGGL(k_norm_grad, grid, dim3(256), 0, stream, g, norm, a, dgamma, dbeta);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
+// k_transposes: [M][A][B] -> [M][B][A], several tensors in one launch
+// ---------------------------------------------------------------------------------------------
+//
+// 64 x 32 tiles through LDS (a row more than a multiple of the banks apart), one dword per lane and access: 128 bytes in a
+// row on both sides, whatever B is (a block's pixel count, mostly odd).
+
+constexpr uint32_t TR_A = 64, TR_B = 32;
+
+struct TransposeProblem {
+    TransposeArgs t;
+    uint32_t tilesB, tiles, firstWg;
+};
+
+struct TransposeKernelArgs {
+    TransposeProblem p[10];
+    int count;
+};
+
+__global__ __launch_bounds__(256) void k_transposes(TransposeKernelArgs k)
+{
+    __shared__ float tile[TR_A * (TR_B + 1)];
+    int i = 0;
+    while (i + 1 < k.count && blockIdx.x >= k.p[i + 1].firstWg) ++i;
+    const TransposeProblem& q = k.p[i];
+    const uint32_t A = q.t.A, B = q.t.B;
+    const uint32_t local = blockIdx.x - q.firstWg, m = local / q.tiles, rest = local - m * q.tiles;
+    const uint32_t ta = rest / q.tilesB, a0 = ta * TR_A, b0 = (rest - ta * q.tilesB) * TR_B;
+    const float* __restrict__ from = q.t.from + (size_t)m * A * B;
+    float* __restrict__ to = q.t.to + (size_t)m * A * B;
+    const uint32_t tid = threadIdx.x;
+    float v[TR_A * TR_B / 256];
+#pragma unroll
+    for (uint32_t j = 0; j < TR_A * TR_B / 256; ++j) {
+        const uint32_t r = a0 + (tid >> 5) + 8 * j, c = b0 + (tid & 31);
+        v[j] = r < A && c < B ? from[(size_t)r * B + c] : 0.f;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < TR_A * TR_B / 256; ++j) tile[((tid >> 5) + 8 * j) * (TR_B + 1) + (tid & 31)] = v[j];
+    lds_barrier();
+#pragma unroll
+    for (uint32_t j = 0; j < TR_A * TR_B / 256; ++j) {
+        const uint32_t r = (tid >> 6) + 4 * j, c = tid & 63;
+        if (b0 + r < B && a0 + c < A) to[(size_t)(b0 + r) * A + a0 + c] = tile[c * (TR_B + 1) + r];
+    }
+}
+
+hipError_t launch_transposes(const TransposeArgs* t, int count, hipStream_t stream)
+{
+    if (count < 1 || count > 10) return hipErrorInvalidValue;
+    TransposeKernelArgs k;
+    uint64_t wgs = 0;
+    for (int i = 0; i < count; ++i) {
+        TransposeProblem& q = k.p[i];
+        q.t = t[i];
+        q.tilesB = (t[i].B + TR_B - 1) / TR_B;
+        q.tiles = (t[i].A + TR_A - 1) / TR_A * q.tilesB;
+        q.firstWg = (uint32_t)wgs;
+        wgs += (uint64_t)t[i].M * q.tiles;
+    }
+    if (wgs >= (1ull << 31)) return hipErrorInvalidConfiguration;
+    k.count = count;
+    hipLaunchKernelGGL(k_transposes, dim3((unsigned)wgs), dim3(256), 0, stream, k);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
+// k_wgrad: dw[m, n] = sum over output pixels p of act[p + tap, c] * dz[p, n], m = (tap, c)
+// ---------------------------------------------------------------------------------------------
+//
+// The sum runs over thousands of pixels and the result is small, so the pixels are what is split: a workgroup takes one
+// 64 x 64 (or 64 x 32) tile of one kernel's gradient over one range of pixels, its four waves every fourth quadruple of
+// pixels, and writes a partial tile that k_wgrad_sum adds to the others.  All three kernels of a bottleneck share the
+// launch: alone, each would leave part of the chip idle.
+//
+// v_mfma_f32_16x16x4_f32 with the four quads of a wave on four pixels: a lane's 16-byte load of four consecutive channels
+// of its pixel feeds four fragments (fragment i has rows 4 * l + i), so 4 pixels x 64 x 64 products cost two 16-byte loads
+// and 16 matrix instructions per lane, straight from memory.
+//
+// Measured (MI355X, kernel trace; 256-64-64-256 channels on about 85 active 11x11 blocks of [1,100,175,256]): 17.8 us for the
+// three products and 17.6 for the sum of the partial tiles, where the library took 77 us and six transposes of its operands
+// (23 us).  The whole gradient: 127 us in 12 launches; 190 us in 27 with the library's passes.
+
+struct WgradProblem {
+    WgradArgs w;
+    FastDiv dP, dSo, dC, dKw;
+    uint32_t rows, P, So, mTot;
+    uint32_t tilesM, tiles, rowsPerSplit, splits;
+    uint32_t aBytes, dzBytes;
+    uint32_t firstWg;      // of the launch
+    uint32_t firstSum;     // 16-byte pieces of the results before this one
+    int jb;                // output channels per lane: 4 or 2
+    float* part;           // [splits][tiles][4 * jb][64] x 4
+};
+
+struct WgradKernelArgs {
+    WgradProblem p[3];
+    int count;
+    uint32_t sums;
+};
+
+constexpr int WG_DEPTH = 4;   // pixel quadruples in flight per wave
+
+template <int JB, bool TAPS>
+__device__ __forceinline__ void wgrad_tile(const WgradProblem& q, uint32_t local, float* lds)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4, wave = tid >> 6;
+    const uint32_t split = local / q.tiles, tile = local - split * q.tiles;
+    const uint32_t tn = tile / q.tilesM, tm = tile - tn * q.tilesM;
+    const uint32_t C = (uint32_t)q.w.C, K = (uint32_t)q.w.K;
+
+    const uint32_t m = tm * 64u + l16 * 4u;
+    const bool mOk = m < q.mTot;
+    const uint32_t tap = TAPS ? fdiv(mOk ? m : 0u, q.dC) : 0u, c = (mOk ? m : 0u) - tap * C;
+    const uint32_t dr = TAPS ? fdiv(tap, q.dKw) : 0u, ds = tap - dr * (uint32_t)q.w.kw;
+    const uint32_t aOff = mOk ? (TAPS ? (dr * (uint32_t)q.w.S + ds) * C + c : c) * 4u : 0u;
+    const uint32_t n = tn * (16u * JB) + l16 * JB;
+    const bool nOk = n < K;
+    const rsrc_t ra = make_rsrc(q.w.act, q.aBytes), rd = make_rsrc(q.w.dz, q.dzBytes);
+
+    const uint32_t beg = split * q.rowsPerSplit, end = min(beg + q.rowsPerSplit, q.rows);
+    struct Operands {
+        acc_t v;
+        float d[JB];
+    };
+    // Rows past the range read zeros on both sides.
+    auto load = [&](uint32_t row, Operands& o) {
+        const bool ok = row < end;
+        uint32_t pix = row;
+        if constexpr (TAPS) {
+            const uint32_t ib = fdiv(ok ? row : 0u, q.dP), p = (ok ? row : 0u) - ib * q.P;
+            const uint32_t r = fdiv(p, q.dSo), s = p - r * q.So;
+            pix = (ib * (uint32_t)q.w.R + r) * (uint32_t)q.w.S + s;
+        }
+        o.v = (acc_t)buf_load<4>(ra, ok && mOk ? pix * C * 4u + aOff : BUF_OOB);
+        const uint32_t od = ok && nOk ? (row * K + n) * 4u : BUF_OOB;
+        if constexpr (JB == 4) {
+            const f4 t = buf_load<4>(rd, od);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o.d[j] = t[j];
+        } else {
+            const f2 t = buf_load<2>(rd, od);
+            o.d[0] = t[0];
+            o.d[1] = t[1];
+        }
+    };
+
+    acc_t acc[4][JB];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < JB; ++j) acc[i][j] = (acc_t)(0.f);
+    Operands ops[WG_DEPTH];
+    uint32_t row = beg + wave * 4u + quad;
+#pragma unroll
+    for (int d = 0; d < WG_DEPTH; ++d) load(row + d * 16u, ops[d]);
+    for (uint32_t first = beg + wave * 4u; first < end; first += WG_DEPTH * 16u) {
+#pragma unroll
+        for (int d = 0; d < WG_DEPTH; ++d) {
+            Operands& o = ops[d];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.v[i], o.d[j], acc[i][j], 0, 0, 0);
+            load(row + (WG_DEPTH + d) * 16u, o);
+        }
+        row += WG_DEPTH * 16u;
+    }
+
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+            *reinterpret_cast<acc_t*>(lds + ((wave * (4 * JB) + i * JB + j) * 64 + lane) * 4) = acc[i][j];
+    lds_barrier();
+    float* const out = q.part + (size_t)local * (4 * JB * 256);
+#pragma unroll
+    for (int f = 0; f < JB; ++f) {
+        const uint32_t frag = f * 4 + wave;
+        acc_t v = (acc_t)(0.f);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v += (acc_t)lds_read4(lds + ((k * (4 * JB) + frag) * 64 + lane) * 4);
+        *reinterpret_cast<acc_t*>(out + (frag * 64 + lane) * 4) = v;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_wgrad(WgradKernelArgs a)
+{
+    extern __shared__ float lds[];
+    int i = 0;
+    while (i + 1 < a.count && blockIdx.x >= a.p[i + 1].firstWg) ++i;
+    const WgradProblem& q = a.p[i];
+    const uint32_t local = blockIdx.x - q.firstWg;
+    const bool taps = q.w.kh * q.w.kw > 1;
+    if (q.jb == 4) {
+        if (taps) wgrad_tile<4, true>(q, local, lds);
+        else wgrad_tile<4, false>(q, local, lds);
+    } else {
+        if (taps) wgrad_tile<2, true>(q, local, lds);
+        else wgrad_tile<2, false>(q, local, lds);
+    }
+}
+
+// Adds the partial tiles, in double, and writes the gradients.
+__global__ __launch_bounds__(256) void k_wgrad_sum(WgradKernelArgs a)
+{
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+    if (id >= a.sums) return;
+    int k = 0;
+    while (k + 1 < a.count && id >= a.p[k + 1].firstSum) ++k;
+    const WgradProblem& q = a.p[k];
+    const uint32_t local = id - q.firstSum, frags = 4u * (uint32_t)q.jb;
+    const uint32_t lane = local & 63, l16 = lane & 15, quad = lane >> 4;
+    const uint32_t tile = (local >> 6) / frags, frag = (local >> 6) - tile * frags;
+    const uint32_t tn = tile / q.tilesM, tm = tile - tn * q.tilesM;
+    const float* p = q.part + (size_t)local * 4;
+    const size_t step = (size_t)q.tiles * frags * 256;
+    double s[4] = {};
+#pragma unroll 8
+    for (uint32_t i = 0; i < q.splits; ++i) {
+        const f4 v = *reinterpret_cast<const f4*>(p + i * step);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += (double)v[j];
+    }
+    const uint32_t i = frag / (uint32_t)q.jb, j = frag - i * (uint32_t)q.jb;
+    const uint32_t n = (tn * 16u + l16) * (uint32_t)q.jb + j;
+    if (n >= (uint32_t)q.w.K) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint32_t m = tm * 64u + (quad * 4u + r) * 4u + i;
+        if (m < q.mTot) q.w.dw[(size_t)m * q.w.K + n] = (float)s[r];
+    }
+}
+
+// About 640 workgroups in all, each of at least 64 pixels, the pixels' ranges of all problems equally long.
+static void wgrad_plan(const WgradArgs* w, int count, WgradKernelArgs& a)
+{
+    uint64_t cost = 0;
+    for (int i = 0; i < count; ++i) {
+        WgradProblem& q = a.p[i];
+        q.w = w[i];
+        q.P = (uint32_t)((w[i].R - w[i].kh + 1) * (w[i].S - w[i].kw + 1));
+        q.So = (uint32_t)(w[i].S - w[i].kw + 1);
+        q.rows = (uint32_t)w[i].M * q.P;
+        q.mTot = (uint32_t)(w[i].kh * w[i].kw * w[i].C);
+        q.jb = w[i].K > 32 ? 4 : 2;
+        q.tilesM = (q.mTot + 63) / 64;
+        q.tiles = q.tilesM * (((uint32_t)w[i].K + 16 * q.jb - 1) / (16 * q.jb));
+        cost += (uint64_t)q.rows * q.tiles;
+    }
+    uint64_t per = (cost + 639) / 640;
+    per = per < 64 ? 64 : (per + 15) / 16 * 16;
+    uint32_t wg = 0, sum = 0;
+    for (int i = 0; i < count; ++i) {
+        WgradProblem& q = a.p[i];
+        q.rowsPerSplit = (uint32_t)per;
+        q.splits = (uint32_t)((q.rows + per - 1) / per);
+        q.firstWg = wg;
+        q.firstSum = sum;
+        wg += q.splits * q.tiles;
+        sum += q.tiles * 4 * q.jb * 64;
+    }
+    a.count = count;
+    a.sums = sum;
+}
+
+size_t wgrad_workspace_bytes(const WgradArgs* w, int count)
+{
+    WgradKernelArgs a;
+    wgrad_plan(w, count, a);
+    size_t total = 0;
+    for (int i = 0; i < count; ++i) total += (size_t)a.p[i].splits * a.p[i].tiles * (4 * a.p[i].jb * 256) * sizeof(float);
+    return total;
+}
+
+hipError_t launch_wgrad(const WgradArgs* w, int count, void* workspace, hipStream_t stream)
+{
+    if (count < 1 || count > 3) return hipErrorInvalidValue;
+    WgradKernelArgs a;
+    wgrad_plan(w, count, a);
+    float* part = static_cast<float*>(workspace);
+    for (int i = 0; i < count; ++i) {
+        WgradProblem& q = a.p[i];
+        q.dP = make_fastdiv(q.P);
+        q.dSo = make_fastdiv(q.So);
+        q.dC = make_fastdiv((uint32_t)w[i].C);
+        q.dKw = make_fastdiv((uint32_t)w[i].kw);
+        q.aBytes = (uint32_t)((uint64_t)w[i].M * w[i].R * w[i].S * w[i].C * 4);
+        q.dzBytes = (uint32_t)((uint64_t)q.rows * w[i].K * 4);
+        q.part = part;
+        part += (size_t)q.splits * q.tiles * (4 * q.jb * 256);
+    }
+    const WgradProblem& last = a.p[count - 1];
+    const uint32_t wgs = last.firstWg + last.splits * last.tiles;
+    hipLaunchKernelGGL(k_wgrad, dim3(wgs), dim3(256), 65536, stream, a);
+    hipLaunchKernelGGL(k_wgrad_sum, dim3((a.sums + 255) / 256), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+}  // namespace sbnet

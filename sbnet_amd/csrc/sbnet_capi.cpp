@@ -702,6 +702,112 @@ int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_ac
     return SBNET_OK;
 }
 
+// The gradients of a bottleneck's three convolutions as launch_block_conv_grad takes them (c[i]: from the gradient of
+// result i to that of its input), the kernels' gradients, and where what lies between them is in the scratch.
+struct BottleneckGrad {
+    sbnet::ConvArgs c[3];
+    sbnet::WgradArgs w[3];
+    size_t sums[3], sumBytes;                 // of the batch norms
+    size_t z[3], act[3], kernel[3], dz[4];    // NHWC stacks (dz[3]: dq), kernels [C,kh,kw,K]
+    size_t part, total;
+};
+
+static bool bottleneck_grad_plan(int32_t num_blocks, const int32_t* bsize, const int32_t* w_dims, BottleneckGrad& b)
+{
+    if (num_blocks <= 0 || !bsize || !w_dims || bsize[0] <= 0 || bsize[1] <= 0) return false;
+    auto take = [](size_t& at, uint64_t bytes) {
+        const size_t here = at;
+        at += (size_t)((bytes + 255) & ~(uint64_t)255);
+        return here;
+    };
+    int R = bsize[0], S = bsize[1];
+    size_t at = 0;
+    for (int i = 0; i < 3; ++i) {
+        const int32_t* d = w_dims + 4 * i;
+        if (d[0] <= 0 || d[1] <= 0 || d[2] <= 0 || d[3] <= 0 || d[0] > R || d[1] > S || (i && d[2] != w_dims[4 * i - 1])) return false;
+        sbnet::ConvArgs& c = b.c[i];
+        c = sbnet::ConvArgs();
+        c.N = c.M = num_blocks;
+        c.kh = d[0]; c.kw = d[1]; c.K = d[2]; c.C = d[3];
+        c.Ro = R; c.So = S;
+        c.H = R -= d[0] - 1;
+        c.W = S -= d[1] - 1;
+        if (!sbnet::conv_grad_fits(c) || (int64_t)num_blocks * c.Ro * c.So < 2) return false;
+        sbnet::WgradArgs& w = b.w[i];
+        w = sbnet::WgradArgs();
+        w.M = num_blocks; w.R = c.Ro; w.S = c.So; w.C = c.K; w.K = c.C; w.kh = c.kh; w.kw = c.kw;
+        b.sums[i] = take(at, sizeof(double) * sbnet::GRAD_SLOTS * 2 * c.K);
+    }
+    b.sumBytes = at;
+    for (int i = 0; i < 3; ++i) {
+        const sbnet::ConvArgs& c = b.c[i];
+        const uint64_t stack = sizeof(float) * (uint64_t)num_blocks * c.Ro * c.So * c.K;
+        b.z[i] = take(at, stack);
+        b.act[i] = take(at, stack);
+        b.dz[i] = take(at, stack);
+        b.kernel[i] = take(at, sizeof(float) * (uint64_t)c.K * c.kh * c.kw * c.C);
+    }
+    b.dz[3] = take(at, sizeof(float) * (uint64_t)num_blocks * R * S * b.c[2].C);
+    b.part = take(at, sbnet::wgrad_workspace_bytes(b.w, 3));
+    b.total = at;
+    return true;
+}
+
+size_t sbnet_bottleneck_grad_workspace_bytes(int32_t num_blocks, const int32_t* bsize, const int32_t* w_dims)
+{
+    BottleneckGrad b;
+    return bottleneck_grad_plan(num_blocks, bsize, w_dims, b) ? b.total : 0;
+}
+
+int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bsize, const float* const* z,
+                          const float* const* act, const float* const* mean, const float* const* inv,
+                          const float* const* gamma, const float* const* weights, const int32_t* w_dims, float* dp,
+                          float* const* dw, float* const* dgamma, float* const* dbeta, void* workspace,
+                          size_t workspace_bytes, void* stream)
+{
+    BottleneckGrad b;
+    if (!dq || !z || !act || !mean || !inv || !gamma || !weights || !dp || !dw || !dgamma || !dbeta || !workspace ||
+        (reinterpret_cast<uintptr_t>(workspace) & 15) || !bottleneck_grad_plan(num_blocks, bsize, w_dims, b) ||
+        workspace_bytes < b.total)
+        return SBNET_EINVAL_ARG;
+    for (int i = 0; i < 3; ++i)
+        if (!z[i] || !act[i] || !mean[i] || !inv[i] || !gamma[i] || !weights[i] || !dw[i] || !dgamma[i] || !dbeta[i] ||
+            (reinterpret_cast<uintptr_t>(dw[i]) & 15))
+            return SBNET_EINVAL_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    uint8_t* const ws = static_cast<uint8_t*>(workspace);
+    auto at = [&](size_t offset) { return reinterpret_cast<float*>(ws + offset); };
+
+    sbnet::TransposeArgs t[10];
+    int n = 0;
+    for (int i = 0; i < 3; ++i) {
+        const sbnet::ConvArgs& c = b.c[i];
+        const uint32_t M = (uint32_t)num_blocks, C = (uint32_t)c.K, P = (uint32_t)(c.Ro * c.So);
+        t[n++] = sbnet::TransposeArgs{z[i], at(b.z[i]), M, C, P};
+        t[n++] = sbnet::TransposeArgs{act[i], at(b.act[i]), M, C, P};
+        t[n++] = sbnet::TransposeArgs{weights[i], at(b.kernel[i]), 1, (uint32_t)c.C, C * (uint32_t)(c.kh * c.kw)};
+    }
+    t[n++] = sbnet::TransposeArgs{dq, at(b.dz[3]), (uint32_t)num_blocks, (uint32_t)b.c[2].C, (uint32_t)(b.c[2].H * b.c[2].W)};
+    SBNET_HIP(sbnet::launch_zero(at(0), b.sumBytes / sizeof(float), s));
+    SBNET_HIP(sbnet::launch_transposes(t, n, s));
+    for (int i = 2; i >= 0; --i) {
+        sbnet::ConvArgs& c = b.c[i];
+        c.a = at(b.dz[i + 1]);
+        c.w = at(b.kernel[i]);
+        c.y = at(b.dz[i]);
+        c.norm = sbnet::NormGradArgs{at(b.z[i]), at(b.act[i]), mean[i], inv[i], gamma[i], reinterpret_cast<double*>(ws + b.sums[i])};
+        SBNET_HIP(sbnet::launch_block_conv_grad(c, s));
+        SBNET_HIP(sbnet::launch_norm_grad(at(b.dz[i]), c.norm, (uint32_t)(c.M * c.Ro * c.So), c.K, dgamma[i], dbeta[i], s));
+        b.w[i].act = at(b.act[i]);
+        b.w[i].dz = at(b.dz[i + 1]);
+        b.w[i].dw = dw[i];
+    }
+    SBNET_HIP(sbnet::launch_wgrad(b.w, 3, ws + b.part, s));
+    t[0] = sbnet::TransposeArgs{at(b.dz[0]), dp, (uint32_t)num_blocks, (uint32_t)(b.c[0].Ro * b.c[0].So), (uint32_t)b.c[0].K};
+    SBNET_HIP(sbnet::launch_transposes(t, 1, s));
+    return SBNET_OK;
+}
+
 int sbnet_sparse_scatter_functor(const float* x, int N, int H, int W, int C, float* y, int bOffsH0,
                                  int bOffsW0, int bSzH, int bSzW, int bStrH, int bStrW, int numActive,
                                  const int16_t* activeBlockIndices, int add, int transpose, int atomic,

@@ -61,7 +61,10 @@ __device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& sca
     shift = bn.beta[c] - bn.mean[c] * scale;
 }
 
-template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS>
+// GRAD: the gradient of a convolution's input.  The same product with the kernel turned around, w [K, kh, kw, C] (n, then
+// k: a lane's four k are one 16-byte load of w, too); the epilogue masks the result where the ReLU did and adds up what
+// the batch norm's gradient needs, in fp32 over 16 pixels and in double from there on.
+template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS, bool GRAD>
 __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKernelArgs a)
 {
     constexpr int WAVES = WK > 4 ? WK : 4, WP = WAVES / WK;
@@ -72,7 +75,8 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     float* const preShift = lds + cPad;
     float* const postScale = lds + 2 * cPad;
     float* const postShift = postScale + TN;
-    float* const red = postScale + 2 * TN;   // [WP][WK][FP * FN][64] x 4, WK > 1 only
+    double* const sums = reinterpret_cast<double*>(postScale + 2 * TN);   // [WP * FP][TN][2], GRAD only
+    float* const red = postScale + (GRAD ? 2 + 4 * WP * FP : 2) * TN;     // [WP][WK][FP * FN][64] x 4, WK > 1 only
 
     // Eight consecutive workgroups go to eight XCDs; the tiles of one pixel range that differ in channels only follow
     // each other on one XCD, whose L2 then holds the pixels once.
@@ -117,7 +121,10 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     const uint32_t K = (uint32_t)a.c.K;
     uint32_t wCol[FN];
 #pragma unroll
-    for (int f = 0; f < FN; ++f) wCol[f] = n0 + f * 16 + l16 < K ? (n0 + f * 16 + l16) * 4u : W_OOB;
+    for (int f = 0; f < FN; ++f) {
+        const uint32_t n = n0 + f * 16 + l16;
+        wCol[f] = n < K ? n * (GRAD ? a.kTot : 1u) * 4u : W_OOB;
+    }
 
     struct Operands {
         acc_t px[FP];
@@ -143,6 +150,17 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
                 c = min(c, (uint32_t)a.c.C - (VEC == 4 ? 4u : 1u));   // (a channel to look scale and shift up for, past the end)
             }
             o.c[j] = c;
+            if constexpr (GRAD) {
+                const uint32_t row = kj < kEnd ? kj * 4u : W_OOB;
+#pragma unroll
+                for (int f = 0; f < FN; ++f) {
+                    const f4 t = buf_load<4>(rw, row + wCol[f]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o.wv[f][i] = t[i];
+                }
+                dr = -dr;   // (the output pixel that this tap took the input pixel to)
+                ds = -ds;
+            }
             const uint32_t toff = (((uint32_t)dr * (uint32_t)a.c.W + (uint32_t)ds) * (uint32_t)a.c.C + c) * 4u;
 #pragma unroll
             for (int f = 0; f < FP; ++f) {
@@ -153,11 +171,13 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
                 else o.px[f][j] = buf_load<1>(ra, off);
             }
         }
+        if constexpr (!GRAD) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t row = (k + j < kEnd) ? (k + j) * K * 4u : W_OOB;
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t row = (k + j < kEnd) ? (k + j) * K * 4u : W_OOB;
 #pragma unroll
-            for (int f = 0; f < FN; ++f) o.wv[f][j] = buf_load<1>(rw, row + wCol[f]);
+                for (int f = 0; f < FN; ++f) o.wv[f][j] = buf_load<1>(rw, row + wCol[f]);
+            }
         }
     };
 
@@ -173,10 +193,17 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
 
     if (PRE)
         for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_fold(a.c.pre, c, preScale[c], preShift[c]);
-    if (post)
+    if constexpr (GRAD) {   // mean and 1 / sigma
+        for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES) {
+            const uint32_t n = min(n0 + i, K - 1);
+            postScale[i] = a.c.norm.mean[n];
+            postShift[i] = a.c.norm.inv[n];
+        }
+    } else if (post) {
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES)
             if (n0 + i < K) bn_fold(a.c.post, n0 + i, postScale[i], postShift[i]);
-    if (PRE || post) lds_barrier();
+    }
+    if (PRE || GRAD || post) lds_barrier();
 
     for (uint32_t step = sBeg; step < sEnd; step += CONV_DEPTH) {
 #pragma unroll
@@ -214,6 +241,34 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     const rsrc_t ry = make_rsrc(a.c.y, a.yBytes);
     auto finish = [&](int i, int f, acc_t v) {
         const uint32_t nl = i * 16 + quad * 4, n = n0 + nl;
+        if constexpr (GRAD) {
+            const uint32_t group = wp * FP + f, row = tp * TP + group * 16 + l16;
+            const uint32_t o = row < rows && n < K ? (row * K + n) * 4u : BUF_OOB;
+            const acc_t z = (acc_t)buf_load<4>(make_rsrc(a.c.norm.z, a.yBytes), o);
+            const acc_t act = (acc_t)buf_load<4>(make_rsrc(a.c.norm.act, a.yBytes), o);   // (0 past the end: masked)
+            const acc_t xhat = (z - (acc_t)lds_read4(postScale + nl)) * (acc_t)lds_read4(postShift + nl);
+            acc_t s1, s2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s1[j] = act[j] <= 0.f ? 0.f : v[j];
+                s2[j] = s1[j] * xhat[j];
+            }
+            buf_store<0>(ry, o, (f4)s1);
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    s1[j] += __shfl_xor(s1[j], off);
+                    s2[j] += __shfl_xor(s2[j], off);
+                }
+            if (l16 == 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    sums[(group * TN + nl + j) * 2] = s1[j];
+                    sums[(group * TN + nl + j) * 2 + 1] = s2[j];
+                }
+            return;
+        }
         if (post) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan(v[j] * postScale[nl + j] + postShift[nl + j]);
@@ -267,18 +322,30 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
             finish(q / FP, q % FP, v);
         }
     }
+
+    if constexpr (GRAD) {
+        lds_barrier();
+        // one atomic per channel, sum and workgroup; consecutive threads to consecutive doubles
+        for (uint32_t i = tid; i < 2u * TN; i += 64 * WAVES) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < WP * FP; ++k) s += sums[k * TN * 2 + i];
+            if (n0 + (i >> 1) < K)
+                unsafeAtomicAdd(a.c.norm.sums + ((size_t)(blockIdx.x & (GRAD_SLOTS - 1)) * K + n0) * 2 + i, s);
+        }
+    }
 }
 
-template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS>
+template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS, bool GRAD = false>
 static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
 {
     constexpr int WAVES = WK > 4 ? WK : 4, TP = 16 * FP * (WAVES / WK), TN = 16 * FN;
     a.tilesP = (a.rows + TP - 1) / TP;
     a.tilesN = ((uint32_t)a.c.K + TN - 1) / TN;
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
-    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + 2 * TN + (WK > 1 ? (size_t)WAVES * FP * FN * 256 : 0));
+    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * FP * (WAVES / WK) : 2) * TN + (WK > 1 ? (size_t)WAVES * FP * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC, PRE, TAPS>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
+    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC, PRE, TAPS, GRAD>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();
 }
 
@@ -318,22 +385,29 @@ static bool make_conv_args(const ConvArgs& c, ConvKernelArgs& a)
     return c.C % 4 == 0 && c.K % 4 == 0 && (bits & 15) == 0;   // 16-byte accesses on both sides
 }
 
-hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
+// fn: fragments of 16 channels per wave; wk: waves that split k.
+static void conv_tile(const ConvKernelArgs& a, bool vec, int& fn, int& wk)
 {
-    if (c.M <= 0) return hipSuccess;
-    if (!conv_fits(c)) return hipErrorInvalidValue;
-    ConvKernelArgs a;
-    const bool vec = make_conv_args(c, a);
     // Narrow wave tiles (16 pixels x 32 channels; 48 where that leaves no channel over, 16 where there are no more) and as
     // many waves per tile as it takes to occupy the SIMDs: a launch of fewer than about 1500 waves is four times shorter
     // with k split four ways than its occupancy would suggest, and one with few steps per wave has nothing to split.
     // Wider tiles read less and wait more: 32x32 is 10-40 % slower on all but the narrowest and largest problems (us for
     // 16x32 / 32x32, best split: 2450 pixels, k 1152, 128 channels 16.4 / 19.0; 4860, 576, 64: 10.3 / 12.0; 45 000, 216, 24:
     // 13.2 / 12.6; 38 400, 600, 24: 24.7 / 22.7).
-    const uint32_t nFrag = ((uint32_t)c.K + 15) / 16;
-    const int fn = nFrag == 1 ? 1 : (vec && nFrag % 3 == 0 && nFrag % 2 == 1 ? 3 : 2);
+    const uint32_t nFrag = ((uint32_t)a.c.K + 15) / 16;
+    fn = nFrag == 1 ? 1 : (vec && nFrag % 3 == 0 && nFrag % 2 == 1 ? 3 : 2);
     const uint64_t waves = (uint64_t)((a.rows + 15) / 16) * ((nFrag + fn - 1) / fn);
-    const int wk = a.kSteps < 8 ? 1 : (waves < 1536 ? 4 : (waves < 3072 && a.kSteps >= 16 ? 2 : 1));
+    wk = a.kSteps < 8 ? 1 : (waves < 1536 ? 4 : (waves < 3072 && a.kSteps >= 16 ? 2 : 1));
+}
+
+hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
+{
+    if (c.M <= 0) return hipSuccess;
+    if (!conv_fits(c)) return hipErrorInvalidValue;
+    ConvKernelArgs a;
+    const bool vec = make_conv_args(c, a);
+    int fn, wk;
+    conv_tile(a, vec, fn, wk);
     if (!vec) {
         if (fn == 1) return wk > 1 ? launch_conv_one<1, 1, 4, 1>(a, stream) : launch_conv_one<1, 1, 1, 1>(a, stream);
         return wk > 1 ? launch_conv_one<1, 2, 4, 1>(a, stream) : launch_conv_one<1, 2, 1, 1>(a, stream);
@@ -348,6 +422,41 @@ hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
     case 24 + 1: return launch_conv_one<1, 3, 1, 4>(a, stream);
     case 24 + 2: return launch_conv_one<1, 3, 2, 4>(a, stream);
     default: return launch_conv_one<1, 3, 4, 4>(a, stream);
+    }
+}
+
+template <int FN, int WK>
+static hipError_t launch_conv_grad_one(ConvKernelArgs& a, hipStream_t stream)
+{
+    if (a.c.kh * a.c.kw > 1) return launch_conv_as<1, FN, WK, 4, false, true, true>(a, stream);
+    return launch_conv_as<1, FN, WK, 4, false, false, true>(a, stream);
+}
+
+bool conv_grad_fits(const ConvArgs& c)
+{
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(c.a) | reinterpret_cast<uintptr_t>(c.y) | reinterpret_cast<uintptr_t>(c.w) |
+                           reinterpret_cast<uintptr_t>(c.norm.z) | reinterpret_cast<uintptr_t>(c.norm.act);
+    return conv_fits(c) && c.M > 0 && c.C % 4 == 0 && c.K % 4 == 0 && (bits & 15) == 0 && !c.idx && !c.oidx && !c.countDev &&
+           c.Ro == c.H + c.kh - 1 && c.So == c.W + c.kw - 1;
+}
+
+hipError_t launch_block_conv_grad(const ConvArgs& c, hipStream_t stream)
+{
+    if (!conv_grad_fits(c)) return hipErrorInvalidValue;
+    ConvKernelArgs a;
+    if (!make_conv_args(c, a)) return hipErrorInvalidValue;
+    int fn, wk;
+    conv_tile(a, true, fn, wk);
+    switch (fn * 8 + wk) {
+    case 8 + 1: return launch_conv_grad_one<1, 1>(a, stream);
+    case 8 + 2: return launch_conv_grad_one<1, 2>(a, stream);
+    case 8 + 4: return launch_conv_grad_one<1, 4>(a, stream);
+    case 16 + 1: return launch_conv_grad_one<2, 1>(a, stream);
+    case 16 + 2: return launch_conv_grad_one<2, 2>(a, stream);
+    case 16 + 4: return launch_conv_grad_one<2, 4>(a, stream);
+    case 24 + 1: return launch_conv_grad_one<3, 1>(a, stream);
+    case 24 + 2: return launch_conv_grad_one<3, 2>(a, stream);
+    default: return launch_conv_grad_one<3, 4>(a, stream);
     }
 }
 

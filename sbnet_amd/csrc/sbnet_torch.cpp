@@ -424,6 +424,73 @@ PyObject* block_bottleneck(PyObject*, PyObject* const* a, Py_ssize_t n)
     });
 }
 
+// bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1, ...), on
+// planar stacks, or None where the kernels do not take the sizes.
+PyObject* bottleneck_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 2)) return nullptr;
+    const at::Tensor* dq = dev_f32(a[0]);
+    if (!dq || dq->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 18) Py_RETURN_NONE;
+    const at::Tensor* t[18];
+    const float* ptr[6][3];
+    for (int i = 0; i < 18; ++i) {
+        t[i] = dev_f32(PyList_GET_ITEM(a[1], i));
+        if (!t[i] || t[i]->device() != dq->device()) Py_RETURN_NONE;
+        ptr[i % 6][i / 6] = static_cast<const float*>(t[i]->data_ptr());
+    }
+    if (t[0]->dim() != 4 || t[0]->size(0) > INT32_MAX) Py_RETURN_NONE;
+    const int64_t M = t[0]->size(0);
+    int64_t C = t[0]->size(1), R = t[0]->size(2), S = t[0]->size(3);
+    if (M <= 0 || C <= 0 || R <= 0 || S <= 0 || R > INT32_MAX || S > INT32_MAX) Py_RETURN_NONE;
+    const int32_t bs[2] = {(int32_t)R, (int32_t)S};
+    int32_t wd[12];
+    for (int i = 0; i < 3; ++i) {
+        const at::Tensor* const* q = t + 6 * i;
+        const at::Tensor* w = q[4];
+        if (q[0]->dim() != 4 || q[0]->sizes() != at::IntArrayRef({M, C, R, S}) || q[1]->sizes() != q[0]->sizes() ||
+            q[0]->numel() >= 2 * CONV_MOST || q[2]->numel() != C || q[3]->numel() != C || q[5]->numel() != C || w->dim() != 4 ||
+            w->size(1) != C || w->size(2) > R || w->size(3) > S || w->numel() <= 0 || w->numel() >= CONV_MOST)
+            Py_RETURN_NONE;
+        wd[4 * i] = (int32_t)w->size(2);
+        wd[4 * i + 1] = (int32_t)w->size(3);
+        wd[4 * i + 2] = (int32_t)C;
+        wd[4 * i + 3] = (int32_t)w->size(0);
+        R -= w->size(2) - 1;
+        S -= w->size(3) - 1;
+        C = w->size(0);
+    }
+    if (dq->sizes() != at::IntArrayRef({M, C, R, S}) || dq->numel() >= 2 * CONV_MOST) Py_RETURN_NONE;
+    const size_t need = sbnet_bottleneck_grad_workspace_bytes((int32_t)M, bs, wd);
+    if (!need) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(dq->device());
+        at::Tensor res[10];
+        float *out[10];
+        res[0] = empty_f32(t[0]->sizes(), *dq);
+        for (int i = 0; i < 3; ++i) {
+            const int32_t* d = wd + 4 * i;
+            res[1 + i] = empty_f32({d[0], d[1], d[2], d[3]}, *dq);
+            res[4 + 2 * i] = empty_f32({d[2]}, *dq);
+            res[5 + 2 * i] = empty_f32({d[2]}, *dq);
+        }
+        for (int i = 0; i < 10; ++i) out[i] = static_cast<float*>(res[i].data_ptr());
+        float *const dgamma[3] = {out[4], out[6], out[8]}, *const dbeta[3] = {out[5], out[7], out[9]};
+        // (as large as the stacks: from the allocator on each call, not kept)
+        at::Tensor ws = at::detail::empty_cuda({(int64_t)need}, at::kByte, dq->device(), c10::nullopt);
+        const float* const dqp = static_cast<const float*>(dq->data_ptr());
+        void *const wp = ws.data_ptr(), *const stream = stream_of(*dq);
+        if (!call([&] {
+                return sbnet_bottleneck_grad(dqp, (int32_t)M, bs, ptr[0], ptr[1], ptr[2], ptr[3], ptr[5], ptr[4], wd, out[0],
+                                             out + 1, dgamma, dbeta, wp, need, stream);
+            }))
+            return nullptr;
+        PyObject* r = PyTuple_New(10);
+        if (!r) return nullptr;
+        for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(res[i])));
+        return r;
+    });
+}
+
 // workspace(device index, bytes) -> uint8 tensor: the scratch of the current stream, for the wrappers in Python
 PyObject* workspace_py(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
@@ -463,6 +530,7 @@ PyMethodDef methods[] = {
     {"scatter", fast(scatter), METH_FASTCALL, nullptr},
     {"block_conv", fast(block_conv), METH_FASTCALL, nullptr},
     {"block_bottleneck", fast(block_bottleneck), METH_FASTCALL, nullptr},
+    {"bottleneck_grad", fast(bottleneck_grad), METH_FASTCALL, nullptr},
     {"workspace", fast(workspace_py), METH_FASTCALL, nullptr},
     {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},

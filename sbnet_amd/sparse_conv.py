@@ -19,10 +19,12 @@ sbnet_amd.autograd).
 Where no gradient is asked for, `sparse_conv2d_custom` and `sparse_res_block_bottleneck` (in inference) run this
 package's own convolution kernels instead (sbnet_amd/csrc/sbnet_conv.hip), which read the active blocks straight from x
 and keep what lies between two convolutions of a residual block in NHWC stacks; the stack's layout is then nobody's to
-see, and `transpose` / `data_format` select nothing.
+see, and `transpose` / `data_format` select nothing.  The gradients of a residual block's training step on planar stacks
+are in own kernels, too (sbnet_block_grad.hip).
 """
 import collections
 import ctypes
+import types
 
 import torch
 import torch.nn.functional as F
@@ -336,6 +338,64 @@ def _block_bottleneck(x, params, indices, block_params, no_activation, in_place)
         block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
+class _ResidualInTraining(torch.autograd.Function):
+    """_bottleneck_residual of a planar block stack with batch statistics: forward as there, the gradients in this package's
+    own kernels (sbnet_block_grad.hip)."""
+
+    @staticmethod
+    def forward(ctx, p, moving, *tensors):   # tensors: kernel, gamma and beta of each layer
+        z, saved = p, []
+        for i in range(3):
+            w, gamma, beta = tensors[3 * i:3 * i + 3]
+            a, mean, inv, _, _ = torch._batch_norm_impl_index(z, gamma, beta, *moving[i], True, 1.0 - BN_DECAY, BN_EPS,
+                                                              torch.backends.cudnn.enabled)
+            w_ = _hwio_to_oihw(w)
+            saved += [z, a.relu_(), mean, inv, w_, gamma]
+            z = F.conv2d(a, w_, stride=(1, 1))
+        ctx.save_for_backward(*saved, *tensors[2::3])
+        ctx.kernels = [(w, w._version) for w in tensors[::3]]   # for a graph of the gradients alone
+        return z
+
+    @staticmethod
+    def backward(ctx, dq):
+        saved = ctx.saved_tensors
+        create_graph = torch.is_grad_enabled()
+        if not create_graph:
+            grads = ops._native.bottleneck_grad(dq.contiguous(), list(saved[:18]))
+            if grads is not None:
+                dp, dw1, dw2, dw3, *norms = grads
+                return dp, None, dw1, norms[0], norms[1], dw2, norms[2], norms[3], dw3, norms[4], norms[5]
+        # a graph of the gradients is asked for, or sizes that the kernels do not take: through the layers one by one
+        wanted = [ctx.needs_input_grad[0], *ctx.needs_input_grad[2:]]
+        with torch.enable_grad():
+            inputs = [saved[0]]
+            for i, (w, version) in enumerate(ctx.kernels):
+                if create_graph and w._version != version:
+                    raise RuntimeError("a kernel needed for gradient computation has been modified by an inplace operation")
+                inputs += [w if create_graph else saved[6 * i + 4].permute(2, 3, 1, 0), saved[6 * i + 5], saved[18 + i]]
+            if not create_graph:
+                inputs = [t.detach().requires_grad_() for t in inputs]
+            layers = types.SimpleNamespace(w=inputs[1::3], bn=[BatchNormParams(*inputs[i:i + 2], None, None) for i in (2, 5, 8)])
+            q = _bottleneck_residual(inputs[0], layers, [1, 1, 1, 1], "VALID", True, "NCHW")
+            found = iter(torch.autograd.grad(q, [t for t, n in zip(inputs, wanted) if n], dq, create_graph=create_graph))
+        grads = [next(found) if n else None for n in wanted]
+        return (grads[0], None, *grads[1:])
+
+
+def _own_residual_gradient(p, params):
+    """Whether _ResidualInTraining applies: not under forward-mode or functorch transforms, autocast, or where deterministic
+    algorithms are asked for (its batch norm sums are added up with atomics, in double)."""
+    tensors = [p, *params.w, *(t for b in params.bn for t in b)]
+    return (torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
+            torch._C._functorch.peek_interpreter_stack() is None and not torch.is_autocast_enabled("cuda") and
+            not torch.are_deterministic_algorithms_enabled() and len(tensors) == 16 and
+            all(t.is_cuda and t.dtype is torch.float32 and t.is_contiguous() for t in tensors) and
+            all(w.dim() == 4 and w.shape[2] % 4 == 0 and w.shape[3] % 4 == 0 for w in params.w) and
+            not any(b.moving_mean.requires_grad or b.moving_var.requires_grad for b in params.bn) and
+            p.shape[0] * (p.shape[2] - sum(w.shape[0] - 1 for w in params.w[:2])) *
+            (p.shape[3] - sum(w.shape[1] - 1 for w in params.w[:2])) >= 2)
+
+
 def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_training, data_format="NHWC",
                                 w_project=None, no_activation=False, use_var=False):
     """sparse_conv_lib.py:751-824: y = x + F(x) evaluated on the active blocks only.
@@ -353,7 +413,12 @@ def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_tr
                           block_params.bstrides, block_params.boffset, transpose=transpose)
     if w_project is not None:
         x = _conv_layer(x, w_project, strides[2], "SAME", False)
-    q = _bottleneck_residual(p, params, strides, "VALID", is_training, data_format, no_activation)
+    if (is_training and transpose and not no_activation and strides[1] == strides[2] == 1 and
+            _own_residual_gradient(p, params)):
+        q = _ResidualInTraining.apply(p, [(b.moving_mean, b.moving_var) for b in params.bn],
+                                      *(t for w, b in zip(params.w, params.bn) for t in (w, b.gamma, b.beta)))
+    else:
+        q = _bottleneck_residual(p, params, strides, "VALID", is_training, data_format, no_activation)
     q = q.contiguous()
     fn = ops.sparse_scatter_var if use_var else ops.sparse_scatter
     return fn(q, indices.bin_counts, indices.active_block_indices, x, block_params.bsize_out,
