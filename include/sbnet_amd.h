@@ -337,6 +337,16 @@ int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_ac
                            const float* const* batch_norms, float bn_eps, float* q, float* y,
                            const int32_t* out_bstride, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Gradient of sbnet_sparse_scatter (plain writes, add = 0) with respect to its base: dbase [dims] = dy, times zero on the
+   pixels that a listed block covers (replaces the stamped-out mask of sparse_conv_lib.py:131-147).  workspace: of
+   sbnet_sparse_scatter_base_grad_workspace_bytes(), 4-byte aligned, any contents; that is 0 where the call does not apply
+   (no block, more than 2x2 blocks over a pixel, channels or images beyond the kernel's range).  dy, dbase: 16-byte aligned. */
+size_t sbnet_sparse_scatter_base_grad_workspace_bytes(int32_t num_active, const int64_t* dims, const int32_t* bsize,
+                                                      const int32_t* bstride, const int32_t* boffset);
+int sbnet_sparse_scatter_base_grad(const float* dy, int32_t num_active, const int16_t* active_block_indices, float* dbase,
+                                   const int64_t* dims, const int32_t* bsize, const int32_t* bstride, const int32_t* boffset,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* Gradient of the same bottleneck's residual function on planar block stacks in training, batch norms with the statistics
    of the stack (replaces the backward of the layers of sparse_conv_lib.py:677-723 with is_training).  For i = 0, 1, 2:
    z[i] [num_blocks, C, R, S] in front of batch norm i (z[0] is the gathered stack), act[i] behind its ReLU, mean[i] and

@@ -65,6 +65,8 @@ SIGNATURES = {
     "sbnet_block_bottleneck_workspace_bytes": (_sz, [_i32, _i32p, _i32p]),
     "sbnet_block_bottleneck": (_int, [_vp, _i64p, _i32, _vp, _vp, _i32p, _i32p, _i32p, _vp, _i32p, _vp, _f, _vp, _vp,
                                       _i32p, _vp, _sz, _vp]),
+    "sbnet_sparse_scatter_base_grad_workspace_bytes": (_sz, [_i32, _i64p, _i32p, _i32p, _i32p]),
+    "sbnet_sparse_scatter_base_grad": (_int, [_vp, _i32, _vp, _vp, _i64p, _i32p, _i32p, _i32p, _vp, _sz, _vp]),
     "sbnet_bottleneck_grad_workspace_bytes": (_sz, [_i32, _i32p, _i32p]),
     "sbnet_bottleneck_grad": (_int, [_vp, _i32, _i32p, _vp, _vp, _vp, _vp, _vp, _vp, _i32p, _vp, _vp, _vp, _vp, _vp, _sz,
                                      _vp]),

@@ -9,7 +9,8 @@ backward pass runs the HIP kernels of the forward ops:
                               computed by one entry point that writes zeros only where no block lies
 * d SparseScatter / dblocks = sparse_gather(grad, ...)
 * d SparseScatter / dybase  = grad                       (add=True)
-                            = grad * stamp-out mask      (add=False; mask = blocks of zeros scattered over ones)
+                            = grad * stamp-out mask      (add=False; mask = blocks of zeros scattered over ones),
+                              in one pass over grad where at most 2x2 blocks cover a pixel
 
 No gradient flows to the index list, the count or the block parameters, as in the reference.
 
@@ -70,7 +71,9 @@ class SparseScatterFunction(torch.autograd.Function):
         if ctx.needs_input_grad[3]:
             if add:
                 d_ybase = grad
-            else:
+            elif not (torch.is_grad_enabled() and grad.requires_grad):
+                d_ybase = ops.scatter_base_backward(grad, [M], idx, bsize, bstride, boffset)
+            if d_ybase is None:   # a graph of the gradients is asked for, or a geometry that the one pass does not take
                 stamp = torch.ones_like(grad)
                 zeros = torch.zeros(ctx.blocks_shape, dtype=torch.float32, device=grad.device)
                 ops.scatter_forward(zeros, [M], idx, stamp, bsize, bstride, boffset, add=False, atomic=False,

@@ -581,6 +581,32 @@ int sbnet_sparse_gather_grad(const float* dy, int32_t num_active, const int16_t*
                         workspace, workspace_bytes, s);
 }
 
+static bool aligned16(const void* p) { return p && (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+size_t sbnet_sparse_scatter_base_grad_workspace_bytes(int32_t num_active, const int64_t* dims, const int32_t* bsize,
+                                                      const int32_t* bstride, const int32_t* boffset)
+{
+    if (num_active <= 0 || !dims || !dims_fit_int(dims) || !bsize || !bstride || !boffset ||
+        !geom_ok((int)dims[0], (int)dims[1], (int)dims[2], (int)dims[3], bsize, bstride))
+        return 0;
+    return sbnet::scatter_base_grad_workspace_bytes(
+        make_geom((int)dims[0], (int)dims[1], (int)dims[2], (int)dims[3], bsize, bstride, boffset), num_active);
+}
+
+int sbnet_sparse_scatter_base_grad(const float* dy, int32_t num_active, const int16_t* active_block_indices, float* dbase,
+                                   const int64_t* dims, const int32_t* bsize, const int32_t* bstride, const int32_t* boffset,
+                                   void* workspace, size_t workspace_bytes, void* stream)
+{
+    const size_t need = sbnet_sparse_scatter_base_grad_workspace_bytes(num_active, dims, bsize, bstride, boffset);
+    if (!need || !active_block_indices || !workspace || workspace_bytes < need || !aligned16(dy) || !aligned16(dbase))
+        return SBNET_EINVAL_ARG;
+    const sbnet::Geom g = make_geom((int)dims[0], (int)dims[1], (int)dims[2], (int)dims[3], bsize, bstride, boffset);
+    bool done = false;
+    SBNET_HIP(sbnet::launch_scatter_base_grad(dy, dbase, active_block_indices, num_active, g, workspace, workspace_bytes,
+                                              static_cast<hipStream_t>(stream), done));
+    return done ? SBNET_OK : SBNET_EINVAL_ARG;
+}
+
 // The input side of a block convolution: checks, and the geometry of [N,H,W,C] read at the listed blocks.
 static int conv_input(const float* x, const int64_t* x_dims, int32_t num_active, const int32_t* bin_counts_device,
                       const int16_t* active_block_indices, const int32_t* bsize, const int32_t* bstride,

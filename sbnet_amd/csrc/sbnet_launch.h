@@ -78,6 +78,12 @@ hipError_t launch_zero(float* y, size_t count, hipStream_t stream);
 hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* idx, int numActive, const Geom& g,
                                      bool transpose, void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done);
 
+// dbase = dy with the pixels that a listed block covers multiplied by zero (the gradient of plain writes with respect to
+// the base); at most 2x2 blocks over a pixel, scratch of scatter_base_grad_workspace_bytes() (0: does not apply).
+size_t scatter_base_grad_workspace_bytes(const Geom& g, int numActive);
+hipError_t launch_scatter_base_grad(const float* dy, float* dbase, const int16_t* idx, int numActive, const Geom& g,
+                                    void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done);
+
 // Plain writes ("=") of overlapping blocks in the order of the sequential CPU functor: on a pixel that several
 // blocks cover, the block listed last wins (sparse_gather.cc:105-129), for either stack layout and for lists that
 // name a block twice.  Needs scratch of scatter_owner_workspace_bytes() (one int32 per pixel; 0 when the blocks do

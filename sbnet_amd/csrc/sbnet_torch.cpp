@@ -320,6 +320,34 @@ PyObject* scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
     });
 }
 
+// scatter_base_grad(grad, bin_counts, active_block_indices, bsize, bstride, boffset) -> gradient of the base of plain writes
+PyObject* scatter_base_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+{
+    if (!expect(n, 6)) return nullptr;
+    const at::Tensor* g = dev_f32(a[0]);
+    Blocks b;
+    Pair bs, bt, bo;
+    if (!g || g->dim() != 4 || reinterpret_cast<uintptr_t>(g->data_ptr()) & 15 || !blocks_of(a[1], a[2], b) || b.count ||
+        b.idx->device() != g->device() || !pair_of(a[3], bs) || !pair_of(a[4], bt) || !pair_of(a[5], bo))
+        Py_RETURN_NONE;
+    const int64_t* const dims = g->sizes().data();
+    const size_t need = sbnet_sparse_scatter_base_grad_workspace_bytes(b.M, dims, bs.v, bt.v, bo.v);
+    if (!need) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        c10::DeviceGuard guard(g->device());
+        at::Tensor d = empty_f32(g->sizes(), *g);
+        at::Tensor ws = workspace(g->device(), (int64_t)need);
+        const float* const gp = static_cast<const float*>(g->data_ptr());
+        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+        float* const dp = static_cast<float*>(d.data_ptr());
+        void *const wp = ws.data_ptr(), *const stream = stream_of(*g);
+        const size_t wn = (size_t)ws.numel();
+        if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, wn, stream); }))
+            return nullptr;
+        return THPVariable_Wrap(std::move(d));
+    });
+}
+
 // Contiguous, on the GPU, float32, with no gradient asked for.
 const at::Tensor* plain_f32(PyObject* o)
 {
@@ -528,6 +556,7 @@ PyMethodDef methods[] = {
     {"gather", fast(gather), METH_FASTCALL, nullptr},
     {"gather_grad", fast(gather_grad), METH_FASTCALL, nullptr},
     {"scatter", fast(scatter), METH_FASTCALL, nullptr},
+    {"scatter_base_grad", fast(scatter_base_grad), METH_FASTCALL, nullptr},
     {"block_conv", fast(block_conv), METH_FASTCALL, nullptr},
     {"block_bottleneck", fast(block_bottleneck), METH_FASTCALL, nullptr},
     {"bottleneck_grad", fast(bottleneck_grad), METH_FASTCALL, nullptr},

@@ -301,6 +301,12 @@ def gather_backward(grad, bin_counts, active_block_indices, x_shape, dynamic_bsi
     return dx
 
 
+def scatter_base_backward(grad, bin_counts, active_block_indices, bsize, bstride, boffset):
+    """Gradient of sparse_scatter (plain writes) with respect to ybase (sparse_conv_lib.py:131-147): grad times a mask that
+    is zero under the listed blocks, or None for a geometry that the kernel does not take."""
+    return (_native or _load_native()).scatter_base_grad(grad, bin_counts, active_block_indices, bsize, bstride, boffset)
+
+
 def scatter_forward(x, bin_counts, active_block_indices, ybase, dynamic_bsize, dynamic_bstride, dynamic_boffset, add,
                     atomic, transpose, use_var, scratch=True):
     """The scatter without autograd bookkeeping.  scratch=False passes no workspace to the library (hardware

@@ -277,3 +277,41 @@ def test_scatter_var_refuses_gradients():
         sbnet_amd.sparse_scatter_var(blocks, [1], idx, base, (2, 2), (2, 2), (0, 0), add=False)
     with torch.no_grad():
         sbnet_amd.sparse_scatter_var(blocks, [1], idx, base, (2, 2), (2, 2), (0, 0), add=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,bsize,bstride,boffset,M,twice", [
+    ((2, 30, 41, 16), (10, 10), (8, 8), (-1, -1), 17, False),    # overlapping, blocks over the borders
+    ((1, 33, 29, 15), (9, 13), (10, 14), (-3, -2), 9, False),    # gaps, odd channels
+    ((1, 64, 64, 6), (8, 8), (8, 8), (0, 0), 64, False),         # every pixel covered
+    ((3, 21, 50, 1), (6, 4), (3, 2), (-5, 1), 60, True),         # twice as large as the stride, a repeated block
+    ((1, 20, 20, 1024), (5, 5), (4, 4), (-2, -2), 5, False),     # the most channels of one strip
+    ((1, 20, 20, 2048), (5, 5), (4, 4), (-2, -2), 5, False),     # more: the composed way
+    ((1, 25, 26, 4), (7, 7), (3, 3), (0, 0), 30, False),         # three blocks over a pixel: the composed way
+    ((2, 17, 19, 8), (5, 6), (3, 40), (-2, -2), 4, False),       # stride larger than the image on one side only
+    ((5, 120, 130, 4), (4, 4), (2, 3), (0, -1), 8000, False),    # map built by two launches
+])
+def test_base_gradient_of_plain_writes_is_the_masked_product(shape, bsize, bstride, boffset, M, twice):
+    """Bit for bit, infinities, NaN and the sign of zero included."""
+    import sbnet_amd
+    rng = np.random.default_rng(M)
+    N, H, W, C = shape
+    bc = [1 + (H - boffset[0] - 1) // bstride[0], 1 + (W - boffset[1] - 1) // bstride[1]]
+    pick = rng.permutation(N * bc[0] * bc[1])[:M]
+    idx = np.stack([pick // (bc[0] * bc[1]), pick // bc[1] % bc[0], pick % bc[1]], 1).astype(np.int16)
+    if twice:
+        idx[-1] = idx[0]
+    idx, M = torch.from_numpy(idx).to("cuda:0"), len(idx)
+    dy = torch.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    dy.view(-1)[::7] = float("inf")
+    dy.view(-1)[3::11] = float("nan")
+    dy = dy.to("cuda:0")
+    q = torch.zeros((M, *bsize, C), device="cuda:0")
+    base = torch.zeros(shape, device="cuda:0", requires_grad=True)
+    y = sbnet_amd.sparse_scatter(q, [M], idx, base, list(bsize), list(bstride), list(boffset), add=False)
+    got, = torch.autograd.grad(y, base, dy)
+    stamp = sbnet_amd.sparse_scatter_var(q, [M], idx, torch.ones(shape, device="cuda:0"), list(bsize), list(bstride),
+                                         list(boffset), add=False)
+    want = dy * stamp
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.nan_to_num(got, nan=1.0).view(torch.int32), torch.nan_to_num(want, nan=1.0).view(torch.int32))
