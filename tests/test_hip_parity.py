@@ -1307,3 +1307,11 @@ def test_config4_overlapping_atomic_add():
 def test_config5_many_small_images(kernel_path):
     M = run_workload(workloads.config5())
     assert M > 10000
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 4095, 4096, 4097, 16383, 16384, 16385, 100003])
+def test_flat_copy_of_any_length(n):
+    """Around whole vectors and whole workgroups: every float copied, none beyond the end."""
+    src, dst = torch.randn(n + 8, device="cuda"), torch.full((n + 8,), 7.0, device="cuda")
+    ops._check(ops._lib.load().sbnet_copy_tensor(dst.data_ptr(), src.data_ptr(), n, ops._stream()))
+    assert torch.equal(dst[:n], src[:n]) and bool((dst[n:] == 7.0).all())
