@@ -18,7 +18,7 @@ namespace sbnet {
 // counts need no padding to a tap.  The input is an NHWC image read at the blocks' positions (pixels outside it are
 // zeros, as sparse_gather has them) or a block stack [M, R, S, C].
 //
-// A wave computes 16*FP pixels x 16*FN channels with v_mfma_f32_16x16x4_f32 (full fp32 products and sums: the precision
+// A wave computes 16 pixels x 16*FN channels with v_mfma_f32_16x16x4_f32 (full fp32 products and sums: the precision
 // of the convolution it replaces).  Channels are the rows of the matrix instruction and pixels its columns, so that a
 // lane ends with four consecutive channels of one pixel: 16-byte stores into NHWC memory.  Both operands go from memory
 // straight to registers: with the instruction's k index spread as (lane / 16) * 4 + step, a lane's four pixel values
@@ -28,9 +28,10 @@ namespace sbnet {
 // CONV_DEPTH sets of operands are in flight per wave.
 //
 // Measured (MI355X, kernel trace): 85 blocks of 17x17x48, 3x3 to 48 channels (19 000 pixels, 0.8 GFLOP; 5.2 us at the
-// rate of a large fp32 product): 19 us, 27 us while the loads of a step sat behind branches; the library convolution
-// took 21 us behind 5 us of layout copies, and up to 800 us the first time a block count occurred.  A bottleneck block of
-// 200 17x17x96 blocks: 39 us in three launches against about 300 us in 17.
+// rate of a large fp32 product): 15.7 us; 20.5 us with an exit inside a round of the loop and places found by division, 27 us
+// while the loads of a step sat behind branches; the library convolution took 21 us behind 5 us of layout copies, and up
+// to 800 us the first time a block count occurred.  A bottleneck block of 200 17x17x96 blocks: 33 us in three launches
+// against about 300 us in 17.
 //
 // WK > 1: the WK waves of a workgroup split k among them and add up through LDS.  For launches whose tiles alone would
 // leave most of the 1024 SIMDs idle.
@@ -40,8 +41,11 @@ namespace sbnet {
 
 typedef float acc_t __attribute__((ext_vector_type(4)));
 
-constexpr int CONV_DEPTH = 3;   // operand sets in flight per wave
+constexpr int CONV_DEPTH = 2;   // operand sets in flight per wave (3: 1-8 % slower, 4: 2-10 %)
 constexpr uint32_t W_OOB = 0x40000000u;   // beyond any kernel (conv_fits), alone and added to itself
+
+// Kernels of one tap; of several, each at least the 16 k of a step long; of several shorter ones.
+enum ConvTaps { TAPS_ONE = 0, TAPS_WIDE = 1, TAPS_NARROW = 2 };
 
 struct ConvKernelArgs {
     ConvArgs c;
@@ -64,19 +68,19 @@ __device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& sca
 // GRAD: the gradient of a convolution's input.  The same product with the kernel turned around, w [K, kh, kw, C] (n, then
 // k: a lane's four k are one 16-byte load of w, too); the epilogue masks the result where the ReLU did and adds up what
 // the batch norm's gradient needs, in fp32 over 16 pixels and in double from there on.
-template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS, bool GRAD>
-__global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKernelArgs a)
+template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD>
+__global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
 {
-    constexpr int WAVES = WK > 4 ? WK : 4, WP = WAVES / WK;
-    constexpr int TP = 16 * FP * WP, TN = 16 * FN;
+    constexpr int WAVES = 4, WP = WAVES / WK;
+    constexpr int TP = 16 * WP, TN = 16 * FN;
     extern __shared__ float lds[];
     const uint32_t cPad = PRE ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
     float* const preScale = lds;
     float* const preShift = lds + cPad;
     float* const postScale = lds + 2 * cPad;
     float* const postShift = postScale + TN;
-    double* const sums = reinterpret_cast<double*>(postScale + 2 * TN);   // [WP * FP][TN][2], GRAD only
-    float* const red = postScale + (GRAD ? 2 + 4 * WP * FP : 2) * TN;     // [WP][WK][FP * FN][64] x 4, WK > 1 only
+    double* const sums = reinterpret_cast<double*>(postScale + 2 * TN);   // [WP][TN][2], GRAD only
+    float* const red = postScale + (GRAD ? 2 + 4 * WP : 2) * TN;     // [WP][WK][FN][64] x 4, WK > 1 only
 
     // Eight consecutive workgroups go to eight XCDs; the tiles of one pixel range that differ in channels only follow
     // each other on one XCD, whose L2 then holds the pixels once.
@@ -87,109 +91,137 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     if (tp * TP >= rows) return;   // (the whole workgroup)
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, quad = lane >> 4;
-    const uint32_t wave = tid >> 6, wk = wave % WK, wp = wave / WK;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), wk = wave % WK, wp = wave / WK;
     const uint32_t n0 = tn * TN;
     const bool post = a.c.post.gamma != nullptr;
 
-    // The wave's pixels: one per lane and fragment, the same for the four quads.
-    int h[FP], w[FP];
-    uint32_t base[FP];   // byte offset of channel 0 of the pixel under tap (0, 0)
-#pragma unroll
-    for (int f = 0; f < FP; ++f) {
-        const uint32_t row = tp * TP + (wp * FP + f) * 16 + l16;
+    // The wave's pixels: one per lane, the same for the four quads.
+    int h0, w0;
+    uint32_t base;   // byte offset of channel 0 of the pixel under tap (0, 0)
+    {
+        const uint32_t row = tp * TP + wp * 16 + l16;
         bool ok = row < rows;
         const uint32_t ib = fdiv(ok ? row : 0u, a.dP), p = (ok ? row : 0u) - ib * a.P;
         const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
         int n = (int)ib;
-        h[f] = (int)r;
-        w[f] = (int)s;
+        h0 = (int)r;
+        w0 = (int)s;
         if (a.c.idx) {
             const int16_t* t = a.c.idx + (size_t)ib * 3;
             n = t[0];
-            h[f] += a.c.oh + t[1] * a.c.U;
-            w[f] += a.c.ow + t[2] * a.c.V;
+            h0 += a.c.oh + t[1] * a.c.U;
+            w0 += a.c.ow + t[2] * a.c.V;
             ok = ok && (unsigned)n < (unsigned)a.c.N;
         }
-        base[f] = (((uint32_t)n * (uint32_t)a.c.H + (uint32_t)h[f]) * (uint32_t)a.c.W + (uint32_t)w[f]) * (uint32_t)a.c.C * 4u;
-        if (!ok) h[f] = -0x40000000;   // outside the image under every tap
+        base = (((uint32_t)n * (uint32_t)a.c.H + (uint32_t)h0) * (uint32_t)a.c.W + (uint32_t)w0) * (uint32_t)a.c.C * 4u;
+        if (!ok) h0 = -0x40000000;   // outside the image under every tap
     }
 
-    const rsrc_t ra = make_rsrc(a.c.a, a.aBytes), rw = make_rsrc(a.c.w, a.wBytes);
+    const rsrc_t ra = make_rsrc(a.c.a, a.aBytes);
     const uint32_t per = (a.kSteps + WK - 1) / WK;
     const uint32_t sBeg = wk * per, sEnd = min(sBeg + per, a.kSteps);
-    const uint32_t kEnd = min(sEnd * 16u, a.kTot);
-    const uint32_t K = (uint32_t)a.c.K;
-    uint32_t wCol[FN];
+    const uint32_t K = (uint32_t)a.c.K, C = (uint32_t)a.c.C;
+
+    // Where the lane's k of the next step to load is: pixel, channel and byte offset, moved on by 16 k a step.  Found by
+    // division once: divisions and products per step cost more cycles than the matrix instructions.  Within a row of taps
+    // the input lies in the order of k (backwards in GRAD, tap by tap).
+    constexpr int DIR = GRAD ? -1 : 1, LANE_K = VEC == 4 ? 1 : 4;   // (four k share a tap, or each has its own)
+    struct Place {
+        uint32_t k, c, off;
+        int h, w;
+    } at[LANE_K];
 #pragma unroll
-    for (int f = 0; f < FN; ++f) {
-        const uint32_t n = n0 + f * 16 + l16;
-        wCol[f] = n < K ? n * (GRAD ? a.kTot : 1u) * 4u : W_OOB;
+    for (int j = 0; j < LANE_K; ++j) {
+        Place& t = at[j];
+        t.k = sBeg * 16u + quad * 4u + j;
+        const uint32_t tap = TAPS ? fdiv(t.k, a.dC) : 0u;
+        const int dr = TAPS ? (int)fdiv(tap, a.dKw) : 0, ds = (int)tap - dr * a.c.kw;
+        t.c = t.k - tap * C;
+        t.h = h0 + DIR * dr;
+        t.w = w0 + (TAPS ? DIR * ds : 0);
+        t.off = base + (TAPS ? (uint32_t)(DIR * (dr * a.c.W + ds)) * C * 4u : 0u) + t.c * 4u;
+    }
+    const int wEnd = w0 + DIR * a.c.kw;
+    const uint32_t tapStep = GRAD ? 0u - 2u * C * 4u : 0u;   // besides the 64 bytes of a step
+    const uint32_t rowStep = (uint32_t)(DIR * (a.c.W - a.c.kw)) * C * 4u;
+    const int wraps = TAPS == TAPS_NARROW ? (int)((15u + C) / C) : TAPS ? 1 : 0;   // taps a step can pass
+    const bool pixelOk = (unsigned)h0 < (unsigned)a.c.H && (unsigned)w0 < (unsigned)a.c.W;   // (of a single tap)
+
+    // Weights: the lane's offset inside the 16 k of a step; the step is in the descriptor.  Columns past the last channel
+    // read something or other for results that are not stored.
+    uint32_t wOff[GRAD ? FN : 4];
+    if constexpr (GRAD) {
+#pragma unroll
+        for (int f = 0; f < FN; ++f) wOff[f] = n0 + f * 16 + l16 < K ? ((n0 + f * 16 + l16) * a.kTot + quad * 4u) * 4u : W_OOB;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wOff[j] = ((quad * 4u + j) * K + n0 + l16) * 4u;
     }
 
     struct Operands {
-        acc_t px[FP];
+        acc_t px;
         float wv[FN][4];
-        uint32_t c[VEC == 4 ? 1 : 4];   // input channel of the lane's k (its first, where four share a tap)
+        uint32_t c[PRE ? LANE_K : 1];   // input channel of the lane's k (its first, where four share a tap)
     };
 
-    // Loads of a step: out-of-range k, channels, rows and pixels get an offset outside the descriptor and read as 0.
-    // All by selects: written with && the compiler branches around each load and waits inside the branch.
+    // Loads of a step: out-of-range k, channels, rows and pixels get an offset outside the descriptor and read as 0; steps
+    // past the wave's last get empty descriptors.  All by selects: written with && the compiler branches around each load
+    // and waits inside the branch.
     auto load = [&](uint32_t step, Operands& o) {
-        const uint32_t k = step * 16u + quad * 4u;
+        const bool run = step < sEnd;   // (wave-uniform)
+        const uint32_t first = step * 16u * (GRAD ? 1u : K) * 4u;
+        const rsrc_t rw = make_rsrc(reinterpret_cast<const char*>(a.c.w) + (run ? first : 0u), run ? a.wBytes - first : 0u);
 #pragma unroll
-        for (int j = 0; j < (VEC == 4 ? 1 : 4); ++j) {
-            const uint32_t kj = k + j;
-            uint32_t c = kj;
-            int dr = 0, ds = 0;
-            if constexpr (TAPS) {
-                const uint32_t tap = fdiv(kj, a.dC);
-                c = kj - tap * (uint32_t)a.c.C;
-                dr = (int)fdiv(tap, a.dKw);
-                ds = (int)tap - dr * a.c.kw;
-            } else {
-                c = min(c, (uint32_t)a.c.C - (VEC == 4 ? 4u : 1u));   // (a channel to look scale and shift up for, past the end)
-            }
-            o.c[j] = c;
+        for (int j = 0; j < LANE_K; ++j) {
+            Place& t = at[j];
+            uint32_t bad = (uint32_t)(t.k >= a.kTot) | (uint32_t)!run;
             if constexpr (GRAD) {
-                const uint32_t row = kj < kEnd ? kj * 4u : W_OOB;
 #pragma unroll
                 for (int f = 0; f < FN; ++f) {
-                    const f4 t = buf_load<4>(rw, row + wCol[f]);
+                    const f4 v = buf_load<4>(rw, wOff[f] | (0u - (uint32_t)(t.k >= a.kTot)));
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) o.wv[f][i] = t[i];
+                    for (int i = 0; i < 4; ++i) o.wv[f][i] = v[i];
                 }
-                dr = -dr;   // (the output pixel that this tap took the input pixel to)
-                ds = -ds;
             }
-            const uint32_t toff = (((uint32_t)dr * (uint32_t)a.c.W + (uint32_t)ds) * (uint32_t)a.c.C + c) * 4u;
-#pragma unroll
-            for (int f = 0; f < FP; ++f) {
-                const uint32_t bad = (uint32_t)((unsigned)(h[f] + dr) >= (unsigned)a.c.H) |
-                                     (uint32_t)((unsigned)(w[f] + ds) >= (unsigned)a.c.W) | (uint32_t)(kj >= kEnd);
-                const uint32_t off = (base[f] + toff) | (0u - bad);
-                if constexpr (VEC == 4) o.px[f] = buf_load<4>(ra, off);
-                else o.px[f][j] = buf_load<1>(ra, off);
+            if constexpr (PRE) o.c[j] = TAPS ? t.c : min(t.c, C - (VEC == 4 ? 4u : 1u));   // (scale and shift of some channel, past the end)
+            if constexpr (TAPS) bad |= (uint32_t)((unsigned)t.h >= (unsigned)a.c.H) | (uint32_t)((unsigned)t.w >= (unsigned)a.c.W);
+            else bad |= (uint32_t)!pixelOk;
+            const uint32_t off = t.off | (0u - bad);
+            if constexpr (VEC == 4) o.px = buf_load<4>(ra, off);
+            else o.px[j] = buf_load<1>(ra, off);
+            t.k += 16u;
+            t.c += 16u;
+            t.off += 64u;
+            for (int i = 0; i < wraps; ++i) {
+                const bool next = t.c >= C;
+                t.c -= next ? C : 0u;
+                t.w += next ? DIR : 0;
+                if constexpr (GRAD) t.off += next ? tapStep : 0u;
+                const bool turn = t.w == wEnd;
+                t.w = turn ? w0 : t.w;
+                t.h += turn ? DIR : 0;
+                t.off += turn ? rowStep : 0u;
             }
         }
         if constexpr (!GRAD) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t row = (k + j < kEnd) ? (k + j) * K * 4u : W_OOB;
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int f = 0; f < FN; ++f) o.wv[f][j] = buf_load<1>(rw, row + wCol[f]);
-            }
+                for (int f = 0; f < FN; ++f) o.wv[f][j] = buf_load<1>(rw, wOff[j] + f * 64u);
         }
     };
 
-    acc_t acc[FN][FP];
+    acc_t acc[FN];
 #pragma unroll
-    for (int i = 0; i < FN; ++i)
-#pragma unroll
-        for (int f = 0; f < FP; ++f) acc[i][f] = (acc_t)(0.f);
+    for (int i = 0; i < FN; ++i) acc[i] = (acc_t)(0.f);
 
     Operands ops[CONV_DEPTH];
 #pragma unroll
-    for (int d = 0; d < CONV_DEPTH; ++d) load(sBeg + d, ops[d]);
+    for (int d = 0; d < CONV_DEPTH; ++d) {
+        load(sBeg + d, ops[d]);
+        // (in this order: shuffled, the waits of the loop would be for the set that was loaded last)
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
     if (PRE)
         for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_fold(a.c.pre, c, preScale[c], preShift[c]);
@@ -205,44 +237,47 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
     }
     if (PRE || GRAD || post) lds_barrier();
 
-    for (uint32_t step = sBeg; step < sEnd; step += CONV_DEPTH) {
+    auto multiply = [&](Operands& o) {
+        if constexpr (PRE) {
+            acc_t sc, sh;
+            if constexpr (VEC == 4) {
+                sc = lds_read4(preScale + o.c[0]);
+                sh = lds_read4(preShift + o.c[0]);
+            } else {
 #pragma unroll
-        for (int d = 0; d < CONV_DEPTH; ++d) {
-            if (d && step + d >= sEnd) break;   // (wave-uniform; a round of multiplying zeros would cost as much as a full one)
-            Operands& o = ops[d];
-            if constexpr (PRE) {
-                acc_t sc, sh;
-                if constexpr (VEC == 4) {
-                    sc = lds_read4(preScale + o.c[0]);
-                    sh = lds_read4(preShift + o.c[0]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        sc[j] = preScale[o.c[j]];
-                        sh[j] = preShift[o.c[j]];
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    sc[j] = preScale[o.c[j]];
+                    sh[j] = preShift[o.c[j]];
                 }
-#pragma unroll
-                for (int f = 0; f < FP; ++f)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) o.px[f][j] = relu_keep_nan(o.px[f][j] * sc[j] + sh[j]);
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 4; ++j) o.px[j] = relu_keep_nan(o.px[j] * sc[j] + sh[j]);
+        }
 #pragma unroll
-                for (int i = 0; i < FN; ++i)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int f = 0; f < FP; ++f)
-                        acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.wv[i][j], o.px[f][j], acc[i][f], 0, 0, 0);
-            load(step + d + CONV_DEPTH, o);   // past the wave's last step: all out of range, no traffic
+            for (int i = 0; i < FN; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.wv[i][j], o.px[j], acc[i], 0, 0, 0);
+    };
+    // Whole rounds without a way out, then what is left.  With an exit inside a round the compiler waits for all loads at
+    // the head of the loop, or moves a round's loads to its end: either way nothing stays in flight.
+    uint32_t step = sBeg;
+    for (; step + CONV_DEPTH <= sEnd; step += CONV_DEPTH) {
+#pragma unroll
+        for (int d = 0; d < CONV_DEPTH; ++d) {
+            multiply(ops[d]);
+            load(step + d + CONV_DEPTH, ops[d]);   // past the wave's last step: all out of range, no traffic
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+#pragma unroll
+    for (int d = 0; d < CONV_DEPTH - 1; ++d)
+        if (step + d < sEnd) multiply(ops[d]);   // (wave-uniform)
 
     const rsrc_t ry = make_rsrc(a.c.y, a.yBytes);
-    auto finish = [&](int i, int f, acc_t v) {
+    auto finish = [&](int i, acc_t v) {
         const uint32_t nl = i * 16 + quad * 4, n = n0 + nl;
         if constexpr (GRAD) {
-            const uint32_t group = wp * FP + f, row = tp * TP + group * 16 + l16;
+            const uint32_t row = tp * TP + wp * 16 + l16;
             const uint32_t o = row < rows && n < K ? (row * K + n) * 4u : BUF_OOB;
             const acc_t z = (acc_t)buf_load<4>(make_rsrc(a.c.norm.z, a.yBytes), o);
             const acc_t act = (acc_t)buf_load<4>(make_rsrc(a.c.norm.act, a.yBytes), o);   // (0 past the end: masked)
@@ -264,8 +299,8 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
             if (l16 == 0)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    sums[(group * TN + nl + j) * 2] = s1[j];
-                    sums[(group * TN + nl + j) * 2 + 1] = s2[j];
+                    sums[(wp * TN + nl + j) * 2] = s1[j];
+                    sums[(wp * TN + nl + j) * 2 + 1] = s2[j];
                 }
             return;
         }
@@ -273,7 +308,7 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan(v[j] * postScale[nl + j] + postShift[nl + j]);
         }
-        const uint32_t row = tp * TP + (wp * FP + f) * 16 + l16;
+        const uint32_t row = tp * TP + wp * 16 + l16;
         bool ok = row < rows;
         uint32_t pix = row;
         if (a.c.oidx) {
@@ -302,24 +337,18 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
 
     if constexpr (WK == 1) {
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
-#pragma unroll
-            for (int f = 0; f < FP; ++f) finish(i, f, acc[i][f]);
+        for (int i = 0; i < FN; ++i) finish(i, acc[i]);
     } else {
 #pragma unroll
-        for (int i = 0; i < FN; ++i)
-#pragma unroll
-            for (int f = 0; f < FP; ++f)
-                *reinterpret_cast<acc_t*>(red + (((wp * WK + wk) * (FP * FN) + i * FP + f) * 64 + lane) * 4) = acc[i][f];
+        for (int i = 0; i < FN; ++i) *reinterpret_cast<acc_t*>(red + (((wp * WK + wk) * FN + i) * 64 + lane) * 4) = acc[i];
         lds_barrier();
 #pragma unroll
-        for (int q = 0; q < FP * FN; ++q) {
-            if (q % WK != (int)wk) continue;   // (wave-uniform)
+        for (int i = 0; i < FN; ++i) {
+            if (i % WK != (int)wk) continue;   // (wave-uniform)
             acc_t v = (acc_t)(0.f);
 #pragma unroll
-            for (int k = 0; k < WK; ++k)
-                v += (acc_t)lds_read4(red + (((wp * WK + k) * (FP * FN) + q) * 64 + lane) * 4);
-            finish(q / FP, q % FP, v);
+            for (int k = 0; k < WK; ++k) v += (acc_t)lds_read4(red + (((wp * WK + k) * FN + i) * 64 + lane) * 4);
+            finish(i, v);
         }
     }
 
@@ -329,32 +358,38 @@ __global__ __launch_bounds__(WK > 4 ? 64 * WK : 256) void k_block_conv(ConvKerne
         for (uint32_t i = tid; i < 2u * TN; i += 64 * WAVES) {
             double s = 0.0;
 #pragma unroll
-            for (int k = 0; k < WP * FP; ++k) s += sums[k * TN * 2 + i];
+            for (int k = 0; k < WP; ++k) s += sums[k * TN * 2 + i];
             if (n0 + (i >> 1) < K)
                 unsafeAtomicAdd(a.c.norm.sums + ((size_t)(blockIdx.x & (GRAD_SLOTS - 1)) * K + n0) * 2 + i, s);
         }
     }
 }
 
-template <int FP, int FN, int WK, int VEC, bool PRE, bool TAPS, bool GRAD = false>
+template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD = false>
 static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
 {
-    constexpr int WAVES = WK > 4 ? WK : 4, TP = 16 * FP * (WAVES / WK), TN = 16 * FN;
+    constexpr int WAVES = 4, TP = 16 * (WAVES / WK), TN = 16 * FN;
     a.tilesP = (a.rows + TP - 1) / TP;
     a.tilesN = ((uint32_t)a.c.K + TN - 1) / TN;
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
-    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * FP * (WAVES / WK) : 2) * TN + (WK > 1 ? (size_t)WAVES * FP * FN * 256 : 0));
+    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 2) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_block_conv<FP, FN, WK, VEC, PRE, TAPS, GRAD>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
+    hipLaunchKernelGGL((k_block_conv<FN, WK, VEC, PRE, TAPS, GRAD>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();
 }
 
-template <int FP, int FN, int WK, int VEC>
+template <int FN, int WK, int VEC, bool PRE, bool GRAD>
+static hipError_t launch_conv_taps(ConvKernelArgs& a, hipStream_t stream)
+{
+    if (a.c.kh * a.c.kw == 1) return launch_conv_as<FN, WK, VEC, PRE, TAPS_ONE, GRAD>(a, stream);
+    if (a.c.C >= 16) return launch_conv_as<FN, WK, VEC, PRE, TAPS_WIDE, GRAD>(a, stream);
+    return launch_conv_as<FN, WK, VEC, PRE, TAPS_NARROW, GRAD>(a, stream);
+}
+
+template <int FN, int WK, int VEC>
 static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
 {
-    const bool taps = a.c.kh * a.c.kw > 1;
-    if (a.c.pre.gamma) return taps ? launch_conv_as<FP, FN, WK, VEC, true, true>(a, stream) : launch_conv_as<FP, FN, WK, VEC, true, false>(a, stream);
-    return taps ? launch_conv_as<FP, FN, WK, VEC, false, true>(a, stream) : launch_conv_as<FP, FN, WK, VEC, false, false>(a, stream);
+    return a.c.pre.gamma ? launch_conv_taps<FN, WK, VEC, true, false>(a, stream) : launch_conv_taps<FN, WK, VEC, false, false>(a, stream);
 }
 
 bool conv_fits(const ConvArgs& c)
@@ -391,9 +426,8 @@ static void conv_tile(const ConvKernelArgs& a, bool vec, int& fn, int& wk)
     // Narrow wave tiles (16 pixels x 32 channels; 48 where that leaves no channel over, 16 where there are no more) and as
     // many waves per tile as it takes to occupy the SIMDs: a launch of fewer than about 1500 waves is four times shorter
     // with k split four ways than its occupancy would suggest, and one with few steps per wave has nothing to split.
-    // Wider tiles read less and wait more: 32x32 is 10-40 % slower on all but the narrowest and largest problems (us for
-    // 16x32 / 32x32, best split: 2450 pixels, k 1152, 128 channels 16.4 / 19.0; 4860, 576, 64: 10.3 / 12.0; 45 000, 216, 24:
-    // 13.2 / 12.6; 38 400, 600, 24: 24.7 / 22.7).
+    // Tiles of 64 channels are no faster (us for 32 / 64: 2350 pixels, k 1152, 128 channels 13.5 / 14.9; 3850, 512, 128:
+    // 12.4 / 11.7; 2350, 128, 512: 8.7 / 9.0), of 16 slower (17.6; 16.4; 10.1), for all that splits.
     const uint32_t nFrag = ((uint32_t)a.c.K + 15) / 16;
     fn = nFrag == 1 ? 1 : (vec && nFrag % 3 == 0 && nFrag % 2 == 1 ? 3 : 2);
     const uint64_t waves = (uint64_t)((a.rows + 15) / 16) * ((nFrag + fn - 1) / fn);
@@ -409,27 +443,20 @@ hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
     int fn, wk;
     conv_tile(a, vec, fn, wk);
     if (!vec) {
-        if (fn == 1) return wk > 1 ? launch_conv_one<1, 1, 4, 1>(a, stream) : launch_conv_one<1, 1, 1, 1>(a, stream);
-        return wk > 1 ? launch_conv_one<1, 2, 4, 1>(a, stream) : launch_conv_one<1, 2, 1, 1>(a, stream);
+        if (fn == 1) return wk > 1 ? launch_conv_one<1, 4, 1>(a, stream) : launch_conv_one<1, 1, 1>(a, stream);
+        return wk > 1 ? launch_conv_one<2, 4, 1>(a, stream) : launch_conv_one<2, 1, 1>(a, stream);
     }
     switch (fn * 8 + wk) {
-    case 8 + 1: return launch_conv_one<1, 1, 1, 4>(a, stream);
-    case 8 + 2: return launch_conv_one<1, 1, 2, 4>(a, stream);
-    case 8 + 4: return launch_conv_one<1, 1, 4, 4>(a, stream);
-    case 16 + 1: return launch_conv_one<1, 2, 1, 4>(a, stream);
-    case 16 + 2: return launch_conv_one<1, 2, 2, 4>(a, stream);
-    case 16 + 4: return launch_conv_one<1, 2, 4, 4>(a, stream);
-    case 24 + 1: return launch_conv_one<1, 3, 1, 4>(a, stream);
-    case 24 + 2: return launch_conv_one<1, 3, 2, 4>(a, stream);
-    default: return launch_conv_one<1, 3, 4, 4>(a, stream);
+    case 8 + 1: return launch_conv_one<1, 1, 4>(a, stream);
+    case 8 + 2: return launch_conv_one<1, 2, 4>(a, stream);
+    case 8 + 4: return launch_conv_one<1, 4, 4>(a, stream);
+    case 16 + 1: return launch_conv_one<2, 1, 4>(a, stream);
+    case 16 + 2: return launch_conv_one<2, 2, 4>(a, stream);
+    case 16 + 4: return launch_conv_one<2, 4, 4>(a, stream);
+    case 24 + 1: return launch_conv_one<3, 1, 4>(a, stream);
+    case 24 + 2: return launch_conv_one<3, 2, 4>(a, stream);
+    default: return launch_conv_one<3, 4, 4>(a, stream);
     }
-}
-
-template <int FN, int WK>
-static hipError_t launch_conv_grad_one(ConvKernelArgs& a, hipStream_t stream)
-{
-    if (a.c.kh * a.c.kw > 1) return launch_conv_as<1, FN, WK, 4, false, true, true>(a, stream);
-    return launch_conv_as<1, FN, WK, 4, false, false, true>(a, stream);
 }
 
 bool conv_grad_fits(const ConvArgs& c)
@@ -448,15 +475,15 @@ hipError_t launch_block_conv_grad(const ConvArgs& c, hipStream_t stream)
     int fn, wk;
     conv_tile(a, true, fn, wk);
     switch (fn * 8 + wk) {
-    case 8 + 1: return launch_conv_grad_one<1, 1>(a, stream);
-    case 8 + 2: return launch_conv_grad_one<1, 2>(a, stream);
-    case 8 + 4: return launch_conv_grad_one<1, 4>(a, stream);
-    case 16 + 1: return launch_conv_grad_one<2, 1>(a, stream);
-    case 16 + 2: return launch_conv_grad_one<2, 2>(a, stream);
-    case 16 + 4: return launch_conv_grad_one<2, 4>(a, stream);
-    case 24 + 1: return launch_conv_grad_one<3, 1>(a, stream);
-    case 24 + 2: return launch_conv_grad_one<3, 2>(a, stream);
-    default: return launch_conv_grad_one<3, 4>(a, stream);
+    case 8 + 1: return launch_conv_taps<1, 1, 4, false, true>(a, stream);
+    case 8 + 2: return launch_conv_taps<1, 2, 4, false, true>(a, stream);
+    case 8 + 4: return launch_conv_taps<1, 4, 4, false, true>(a, stream);
+    case 16 + 1: return launch_conv_taps<2, 1, 4, false, true>(a, stream);
+    case 16 + 2: return launch_conv_taps<2, 2, 4, false, true>(a, stream);
+    case 16 + 4: return launch_conv_taps<2, 4, 4, false, true>(a, stream);
+    case 24 + 1: return launch_conv_taps<3, 1, 4, false, true>(a, stream);
+    case 24 + 2: return launch_conv_taps<3, 2, 4, false, true>(a, stream);
+    default: return launch_conv_taps<3, 4, 4, false, true>(a, stream);
     }
 }
 
