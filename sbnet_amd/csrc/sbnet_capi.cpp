@@ -724,7 +724,11 @@ int sbnet_block_bottleneck(const float* x, const int64_t* x_dims, int32_t num_ac
     } else {
         c[2].y = q;
     }
-    for (int i = 0; i < 3; ++i) SBNET_HIP(sbnet::launch_block_conv(c[i], static_cast<hipStream_t>(stream)));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    SBNET_HIP(sbnet::launch_block_conv(c[0], s));
+    bool done = false;
+    SBNET_HIP(sbnet::launch_block_conv_next(c[1], c[2], s, done));
+    for (int i = 1; i < 3 && !done; ++i) SBNET_HIP(sbnet::launch_block_conv(c[i], s));
     return SBNET_OK;
 }
 

@@ -50,6 +50,11 @@ struct ConvArgs {
 bool conv_fits(const ConvArgs& c);
 hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream);
 
+// c and, on its result, the 1x1 convolution `next` (whose input is not looked at) in one launch; `done` is false, and nothing
+// launched, where that does not apply: c must be larger than 1x1, with 16 input channels or more, 128 output channels or
+// fewer and all channels multiples of four.
+hipError_t launch_block_conv_next(const ConvArgs& c, const ConvArgs& next, hipStream_t stream, bool& done);
+
 // Gradient of a convolution's input on block stacks, masked by the ReLU in front of it: a is the gradient of the output
 // [M,H,W,C], w [K,kh,kw,C] the convolution's kernel, y [M,Ro,So,K] the result (Ro = H + kh - 1, So = W + kw - 1); adds to
 // norm.sums.  Channels multiples of four, pointers 16-byte aligned (conv_grad_fits).

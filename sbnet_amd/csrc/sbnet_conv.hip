@@ -31,7 +31,7 @@ namespace sbnet {
 // rate of a large fp32 product): 15.7 us; 20.5 us with an exit inside a round of the loop and places found by division, 27 us
 // while the loads of a step sat behind branches; the library convolution took 21 us behind 5 us of layout copies, and up
 // to 800 us the first time a block count occurred.  A bottleneck block of 200 17x17x96 blocks: 33 us in three launches
-// against about 300 us in 17.
+// against about 300 us in 17 (31 us in two with NEXT, below).
 //
 // WK > 1: the WK waves of a workgroup split k among them and add up through LDS.  For launches whose tiles alone would
 // leave most of the 1024 SIMDs idle.
@@ -54,6 +54,9 @@ struct ConvKernelArgs {
     uint32_t rows, P;           // output pixels in all, per block
     uint32_t tilesP, tilesN;
     uint32_t aBytes, wBytes, yBytes;
+    const float* w2;            // NEXT: the second kernel [K, K2]
+    int K2;
+    uint32_t w2Bytes;
 };
 
 __device__ __forceinline__ float relu_keep_nan(float v) { return v < 0.f ? 0.f : v; }
@@ -68,7 +71,13 @@ __device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& sca
 // GRAD: the gradient of a convolution's input.  The same product with the kernel turned around, w [K, kh, kw, C] (n, then
 // k: a lane's four k are one 16-byte load of w, too); the epilogue masks the result where the ReLU did and adds up what
 // the batch norm's gradient needs, in fp32 over 16 pixels and in double from there on.
-template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD>
+//
+// NEXT: a 1x1 convolution on top, on the workgroup's own pixels, before anything is written: the result of the first is
+// laid out as the matrix instructions want their input (a lane holds channels 16 * i + 4 * quad + 0..3 of its pixel, the
+// four k of step i) and stays in registers.  All its channels are in one tile.
+// Saves a launch, the stack in between and the second kernel's start: the 3x3 and the last 1x1 of a bottleneck on 200
+// 17x17x96 blocks, 24 channels in between, take 20.1 us; 22.5 us one after the other (MI355X, kernel trace).
+template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD, bool NEXT>
 __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
 {
     constexpr int WAVES = 4, WP = WAVES / WK;
@@ -115,6 +124,18 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
         }
         base = (((uint32_t)n * (uint32_t)a.c.H + (uint32_t)h0) * (uint32_t)a.c.W + (uint32_t)w0) * (uint32_t)a.c.C * 4u;
         if (!ok) h0 = -0x40000000;   // outside the image under every tap
+    }
+
+    // Where the lane's pixel goes (the list is read here, not behind the products).
+    bool outOk = tp * TP + wp * 16 + l16 < rows;
+    uint32_t outPix = tp * TP + wp * 16 + l16;
+    if (!GRAD && a.c.oidx) {
+        const uint32_t row = outOk ? outPix : 0u, ib = fdiv(row, a.dP), p = row - ib * a.P;
+        const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
+        const int16_t* t = a.c.oidx + (size_t)ib * 3;
+        const int on = t[0], oh = t[1] * a.c.oU + (int)r, ow = t[2] * a.c.oV + (int)s;
+        outOk = outOk && (unsigned)on < (unsigned)a.c.oN && (unsigned)oh < (unsigned)a.c.oH && (unsigned)ow < (unsigned)a.c.oW;
+        outPix = ((uint32_t)on * (uint32_t)a.c.oH + (uint32_t)oh) * (uint32_t)a.c.oW + (uint32_t)ow;
     }
 
     const rsrc_t ra = make_rsrc(a.c.a, a.aBytes);
@@ -274,6 +295,23 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
         if (step + d < sEnd) multiply(ops[d]);   // (wave-uniform)
 
     const rsrc_t ry = make_rsrc(a.c.y, a.yBytes);
+    // Four channels from n on of the lane's pixel.
+    auto emit = [&](uint32_t n, uint32_t channels, acc_t v) {
+        const uint32_t off = (outPix * channels + n) * 4u;
+        if constexpr (VEC == 4) {
+            const uint32_t o = outOk && n < channels ? off : BUF_OOB;   // channels are a multiple of 4 here
+            if (!NEXT && a.c.add) v += buf_load<4>(ry, o);
+            buf_store<0>(ry, o, (f4)v);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t o = outOk && n + j < channels ? off + 4u * j : BUF_OOB;
+                float t = v[j];
+                if (a.c.add) t += buf_load<1>(ry, o);
+                buf_store<0>(ry, o, t);
+            }
+        }
+    };
     auto finish = [&](int i, acc_t v) {
         const uint32_t nl = i * 16 + quad * 4, n = n0 + nl;
         if constexpr (GRAD) {
@@ -308,34 +346,52 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan(v[j] * postScale[nl + j] + postShift[nl + j]);
         }
-        const uint32_t row = tp * TP + wp * 16 + l16;
-        bool ok = row < rows;
-        uint32_t pix = row;
-        if (a.c.oidx) {
-            const uint32_t ib = fdiv(ok ? row : 0u, a.dP), p = (ok ? row : 0u) - ib * a.P;
-            const uint32_t r = fdiv(p, a.dSo), s = p - r * (uint32_t)a.c.So;
-            const int16_t* t = a.c.oidx + (size_t)ib * 3;
-            const int on = t[0], oh = t[1] * a.c.oU + (int)r, ow = t[2] * a.c.oV + (int)s;
-            ok = ok && (unsigned)on < (unsigned)a.c.oN && (unsigned)oh < (unsigned)a.c.oH && (unsigned)ow < (unsigned)a.c.oW;
-            pix = ((uint32_t)on * (uint32_t)a.c.oH + (uint32_t)oh) * (uint32_t)a.c.oW + (uint32_t)ow;
-        }
-        const uint32_t off = (pix * K + n) * 4u;
-        if constexpr (VEC == 4) {
-            const uint32_t o = ok && n < K ? off : BUF_OOB;   // K is a multiple of 4 here
-            if (a.c.add) v += buf_load<4>(ry, o);
-            buf_store<0>(ry, o, (f4)v);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t o = ok && n + j < K ? off + 4u * j : BUF_OOB;
-                float t = v[j];
-                if (a.c.add) t += buf_load<1>(ry, o);
-                buf_store<0>(ry, o, t);
-            }
-        }
+        emit(n, K, v);
     };
 
-    if constexpr (WK == 1) {
+    if constexpr (NEXT) {
+        auto between = [&](int i, acc_t v) {   // (columns past the last channel hold something or other: cleared)
+            const uint32_t nl = i * 16 + quad * 4;
+            const acc_t sc = lds_read4(postScale + nl), sh = lds_read4(postShift + nl);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = nl < K ? (post ? relu_keep_nan(v[j] * sc[j] + sh[j]) : v[j]) : 0.f;
+            return v;
+        };
+#pragma unroll
+        for (int i = 0; i < FN; ++i) acc[i] = between(i, acc[i]);
+        const uint32_t K2 = (uint32_t)a.K2;
+        const rsrc_t rw2 = make_rsrc(a.w2, a.w2Bytes);
+        constexpr int FO = 4;
+        for (uint32_t t0 = 0; t0 < K2; t0 += 16u * FO) {
+            float wv[2][4][FO];
+            auto fetch = [&](int i) {   // (rows past the last channel read as zeros)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int f = 0; f < FO; ++f)
+                        wv[i & 1][j][f] = buf_load<1>(rw2, ((i * 16u + quad * 4u + j) * K2 + t0 + l16) * 4u + f * 64u);
+            };
+            acc_t out[FO], y[FO];   // (y: what the result is added to, loaded ahead of the products)
+#pragma unroll
+            for (int f = 0; f < FO; ++f) {
+                const uint32_t n = t0 + f * 16u + quad * 4u;
+                out[f] = (acc_t)(0.f);
+                y[f] = buf_load<4>(ry, a.c.add && outOk && n < K2 ? (outPix * K2 + n) * 4u : BUF_OOB);
+            }
+            fetch(0);
+#pragma unroll
+            for (int i = 0; i < FN; ++i) {
+                if (i + 1 < FN) fetch(i + 1);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int f = 0; f < FO; ++f)
+                        out[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i & 1][j][f], acc[i][j], out[f], 0, 0, 0);
+            }
+#pragma unroll
+            for (int f = 0; f < FO; ++f) emit(t0 + f * 16u + quad * 4u, K2, out[f] + y[f]);
+        }
+    } else if constexpr (WK == 1) {
 #pragma unroll
         for (int i = 0; i < FN; ++i) finish(i, acc[i]);
     } else {
@@ -365,7 +421,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     }
 }
 
-template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD = false>
+template <int FN, int WK, int VEC, bool PRE, int TAPS, bool GRAD = false, bool NEXT = false>
 static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
 {
     constexpr int WAVES = 4, TP = 16 * (WAVES / WK), TN = 16 * FN;
@@ -374,7 +430,7 @@ static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
     const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 2) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_block_conv<FN, WK, VEC, PRE, TAPS, GRAD>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
+    hipLaunchKernelGGL((k_block_conv<FN, WK, VEC, PRE, TAPS, GRAD, NEXT>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();
 }
 
@@ -456,6 +512,38 @@ hipError_t launch_block_conv(const ConvArgs& c, hipStream_t stream)
     case 24 + 1: return launch_conv_one<3, 1, 4>(a, stream);
     case 24 + 2: return launch_conv_one<3, 2, 4>(a, stream);
     default: return launch_conv_one<3, 4, 4>(a, stream);
+    }
+}
+
+hipError_t launch_block_conv_next(const ConvArgs& c, const ConvArgs& next, hipStream_t stream, bool& done)
+{
+    done = false;
+    if (c.M <= 0 || c.pre.gamma || next.pre.gamma || next.post.gamma || next.kh != 1 || next.kw != 1 || c.kh * c.kw == 1 ||
+        c.C < 16 || c.K > 128 || next.C != c.K || next.K % 4 != 0 || !conv_fits(c) || !conv_fits(next))
+        return hipSuccess;
+    ConvArgs both = c;   // input and kernel of the first, output of the second
+    both.y = next.y;
+    both.oidx = next.oidx;
+    both.oN = next.oN; both.oH = next.oH; both.oW = next.oW; both.oU = next.oU; both.oV = next.oV;
+    both.add = next.add;
+    ConvKernelArgs a;
+    if (!make_conv_args(both, a)) return hipSuccess;
+    a.yBytes = (uint32_t)((next.oidx ? (uint64_t)next.oN * next.oH * next.oW : (uint64_t)a.rows) * next.K * 4);
+    a.w2 = next.w;
+    a.K2 = next.K;
+    a.w2Bytes = (uint32_t)(next.C * next.K * 4);
+    // A wave per 16 pixels and all channels: with fewer of them than SIMDs to fill, two launches that split further are
+    // faster (2350 pixels, 128 channels in between: 22.2 against 28 us, four waves to 16 pixels).
+    if ((a.rows + 15) / 16 < 1536) return hipSuccess;
+    done = true;
+    switch ((c.K + 15) / 16) {
+    case 1: return launch_conv_as<1, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
+    case 2: return launch_conv_as<2, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
+    case 3: return launch_conv_as<3, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
+    case 4: return launch_conv_as<4, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
+    case 5:
+    case 6: return launch_conv_as<6, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
+    default: return launch_conv_as<8, 1, 4, false, TAPS_WIDE, false, true>(a, stream);
     }
 }
 

@@ -124,3 +124,13 @@ def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
         most[n, bh * Ro:(bh + 1) * Ro, bw * So:(bw + 1) * So] = bound[i, :part.shape[0], :part.shape[1]] + U * part.abs()
     err = (y.cpu().double() - want).abs()
     assert bool((err <= most + 1e-30).all()), float((err / (most + 1e-30)).max())
+
+
+@pytest.mark.parametrize("use_var", [False, True])
+@pytest.mark.parametrize("C,mid,bsize,shape", [(40, 36, 9, (2, 33, 41)),       # three fragments in between, the last a quarter full
+                                               (132, 84, 11, (1, 60, 44)),     # six; output tiles of 64 channels and a rest
+                                               (64, 100, 8, (1, 40, 40)),      # seven of eight
+                                               (20, 132, 8, (1, 40, 40)),      # more than one tile: not in one launch
+                                               (64, 128, 24, (1, 180, 185))])  # eight, a wave for every 16 pixels
+def test_last_two_convolutions_in_one_launch(C, mid, bsize, shape, use_var):
+    test_bottleneck_in_inference(C, mid, bsize, shape, False, use_var)
