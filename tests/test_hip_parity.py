@@ -1315,3 +1315,14 @@ def test_flat_copy_of_any_length(n):
     src, dst = torch.randn(n + 8, device="cuda"), torch.full((n + 8,), 7.0, device="cuda")
     ops._check(ops._lib.load().sbnet_copy_tensor(dst.data_ptr(), src.data_ptr(), n, ops._stream()))
     assert torch.equal(dst[:n], src[:n]) and bool((dst[n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("avgpool", [False, True])
+@pytest.mark.parametrize("N,H,W,bsize,bstride,boffset", [
+    (64, 128, 128, (6, 6), (4, 4), (-1, -1)),    # 1089 counts, added up by each workgroup of the compaction
+    (1, 1020, 1028, (2, 2), (1, 1), (0, 0)),     # 4096
+    (1, 1021, 1028, (2, 2), (1, 1), (0, 0)),     # 4101: scanned
+])
+def test_reduce_mask_around_the_scan(N, H, W, bsize, bstride, boffset, avgpool):
+    mask = (np.random.default_rng(H).random((N, H, W, 1)) < 0.2).astype(np.float32)
+    check_reduce(mask, bcount_covering(H, W, bstride, boffset), bsize, bstride, boffset, 0.2, avgpool)
