@@ -10,6 +10,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
@@ -348,11 +349,12 @@ PyObject* scatter_base_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
     });
 }
 
-// Contiguous, on the GPU, float32, with no gradient asked for.
+// Contiguous, on the GPU, float32, with no gradient asked for, and not under autocast, where the layers' convolutions
+// would compute in another type.
 const at::Tensor* plain_f32(PyObject* o)
 {
     const at::Tensor* t = dev_f32(o);
-    return t && !(t->requires_grad() && at::GradMode::is_enabled()) ? t : nullptr;
+    return t && !at::autocast::is_autocast_enabled(at::kCUDA) && !(t->requires_grad() && at::GradMode::is_enabled()) ? t : nullptr;
 }
 
 constexpr int64_t CONV_MOST = 1ll << 28, ROWS_MOST = 1ll << 28;   // elements, output pixels: inside what the kernels take

@@ -134,3 +134,14 @@ def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
                                                (64, 128, 24, (1, 180, 185))])  # eight, a wave for every 16 pixels
 def test_last_two_convolutions_in_one_launch(C, mid, bsize, shape, use_var):
     test_bottleneck_in_inference(C, mid, bsize, shape, False, use_var)
+
+
+def test_layers_under_autocast_take_the_layers_own_way():
+    """Autocast makes the composed convolutions compute in half precision, which the scatter refuses: so does the layer."""
+    bp = sbnet_amd.calc_block_params([1, 20, 20, 16], [1, 8, 8, 1], [3, 3, 16, 16], [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(1, 20, 20, 1, device=DEV), bp, 0.0)
+    x, w = torch.randn(1, 20, 20, 16, device=DEV), torch.randn(3, 3, 16, 16, device=DEV)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16), pytest.raises(TypeError):
+        sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
+    with torch.no_grad():
+        sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
