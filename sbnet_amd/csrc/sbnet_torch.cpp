@@ -126,6 +126,14 @@ at::Tensor workspace(const at::Device& device, int64_t bytes)
     return ws;
 }
 
+// Scratch of one call, as the tensors between torch's operators are: for the layers, whose stacks are large, may belong to a
+// captured graph, and must not be shared with another thread that enqueues on the same stream.  Given back at the end of
+// the call, in the order of the stream.
+at::Tensor own_scratch(const at::Tensor& like, size_t bytes)
+{
+    return at::detail::empty_cuda({(int64_t)bytes}, at::kByte, like.device(), c10::nullopt);
+}
+
 // Runs a library call without the GIL, as ctypes does; raises on a status other than SBNET_OK.
 template <typename F>
 bool call(F f)
@@ -337,13 +345,12 @@ PyObject* scatter_base_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
     return guarded([&]() -> PyObject* {
         c10::DeviceGuard guard(g->device());
         at::Tensor d = empty_f32(g->sizes(), *g);
-        at::Tensor ws = workspace(g->device(), (int64_t)need);
+        at::Tensor ws = own_scratch(*g, need);
         const float* const gp = static_cast<const float*>(g->data_ptr());
         const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
         float* const dp = static_cast<float*>(d.data_ptr());
         void *const wp = ws.data_ptr(), *const stream = stream_of(*g);
-        const size_t wn = (size_t)ws.numel();
-        if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, wn, stream); }))
+        if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, need, stream); }))
             return nullptr;
         return THPVariable_Wrap(std::move(d));
     });
@@ -433,7 +440,7 @@ PyObject* block_bottleneck(PyObject*, PyObject* const* a, Py_ssize_t n)
     return guarded([&]() -> PyObject* {
         c10::DeviceGuard guard(x->device());
         at::Tensor q = in_place ? *x : empty_f32({b.M, R, S, C}, *x);
-        at::Tensor ws = workspace(x->device(), (int64_t)sbnet_block_bottleneck_workspace_bytes(b.M, bs.v, wd));
+        at::Tensor ws = own_scratch(*x, sbnet_block_bottleneck_workspace_bytes(b.M, bs.v, wd));
         const float* const xp = static_cast<const float*>(x->data_ptr());
         const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
         float* const qp = static_cast<float*>(q.data_ptr());
@@ -505,8 +512,7 @@ PyObject* bottleneck_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
         }
         for (int i = 0; i < 10; ++i) out[i] = static_cast<float*>(res[i].data_ptr());
         float *const dgamma[3] = {out[4], out[6], out[8]}, *const dbeta[3] = {out[5], out[7], out[9]};
-        // (as large as the stacks: from the allocator on each call, not kept)
-        at::Tensor ws = at::detail::empty_cuda({(int64_t)need}, at::kByte, dq->device(), c10::nullopt);
+        at::Tensor ws = own_scratch(*dq, need);
         const float* const dqp = static_cast<const float*>(dq->data_ptr());
         void *const wp = ws.data_ptr(), *const stream = stream_of(*dq);
         if (!call([&] {

@@ -4,12 +4,15 @@ The bound on a float32 sum of n products in any order is n * 2^-24 * sum |a| * |
 none here); through batch norm and ReLU the same argument runs with the folded scale, so the tests compare with that
 bound evaluated per element on the absolute values, in float64.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
 
 import sbnet_amd
+from sbnet_amd import ops
 from sbnet_amd import sparse_conv as sc
 from sbnet_amd.block_params import BlockParams
 
@@ -145,3 +148,77 @@ def test_layers_under_autocast_take_the_layers_own_way():
         sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
     with torch.no_grad():
         sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
+
+
+def residual_layer(seed, shape=(1, 60, 70), C=32, mid=8, bsize=9):
+    """A residual layer in place on a tensor, its input, and what it gives by itself."""
+    ksizes = [[1, 1, C, mid], [3, 3, mid, mid], [1, 1, mid, C]]
+    bp = sbnet_amd.calc_block_params_res_block([*shape, C], [1, bsize, bsize, 1], ksizes, [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(*shape, 1, device=DEV), bp, 0.0)
+    params = sc.BottleneckParams(ksizes, DEV, seed=seed)
+    x = torch.randn(*shape, C, device=DEV, generator=torch.Generator(DEV).manual_seed(seed))
+
+    def layer(t):
+        with torch.no_grad():
+            return sc.sparse_res_block_bottleneck(t, params, ind, bp, [1, 1, 1, 1], False, use_var=True)
+
+    return layer, x, layer(x.clone())
+
+
+def test_layers_share_no_scratch_between_calls():
+    """The stacks between a block's convolutions and the map of the base's gradient are tensors of the call, not a buffer kept
+    for the stream: another thread on the stream, or a captured graph, would find another call's values in it."""
+    layer, x, want = residual_layer(1)
+    base = torch.zeros(1, 16, 16, 4, device=DEV, requires_grad=True)
+    idx = torch.tensor([[0, 0, 0], [0, 1, 1]], dtype=torch.int16, device=DEV)
+    y = sbnet_amd.sparse_scatter(torch.ones(2, 8, 8, 4, device=DEV), [2], idx, base, [8, 8], [8, 8], [0, 0], add=False)
+    ops.release_workspaces()
+    assert torch.equal(layer(x.clone()), want)
+    torch.autograd.grad(y, base, torch.ones_like(y))
+    assert not ops._load_native().has_workspaces()
+
+
+def test_layers_from_two_threads_on_one_stream():
+    work = [residual_layer(seed) for seed in (1, 2)]
+    wrong = []
+
+    def run(layer, x, want):
+        for _ in range(100):
+            if not torch.equal(layer(x.clone()), want):
+                wrong.append(1)
+
+    threads = [threading.Thread(target=run, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+def test_captured_layers_own_their_stacks():
+    """Two layers captured on one stream, replayed side by side, after the eager calls' scratch has been given back."""
+    work = [residual_layer(seed) for seed in (1, 2)]
+    side = torch.cuda.Stream()
+    graphs = []
+    for layer, x, _ in work:
+        t, g = x.clone(), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            layer(x.clone())
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            layer(t)
+        graphs.append((t, g, torch.cuda.Stream()))
+    ops.release_workspaces()
+    held = [torch.full((1 << 20,), 7.0, device=DEV) for _ in range(8)]
+    for _ in range(4):
+        for (t, _, _), (_, x, _) in zip(graphs, work):
+            t.copy_(x)
+        torch.cuda.synchronize()
+        for _, g, stream in graphs:
+            with torch.cuda.stream(stream):
+                g.replay()
+        torch.cuda.synchronize()
+        for (t, _, _), (_, _, want) in zip(graphs, work):
+            assert torch.equal(t, want)
+    assert all(bool((h == 7.0).all()) for h in held)
