@@ -14,6 +14,7 @@
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -51,13 +52,20 @@ bool pair_of(PyObject* o, Pair& p)
     return false;
 }
 
-// A contiguous tensor of the type on the GPU.
+// A tensor (or parameter) with memory behind it: no subclass and no wrapper of a transform (vmap, grad, fake tensors).
+const at::Tensor* plain_tensor(PyObject* o, at::ScalarType type)
+{
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.defined() || t.scalar_type() != type || t.layout() != at::kStrided || !t.has_storage()) return nullptr;
+    return t.numel() == 0 || t.const_data_ptr() ? &t : nullptr;
+}
+
+// A contiguous one on the GPU.
 const at::Tensor* dev_tensor(PyObject* o, at::ScalarType type)
 {
-    if (!THPVariable_Check(o)) return nullptr;
-    const at::Tensor& t = THPVariable_Unpack(o);
-    if (!t.defined() || !t.is_cuda() || t.scalar_type() != type || t.layout() != at::kStrided || !t.is_contiguous()) return nullptr;
-    return &t;
+    const at::Tensor* t = plain_tensor(o, type);
+    return t && t->is_cuda() && t->is_contiguous() ? t : nullptr;
 }
 
 const at::Tensor* dev_f32(PyObject* o) { return dev_tensor(o, at::kFloat); }
@@ -75,16 +83,16 @@ bool blocks_of(PyObject* counts, PyObject* list, Blocks& b)
     if (!b.idx || b.idx->dim() != 2 || b.idx->size(1) != 3 || b.idx->size(0) > INT32_MAX) return false;
     b.count = nullptr;
     if (THPVariable_Check(counts)) {
-        const at::Tensor& c = THPVariable_Unpack(counts);
-        if (!c.defined() || c.scalar_type() != at::kInt || c.layout() != at::kStrided || c.numel() < 1) return false;
-        if (c.is_cuda()) {
-            if (c.device() != b.idx->device()) return false;
-            b.count = static_cast<const int32_t*>(c.data_ptr());
+        const at::Tensor* c = plain_tensor(counts, at::kInt);
+        if (!c || c->numel() < 1) return false;
+        if (c->is_cuda()) {
+            if (c->device() != b.idx->device()) return false;
+            b.count = static_cast<const int32_t*>(c->data_ptr());
             b.M = (int32_t)b.idx->size(0);
             return true;
         }
-        if (!c.is_cpu()) return false;
-        b.M = *static_cast<const int32_t*>(c.data_ptr());
+        if (!c->is_cpu()) return false;
+        b.M = *static_cast<const int32_t*>(c->const_data_ptr());
     } else if (PyList_CheckExact(counts) && PyList_GET_SIZE(counts) >= 1) {
         if (!int_of(PyList_GET_ITEM(counts, 0), &b.M)) return false;
     } else {
@@ -151,28 +159,33 @@ bool call(F f)
     return false;
 }
 
-template <typename F>
-PyObject* guarded(F f)
+// A function of the module: N arguments, and no C++ exception through the interpreter's frames.
+template <PyObject* (*F)(PyObject* const*), Py_ssize_t N>
+PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", N, n);
+        return nullptr;
+    }
     try {
-        return f();
+        return F(a);
     } catch (...) {
         torch::translate_exception_to_python(std::current_exception());
     }
     return nullptr;
 }
 
-bool expect(Py_ssize_t n, Py_ssize_t want)
+// The same for an op: left to the general wrappers while something looks on at torch's operators.
+template <PyObject* (*F)(PyObject* const*), Py_ssize_t N>
+PyObject* op_entry(PyObject* self, PyObject* const* a, Py_ssize_t n)
 {
-    if (n == want) return true;
-    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
-    return false;
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set()) Py_RETURN_NONE;
+    return entry<F, N>(self, a, n);
 }
 
 // reduce_mask(mask, bcount, bsize, bstride, boffset, tol, avgpool, sync) -> (active_block_indices, bin_counts)
-PyObject* reduce_mask(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* reduce_mask(PyObject* const* a)
 {
-    if (!expect(n, 8)) return nullptr;
     const at::Tensor* mask = dev_f32(a[0]);
     Pair bc, bs, bt, bo;
     if (!mask || !pair_of(a[1], bc) || !pair_of(a[2], bs) || !pair_of(a[3], bt) || !pair_of(a[4], bo)) Py_RETURN_NONE;
@@ -186,32 +199,29 @@ PyObject* reduce_mask(PyObject*, PyObject* const* a, Py_ssize_t n)
     const float tol = (float)PyFloat_AS_DOUBLE(a[5]);
     const int avgpool = PyObject_IsTrue(a[6]), sync = PyObject_IsTrue(a[7]);
     if (avgpool < 0 || sync < 0) return nullptr;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(mask->device());
-        at::Tensor idx = at::detail::empty_cuda({T, 3}, at::kShort, mask->device(), c10::nullopt);
-        at::Tensor count = sync ? at::empty({1}, at::kInt) : at::detail::empty_cuda({1}, at::kInt, mask->device(), c10::nullopt);
-        int32_t* const cp = static_cast<int32_t*>(count.data_ptr());
-        at::Tensor ws = workspace(mask->device(), (int64_t)sbnet_reduce_mask_workspace_bytes(N, bc.v, 2));
-        void* const stream = stream_of(*mask);
-        if (!call([&] {
-                return sbnet_reduce_mask(static_cast<const float*>(mask->data_ptr()), N, H, W, bc.v, 2, bs.v, 2, bt.v, 2, bo.v,
-                                         2, tol, avgpool, static_cast<int16_t*>(idx.data_ptr()), sync ? cp : nullptr,
-                                         sync ? nullptr : cp, ws.data_ptr(), (size_t)ws.numel(), stream);
-            }))
-            return nullptr;
-        PyObject* pi = THPVariable_Wrap(std::move(idx));
-        PyObject* pc = THPVariable_Wrap(std::move(count));
-        PyObject* t = pi && pc ? PyTuple_Pack(2, pi, pc) : nullptr;
-        Py_XDECREF(pi);
-        Py_XDECREF(pc);
-        return t;
-    });
+    c10::DeviceGuard guard(mask->device());
+    at::Tensor idx = at::detail::empty_cuda({T, 3}, at::kShort, mask->device(), c10::nullopt);
+    at::Tensor count = sync ? at::empty({1}, at::kInt) : at::detail::empty_cuda({1}, at::kInt, mask->device(), c10::nullopt);
+    int32_t* const cp = static_cast<int32_t*>(count.data_ptr());
+    at::Tensor ws = workspace(mask->device(), (int64_t)sbnet_reduce_mask_workspace_bytes(N, bc.v, 2));
+    void* const stream = stream_of(*mask);
+    if (!call([&] {
+            return sbnet_reduce_mask(static_cast<const float*>(mask->data_ptr()), N, H, W, bc.v, 2, bs.v, 2, bt.v, 2, bo.v,
+                                     2, tol, avgpool, static_cast<int16_t*>(idx.data_ptr()), sync ? cp : nullptr,
+                                     sync ? nullptr : cp, ws.data_ptr(), (size_t)ws.numel(), stream);
+        }))
+        return nullptr;
+    PyObject* pi = THPVariable_Wrap(std::move(idx));
+    PyObject* pc = THPVariable_Wrap(std::move(count));
+    PyObject* t = pi && pc ? PyTuple_Pack(2, pi, pc) : nullptr;
+    Py_XDECREF(pi);
+    Py_XDECREF(pc);
+    return t;
 }
 
 // gather(x, bin_counts, active_block_indices, bsize, bstride, boffset, transpose, out) -> stack
-PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* gather(PyObject* const* a)
 {
-    if (!expect(n, 8)) return nullptr;
     const at::Tensor* x = dev_f32(a[0]);
     Blocks b;
     Pair bs, bt, bo;
@@ -225,28 +235,25 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n)
         out = dev_f32(a[7]);
         if (!out || out->device() != x->device() || !is_stack(*out, b.M, x->size(3), bs, transpose)) Py_RETURN_NONE;
     }
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(x->device());
-        at::Tensor y = out ? *out : empty_stack(b.M, x->size(3), bs, transpose, *x);
-        const float* const xp = static_cast<const float*>(x->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const yp = static_cast<float*>(y.data_ptr());
-        const int64_t* const dims = x->sizes().data();
-        void* const stream = stream_of(*x);
-        if (!call([&] {
-                return b.count ? sbnet_sparse_gather_device_count(xp, dims, 4, b.count, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2,
-                                                                  transpose, yp, stream)
-                               : sbnet_sparse_gather(xp, dims, 4, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2, transpose, yp, stream);
-            }))
-            return nullptr;
-        return THPVariable_Wrap(std::move(y));
-    });
+    c10::DeviceGuard guard(x->device());
+    at::Tensor y = out ? *out : empty_stack(b.M, x->size(3), bs, transpose, *x);
+    const float* const xp = static_cast<const float*>(x->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const yp = static_cast<float*>(y.data_ptr());
+    const int64_t* const dims = x->sizes().data();
+    void* const stream = stream_of(*x);
+    if (!call([&] {
+            return b.count ? sbnet_sparse_gather_device_count(xp, dims, 4, b.count, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2,
+                                                              transpose, yp, stream)
+                           : sbnet_sparse_gather(xp, dims, 4, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2, transpose, yp, stream);
+        }))
+        return nullptr;
+    return THPVariable_Wrap(std::move(y));
 }
 
 // gather_grad(grad, bin_counts, active_block_indices, x_shape, bsize, bstride, boffset, transpose) -> dx
-PyObject* gather_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* gather_grad(PyObject* const* a)
 {
-    if (!expect(n, 8)) return nullptr;
     const at::Tensor* g = dev_f32(a[0]);
     Blocks b;
     Pair bs, bt, bo;
@@ -262,28 +269,25 @@ PyObject* gather_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
     const int transpose = PyObject_IsTrue(a[7]);
     if (transpose < 0) return nullptr;
     if (!is_stack(*g, b.M, dims[3], bs, transpose)) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(g->device());
-        at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, *g);
-        const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
-        at::Tensor ws = need ? workspace(g->device(), need) : at::Tensor();
-        const float* const gp = static_cast<const float*>(g->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const dp = static_cast<float*>(dx.data_ptr());
-        void* const stream = stream_of(*g);
-        if (!call([&] {
-                return sbnet_sparse_gather_grad(gp, b.M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
-                                                need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
-            }))
-            return nullptr;
-        return THPVariable_Wrap(std::move(dx));
-    });
+    c10::DeviceGuard guard(g->device());
+    at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, *g);
+    const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
+    at::Tensor ws = need ? workspace(g->device(), need) : at::Tensor();
+    const float* const gp = static_cast<const float*>(g->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const dp = static_cast<float*>(dx.data_ptr());
+    void* const stream = stream_of(*g);
+    if (!call([&] {
+            return sbnet_sparse_gather_grad(gp, b.M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
+                                            need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
+        }))
+        return nullptr;
+    return THPVariable_Wrap(std::move(dx));
 }
 
 // scatter(x, bin_counts, active_block_indices, ybase, bsize, bstride, boffset, add, atomic, transpose, use_var) -> y
-PyObject* scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* scatter(PyObject* const* a)
 {
-    if (!expect(n, 11)) return nullptr;
     const at::Tensor *x = dev_f32(a[0]), *base = dev_f32(a[3]);
     Blocks b;
     Pair bs, bt, bo;
@@ -296,43 +300,40 @@ PyObject* scatter(PyObject*, PyObject* const* a, Py_ssize_t n)
     if (b.count && x->dim() > 0 && x->size(0) < b.M) b.M = (int32_t)x->size(0);
     if (!is_stack(*x, b.M, base->size(3), bs, transpose)) Py_RETURN_NONE;
     const bool overlap = bt.v[0] < bs.v[0] || bt.v[1] < bs.v[1];
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(base->device());
-        const int64_t* const dims = base->sizes().data();
-        const bool scratch = (add && atomic) || !in_place || (!add && overlap);
-        const int64_t need = scratch ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
-        at::Tensor ws = need ? workspace(base->device(), need) : at::Tensor();
-        void* const wp = need ? ws.data_ptr() : nullptr;
-        const size_t wn = need ? (size_t)ws.numel() : 0;
-        at::Tensor y = in_place ? *base : empty_f32(base->sizes(), *base);
-        const float *const xp = static_cast<const float*>(x->data_ptr()), *const bp = static_cast<const float*>(base->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const yp = static_cast<float*>(y.data_ptr());
-        void* const stream = stream_of(*base);
-        if (!call([&] {
-                if (in_place)
-                    return b.count ? sbnet_sparse_scatter_var_device_count(xp, b.count, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2,
-                                                                           bo.v, 2, add, atomic, transpose, wp, wn, stream)
-                                   : sbnet_sparse_scatter_var(xp, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
-                                                              transpose, wp, wn, stream);
-                return b.count ? sbnet_sparse_scatter_device_count(xp, b.count, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2,
-                                                                   add, atomic, transpose, yp, wp, wn, stream)
-                               : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
-                                                      transpose, yp, wp, wn, stream);
-            }))
-            return nullptr;
-        if (in_place) {
-            Py_INCREF(a[3]);   // the caller's own tensor object, as the Python wrapper returns it
-            return a[3];
-        }
-        return THPVariable_Wrap(std::move(y));
-    });
+    c10::DeviceGuard guard(base->device());
+    const int64_t* const dims = base->sizes().data();
+    const bool scratch = (add && atomic) || !in_place || (!add && overlap);
+    const int64_t need = scratch ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
+    at::Tensor ws = need ? workspace(base->device(), need) : at::Tensor();
+    void* const wp = need ? ws.data_ptr() : nullptr;
+    const size_t wn = need ? (size_t)ws.numel() : 0;
+    at::Tensor y = in_place ? *base : empty_f32(base->sizes(), *base);
+    const float *const xp = static_cast<const float*>(x->data_ptr()), *const bp = static_cast<const float*>(base->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const yp = static_cast<float*>(y.data_ptr());
+    void* const stream = stream_of(*base);
+    if (!call([&] {
+            if (in_place)
+                return b.count ? sbnet_sparse_scatter_var_device_count(xp, b.count, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2,
+                                                                       bo.v, 2, add, atomic, transpose, wp, wn, stream)
+                               : sbnet_sparse_scatter_var(xp, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
+                                                          transpose, wp, wn, stream);
+            return b.count ? sbnet_sparse_scatter_device_count(xp, b.count, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2,
+                                                               add, atomic, transpose, yp, wp, wn, stream)
+                           : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
+                                                  transpose, yp, wp, wn, stream);
+        }))
+        return nullptr;
+    if (in_place) {
+        Py_INCREF(a[3]);   // the caller's own tensor object, as the Python wrapper returns it
+        return a[3];
+    }
+    return THPVariable_Wrap(std::move(y));
 }
 
 // scatter_base_grad(grad, bin_counts, active_block_indices, bsize, bstride, boffset) -> gradient of the base of plain writes
-PyObject* scatter_base_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* scatter_base_grad(PyObject* const* a)
 {
-    if (!expect(n, 6)) return nullptr;
     const at::Tensor* g = dev_f32(a[0]);
     Blocks b;
     Pair bs, bt, bo;
@@ -342,18 +343,16 @@ PyObject* scatter_base_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
     const int64_t* const dims = g->sizes().data();
     const size_t need = sbnet_sparse_scatter_base_grad_workspace_bytes(b.M, dims, bs.v, bt.v, bo.v);
     if (!need) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(g->device());
-        at::Tensor d = empty_f32(g->sizes(), *g);
-        at::Tensor ws = own_scratch(*g, need);
-        const float* const gp = static_cast<const float*>(g->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const dp = static_cast<float*>(d.data_ptr());
-        void *const wp = ws.data_ptr(), *const stream = stream_of(*g);
-        if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, need, stream); }))
-            return nullptr;
-        return THPVariable_Wrap(std::move(d));
-    });
+    c10::DeviceGuard guard(g->device());
+    at::Tensor d = empty_f32(g->sizes(), *g);
+    at::Tensor ws = own_scratch(*g, need);
+    const float* const gp = static_cast<const float*>(g->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const dp = static_cast<float*>(d.data_ptr());
+    void *const wp = ws.data_ptr(), *const stream = stream_of(*g);
+    if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, need, stream); }))
+        return nullptr;
+    return THPVariable_Wrap(std::move(d));
 }
 
 // Contiguous, on the GPU, float32, with no gradient asked for, and not under autocast, where the layers' convolutions
@@ -377,9 +376,8 @@ bool kernel_of(const at::Tensor& w, int64_t C, int64_t R, int64_t S, int32_t* di
 bool positive(const Pair& p) { return p.v[0] > 0 && p.v[1] > 0; }
 
 // block_conv(x, w, bin_counts, active_block_indices, bsize, bstride, boffset) -> NHWC stack
-PyObject* block_conv(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* block_conv(PyObject* const* a)
 {
-    if (!expect(n, 7)) return nullptr;
     const at::Tensor *x = plain_f32(a[0]), *w = plain_f32(a[1]);
     Blocks b;
     Pair bs, bt, bo;
@@ -390,25 +388,22 @@ PyObject* block_conv(PyObject*, PyObject* const* a, Py_ssize_t n)
         Py_RETURN_NONE;
     const int64_t R = bs.v[0] - wd[0] + 1, S = bs.v[1] - wd[1] + 1;
     if (R * S >= ROWS_MOST || b.M * R * S >= ROWS_MOST || b.M * R * S * wd[3] >= 2 * CONV_MOST) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(x->device());
-        at::Tensor q = empty_f32({b.M, R, S, wd[3]}, *x);
-        const float *const xp = static_cast<const float*>(x->data_ptr()), *const kp = static_cast<const float*>(w->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const qp = static_cast<float*>(q.data_ptr());
-        const int64_t* const dims = x->sizes().data();
-        void* const stream = stream_of(*x);
-        if (b.M && !call([&] { return sbnet_block_conv(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, kp, wd, qp, stream); }))
-            return nullptr;
-        return THPVariable_Wrap(std::move(q));
-    });
+    c10::DeviceGuard guard(x->device());
+    at::Tensor q = empty_f32({b.M, R, S, wd[3]}, *x);
+    const float *const xp = static_cast<const float*>(x->data_ptr()), *const kp = static_cast<const float*>(w->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const qp = static_cast<float*>(q.data_ptr());
+    const int64_t* const dims = x->sizes().data();
+    void* const stream = stream_of(*x);
+    if (b.M && !call([&] { return sbnet_block_conv(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, kp, wd, qp, stream); }))
+        return nullptr;
+    return THPVariable_Wrap(std::move(q));
 }
 
 // block_bottleneck(x, [w1, w2, w3], [gamma, beta, mean, var] * 3, bin_counts, active_block_indices, bsize, bstride,
 //                  boffset, out_stride, eps, no_activation, in_place) -> NHWC stack, or x with the result added
-PyObject* block_bottleneck(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* block_bottleneck(PyObject* const* a)
 {
-    if (!expect(n, 12)) return nullptr;
     const at::Tensor* x = plain_f32(a[0]);
     Blocks b;
     Pair bs, bt, bo, os;
@@ -437,35 +432,32 @@ PyObject* block_bottleneck(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (R * S >= ROWS_MOST || b.M * R * S >= ROWS_MOST || b.M * R * S * C >= 2 * CONV_MOST) Py_RETURN_NONE;
     }
     if (in_place && (C != x->size(3) || os.v[0] != R || os.v[1] != S)) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(x->device());
-        at::Tensor q = in_place ? *x : empty_f32({b.M, R, S, C}, *x);
-        at::Tensor ws = own_scratch(*x, sbnet_block_bottleneck_workspace_bytes(b.M, bs.v, wd));
-        const float* const xp = static_cast<const float*>(x->data_ptr());
-        const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-        float* const qp = static_cast<float*>(q.data_ptr());
-        const int64_t* const dims = x->sizes().data();
-        const float eps = (float)PyFloat_AS_DOUBLE(a[9]);
-        void* const stream = stream_of(*x);
-        if (b.M && !call([&] {
-                return sbnet_block_bottleneck(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, weights, wd, norms, eps,
-                                              in_place ? nullptr : qp, in_place ? qp : nullptr, os.v, ws.data_ptr(),
-                                              (size_t)ws.numel(), stream);
-            }))
-            return nullptr;
-        if (in_place) {
-            Py_INCREF(a[0]);
-            return a[0];
-        }
-        return THPVariable_Wrap(std::move(q));
-    });
+    c10::DeviceGuard guard(x->device());
+    at::Tensor q = in_place ? *x : empty_f32({b.M, R, S, C}, *x);
+    at::Tensor ws = own_scratch(*x, sbnet_block_bottleneck_workspace_bytes(b.M, bs.v, wd));
+    const float* const xp = static_cast<const float*>(x->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const qp = static_cast<float*>(q.data_ptr());
+    const int64_t* const dims = x->sizes().data();
+    const float eps = (float)PyFloat_AS_DOUBLE(a[9]);
+    void* const stream = stream_of(*x);
+    if (b.M && !call([&] {
+            return sbnet_block_bottleneck(xp, dims, b.M, b.count, ip, bs.v, bt.v, bo.v, weights, wd, norms, eps,
+                                          in_place ? nullptr : qp, in_place ? qp : nullptr, os.v, ws.data_ptr(),
+                                          (size_t)ws.numel(), stream);
+        }))
+        return nullptr;
+    if (in_place) {
+        Py_INCREF(a[0]);
+        return a[0];
+    }
+    return THPVariable_Wrap(std::move(q));
 }
 
 // bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1, ...), on
 // planar stacks, or None where the kernels do not take the sizes.
-PyObject* bottleneck_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* bottleneck_grad(PyObject* const* a)
 {
-    if (!expect(n, 2)) return nullptr;
     const at::Tensor* dq = dev_f32(a[0]);
     if (!dq || dq->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 18) Py_RETURN_NONE;
     const at::Tensor* t[18];
@@ -499,46 +491,41 @@ PyObject* bottleneck_grad(PyObject*, PyObject* const* a, Py_ssize_t n)
     if (dq->sizes() != at::IntArrayRef({M, C, R, S}) || dq->numel() >= 2 * CONV_MOST) Py_RETURN_NONE;
     const size_t need = sbnet_bottleneck_grad_workspace_bytes((int32_t)M, bs, wd);
     if (!need) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        c10::DeviceGuard guard(dq->device());
-        at::Tensor res[10];
-        float *out[10];
-        res[0] = empty_f32(t[0]->sizes(), *dq);
-        for (int i = 0; i < 3; ++i) {
-            const int32_t* d = wd + 4 * i;
-            res[1 + i] = empty_f32({d[0], d[1], d[2], d[3]}, *dq);
-            res[4 + 2 * i] = empty_f32({d[2]}, *dq);
-            res[5 + 2 * i] = empty_f32({d[2]}, *dq);
-        }
-        for (int i = 0; i < 10; ++i) out[i] = static_cast<float*>(res[i].data_ptr());
-        float *const dgamma[3] = {out[4], out[6], out[8]}, *const dbeta[3] = {out[5], out[7], out[9]};
-        at::Tensor ws = own_scratch(*dq, need);
-        const float* const dqp = static_cast<const float*>(dq->data_ptr());
-        void *const wp = ws.data_ptr(), *const stream = stream_of(*dq);
-        if (!call([&] {
-                return sbnet_bottleneck_grad(dqp, (int32_t)M, bs, ptr[0], ptr[1], ptr[2], ptr[3], ptr[5], ptr[4], wd, out[0],
-                                             out + 1, dgamma, dbeta, wp, need, stream);
-            }))
-            return nullptr;
-        PyObject* r = PyTuple_New(10);
-        if (!r) return nullptr;
-        for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(res[i])));
-        return r;
-    });
+    c10::DeviceGuard guard(dq->device());
+    at::Tensor res[10];
+    float *out[10];
+    res[0] = empty_f32(t[0]->sizes(), *dq);
+    for (int i = 0; i < 3; ++i) {
+        const int32_t* d = wd + 4 * i;
+        res[1 + i] = empty_f32({d[0], d[1], d[2], d[3]}, *dq);
+        res[4 + 2 * i] = empty_f32({d[2]}, *dq);
+        res[5 + 2 * i] = empty_f32({d[2]}, *dq);
+    }
+    for (int i = 0; i < 10; ++i) out[i] = static_cast<float*>(res[i].data_ptr());
+    float *const dgamma[3] = {out[4], out[6], out[8]}, *const dbeta[3] = {out[5], out[7], out[9]};
+    at::Tensor ws = own_scratch(*dq, need);
+    const float* const dqp = static_cast<const float*>(dq->data_ptr());
+    void *const wp = ws.data_ptr(), *const stream = stream_of(*dq);
+    if (!call([&] {
+            return sbnet_bottleneck_grad(dqp, (int32_t)M, bs, ptr[0], ptr[1], ptr[2], ptr[3], ptr[5], ptr[4], wd, out[0],
+                                         out + 1, dgamma, dbeta, wp, need, stream);
+        }))
+        return nullptr;
+    PyObject* r = PyTuple_New(10);
+    if (!r) return nullptr;
+    for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(res[i])));
+    return r;
 }
 
 // workspace(device index, bytes) -> uint8 tensor: the scratch of the current stream, for the wrappers in Python
-PyObject* workspace_py(PyObject*, PyObject* const* a, Py_ssize_t n)
+PyObject* workspace_py(PyObject* const* a)
 {
-    if (!expect(n, 2)) return nullptr;
     const long dev = PyLong_AsLong(a[0]);
     const long long bytes = PyLong_AsLongLong(a[1]);
     if (PyErr_Occurred()) return nullptr;
-    return guarded([&]() -> PyObject* {
-        const at::Device device(at::kCUDA, (c10::DeviceIndex)dev);
-        c10::DeviceGuard guard(device);
-        return THPVariable_Wrap(workspace(device, bytes));
-    });
+    const at::Device device(at::kCUDA, (c10::DeviceIndex)dev);
+    c10::DeviceGuard guard(device);
+    return THPVariable_Wrap(workspace(device, bytes));
 }
 
 PyObject* release_workspaces(PyObject*, PyObject*)
@@ -560,15 +547,15 @@ template <typename F>
 PyCFunction fast(F f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)); }
 
 PyMethodDef methods[] = {
-    {"reduce_mask", fast(reduce_mask), METH_FASTCALL, nullptr},
-    {"gather", fast(gather), METH_FASTCALL, nullptr},
-    {"gather_grad", fast(gather_grad), METH_FASTCALL, nullptr},
-    {"scatter", fast(scatter), METH_FASTCALL, nullptr},
-    {"scatter_base_grad", fast(scatter_base_grad), METH_FASTCALL, nullptr},
-    {"block_conv", fast(block_conv), METH_FASTCALL, nullptr},
-    {"block_bottleneck", fast(block_bottleneck), METH_FASTCALL, nullptr},
-    {"bottleneck_grad", fast(bottleneck_grad), METH_FASTCALL, nullptr},
-    {"workspace", fast(workspace_py), METH_FASTCALL, nullptr},
+    {"reduce_mask", fast(op_entry<reduce_mask, 8>), METH_FASTCALL, nullptr},
+    {"gather", fast(op_entry<gather, 8>), METH_FASTCALL, nullptr},
+    {"gather_grad", fast(op_entry<gather_grad, 8>), METH_FASTCALL, nullptr},
+    {"scatter", fast(op_entry<scatter, 11>), METH_FASTCALL, nullptr},
+    {"scatter_base_grad", fast(op_entry<scatter_base_grad, 6>), METH_FASTCALL, nullptr},
+    {"block_conv", fast(op_entry<block_conv, 7>), METH_FASTCALL, nullptr},
+    {"block_bottleneck", fast(op_entry<block_bottleneck, 12>), METH_FASTCALL, nullptr},
+    {"bottleneck_grad", fast(op_entry<bottleneck_grad, 2>), METH_FASTCALL, nullptr},
+    {"workspace", fast(entry<workspace_py, 2>), METH_FASTCALL, nullptr},
     {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},
     {"set_check", set_check, METH_O, nullptr},

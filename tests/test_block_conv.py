@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
+from torch.utils.flop_counter import FlopCounterMode
 
 import sbnet_amd
 from sbnet_amd import ops
@@ -148,6 +149,16 @@ def test_layers_under_autocast_take_the_layers_own_way():
         sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
     with torch.no_grad():
         sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
+
+
+def test_layers_under_a_dispatch_mode_take_the_layers_own_way():
+    """What looks on at torch's operators (here: counts their operations) sees a layer's convolution."""
+    bp = sbnet_amd.calc_block_params([1, 20, 20, 16], [1, 8, 8, 1], [3, 3, 16, 16], [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(1, 20, 20, 1, device=DEV), bp, 0.0)
+    x, w = torch.randn(1, 20, 20, 16, device=DEV), torch.randn(3, 3, 16, 16, device=DEV)
+    with torch.no_grad(), FlopCounterMode(display=False) as flops:
+        sc.sparse_conv2d_custom(x, w, ind, bp, [1, 1, 1, 1])
+    assert flops.get_total_flops() == 2 * int(ind.bin_counts[0]) * 36 * 9 * 16 * 16
 
 
 def residual_layer(seed, shape=(1, 60, 70), C=32, mid=8, bsize=9):

@@ -263,6 +263,38 @@ def test_native_wrappers_leave_what_they_do_not_take():
         ops.sparse_gather(x, [1], idx, pair, pair, [0, 0])
 
 
+def test_native_wrappers_leave_tensors_without_memory():
+    """Fake tensors and those of a transform go the general way, which raises what it raises: nothing is read through their
+    pointers, and no C++ exception leaves the module."""
+    import torch
+    from torch._subclasses.fake_tensor import DataDependentOutputException, FakeTensorMode
+    from sbnet_amd import ops
+
+    native = ops._load_native()
+    pair, zero = [4, 4], [0, 0]
+    with FakeTensorMode():
+        x, q = torch.empty(1, 8, 8, 4, device="cuda:0"), torch.empty(4, 4, 4, 4, device="cuda:0")
+        idx, count = torch.empty(4, 3, dtype=torch.int16, device="cuda:0"), torch.empty(1, dtype=torch.int32)
+        w, v = torch.empty(1, 1, 4, 4, device="cuda:0"), torch.empty(4, device="cuda:0")
+        batch = torch.empty(3, 1, 8, 8, 4, device="cuda:0")
+
+    def calls(x, count):
+        return [native.reduce_mask(x[..., :1].contiguous(), [2, 2], pair, pair, zero, 0.5, False, True),
+                native.gather(x, count, idx, pair, pair, zero, False, None),
+                native.gather_grad(q, count, idx, (1, 8, 8, 4), pair, pair, zero, False),
+                native.scatter(q, count, idx, x, pair, pair, zero, False, False, False, True),
+                native.scatter_base_grad(x, count, idx, pair, pair, zero),
+                native.block_conv(x, w, count, idx, pair, pair, zero),
+                native.block_bottleneck(x, [w] * 3, [v] * 12, count, idx, pair, pair, zero, pair, 1e-3, False, False),
+                native.bottleneck_grad(q, [q, q, v, v, w, v] * 3)]
+
+    results = calls(x, count) + calls(x, [1])
+    torch.vmap(lambda x: results.extend(calls(x, [1])) or x)(batch)
+    assert results == [None] * 24
+    with pytest.raises(DataDependentOutputException):
+        ops.sparse_gather(x, count, idx, pair, pair, zero)
+
+
 @pytest.mark.gpu
 def test_scratch_provider_keeps_outgrown_buffers_until_shutdown():
     """sbnet_scratch_acquire hands one grow-only buffer per stream to callers without an allocator.  A pointer it

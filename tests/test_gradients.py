@@ -315,3 +315,16 @@ def test_base_gradient_of_plain_writes_is_the_masked_product(shape, bsize, bstri
     want = dy * stamp
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     assert torch.equal(torch.nan_to_num(got, nan=1.0).view(torch.int32), torch.nan_to_num(want, nan=1.0).view(torch.int32))
+
+
+@pytest.mark.gpu
+def test_batched_gradients_are_refused():
+    """A vectorised Jacobian's gradients have no memory of their own: an exception, as from any op without a batching rule."""
+    import sbnet_amd
+    idx = torch.tensor([[0, 0, 0], [0, 1, 1]], dtype=torch.int16, device="cuda:0")
+    for leaf in (0, 1):
+        tensors = [torch.zeros(2, 4, 4, 4, device="cuda:0"), torch.zeros(1, 8, 8, 4, device="cuda:0")]
+        tensors[leaf].requires_grad_()
+        y = sbnet_amd.sparse_scatter(tensors[0], [2], idx, tensors[1], [4, 4], [4, 4], [0, 0], add=False)
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(y, tensors[leaf], torch.ones(3, *y.shape, device="cuda:0"), is_grads_batched=True)
