@@ -36,8 +36,8 @@ namespace sbnet {
 // WK > 1: the WK waves of a workgroup split k among them and add up through LDS.  For launches whose tiles alone would
 // leave most of the 1024 SIMDs idle.
 //
-// Batch norm of the input (pre) applies to values after the load, out-of-image zeros included, with scale and shift
-// computed once per workgroup into LDS; batch norm of the result (post), for the convolution that follows, at the end.
+// Batch norm of the input (pre) applies to values after the load, out-of-image zeros included, with mean, scale and shift
+// read once per workgroup into LDS; batch norm of the result (post), for the convolution that follows, at the end.
 
 typedef float acc_t __attribute__((ext_vector_type(4)));
 
@@ -61,11 +61,13 @@ struct ConvKernelArgs {
 
 __device__ __forceinline__ float relu_keep_nan(float v) { return v < 0.f ? 0.f : v; }
 
-// scale and shift of an inference batch norm, y = x * scale + shift
-__device__ __forceinline__ void bn_fold(const BnArgs& bn, uint32_t c, float& scale, float& shift)
+// An inference batch norm, y = (x - mean) * scale + beta, of channel c.  The mean is taken off first: folded into the shift
+// it costs accuracy in proportion to |mean| / sigma (relative error 3e-7 at 10, 3e-5 at 1000; 5e-8 this way).
+__device__ __forceinline__ void bn_read(const BnArgs& bn, uint32_t c, float& mean, float& scale, float& beta)
 {
+    mean = bn.mean[c];
     scale = bn.gamma[c] * (1.f / sqrtf(bn.var[c] + bn.eps));
-    shift = bn.beta[c] - bn.mean[c] * scale;
+    beta = bn.beta[c];
 }
 
 // GRAD: the gradient of a convolution's input.  The same product with the kernel turned around, w [K, kh, kw, C] (n, then
@@ -84,12 +86,11 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     constexpr int TP = 16 * WP, TN = 16 * FN;
     extern __shared__ float lds[];
     const uint32_t cPad = PRE ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
-    float* const preScale = lds;
-    float* const preShift = lds + cPad;
-    float* const postScale = lds + 2 * cPad;
-    float* const postShift = postScale + TN;
-    double* const sums = reinterpret_cast<double*>(postScale + 2 * TN);   // [WP][TN][2], GRAD only
-    float* const red = postScale + (GRAD ? 2 + 4 * WP : 2) * TN;     // [WP][WK][FN][64] x 4, WK > 1 only
+    float *const preMean = lds, *const preScale = lds + cPad, *const preBeta = lds + 2 * cPad;
+    float *const postMean = lds + 3 * cPad, *const postScale = postMean + TN;   // (GRAD: mean and 1 / sigma)
+    float* const postBeta = postMean + 2 * TN;                            // not GRAD
+    double* const sums = reinterpret_cast<double*>(postMean + 2 * TN);    // [WP][TN][2], GRAD only
+    float* const red = postMean + (GRAD ? 2 + 4 * WP : 3) * TN;           // [WP][WK][FN][64] x 4, WK > 1 only
 
     // Eight consecutive workgroups go to eight XCDs; the tiles of one pixel range that differ in channels only follow
     // each other on one XCD, whose L2 then holds the pixels once.
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
                     for (int i = 0; i < 4; ++i) o.wv[f][i] = v[i];
                 }
             }
-            if constexpr (PRE) o.c[j] = TAPS ? t.c : min(t.c, C - (VEC == 4 ? 4u : 1u));   // (scale and shift of some channel, past the end)
+            if constexpr (PRE) o.c[j] = TAPS ? t.c : min(t.c, C - (VEC == 4 ? 4u : 1u));   // (the batch norm of some channel, past the end)
             if constexpr (TAPS) bad |= (uint32_t)((unsigned)t.h >= (unsigned)a.c.H) | (uint32_t)((unsigned)t.w >= (unsigned)a.c.W);
             else bad |= (uint32_t)!pixelOk;
             const uint32_t off = t.off | (0u - bad);
@@ -245,34 +246,36 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     }
 
     if (PRE)
-        for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_fold(a.c.pre, c, preScale[c], preShift[c]);
-    if constexpr (GRAD) {   // mean and 1 / sigma
+        for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_read(a.c.pre, c, preMean[c], preScale[c], preBeta[c]);
+    if constexpr (GRAD) {
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES) {
             const uint32_t n = min(n0 + i, K - 1);
-            postScale[i] = a.c.norm.mean[n];
-            postShift[i] = a.c.norm.inv[n];
+            postMean[i] = a.c.norm.mean[n];
+            postScale[i] = a.c.norm.inv[n];
         }
     } else if (post) {
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES)
-            if (n0 + i < K) bn_fold(a.c.post, n0 + i, postScale[i], postShift[i]);
+            if (n0 + i < K) bn_read(a.c.post, n0 + i, postMean[i], postScale[i], postBeta[i]);
     }
     if (PRE || GRAD || post) lds_barrier();
 
     auto multiply = [&](Operands& o) {
         if constexpr (PRE) {
-            acc_t sc, sh;
+            acc_t mean, sc, beta;
             if constexpr (VEC == 4) {
+                mean = lds_read4(preMean + o.c[0]);
                 sc = lds_read4(preScale + o.c[0]);
-                sh = lds_read4(preShift + o.c[0]);
+                beta = lds_read4(preBeta + o.c[0]);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
+                    mean[j] = preMean[o.c[j]];
                     sc[j] = preScale[o.c[j]];
-                    sh[j] = preShift[o.c[j]];
+                    beta[j] = preBeta[o.c[j]];
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) o.px[j] = relu_keep_nan(o.px[j] * sc[j] + sh[j]);
+            for (int j = 0; j < 4; ++j) o.px[j] = relu_keep_nan((o.px[j] - mean[j]) * sc[j] + beta[j]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -319,7 +322,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
             const uint32_t o = row < rows && n < K ? (row * K + n) * 4u : BUF_OOB;
             const acc_t z = (acc_t)buf_load<4>(make_rsrc(a.c.norm.z, a.yBytes), o);
             const acc_t act = (acc_t)buf_load<4>(make_rsrc(a.c.norm.act, a.yBytes), o);   // (0 past the end: masked)
-            const acc_t xhat = (z - (acc_t)lds_read4(postScale + nl)) * (acc_t)lds_read4(postShift + nl);
+            const acc_t xhat = (z - (acc_t)lds_read4(postMean + nl)) * (acc_t)lds_read4(postScale + nl);
             acc_t s1, s2;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
         }
         if (post) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan(v[j] * postScale[nl + j] + postShift[nl + j]);
+            for (int j = 0; j < 4; ++j) v[j] = relu_keep_nan((v[j] - postMean[nl + j]) * postScale[nl + j] + postBeta[nl + j]);
         }
         emit(n, K, v);
     };
@@ -352,9 +355,9 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     if constexpr (NEXT) {
         auto between = [&](int i, acc_t v) {   // (columns past the last channel hold something or other: cleared)
             const uint32_t nl = i * 16 + quad * 4;
-            const acc_t sc = lds_read4(postScale + nl), sh = lds_read4(postShift + nl);
+            const acc_t mean = lds_read4(postMean + nl), sc = lds_read4(postScale + nl), beta = lds_read4(postBeta + nl);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = nl < K ? (post ? relu_keep_nan(v[j] * sc[j] + sh[j]) : v[j]) : 0.f;
+            for (int j = 0; j < 4; ++j) v[j] = nl < K ? (post ? relu_keep_nan((v[j] - mean[j]) * sc[j] + beta[j]) : v[j]) : 0.f;
             return v;
         };
 #pragma unroll
@@ -428,7 +431,7 @@ static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
     a.tilesP = (a.rows + TP - 1) / TP;
     a.tilesN = ((uint32_t)a.c.K + TN - 1) / TN;
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
-    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 2 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 2) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
+    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 3 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 3) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((k_block_conv<FN, WK, VEC, PRE, TAPS, GRAD, NEXT>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();
@@ -450,7 +453,7 @@ static hipError_t launch_conv_one(ConvKernelArgs& a, hipStream_t stream)
 
 bool conv_fits(const ConvArgs& c)
 {
-    // 32-bit byte offsets in the input, the weights and the output; scale and shift of the input's channels in LDS
+    // 32-bit byte offsets in the input, the weights and the output; the batch norm of the input's channels in LDS
     const uint64_t most = 1ull << 30;
     const uint64_t a = (uint64_t)c.N * c.H * c.W * c.C, w = (uint64_t)c.kh * c.kw * c.C * c.K;
     const uint64_t rows = (uint64_t)c.M * c.Ro * c.So;

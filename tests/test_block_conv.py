@@ -87,10 +87,11 @@ def bottleneck64(p, params, no_activation):
         if i or not no_activation:
             g, b, m, v = (t.detach().cpu().double().view(1, -1, 1, 1) for t in bn)
             scale = g / (v + sc.BN_EPS).sqrt()
-            err = scale.abs() * err + 8 * U * ((p * scale).abs() + (m * scale).abs() + b.abs())
-            p = torch.relu(p * scale + b - m * scale)
+            # the mean comes off first, so what is rounded is the distance from it
+            err = scale.abs() * err + 8 * U * (((p - m) * scale).abs() + b.abs())
+            p = torch.relu((p - m) * scale + b)
         w64 = w.detach().cpu().double().permute(3, 2, 0, 1)
-        n = w64[0].numel()
+        n = int((w64 != 0).sum((1, 2, 3)).max())   # (a product with zero rounds nothing)
         err = F.conv2d(err + n * U * p.abs(), w64.abs())
         p = F.conv2d(p, w64)
     return p.permute(0, 2, 3, 1), err.permute(0, 2, 3, 1)
@@ -128,6 +129,32 @@ def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
         most[n, bh * Ro:(bh + 1) * Ro, bw * So:(bw + 1) * So] = bound[i, :part.shape[0], :part.shape[1]] + U * part.abs()
     err = (y.cpu().double() - want).abs()
     assert bool((err <= most + 1e-30).all()), float((err / (most + 1e-30)).max())
+
+
+@pytest.mark.parametrize("ratio", [10.0, 1000.0])
+@pytest.mark.parametrize("C", [16, 18])
+@pytest.mark.parametrize("no_activation", [False, True])
+def test_batch_norm_of_values_far_from_zero(C, no_activation, ratio):
+    """Channels whose mean is many times their spread, in front of the first convolution or, with kernels that only pass
+    pixels on, behind it: the result is off by the rounding of the distance from the mean, not of the mean."""
+    shape, ksizes = (1, 30, 41), [[1, 1, C, C], [3, 3, C, C], [1, 1, C, C]]
+    bp = sbnet_amd.calc_block_params_res_block([*shape, C], [1, 9, 9, 1], ksizes, [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(*shape, 1, device=DEV), bp, 0.0)
+    M = int(ind.bin_counts[0])
+    params = sc.BottleneckParams(ksizes, DEV, seed=C)
+    rng = np.random.default_rng(C)
+    x = torch.from_numpy((ratio + rng.standard_normal((*shape, C))).astype(np.float32))
+    with torch.no_grad():
+        for w in params.w:
+            w.zero_()[w.shape[0] // 2, w.shape[1] // 2].copy_(torch.eye(C))
+        bn = params.bn[1 if no_activation else 0]
+        bn.moving_mean.copy_(torch.from_numpy((ratio + 0.1 * rng.standard_normal(C)).astype(np.float32)))
+        q = sc._block_bottleneck(x.to(DEV), params, ind, bp, no_activation, False)
+    idx = ind.active_block_indices[:M].cpu()
+    # (nothing is rounded in front of that batch norm; pixels outside the image are as far from the mean as it is from 0)
+    want, bound = bottleneck64(blocks64(x, idx, bp.bsize, bp.bstrides, bp.boffset), params, no_activation)
+    err = (q.cpu().double() - want).abs()
+    assert bool((err <= bound + 1e-30).all()), float((err / (bound + 1e-30)).max())
 
 
 @pytest.mark.parametrize("use_var", [False, True])
