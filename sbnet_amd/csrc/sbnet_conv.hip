@@ -70,6 +70,10 @@ __device__ __forceinline__ void bn_read(const BnArgs& bn, uint32_t c, float& mea
     beta = bn.beta[c];
 }
 
+// Channels of the input's batch norm in LDS: the last four, past the end, make zeros of the zeros that k past the end reads
+// (any channel's own could make an infinity, which the zero weights turn into NaN).
+__host__ __device__ constexpr uint32_t pre_channels(int C) { return (((uint32_t)C + 3u) & ~3u) + 4u; }
+
 // GRAD: the gradient of a convolution's input.  The same product with the kernel turned around, w [K, kh, kw, C] (n, then
 // k: a lane's four k are one 16-byte load of w, too); the epilogue masks the result where the ReLU did and adds up what
 // the batch norm's gradient needs, in fp32 over 16 pixels and in double from there on.
@@ -85,7 +89,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     constexpr int WAVES = 4, WP = WAVES / WK;
     constexpr int TP = 16 * WP, TN = 16 * FN;
     extern __shared__ float lds[];
-    const uint32_t cPad = PRE ? ((uint32_t)a.c.C + 3u) & ~3u : 0u;
+    const uint32_t cPad = PRE ? pre_channels(a.c.C) : 0u;
     float *const preMean = lds, *const preScale = lds + cPad, *const preBeta = lds + 2 * cPad;
     float *const postMean = lds + 3 * cPad, *const postScale = postMean + TN;   // (GRAD: mean and 1 / sigma)
     float* const postBeta = postMean + 2 * TN;                            // not GRAD
@@ -205,7 +209,7 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
                     for (int i = 0; i < 4; ++i) o.wv[f][i] = v[i];
                 }
             }
-            if constexpr (PRE) o.c[j] = TAPS ? t.c : min(t.c, C - (VEC == 4 ? 4u : 1u));   // (the batch norm of some channel, past the end)
+            if constexpr (PRE) o.c[j] = TAPS ? (t.k >= a.kTot ? cPad - 4u : t.c) : min(t.c, cPad - 4u);
             if constexpr (TAPS) bad |= (uint32_t)((unsigned)t.h >= (unsigned)a.c.H) | (uint32_t)((unsigned)t.w >= (unsigned)a.c.W);
             else bad |= (uint32_t)!pixelOk;
             const uint32_t off = t.off | (0u - bad);
@@ -246,7 +250,13 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
     }
 
     if (PRE)
-        for (uint32_t c = tid; c < (uint32_t)a.c.C; c += 64 * WAVES) bn_read(a.c.pre, c, preMean[c], preScale[c], preBeta[c]);
+        for (uint32_t c = tid; c < cPad; c += 64 * WAVES) {
+            float mean = 0.f, scale = 0.f, beta = 0.f;
+            if (c < C) bn_read(a.c.pre, c, mean, scale, beta);
+            preMean[c] = mean;
+            preScale[c] = scale;
+            preBeta[c] = beta;
+        }
     if constexpr (GRAD) {
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES) {
             const uint32_t n = min(n0 + i, K - 1);
@@ -431,7 +441,7 @@ static hipError_t launch_conv_as(ConvKernelArgs& a, hipStream_t stream)
     a.tilesP = (a.rows + TP - 1) / TP;
     a.tilesN = ((uint32_t)a.c.K + TN - 1) / TN;
     const uint64_t grid = (uint64_t)((a.tilesP + 7) / 8 * 8) * a.tilesN;
-    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 3 * (((size_t)a.c.C + 3) & ~(size_t)3) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 3) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
+    const size_t lds = sizeof(float) * ((a.c.pre.gamma ? 3 * (size_t)pre_channels(a.c.C) : 0) + (GRAD ? 2 + 4 * (WAVES / WK) : 3) * TN + (WK > 1 ? (size_t)WAVES * FN * 256 : 0));
     if (grid >= (1ull << 31) || lds > 64 * 1024) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((k_block_conv<FN, WK, VEC, PRE, TAPS, GRAD, NEXT>), dim3((unsigned)grid), dim3(64 * WAVES), lds, stream, a);
     return hipGetLastError();

@@ -157,6 +157,21 @@ def test_batch_norm_of_values_far_from_zero(C, no_activation, ratio):
     assert bool((err <= bound + 1e-30).all()), float((err / (bound + 1e-30)).max())
 
 
+@pytest.mark.parametrize("C,kh", [(18, 1), (20, 1), (20, 3), (18, 3), (5, 3)])   # k ends inside a step of sixteen
+def test_infinite_shift_of_a_channel_stays_infinite(C, kh):
+    """Infinities where the exact result has them, and no NaN out of the places past the last k."""
+    shape, ksizes = (1, 30, 41), [[kh, kh, C, 8], [1, 1, 8, 8], [1, 1, 8, C]]
+    bp = sbnet_amd.calc_block_params_res_block([*shape, C], [1, 9, 9, 1], ksizes, [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(*shape, 1, device=DEV), bp, 0.0)
+    params = sc.BottleneckParams(ksizes, DEV, seed=C)
+    with torch.no_grad():
+        for w in params.w:
+            w.abs_()
+        params.bn[0].beta[-1] = float("inf")
+        q = sc._block_bottleneck(torch.randn(*shape, C, device=DEV), params, ind, bp, False, False)
+    assert bool((q == float("inf")).all())
+
+
 @pytest.mark.parametrize("use_var", [False, True])
 @pytest.mark.parametrize("C,mid,bsize,shape", [(40, 36, 9, (2, 33, 41)),       # three fragments in between, the last a quarter full
                                                (132, 84, 11, (1, 60, 44)),     # six; output tiles of 64 channels and a rest
