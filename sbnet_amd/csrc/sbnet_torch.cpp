@@ -401,7 +401,8 @@ PyObject* block_conv(PyObject* const* a)
 }
 
 // block_bottleneck(x, [w1, w2, w3], [gamma, beta, mean, var] * 3, bin_counts, active_block_indices, bsize, bstride,
-//                  boffset, out_stride, eps, no_activation, in_place) -> NHWC stack, or x with the result added
+//                  boffset, out_stride, eps, no_activation, in_place) -> NHWC stack, or x with the result added; with
+// no_activation the first four are not looked at
 PyObject* block_bottleneck(PyObject* const* a)
 {
     const at::Tensor* x = plain_f32(a[0]);
@@ -422,9 +423,11 @@ PyObject* block_bottleneck(PyObject* const* a)
         if (!w || w->device() != x->device() || !kernel_of(*w, C, R, S, wd + 4 * i)) Py_RETURN_NONE;
         weights[i] = static_cast<const float*>(w->data_ptr());
         for (int j = 0; j < 4; ++j) {
+            norms[4 * i + j] = nullptr;
+            if (i == 0 && no_activation) continue;
             const at::Tensor* t = plain_f32(PyList_GET_ITEM(a[2], 4 * i + j));
             if (!t || t->device() != x->device() || t->numel() != C) Py_RETURN_NONE;
-            norms[4 * i + j] = i == 0 && no_activation ? nullptr : static_cast<const float*>(t->data_ptr());
+            norms[4 * i + j] = static_cast<const float*>(t->data_ptr());
         }
         R -= wd[4 * i] - 1;
         S -= wd[4 * i + 1] - 1;

@@ -333,8 +333,10 @@ def res_block_bottleneck(x, params, strides, is_training, data_format="NHWC", w_
 def _block_bottleneck(x, params, indices, block_params, no_activation, in_place):
     """The residual function of the active blocks in inference: added to x (returns x) or as an NHWC stack; None where
     only the composed path applies."""
+    norms = [[None] * 4 if no_activation and not i else [b.gamma, b.beta, b.moving_mean, b.moving_var]
+             for i, b in enumerate(params.bn)]
     return (ops._native or ops._load_native()).block_bottleneck(
-        x, params.w, [t for b in params.bn for t in b], indices.bin_counts, indices.active_block_indices, block_params.bsize,
+        x, params.w, sum(norms, []), indices.bin_counts, indices.active_block_indices, block_params.bsize,
         block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
@@ -385,13 +387,15 @@ class _ResidualInTraining(torch.autograd.Function):
 def _own_residual_gradient(p, params):
     """Whether _ResidualInTraining applies: not under forward-mode or functorch transforms, autocast, or where deterministic
     algorithms are asked for (its batch norm sums are added up with atomics, in double)."""
-    tensors = [p, *params.w, *(t for b in params.bn for t in b)]
+    tensors = [p, *params.w, *(t for b in params.bn for t in (b.gamma, b.beta))]
+    stats = [t for b in params.bn for t in (b.moving_mean, b.moving_var) if t is not None]
     return (torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
             torch._C._functorch.peek_interpreter_stack() is None and not torch.is_autocast_enabled("cuda") and
-            not torch.are_deterministic_algorithms_enabled() and len(tensors) == 16 and
-            all(t.is_cuda and t.dtype is torch.float32 and t.is_contiguous() for t in tensors) and
+            not torch.are_deterministic_algorithms_enabled() and len(tensors) == 10 and
+            all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32 and t.is_contiguous()
+                for t in tensors + stats) and
             all(w.dim() == 4 and w.shape[2] % 4 == 0 and w.shape[3] % 4 == 0 for w in params.w) and
-            not any(b.moving_mean.requires_grad or b.moving_var.requires_grad for b in params.bn) and
+            not any(t.requires_grad for t in stats) and
             p.shape[0] * (p.shape[2] - sum(w.shape[0] - 1 for w in params.w[:2])) *
             (p.shape[3] - sum(w.shape[1] - 1 for w in params.w[:2])) >= 2)
 

@@ -4,6 +4,8 @@ The bound travels with the values: each step passes on the error it received thr
 coefficients and adds its own sums' n * 2^-24 * sum |a| * |b| (any order of the sum); batch norm's own arithmetic is a
 handful of roundings per value.
 """
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -142,3 +144,21 @@ def test_kernel_changed_between_forward_and_backward():
     second = torch.autograd.grad(y, tensors, torch.ones_like(y))
     for a, b in zip(first, second):
         assert float((a - b).norm()) <= 1e-6 * float(a.norm())
+
+
+@pytest.mark.parametrize("is_training,no_activation", [(True, False), (True, True), (False, True)])
+def test_blocks_without_running_statistics_or_a_first_batch_norm(is_training, no_activation):
+    """What a block does not use may be absent, and the batch norms' parameters may come in any object with their names."""
+    bp, ind, params, x = make_block()
+    x = x.detach()
+    with torch.no_grad():
+        want = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], is_training, "NCHW", no_activation=no_activation)
+    params.bn = [types.SimpleNamespace(**b._asdict()) for b in params.bn]
+    for b in params.bn if is_training else ():
+        b.moving_mean = b.moving_var = None
+    if no_activation:
+        params.bn[0] = None
+    for grad in (False, is_training):
+        with torch.set_grad_enabled(grad):
+            y = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], is_training, "NCHW", no_activation=no_activation)
+        assert torch.equal(y, want)
