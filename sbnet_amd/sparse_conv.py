@@ -24,7 +24,6 @@ are in own kernels, too (sbnet_block_grad.hip).
 """
 import collections
 import ctypes
-import types
 
 import torch
 import torch.nn.functional as F
@@ -340,9 +339,36 @@ def _block_bottleneck(x, params, indices, block_params, no_activation, in_place)
         block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
+class _AsItWas(torch.autograd.Function):
+    """The value a tensor had, with the gradient going to the tensor as it is now."""
+
+    @staticmethod
+    def forward(ctx, tensor, value):
+        return value.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return grad, None
+
+
+class _ReluAsItWas(torch.autograd.Function):
+    """A ReLU whose result is known."""
+
+    @staticmethod
+    def forward(ctx, x, result):
+        ctx.save_for_backward(result)
+        return result.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        result, = ctx.saved_tensors
+        return torch.where(result <= 0, torch.zeros_like(grad), grad), None
+
+
 class _ResidualInTraining(torch.autograd.Function):
     """_bottleneck_residual of a planar block stack with batch statistics: forward as there, the gradients in this package's
-    own kernels (sbnet_block_grad.hip)."""
+    own kernels (sbnet_block_grad.hip).  As there, what is kept of a kernel is a copy and of a beta nothing, so that both may
+    change before backward."""
 
     @staticmethod
     def forward(ctx, p, moving, *tensors):   # tensors: kernel, gamma and beta of each layer
@@ -354,8 +380,8 @@ class _ResidualInTraining(torch.autograd.Function):
             w_ = _hwio_to_oihw(w)
             saved += [z, a.relu_(), mean, inv, w_, gamma]
             z = F.conv2d(a, w_, stride=(1, 1))
-        ctx.save_for_backward(*saved, *tensors[2::3])
-        ctx.kernels = [(w, w._version) for w in tensors[::3]]   # for a graph of the gradients alone
+        ctx.save_for_backward(*saved)
+        ctx.layers = [(tensors[i], tensors[i + 2]) for i in (0, 3, 6)]   # for a graph of the gradients alone
         return z
 
     @staticmethod
@@ -363,7 +389,7 @@ class _ResidualInTraining(torch.autograd.Function):
         saved = ctx.saved_tensors
         create_graph = torch.is_grad_enabled()
         if not create_graph:
-            grads = ops._native.bottleneck_grad(dq.contiguous(), list(saved[:18]))
+            grads = ops._native.bottleneck_grad(dq.contiguous(), list(saved))
             if grads is not None:
                 dp, dw1, dw2, dw3, *norms = grads
                 return dp, None, dw1, norms[0], norms[1], dw2, norms[2], norms[3], dw3, norms[4], norms[5]
@@ -371,14 +397,16 @@ class _ResidualInTraining(torch.autograd.Function):
         wanted = [ctx.needs_input_grad[0], *ctx.needs_input_grad[2:]]
         with torch.enable_grad():
             inputs = [saved[0]]
-            for i, (w, version) in enumerate(ctx.kernels):
-                if create_graph and w._version != version:
-                    raise RuntimeError("a kernel needed for gradient computation has been modified by an inplace operation")
-                inputs += [w if create_graph else saved[6 * i + 4].permute(2, 3, 1, 0), saved[6 * i + 5], saved[18 + i]]
+            for i, (w, beta) in enumerate(ctx.layers):
+                inputs += [w, saved[6 * i + 5], beta]
             if not create_graph:
                 inputs = [t.detach().requires_grad_() for t in inputs]
-            layers = types.SimpleNamespace(w=inputs[1::3], bn=[BatchNormParams(*inputs[i:i + 2], None, None) for i in (2, 5, 8)])
-            q = _bottleneck_residual(inputs[0], layers, [1, 1, 1, 1], "VALID", True, "NCHW")
+            q = inputs[0]
+            for i in range(3):
+                w, gamma, beta = inputs[1 + 3 * i:4 + 3 * i]
+                y = _batch_norm(q, BatchNormParams(gamma, beta, None, None), True, True)
+                w_ = _AsItWas.apply(_hwio_to_oihw(w), saved[6 * i + 4])
+                q = F.conv2d(_ReluAsItWas.apply(y, saved[6 * i + 1]), w_)
             found = iter(torch.autograd.grad(q, [t for t, n in zip(inputs, wanted) if n], dq, create_graph=create_graph))
         grads = [next(found) if n else None for n in wanted]
         return (grads[0], None, *grads[1:])

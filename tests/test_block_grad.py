@@ -146,6 +146,28 @@ def test_kernel_changed_between_forward_and_backward():
         assert float((a - b).norm()) <= 1e-6 * float(a.norm())
 
 
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_kernels_and_betas_changed_between_forward_and_backward(create_graph):
+    """No gradient depends on what a beta or a kernel is by the time of backward; nor does a gradient's gradient."""
+    results = []
+    for change in (False, True):
+        bp, ind, params, x = make_block()
+        tensors = [x, *params.parameters()]
+        y = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], True, data_format="NCHW")
+        if change:
+            with torch.no_grad():
+                for t in [*params.w, *(b.beta for b in params.bn)]:
+                    t.add_(1.0)
+        grads = torch.autograd.grad(y, tensors, torch.ones_like(y), create_graph=create_graph)
+        if create_graph:
+            grads = grads + torch.autograd.grad(sum((g * g).sum() for g in grads), tensors)
+        results.append([g.detach() for g in grads])
+    # The same sums, in an order that the library is free in: six of them one behind the other, over up to 2025 pixels, are
+    # off by about 6 * 2025 ** 0.5 * 2^-24 = 1.6e-5, the gradients' own cancellation not counted.
+    for a, b in zip(*results):
+        assert float((a - b).norm()) <= 1e-4 * float(a.norm())
+
+
 @pytest.mark.parametrize("is_training,no_activation", [(True, False), (True, True), (False, True)])
 def test_blocks_without_running_statistics_or_a_first_batch_norm(is_training, no_activation):
     """What a block does not use may be absent, and the batch norms' parameters may come in any object with their names."""
