@@ -351,7 +351,8 @@ int sbnet_sparse_scatter_base_grad(const float* dy, int32_t num_active, const in
    of the stack (replaces the backward of the layers of sparse_conv_lib.py:677-723 with is_training).  For i = 0, 1, 2:
    z[i] [num_blocks, C, R, S] in front of batch norm i (z[0] is the gathered stack), act[i] behind its ReLU, mean[i] and
    inv[i] = 1 / sqrt(variance + eps) of the batch, gamma[i]; weights[i] [K,C,kh,kw], w_dims[4 * i ...] = kh, kw, C, K.
-   dq: the gradient of the third convolution's result -> dp that of z[0], both planar; dw[i] [kh,kw,C,K]; dgamma, dbeta.
+   dq: the gradient of the third convolution's result -> dp that of z[0], both planar; dw[i] [kh,kw,C,K]; dgamma[i],
+   dbeta[i].  NULL for any of these ten: not asked for, and what only they need is not computed.
    Channels in multiples of four; dw and workspace 16-byte aligned; at least two pixels per channel everywhere.
    workspace: sbnet_bottleneck_grad_workspace_bytes() bytes (0: the sizes are not taken), any contents. */
 size_t sbnet_bottleneck_grad_workspace_bytes(int32_t num_blocks, const int32_t* bsize, const int32_t* w_dims);

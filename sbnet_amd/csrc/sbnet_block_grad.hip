@@ -58,8 +58,8 @@ __global__ __launch_bounds__(256) void k_norm_grad(float* __restrict__ g, NormGr
         c1[j] = (float)(s1 / a.rows);
         c2[j] = (float)(s2 / a.rows * inv);
         if (blockIdx.x == 0 && ty == 0) {
-            dgamma[c + j] = (float)s2;
-            dbeta[c + j] = (float)s1;
+            if (dgamma) dgamma[c + j] = (float)s2;
+            if (dbeta) dbeta[c + j] = (float)s1;
         }
     }
     const float* const z = norm.z;

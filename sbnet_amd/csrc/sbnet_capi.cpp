@@ -11,6 +11,7 @@
 #include <hip/hip_runtime_api.h>
 #include <sched.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -778,7 +779,16 @@ static bool bottleneck_grad_plan(int32_t num_blocks, const int32_t* bsize, const
         b.kernel[i] = take(at, sizeof(float) * (uint64_t)c.K * c.kh * c.kw * c.C);
     }
     b.dz[3] = take(at, sizeof(float) * (uint64_t)num_blocks * R * S * b.c[2].C);
-    b.part = take(at, sbnet::wgrad_workspace_bytes(b.w, 3));
+    // (the pixels are split by how many kernels there are to do: the most that any of them together need)
+    size_t part = 0;
+    for (int s = 1; s < 8; ++s) {
+        sbnet::WgradArgs w[3];
+        int n = 0;
+        for (int i = 0; i < 3; ++i)
+            if (s >> i & 1) w[n++] = b.w[i];
+        part = std::max(part, sbnet::wgrad_workspace_bytes(w, n));
+    }
+    b.part = take(at, part);
     b.total = at;
     return true;
 }
@@ -796,14 +806,20 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
                           size_t workspace_bytes, void* stream)
 {
     BottleneckGrad b;
-    if (!dq || !z || !act || !mean || !inv || !gamma || !weights || !dp || !dw || !dgamma || !dbeta || !workspace ||
+    if (!dq || !z || !act || !mean || !inv || !gamma || !weights || !dw || !dgamma || !dbeta || !workspace ||
         (reinterpret_cast<uintptr_t>(workspace) & 15) || !bottleneck_grad_plan(num_blocks, bsize, w_dims, b) ||
         workspace_bytes < b.total)
         return SBNET_EINVAL_ARG;
     for (int i = 0; i < 3; ++i)
-        if (!z[i] || !act[i] || !mean[i] || !inv[i] || !gamma[i] || !weights[i] || !dw[i] || !dgamma[i] || !dbeta[i] ||
-            (reinterpret_cast<uintptr_t>(dw[i]) & 15))
+        if (!z[i] || !act[i] || !mean[i] || !inv[i] || !gamma[i] || !weights[i] || (reinterpret_cast<uintptr_t>(dw[i]) & 15))
             return SBNET_EINVAL_ARG;
+    // how far down the gradient has to go: whether batch norm i or anything in front of it has one that is asked for
+    bool needs[3], any = dp != nullptr;
+    for (int i = 0; i < 3; ++i) {
+        needs[i] = any = any || dgamma[i] || dbeta[i];
+        any = any || dw[i];
+    }
+    if (!any) return SBNET_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint8_t* const ws = static_cast<uint8_t*>(workspace);
     auto at = [&](size_t offset) { return reinterpret_cast<float*>(ws + offset); };
@@ -813,14 +829,14 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
     for (int i = 0; i < 3; ++i) {
         const sbnet::ConvArgs& c = b.c[i];
         const uint32_t M = (uint32_t)num_blocks, C = (uint32_t)c.K, P = (uint32_t)(c.Ro * c.So);
-        t[n++] = sbnet::TransposeArgs{z[i], at(b.z[i]), M, C, P};
-        t[n++] = sbnet::TransposeArgs{act[i], at(b.act[i]), M, C, P};
-        t[n++] = sbnet::TransposeArgs{weights[i], at(b.kernel[i]), 1, (uint32_t)c.C, C * (uint32_t)(c.kh * c.kw)};
+        if (needs[i]) t[n++] = sbnet::TransposeArgs{z[i], at(b.z[i]), M, C, P};
+        if (needs[i] || dw[i]) t[n++] = sbnet::TransposeArgs{act[i], at(b.act[i]), M, C, P};
+        if (needs[i]) t[n++] = sbnet::TransposeArgs{weights[i], at(b.kernel[i]), 1, (uint32_t)c.C, C * (uint32_t)(c.kh * c.kw)};
     }
     t[n++] = sbnet::TransposeArgs{dq, at(b.dz[3]), (uint32_t)num_blocks, (uint32_t)b.c[2].C, (uint32_t)(b.c[2].H * b.c[2].W)};
-    SBNET_HIP(sbnet::launch_zero(at(0), b.sumBytes / sizeof(float), s));
+    if (needs[2]) SBNET_HIP(sbnet::launch_zero(at(0), b.sumBytes / sizeof(float), s));
     SBNET_HIP(sbnet::launch_transposes(t, n, s));
-    for (int i = 2; i >= 0; --i) {
+    for (int i = 2; i >= 0 && needs[i]; --i) {
         sbnet::ConvArgs& c = b.c[i];
         c.a = at(b.dz[i + 1]);
         c.w = at(b.kernel[i]);
@@ -828,11 +844,18 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
         c.norm = sbnet::NormGradArgs{at(b.z[i]), at(b.act[i]), mean[i], inv[i], gamma[i], reinterpret_cast<double*>(ws + b.sums[i])};
         SBNET_HIP(sbnet::launch_block_conv_grad(c, s));
         SBNET_HIP(sbnet::launch_norm_grad(at(b.dz[i]), c.norm, (uint32_t)(c.M * c.Ro * c.So), c.K, dgamma[i], dbeta[i], s));
+    }
+    sbnet::WgradArgs w[3];
+    int kernels = 0;
+    for (int i = 0; i < 3; ++i) {
+        if (!dw[i]) continue;
         b.w[i].act = at(b.act[i]);
         b.w[i].dz = at(b.dz[i + 1]);
         b.w[i].dw = dw[i];
+        w[kernels++] = b.w[i];
     }
-    SBNET_HIP(sbnet::launch_wgrad(b.w, 3, ws + b.part, s));
+    if (kernels) SBNET_HIP(sbnet::launch_wgrad(w, kernels, ws + b.part, s));
+    if (!dp) return SBNET_OK;
     t[0] = sbnet::TransposeArgs{at(b.dz[0]), dp, (uint32_t)num_blocks, (uint32_t)(b.c[0].Ro * b.c[0].So), (uint32_t)b.c[0].K};
     SBNET_HIP(sbnet::launch_transposes(t, 1, s));
     return SBNET_OK;

@@ -61,7 +61,8 @@ hipError_t launch_block_conv_next(const ConvArgs& c, const ConvArgs& next, hipSt
 bool conv_grad_fits(const ConvArgs& c);
 hipError_t launch_block_conv_grad(const ConvArgs& c, hipStream_t stream);
 
-// Backward of the batch norm: g [rows, C], behind the mask, becomes the gradient of z in place; dgamma, dbeta.
+// Backward of the batch norm: g [rows, C], behind the mask, becomes the gradient of z in place; dgamma, dbeta (nullptr: not
+// asked for).
 hipError_t launch_norm_grad(float* g, const NormGradArgs& norm, uint32_t rows, int C, float* dgamma, float* dbeta,
                             hipStream_t stream);
 

@@ -159,13 +159,19 @@ bool call(F f)
     return false;
 }
 
-// A function of the module: N arguments, and no C++ exception through the interpreter's frames.
-template <PyObject* (*F)(PyObject* const*), Py_ssize_t N>
+// A function of the module: N arguments, of which those after the first FEWEST may be missing (None), and no C++ exception
+// through the interpreter's frames.
+template <PyObject* (*F)(PyObject* const*), Py_ssize_t N, Py_ssize_t FEWEST = N>
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    if (n != N) {
+    if (n > N || n < FEWEST) {
         PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", N, n);
         return nullptr;
+    }
+    PyObject* all[N];
+    if constexpr (FEWEST < N) {
+        for (Py_ssize_t i = 0; i < N; ++i) all[i] = i < n ? a[i] : Py_None;
+        a = all;
     }
     try {
         return F(a);
@@ -176,11 +182,11 @@ PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n)
 }
 
 // The same for an op: left to the general wrappers while something looks on at torch's operators.
-template <PyObject* (*F)(PyObject* const*), Py_ssize_t N>
+template <PyObject* (*F)(PyObject* const*), Py_ssize_t N, Py_ssize_t FEWEST = N>
 PyObject* op_entry(PyObject* self, PyObject* const* a, Py_ssize_t n)
 {
     if (c10::impl::TorchDispatchModeTLS::any_modes_set()) Py_RETURN_NONE;
-    return entry<F, N>(self, a, n);
+    return entry<F, N, FEWEST>(self, a, n);
 }
 
 // reduce_mask(mask, bcount, bsize, bstride, boffset, tol, avgpool, sync) -> (active_block_indices, bin_counts)
@@ -457,12 +463,16 @@ PyObject* block_bottleneck(PyObject* const* a)
     return THPVariable_Wrap(std::move(q));
 }
 
-// bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1, ...), on
-// planar stacks, or None where the kernels do not take the sizes.
+// bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3, wanted) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1,
+// ...), on planar stacks, or None where the kernels do not take the sizes.  wanted: a tuple with the truth of each of the
+// ten, those not wanted are None; all where it is missing.
 PyObject* bottleneck_grad(PyObject* const* a)
 {
     const at::Tensor* dq = dev_f32(a[0]);
     if (!dq || dq->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 18) Py_RETURN_NONE;
+    bool wanted[10];
+    if (a[2] != Py_None && (!PyTuple_CheckExact(a[2]) || PyTuple_GET_SIZE(a[2]) != 10)) Py_RETURN_NONE;
+    for (int i = 0; i < 10; ++i) wanted[i] = a[2] == Py_None || PyTuple_GET_ITEM(a[2], i) == Py_True;
     const at::Tensor* t[18];
     const float* ptr[6][3];
     for (int i = 0; i < 18; ++i) {
@@ -497,14 +507,14 @@ PyObject* bottleneck_grad(PyObject* const* a)
     c10::DeviceGuard guard(dq->device());
     at::Tensor res[10];
     float *out[10];
-    res[0] = empty_f32(t[0]->sizes(), *dq);
+    if (wanted[0]) res[0] = empty_f32(t[0]->sizes(), *dq);
     for (int i = 0; i < 3; ++i) {
         const int32_t* d = wd + 4 * i;
-        res[1 + i] = empty_f32({d[0], d[1], d[2], d[3]}, *dq);
-        res[4 + 2 * i] = empty_f32({d[2]}, *dq);
-        res[5 + 2 * i] = empty_f32({d[2]}, *dq);
+        if (wanted[1 + i]) res[1 + i] = empty_f32({d[0], d[1], d[2], d[3]}, *dq);
+        if (wanted[4 + 2 * i]) res[4 + 2 * i] = empty_f32({d[2]}, *dq);
+        if (wanted[5 + 2 * i]) res[5 + 2 * i] = empty_f32({d[2]}, *dq);
     }
-    for (int i = 0; i < 10; ++i) out[i] = static_cast<float*>(res[i].data_ptr());
+    for (int i = 0; i < 10; ++i) out[i] = wanted[i] ? static_cast<float*>(res[i].data_ptr()) : nullptr;
     float *const dgamma[3] = {out[4], out[6], out[8]}, *const dbeta[3] = {out[5], out[7], out[9]};
     at::Tensor ws = own_scratch(*dq, need);
     const float* const dqp = static_cast<const float*>(dq->data_ptr());
@@ -516,7 +526,10 @@ PyObject* bottleneck_grad(PyObject* const* a)
         return nullptr;
     PyObject* r = PyTuple_New(10);
     if (!r) return nullptr;
-    for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(res[i])));
+    for (int i = 0; i < 10; ++i) {
+        PyObject* const o = wanted[i] ? THPVariable_Wrap(std::move(res[i])) : (Py_INCREF(Py_None), Py_None);
+        PyTuple_SET_ITEM(r, i, o);
+    }
     return r;
 }
 
@@ -557,7 +570,7 @@ PyMethodDef methods[] = {
     {"scatter_base_grad", fast(op_entry<scatter_base_grad, 6>), METH_FASTCALL, nullptr},
     {"block_conv", fast(op_entry<block_conv, 7>), METH_FASTCALL, nullptr},
     {"block_bottleneck", fast(op_entry<block_bottleneck, 12>), METH_FASTCALL, nullptr},
-    {"bottleneck_grad", fast(op_entry<bottleneck_grad, 2>), METH_FASTCALL, nullptr},
+    {"bottleneck_grad", fast(op_entry<bottleneck_grad, 3, 2>), METH_FASTCALL, nullptr},
     {"workspace", fast(entry<workspace_py, 2>), METH_FASTCALL, nullptr},
     {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},

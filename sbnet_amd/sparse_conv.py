@@ -389,7 +389,9 @@ class _ResidualInTraining(torch.autograd.Function):
         saved = ctx.saved_tensors
         create_graph = torch.is_grad_enabled()
         if not create_graph:
-            grads = ops._native.bottleneck_grad(dq.contiguous(), list(saved))
+            n = ctx.needs_input_grad
+            wanted = (n[0], n[2], n[5], n[8], n[3], n[4], n[6], n[7], n[9], n[10])
+            grads = ops._native.bottleneck_grad(dq.contiguous(), list(saved), wanted)
             if grads is not None:
                 dp, dw1, dw2, dw3, *norms = grads
                 return dp, None, dw1, norms[0], norms[1], dw2, norms[2], norms[3], dw3, norms[4], norms[5]

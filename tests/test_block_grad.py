@@ -95,6 +95,39 @@ def test_gradients_of_a_bottleneck(M, bsize, ksizes):
         assert bool((err <= 2 * bound + 1e-30).all()), (k, float((err / (2 * bound + 1e-30)).max()))
 
 
+ALL = range(10)
+
+
+@pytest.mark.parametrize("wanted", [(), (0,), (1,), (2,), (3,), (4,), (7,), (9,), (1, 3), (2, 4), (0, 2, 8), (1, 2, 3), (4, 5, 6, 7, 8, 9)])
+def test_gradients_that_are_not_wanted(wanted):
+    """Any of dp, dw1-3 and the batch norms' six alone: the others are None, and what they need is not in the way."""
+    M, bsize, ksizes = CASES[2]
+    saved, dq = forward32(np.random.default_rng(M), M, bsize, ksizes)
+    dp, dws, norms = backward64(saved, dq)
+    want = [dp, *dws, *(pair for n in norms for pair in n)]
+    got = ops._load_native().bottleneck_grad(dq.to(DEV), [t.to(DEV) for t in saved], tuple(k in wanted for k in ALL))
+    for k, (value, (exact, bound)) in enumerate(zip(got, want)):
+        assert (value is not None) == (k in wanted)
+        if value is not None:
+            err = (value.cpu().double() - exact).abs()
+            assert bool((err <= 2 * bound + 1e-30).all()), (k, float((err / (2 * bound + 1e-30)).max()))
+
+
+def test_frozen_kernels_and_input():
+    """What requires no gradient gets none; the rest is what it is with everything wanted."""
+    results = []
+    for frozen in (False, True):
+        bp, ind, params, x = make_block()
+        if frozen:
+            x = x.detach()
+            for w in params.w:
+                w.requires_grad_(False)
+        y = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], True, data_format="NCHW")
+        results.append(torch.autograd.grad(y, [t for b in params.bn for t in b[:2]], torch.cos(y.detach())))
+    for a, b in zip(*results):   # (the order in which the sums' atomics arrive is free)
+        assert float((a - b).norm()) <= 1e-5 * float(a.norm())
+
+
 def make_block(C=16, mid=8):
     ksizes = [[1, 1, C, mid], [3, 3, mid, mid], [1, 1, mid, C]]
     bp = sbnet_amd.calc_block_params_res_block([1, 30, 33, C], [1, 9, 9, 1], ksizes, [1, 1, 1, 1], "SAME")
