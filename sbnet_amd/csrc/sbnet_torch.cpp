@@ -381,6 +381,26 @@ bool kernel_of(const at::Tensor& w, int64_t C, int64_t R, int64_t S, int32_t* di
 
 bool positive(const Pair& p) { return p.v[0] > 0 && p.v[1] > 0; }
 
+// Whether a convolution of `rows` output pixels is left to the library as the faster way (MI355X; us for library / own, the
+// layer in place on planar stacks, 17x17 and 24x24 blocks).
+bool library_is_faster(const int32_t* w, int64_t rows, bool aligned)
+{
+    const int64_t k = (int64_t)w[0] * w[1] * w[2], K = w[3];
+    if (aligned && w[2] % 4 == 0 && K % 4 == 0) {
+        // 3x3: the library's transforms save multiplications, which pays for many pixels of many channels.  128 channels:
+        // 66 / 61 at 4 GFLOP, 386 / 358 at 32, 691 / 764 at 69, 1391 / 1512 at 137; 256: 368 / 354, 676 / 680 at 64,
+        // 2635 / 2904 at 276; 512: 362 / 390 at 32, 1368 / 1476 at 129, 9874 / 12969 at 1105.  With 80 channels or fewer the
+        // two meet without crossing (406 / 415 with 64 at 34).  1x1 and 5x5 products of any size go either way with the
+        // block count (1x1, 512 channels: 644 / 570, 1284 / 1294; 5x5, 256: 592 / 681, 1790 / 1407, 2169 / 2560).
+        return w[0] == 3 && w[1] == 3 && w[2] > 80 && 2.0 * rows * k * K > 64e9;
+    }
+    // Single-float loads, at a third of the rate: only small products, in steps of 16 k times 16 channels.  30 channels,
+    // 3x3: 39 / 34 at 1.8 M steps, 53 / 55 at 3.7, 144 / 196 at 16; 50: 33 / 30 at 1.7, 46 / 51 at 3.2; 130: 64 / 65 at 4.5,
+    // 89 / 134 at 9.6.  Channels that fill no fragment read as many pixels for less: 3 channels, 3x3: 36 / 33 at 0.5,
+    // 57 / 56 at 0.9 (44 / 56 on NHWC stacks); 7x7: 50 / 38 at 0.9, 83 / 99 at 3.3.
+    return rows * ((k + 15) / 16) * ((K + 15) / 16) > (K < 16 ? 900000 : 2500000);
+}
+
 // block_conv(x, w, bin_counts, active_block_indices, bsize, bstride, boffset) -> NHWC stack
 PyObject* block_conv(PyObject* const* a)
 {
@@ -394,6 +414,8 @@ PyObject* block_conv(PyObject* const* a)
         Py_RETURN_NONE;
     const int64_t R = bs.v[0] - wd[0] + 1, S = bs.v[1] - wd[1] + 1;
     if (R * S >= ROWS_MOST || b.M * R * S >= ROWS_MOST || b.M * R * S * wd[3] >= 2 * CONV_MOST) Py_RETURN_NONE;
+    // (of a count on the device only the capacity is known, which the library would compute in full)
+    if (!b.count && library_is_faster(wd, b.M * R * S, (reinterpret_cast<uintptr_t>(x->const_data_ptr()) & 15) == 0)) Py_RETURN_NONE;
     c10::DeviceGuard guard(x->device());
     at::Tensor q = empty_f32({b.M, R, S, wd[3]}, *x);
     const float *const xp = static_cast<const float*>(x->data_ptr()), *const kp = static_cast<const float*>(w->data_ptr());

@@ -55,7 +55,8 @@ def _conv_blocks(p, w, stride, transpose):
 
 def _block_conv(x, w, indices, block_params):
     """VALID convolution (stride 1) of the active blocks as an NHWC stack, or None where only the composed path applies
-    (a gradient is asked for, tensors that are not contiguous float32, sizes beyond 32-bit byte offsets)."""
+    (a gradient is asked for, tensors that are not contiguous float32, sizes beyond 32-bit byte offsets, products for which
+    the library is faster)."""
     return (ops._native or ops._load_native()).block_conv(x, w, indices.bin_counts, indices.active_block_indices,
                                                           block_params.bsize, block_params.bstrides, block_params.boffset)
 
@@ -71,6 +72,11 @@ def sparse_conv2d_custom(x, w, indices, block_params, strides, use_var=False, tr
     if q is not None:
         transpose = False
     else:
+        # The stack's layout is nobody's to see, and from 16 channels on the library is the faster on planar ones: up to
+        # twice as fast for 3x3 products on most block counts (256 channels, 484 blocks of 24x24: 2635 against 5824 us),
+        # 8 % slower on some; with fewer channels it pays for its layout copies (3 channels, 465 000 pixels: 57 against 44).
+        transpose = transpose or (x.dim() == 4 and x.shape[3] >= 16 and
+                                  not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
         p = ops.sparse_gather(x, indices.bin_counts, indices.active_block_indices, block_params.bsize,
                               block_params.bstrides, block_params.boffset, transpose=transpose)
         q = _conv_blocks(p, w, 1, transpose)

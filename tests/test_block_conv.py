@@ -79,6 +79,34 @@ def test_block_conv(case, device_count):
     assert bool((err <= bound + 1e-30).all()), float((err / (bound + 1e-30)).max())
 
 
+@pytest.mark.parametrize("C,k,M,bsize,own", [
+    (12, 3, 3000, 18, True),      # narrow: however many pixels
+    (96, 3, 1500, 18, True),      # 63.7 GFLOP
+    (96, 3, 1550, 18, False),     # 65.8
+    (80, 3, 2400, 18, True),
+    (128, 1, 1500, 17, True),     # one tap
+    (30, 3, 280, 18, True),       # 2.4 and 2.6 million steps of 16 k times 16 channels
+    (30, 3, 300, 18, False),
+    (3, 7, 350, 22, True),        # 0.90 and 0.92
+    (3, 7, 360, 22, False),
+])
+def test_where_the_library_takes_over(C, k, M, bsize, own):
+    """The route of a product by its size; the two sides agree within the bound of a sum in any order, 2 * k * k * C * 2^-24
+    of the sum of absolute products."""
+    idx = torch.stack([torch.zeros(M, dtype=torch.int64), torch.arange(M) // 40, torch.arange(M) % 40], 1).to(torch.int16).to(DEV)
+    out = bsize - k + 1
+    bp = BlockParams(bsize=[bsize] * 2, bsize_out=[out] * 2, boffset=[-(k // 2)] * 2, bcount=None, bstrides=[out] * 2)
+    g = torch.Generator(DEV).manual_seed(C)
+    x = torch.rand(1, (M // 40 + 1) * out, 40 * out, C, device=DEV, generator=g)   # (positive: the sum itself)
+    w = torch.rand(k, k, C, C, device=DEV, generator=g)
+    ind = sbnet_amd.ReduceMaskResult(idx, torch.tensor([M], dtype=torch.int32))
+    assert (sc._block_conv(x, w, ind, bp) is not None) == own
+    on_device = sbnet_amd.ReduceMaskResult(idx, torch.tensor([M], dtype=torch.int32, device=DEV))
+    results = [sc.sparse_conv2d_custom(x, w, i, bp, [1, 1, 1, 1], transpose=t) for i in (ind, on_device) for t in (False, True)]
+    for y in results[1:]:
+        assert bool(((y - results[0]).abs() <= 2 * k * k * C * U * results[0]).all())
+
+
 def bottleneck64(p, params, no_activation):
     """Residual function in float64 and, beside it, the accumulated rounding bound: each stage adds its own sum's bound and
     passes on the one it received through the absolute values of its scales and weights."""
