@@ -345,6 +345,16 @@ def _block_bottleneck(x, params, indices, block_params, no_activation, in_place)
         block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
+# The forward products, in flops, up to which a training step with the own gradients is the faster one (MI355X; us a step with
+# the library's / the own, everything wanted).  256-64-64-256 channels: 635 / 394 at 1.5 GFLOP, 763 / 684 at 6,
+# 2349 / 2063 at 20, 7565 / 8103 at 82; 512-128: 759 / 517 at 6, 1660 / 1679 at 25, 5155 / 5441 at 81; 1024-256: 781 / 520 at
+# 4.5, 1174 / 1243 at 24; 2048-512: 942 / 872 at 18, 3053 / 3829 at 97.
+OWN_GRADIENT_MOST = 22e9
+# Without gradients of the kernels, which are the own kernels' best part.  256-64: 494 / 377 at 1.5, 544 / 611 at 6.3; 512-128:
+# 619 / 484 at 6.1, 1230 / 1456 at 25; 1024-256: 637 / 493 at 4.5, 860 / 1060 at 24; 2048-512: 699 / 719 at 18.
+OWN_GRADIENT_MOST_FROZEN = 6.2e9
+
+
 class _AsItWas(torch.autograd.Function):
     """The value a tensor had, with the gradient going to the tensor as it is now."""
 
@@ -422,7 +432,8 @@ class _ResidualInTraining(torch.autograd.Function):
 
 def _own_residual_gradient(p, params):
     """Whether _ResidualInTraining applies: not under forward-mode or functorch transforms, autocast, or where deterministic
-    algorithms are asked for (its batch norm sums are added up with atomics, in double)."""
+    algorithms are asked for (its batch norm sums are added up with atomics, in double), and up to the size where the
+    library's gradients become the faster ones."""
     tensors = [p, *params.w, *(t for b in params.bn for t in (b.gamma, b.beta))]
     stats = [t for b in params.bn for t in (b.moving_mean, b.moving_var) if t is not None]
     return (torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
@@ -432,6 +443,8 @@ def _own_residual_gradient(p, params):
                 for t in tensors + stats) and
             all(w.dim() == 4 and w.shape[2] % 4 == 0 and w.shape[3] % 4 == 0 for w in params.w) and
             not any(t.requires_grad for t in stats) and
+            2 * p.shape[0] * p.shape[2] * p.shape[3] * sum(w.numel() for w in params.w) <=
+            (OWN_GRADIENT_MOST if any(w.requires_grad for w in params.w) else OWN_GRADIENT_MOST_FROZEN) and
             p.shape[0] * (p.shape[2] - sum(w.shape[0] - 1 for w in params.w[:2])) *
             (p.shape[3] - sum(w.shape[1] - 1 for w in params.w[:2])) >= 2)
 

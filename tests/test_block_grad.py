@@ -95,6 +95,17 @@ def test_gradients_of_a_bottleneck(M, bsize, ksizes):
         assert bool((err <= 2 * bound + 1e-30).all()), (k, float((err / (2 * bound + 1e-30)).max()))
 
 
+@pytest.mark.parametrize("frozen", [False, True])
+def test_large_steps_take_the_librarys_gradients(frozen):
+    params = sc.BottleneckParams([[1, 1, 256, 64], [3, 3, 64, 64], [1, 1, 64, 256]], DEV)
+    for w in params.w:
+        w.requires_grad_(not frozen)
+    most = sc.OWN_GRADIENT_MOST_FROZEN if frozen else sc.OWN_GRADIENT_MOST
+    blocks = int(most / (2 * 17 * 17 * sum(w.numel() for w in params.w)))
+    for M, own in ((blocks, True), (blocks + 1, False)):
+        assert sc._own_residual_gradient(torch.empty(M, 256, 17, 17, device=DEV), params) == own
+
+
 ALL = range(10)
 
 
