@@ -231,6 +231,46 @@ def test_sparse_res_block_in_a_hip_graph_replays_identically(data_format):
             np.testing.assert_array_equal(got.cpu().numpy(), exp.cpu().numpy())
 
 
+@pytest.mark.parametrize("is_training,grad", [(True, True), (True, False), (False, True)])
+def test_training_on_either_layout_takes_planar_stacks(is_training, grad):
+    """The two data formats are one calculation, bit for bit, forward and backward."""
+    import sbnet_amd
+    from sbnet_amd import sparse_conv as sc
+    shape, ksizes = [1, 30, 33, 16], [[1, 1, 16, 8], [3, 3, 8, 8], [1, 1, 8, 16]]
+    bp = sbnet_amd.calc_block_params_res_block(shape, [1, 9, 9, 1], ksizes, [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(*shape[:3], 1, device=DEV), bp, 0.0)
+    results, layouts = [], []
+    gather = sbnet_amd.ops.sparse_gather
+    for data_format in ("NCHW", "NHWC"):
+        params = sc.BottleneckParams(ksizes, DEV, seed=3)
+        x = torch.randn(shape, device=DEV, generator=torch.Generator(DEV).manual_seed(1)).requires_grad_(grad)
+        sc.ops.sparse_gather = lambda *a, **k: layouts.append(k["transpose"]) or gather(*a, **k)
+        try:
+            with torch.set_grad_enabled(grad):
+                y = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], is_training, data_format=data_format)
+        finally:
+            sc.ops.sparse_gather = gather
+        results.append([y.detach()] + (list(torch.autograd.grad(y, [x, *params.parameters()], torch.ones_like(y))) if grad else []))
+    assert layouts == [True, True]
+    assert torch.equal(results[0][0], results[1][0])
+    for a, b in zip(*results):   # (gradients: the order in which the sums' atomics arrive is free)
+        assert float((a - b).norm()) <= 1e-5 * float(a.norm())
+
+
+@pytest.mark.skip(reason="this step ended the process on an NHWC stack for a reason that is not known; it now runs on a planar "
+                         "stack, and stays unrun until the cause is")
+def test_training_step_that_ended_the_process():
+    import sbnet_amd
+    from sbnet_amd import sparse_conv as sc
+    shape, ksizes = [1, 40, 45, 384], [[1, 1, 384, 96], [3, 3, 96, 96], [1, 1, 96, 384]]
+    bp = sbnet_amd.calc_block_params_res_block(shape, [1, 15, 15, 1], ksizes, [1, 1, 1, 1], "SAME")
+    ind = sc.convert_mask_to_indices_custom(torch.ones(*shape[:3], 1, device=DEV), bp, 0.0)
+    params = sc.BottleneckParams(ksizes, DEV, seed=3)
+    x = torch.randn(shape, device=DEV).requires_grad_()
+    y = sc.sparse_res_block_bottleneck(x, params, ind, bp, [1, 1, 1, 1], True, data_format="NHWC")
+    torch.autograd.grad(y, [x, *params.parameters()], torch.ones_like(y))
+
+
 # ---------------------------------------------------------------------------------------------
 # The reference's index-list interface (convert_mask_to_block_indices / upsample_indices / sparse_conv2d /
 # sparse_conv2d_matmul), pinned by the vectors its own tests hold
