@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <map>
+#include <mutex>
 #include <utility>
 
 #include "../../include/sbnet_amd.h"
@@ -120,18 +121,33 @@ at::Tensor empty_stack(int32_t M, int64_t C, const Pair& bsize, bool planar, con
 void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
 // Scratch of the calls of one stream, which run in order: one buffer per (device, stream) that only grows.  The GIL
-// guards the table.  A buffer that a call still holds when another thread grows it stays alive until that call's
-// work has been enqueued, and torch's allocator hands its memory on in the order of the stream.
-std::map<std::pair<int, void*>, at::Tensor>* g_workspaces = nullptr;
+// guards the table; a call enqueues its launches under the buffer's lock, so that another thread's on the same stream come
+// before or after them and not in between.  A buffer that a call still holds when another thread grows it stays alive
+// until that call's work has been enqueued, and torch's allocator hands its memory on in the order of the stream.
+struct Scratch {
+    at::Tensor buffer;
+    std::recursive_mutex busy;   // (waited for without the GIL, which its holder may want)
+};
 
-at::Tensor workspace(const at::Device& device, int64_t bytes)
+std::map<std::pair<int, void*>, Scratch>* g_workspaces = nullptr;   // entries stay, release_workspaces() drops the buffers
+
+Scratch& stream_scratch(int device)
 {
-    void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
-    if (!g_workspaces) g_workspaces = new std::map<std::pair<int, void*>, at::Tensor>();
-    at::Tensor& ws = (*g_workspaces)[std::make_pair((int)device.index(), stream)];
-    if (!ws.defined() || ws.numel() < bytes)
-        ws = at::detail::empty_cuda({bytes < (1 << 16) ? (1 << 16) : bytes}, at::kByte, device, c10::nullopt);
-    return ws;
+    if (!g_workspaces) g_workspaces = new std::map<std::pair<int, void*>, Scratch>();
+    return (*g_workspaces)[std::make_pair(device, (void*)c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream())];
+}
+
+struct Workspace {
+    at::Tensor buffer;
+    std::recursive_mutex* busy = nullptr;
+};
+
+Workspace workspace(const at::Device& device, int64_t bytes)
+{
+    Scratch& s = stream_scratch(device.index());
+    if (!s.buffer.defined() || s.buffer.numel() < bytes)
+        s.buffer = at::detail::empty_cuda({bytes < (1 << 16) ? (1 << 16) : bytes}, at::kByte, device, c10::nullopt);
+    return {s.buffer, &s.busy};
 }
 
 // Scratch of one call, as the tensors between torch's operators are: for the layers, whose stacks are large, may belong to a
@@ -144,11 +160,13 @@ at::Tensor own_scratch(const at::Tensor& like, size_t bytes)
 
 // Runs a library call without the GIL, as ctypes does; raises on a status other than SBNET_OK.
 template <typename F>
-bool call(F f)
+bool call(F f, std::recursive_mutex* busy = nullptr)
 {
     int status;
     Py_BEGIN_ALLOW_THREADS
+    if (busy) busy->lock();
     status = f();
+    if (busy) busy->unlock();
     Py_END_ALLOW_THREADS
     if (status == SBNET_OK) return true;
     PyObject* r = PyObject_CallFunction(g_check, "i", status);
@@ -209,13 +227,14 @@ PyObject* reduce_mask(PyObject* const* a)
     at::Tensor idx = at::detail::empty_cuda({T, 3}, at::kShort, mask->device(), c10::nullopt);
     at::Tensor count = sync ? at::empty({1}, at::kInt) : at::detail::empty_cuda({1}, at::kInt, mask->device(), c10::nullopt);
     int32_t* const cp = static_cast<int32_t*>(count.data_ptr());
-    at::Tensor ws = workspace(mask->device(), (int64_t)sbnet_reduce_mask_workspace_bytes(N, bc.v, 2));
+    const Workspace scratch = workspace(mask->device(), (int64_t)sbnet_reduce_mask_workspace_bytes(N, bc.v, 2));
+    const at::Tensor& ws = scratch.buffer;
     void* const stream = stream_of(*mask);
     if (!call([&] {
             return sbnet_reduce_mask(static_cast<const float*>(mask->data_ptr()), N, H, W, bc.v, 2, bs.v, 2, bt.v, 2, bo.v,
                                      2, tol, avgpool, static_cast<int16_t*>(idx.data_ptr()), sync ? cp : nullptr,
                                      sync ? nullptr : cp, ws.data_ptr(), (size_t)ws.numel(), stream);
-        }))
+        }, scratch.busy))
         return nullptr;
     PyObject* pi = THPVariable_Wrap(std::move(idx));
     PyObject* pc = THPVariable_Wrap(std::move(count));
@@ -278,7 +297,8 @@ PyObject* gather_grad(PyObject* const* a)
     c10::DeviceGuard guard(g->device());
     at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, *g);
     const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
-    at::Tensor ws = need ? workspace(g->device(), need) : at::Tensor();
+    const Workspace scratch = need ? workspace(g->device(), need) : Workspace();
+    const at::Tensor& ws = scratch.buffer;
     const float* const gp = static_cast<const float*>(g->data_ptr());
     const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
     float* const dp = static_cast<float*>(dx.data_ptr());
@@ -286,7 +306,7 @@ PyObject* gather_grad(PyObject* const* a)
     if (!call([&] {
             return sbnet_sparse_gather_grad(gp, b.M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
                                             need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
-        }))
+        }, scratch.busy))
         return nullptr;
     return THPVariable_Wrap(std::move(dx));
 }
@@ -308,9 +328,10 @@ PyObject* scatter(PyObject* const* a)
     const bool overlap = bt.v[0] < bs.v[0] || bt.v[1] < bs.v[1];
     c10::DeviceGuard guard(base->device());
     const int64_t* const dims = base->sizes().data();
-    const bool scratch = (add && atomic) || !in_place || (!add && overlap);
-    const int64_t need = scratch ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
-    at::Tensor ws = need ? workspace(base->device(), need) : at::Tensor();
+    const bool wants = (add && atomic) || !in_place || (!add && overlap);
+    const int64_t need = wants ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
+    const Workspace scratch = need ? workspace(base->device(), need) : Workspace();
+    const at::Tensor& ws = scratch.buffer;
     void* const wp = need ? ws.data_ptr() : nullptr;
     const size_t wn = need ? (size_t)ws.numel() : 0;
     at::Tensor y = in_place ? *base : empty_f32(base->sizes(), *base);
@@ -328,7 +349,7 @@ PyObject* scatter(PyObject* const* a)
                                                                add, atomic, transpose, yp, wp, wn, stream)
                            : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
                                                   transpose, yp, wp, wn, stream);
-        }))
+        }, scratch.busy))
         return nullptr;
     if (in_place) {
         Py_INCREF(a[3]);   // the caller's own tensor object, as the Python wrapper returns it
@@ -563,16 +584,45 @@ PyObject* workspace_py(PyObject* const* a)
     if (PyErr_Occurred()) return nullptr;
     const at::Device device(at::kCUDA, (c10::DeviceIndex)dev);
     c10::DeviceGuard guard(device);
-    return THPVariable_Wrap(workspace(device, bytes));
+    return THPVariable_Wrap(workspace(device, bytes).buffer);
+}
+
+// lock_workspace(device index) -> what unlock_workspace() takes: the lock of the current stream's scratch
+PyObject* lock_workspace(PyObject* const* a)
+{
+    const long dev = PyLong_AsLong(a[0]);
+    if (PyErr_Occurred()) return nullptr;
+    std::recursive_mutex* const busy = &stream_scratch((int)dev).busy;
+    PyObject* const held = PyCapsule_New(busy, nullptr, nullptr);
+    if (!held) return nullptr;
+    Py_BEGIN_ALLOW_THREADS
+    busy->lock();
+    Py_END_ALLOW_THREADS
+    return held;
+}
+
+PyObject* unlock_workspace(PyObject* const* a)
+{
+    void* const busy = PyCapsule_GetPointer(a[0], nullptr);
+    if (!busy) return nullptr;
+    static_cast<std::recursive_mutex*>(busy)->unlock();
+    Py_RETURN_NONE;
 }
 
 PyObject* release_workspaces(PyObject*, PyObject*)
 {
-    if (g_workspaces) g_workspaces->clear();
+    if (g_workspaces)
+        for (auto& w : *g_workspaces) w.second.buffer.reset();
     Py_RETURN_NONE;
 }
 
-PyObject* has_workspaces(PyObject*, PyObject*) { return PyBool_FromLong(g_workspaces && !g_workspaces->empty()); }
+PyObject* has_workspaces(PyObject*, PyObject*)
+{
+    bool any = false;
+    if (g_workspaces)
+        for (auto& w : *g_workspaces) any = any || w.second.buffer.defined();
+    return PyBool_FromLong(any);
+}
 
 PyObject* set_check(PyObject*, PyObject* f)
 {
@@ -594,6 +644,8 @@ PyMethodDef methods[] = {
     {"block_bottleneck", fast(op_entry<block_bottleneck, 12>), METH_FASTCALL, nullptr},
     {"bottleneck_grad", fast(op_entry<bottleneck_grad, 3, 2>), METH_FASTCALL, nullptr},
     {"workspace", fast(entry<workspace_py, 2>), METH_FASTCALL, nullptr},
+    {"lock_workspace", fast(entry<lock_workspace, 1>), METH_FASTCALL, nullptr},
+    {"unlock_workspace", fast(entry<unlock_workspace, 1>), METH_FASTCALL, nullptr},
     {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},
     {"set_check", set_check, METH_O, nullptr},

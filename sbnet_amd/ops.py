@@ -9,6 +9,7 @@ the current stream only; all computation happens in the HIP kernels behind the C
 no fallback if the library is missing.
 """
 import collections
+import contextlib
 import ctypes
 
 import numpy as np
@@ -114,10 +115,17 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+@contextlib.contextmanager
 def _workspace(device, nbytes):
-    """Scratch of the current stream: one uint8 tensor per (device, stream) that is kept and only grows."""
+    """Scratch of the current stream: one uint8 tensor per (device, stream) that is kept and only grows.  Inside the context
+    no other thread enqueues a call that uses it."""
     index = device.index if device.index is not None else torch.cuda.current_device()
-    return (_native or _load_native()).workspace(index, nbytes)
+    native = _native or _load_native()
+    held = native.lock_workspace(index)
+    try:
+        yield native.workspace(index, nbytes)
+    finally:
+        native.unlock_workspace(held)
 
 
 def release_workspaces():
@@ -173,13 +181,13 @@ def reduce_mask(mask, dynamic_bcount=None, dynamic_bsize=None, dynamic_bstride=N
     with torch.cuda.device(mask.device):
         idx = torch.empty((max(int(max_idx), 1), 3), dtype=torch.int16, device=mask.device)
         nws = lib.sbnet_reduce_mask_workspace_bytes(N, bcp, bcl) if bcl == 2 else 0
-        ws = _workspace(mask.device, nws)
         dev_count = torch.empty(1, dtype=torch.int32, device=mask.device)
         host_count = np.zeros(1, dtype=np.int32)
         hp = host_count.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)) if sync else None
-        _check(lib.sbnet_reduce_mask(mask.data_ptr(), N, H, W, bcp, bcl, bsp, bsl, btp, btl, bop, bol,
-                                     ctypes.c_float(tol), int(bool(avgpool)), idx.data_ptr(), hp,
-                                     dev_count.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
+        with _workspace(mask.device, nws) as ws:
+            _check(lib.sbnet_reduce_mask(mask.data_ptr(), N, H, W, bcp, bcl, bsp, bsl, btp, btl, bop, bol,
+                                         ctypes.c_float(tol), int(bool(avgpool)), idx.data_ptr(), hp,
+                                         dev_count.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
     if sync:
         return ReduceMaskResult(idx, torch.from_numpy(host_count))
     return ReduceMaskResult(idx, dev_count)
@@ -200,12 +208,12 @@ def reduce_mask_functor(mask, bcount, bsize, bstride, boffset, tol, avgpool=Fals
     with torch.cuda.device(mask.device):
         max_idx = lib.sbnet_reduce_mask_max_indices(N, bcp, bcl)
         idx = torch.empty((max(int(max_idx), 1), 3), dtype=torch.int16, device=mask.device)
-        ws = _workspace(mask.device, lib.sbnet_reduce_mask_workspace_bytes(N, bcp, bcl))
         count = torch.empty(1, dtype=torch.int32, device=mask.device)
-        _check(lib.sbnet_reduce_mask_functor(mask.data_ptr(), N, H, W, ctypes.c_float(tol), int(bo[0]), int(bo[1]),
-                                             int(bs[0]), int(bs[1]), int(bt[0]), int(bt[1]), int(bc[0]), int(bc[1]),
-                                             1, 1, idx.data_ptr(), count.data_ptr(), int(bool(avgpool)),
-                                             ws.data_ptr(), ws.numel(), _stream()))
+        with _workspace(mask.device, lib.sbnet_reduce_mask_workspace_bytes(N, bcp, bcl)) as ws:
+            _check(lib.sbnet_reduce_mask_functor(mask.data_ptr(), N, H, W, ctypes.c_float(tol), int(bo[0]), int(bo[1]),
+                                                 int(bs[0]), int(bs[1]), int(bt[0]), int(bt[1]), int(bc[0]), int(bc[1]),
+                                                 1, 1, idx.data_ptr(), count.data_ptr(), int(bool(avgpool)),
+                                                 ws.data_ptr(), ws.numel(), _stream()))
     return idx, count
 
 
@@ -289,12 +297,12 @@ def gather_backward(grad, bin_counts, active_block_indices, x_shape, dynamic_bsi
     if rank == 4 and bsl == 2 and btl == 2 and bol == 2:
         _check_count(M, idx)
         _check_stack(grad, M, x_shape[3], int(bs[0]), int(bs[1]), transpose, "grad")
-    with torch.cuda.device(grad.device):
+    with torch.cuda.device(grad.device), contextlib.ExitStack() as scratch:
         dx = torch.empty(x_shape, dtype=torch.float32, device=grad.device)
         ws_ptr, ws_bytes = None, 0
         need = lib.sbnet_sparse_scatter_workspace_bytes(M, dims, rank, bsp, bsl, btp, btl, bop, bol)
         if need:
-            ws = _workspace(grad.device, need)
+            ws = scratch.enter_context(_workspace(grad.device, need))
             ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         _check(lib.sbnet_sparse_gather_grad(grad.data_ptr(), M, idx.data_ptr(), dx.data_ptr(), dims, rank, bsp, bsl, btp,
                                             btl, bop, bol, int(bool(transpose)), ws_ptr, ws_bytes, _stream()))
@@ -335,7 +343,7 @@ def scatter_forward(x, bin_counts, active_block_indices, ybase, dynamic_bsize, d
     if rank == 4 and bsl == 2 and btl == 2 and bol == 2 and (atomic or not add or not overlap):
         _check_count(M, idx)
         _check_stack(x, M, int(ybase.shape[3]), int(bs[0]), int(bs[1]), transpose, "x")
-    with torch.cuda.device(ybase.device):
+    with torch.cuda.device(ybase.device), contextlib.ExitStack() as held:
         ws_ptr, ws_bytes = None, 0
         if scratch and ((add and atomic) or not use_var or (not add and overlap)):
             # scratch for the atomic-free scatter-add of overlapping blocks, for overlapping plain writes in the
@@ -343,7 +351,7 @@ def scatter_forward(x, bin_counts, active_block_indices, ybase, dynamic_bsize, d
             # pass (uncovered pixels copied, covered ones scattered)
             need = lib.sbnet_sparse_scatter_workspace_bytes(M, dims, rank, bsp, bsl, btp, btl, bop, bol)
             if need:
-                ws = _workspace(ybase.device, need)
+                ws = held.enter_context(_workspace(ybase.device, need))
                 ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         flags = (int(bool(add)), int(bool(atomic)), int(bool(transpose)))
         if use_var:

@@ -1326,3 +1326,42 @@ def test_flat_copy_of_any_length(n):
 def test_reduce_mask_around_the_scan(N, H, W, bsize, bstride, boffset, avgpool):
     mask = (np.random.default_rng(H).random((N, H, W, 1)) < 0.2).astype(np.float32)
     check_reduce(mask, bcount_covering(H, W, bstride, boffset), bsize, bstride, boffset, 0.2, avgpool)
+
+
+def test_two_threads_on_one_stream_share_its_scratch_call_by_call():
+    """Overlapping adds and writes, masks and gradients of two geometries, each call of several launches over the one scratch
+    buffer of the stream: what a thread gets is what it gets alone.  One thread's parameters go the general wrappers' way."""
+    import threading
+
+    def work(seed, C, block, stride, wrap):
+        rng = np.random.default_rng(seed)
+        N, H, W = 2, 90, 110
+        bc = [(H - block) // stride + 1, (W - block) // stride + 1]
+        mask = torch.from_numpy((rng.random((N, H, W, 1)) < 0.01).astype(np.float32)).to("cuda")
+        base = torch.from_numpy(rng.standard_normal((N, H, W, C)).astype(np.float32)).to("cuda")
+        geom = [wrap(v) for v in ([block, block], [stride, stride], [0, 0])]
+
+        def run():
+            ind = sbnet_amd.reduce_mask(mask, wrap(bc), *geom, tol=0.5)
+            q = sbnet_amd.sparse_gather(base, *reversed(ind), *geom)
+            added = sbnet_amd.sparse_scatter_var(q, *reversed(ind), base.clone(), *geom, add=True, atomic=True)
+            written = sbnet_amd.sparse_scatter(2 * q, *reversed(ind), base, *geom, add=False)
+            dx = ops.gather_backward(q, ind.bin_counts, ind.active_block_indices, tuple(base.shape), *geom)
+            return [ind.active_block_indices[:int(ind.bin_counts[0])], added, written, dx]
+
+        return run, run()
+
+    jobs = [work(1, 16, 12, 8, list), work(2, 36, 9, 6, lambda v: np.asarray(v, np.int32))]
+    wrong = []
+
+    def thread(run, want):
+        for _ in range(60):
+            if not all(torch.equal(a, b) for a, b in zip(run(), want)):
+                wrong.append(1)
+
+    threads = [threading.Thread(target=thread, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
