@@ -263,6 +263,14 @@ def test_native_wrappers_leave_what_they_do_not_take():
         ops.sparse_gather(x, [1], idx, pair, pair, [0, 0])
 
 
+def test_extension_module_is_rebuilt_for_another_torch():
+    """It is bound to the Python and the torch that it was compiled against, so these are among what it depends on."""
+    make = ["make", "-n", "-C", os.path.join(ROOT, "sbnet_amd", "csrc"), "-o", "../libsbnet_amd.so", "-o", "sbnet_torch.cpp",
+            "-o", "../../include/sbnet_amd.h", "../_native.so"]
+    assert "g++" not in subprocess.check_output(make, text=True)
+    assert "g++" in subprocess.check_output(make + ["NATIVE_FOR=cpython-311 torch 9.9"], text=True)
+
+
 def test_native_wrappers_leave_tensors_without_memory():
     """Fake tensors and those of a transform go the general way, which raises what it raises: nothing is read through their
     pointers, and no C++ exception leaves the module."""
