@@ -48,7 +48,9 @@ struct PoolArgs {
 };
 
 // Up to here every compacting workgroup adds up the counts before it, at most 16 loads a thread.  The scan is a launch of
-// 4.7 us (1089 counts of 64 128x128 images with 6x6 blocks: the step on them 104.7 us with it, 100.8 without).
+// its own.  us of all launches with it / without: 1089 counts (64 128x128 images, 6x6 blocks) 10.3 / 7.9, 2178: 13.2 / 10.5,
+// 4083: 16.3 / 13.9; one-pixel blocks, 1915 counts: 12.2 / 9.6, 3907: 18.4 / 14.9.  The sums are still the cheaper at 15 625
+// counts (63.5 / 52.7) but grow with the square: the line keeps them few.
 constexpr uint32_t SCAN_MIN_COUNTS = 4096;
 
 // Stores the count (and, for an empty list, the (0,0,0) triple of reduce_mask.cc:206-218) and hands it to a

@@ -53,6 +53,9 @@ CONVS = [
     (1, 60, 60, 132, 68, 1, 1, (6, 6), 40),
     (1, 300, 300, 16, 64, 3, 3, (12, 12), 700),   # enough tiles that k is not split
     (1, 300, 300, 7, 33, 3, 3, (12, 12), 700),
+    (1, 260, 260, 32, 16, 3, 3, (18, 18), 110),   # 1760 wave tiles of 16, 32 and 48 channels: k split in two
+    (1, 260, 260, 32, 32, 3, 3, (18, 18), 110),
+    (1, 260, 260, 32, 48, 3, 3, (18, 18), 110),
 ]
 
 
@@ -130,6 +133,11 @@ def bottleneck64(p, params, no_activation):
 @pytest.mark.parametrize("C,mid,bsize,shape", [(6, 3, 5, (2, 23, 31)), (24, 8, 9, (1, 40, 52)), (96, 24, 17, (1, 70, 64)),
                                                (260, 64, 7, (1, 30, 30)), (16, 16, 24, (1, 220, 220))])
 def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
+    check_bottleneck(C, mid, bsize, shape, no_activation, use_var)
+
+
+def check_bottleneck(C, mid, bsize, shape, no_activation, use_var):
+    """Returns the number of output pixels."""
     rng = np.random.default_rng(C)
     ksizes = [[1, 1, C, mid], [3, 3, mid, mid], [1, 1, mid, C]]
     bp = sbnet_amd.calc_block_params_res_block([shape[0], shape[1], shape[2], C], [1, bsize, bsize, 1], ksizes, [1, 1, 1, 1], "SAME")
@@ -157,6 +165,7 @@ def test_bottleneck_in_inference(C, mid, bsize, shape, no_activation, use_var):
         most[n, bh * Ro:(bh + 1) * Ro, bw * So:(bw + 1) * So] = bound[i, :part.shape[0], :part.shape[1]] + U * part.abs()
     err = (y.cpu().double() - want).abs()
     assert bool((err <= most + 1e-30).all()), float((err / (most + 1e-30)).max())
+    return M * Ro * So
 
 
 @pytest.mark.parametrize("ratio", [10.0, 1000.0])
@@ -200,14 +209,22 @@ def test_infinite_shift_of_a_channel_stays_infinite(C, kh):
     assert bool((q == float("inf")).all())
 
 
+ONE_LAUNCH = 1536 * 16   # output pixels from which on the last two convolutions share a launch, up to 128 channels in between
+
+
 @pytest.mark.parametrize("use_var", [False, True])
-@pytest.mark.parametrize("C,mid,bsize,shape", [(40, 36, 9, (2, 33, 41)),       # three fragments in between, the last a quarter full
-                                               (132, 84, 11, (1, 60, 44)),     # six; output tiles of 64 channels and a rest
-                                               (64, 100, 8, (1, 40, 40)),      # seven of eight
-                                               (20, 132, 8, (1, 40, 40)),      # more than one tile: not in one launch
-                                               (64, 128, 24, (1, 180, 185))])  # eight, a wave for every 16 pixels
-def test_last_two_convolutions_in_one_launch(C, mid, bsize, shape, use_var):
-    test_bottleneck_in_inference(C, mid, bsize, shape, False, use_var)
+@pytest.mark.parametrize("C,mid,bsize,shape,one", [
+    (96, 24, 17, (1, 190, 205), True),      # one fragment of channels in between and half of another
+    (40, 36, 17, (2, 140, 150), True),      # three, the last a quarter full
+    (256, 64, 17, (1, 180, 175), True),     # four
+    (132, 84, 17, (1, 180, 175), True),     # six; output tiles of 64 channels and a rest
+    (64, 100, 17, (1, 180, 175), True),     # seven of eight
+    (64, 128, 24, (1, 180, 185), True),     # eight
+    (132, 84, 11, (1, 60, 44), False),      # few pixels: two launches
+    (20, 132, 17, (1, 180, 175), False),    # more than one tile of channels in between: two launches
+])
+def test_last_two_convolutions_in_one_launch(C, mid, bsize, shape, one, use_var):
+    assert (check_bottleneck(C, mid, bsize, shape, False, use_var) >= ONE_LAUNCH and mid <= 128) == one
 
 
 def test_layers_under_autocast_take_the_layers_own_way():

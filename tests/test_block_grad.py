@@ -78,6 +78,9 @@ CASES = [
     (3, (9, 7), [[3, 1, 20, 16], [1, 5, 16, 28], [3, 3, 28, 20]]),        # unequal and multiple taps everywhere
     (5, (8, 8), [[1, 1, 260, 132], [3, 3, 132, 132], [1, 1, 132, 260]]),  # second chunk of channels in the batch norm's backward
     (300, (14, 14), [[1, 1, 16, 16], [3, 3, 16, 16], [1, 1, 16, 16]]),    # enough pixels that k is not split
+    (100, (18, 18), [[1, 1, 16, 16], [3, 3, 16, 32], [1, 1, 32, 16]]),    # 2025 wave tiles of 16, 32 and 48 channels and 18
+    (100, (18, 18), [[1, 1, 16, 32], [3, 3, 32, 32], [1, 1, 32, 16]]),    # steps in the middle: k split in two
+    (100, (18, 18), [[1, 1, 16, 48], [3, 3, 48, 32], [1, 1, 32, 16]]),
 ]
 
 

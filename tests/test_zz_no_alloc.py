@@ -47,8 +47,10 @@ def both(lib, mask, bcount, bsize, bstride, boffset, tol, avgpool):
      ((1, 64, 64), (8, 8), (10, 10), (8, 8), (-1, -1), False)],      # 64 blocks: one compaction workgroup
     [((1, 800, 800), (32, 32), (27, 27), (25, 25), (-1, -1), False),  # 1024 blocks, a wave per block
      ((2, 40, 52), (7, 9), (6, 6), (6, 6), (-2, -1), True)],
-    [((2, 400, 400), (400, 400), (1, 1), (1, 1), (0, 0), False),     # 320 000 one-pixel blocks: more than 1024 pooling
-     ((1, 30, 30), (10, 10), (3, 3), (3, 3), (0, 0), True)],         # workgroups, so the counts are scanned first
+    [((2, 400, 400), (400, 400), (1, 1), (1, 1), (0, 0), False),     # 320 000 one-pixel blocks: 1250 pooling workgroups,
+     ((1, 30, 30), (10, 10), (3, 3), (3, 3), (0, 0), True)],         # whose counts each compacting workgroup adds up
+    [((2, 800, 800), (260, 260), (23, 23), (3, 3), (0, 0), False),   # 135 200 blocks, 32 to a pooling workgroup: 4225 of
+     ((1, 30, 30), (10, 10), (3, 3), (3, 3), (0, 0), True)],         # these, so the counts are scanned first
 ])
 def test_static_scratch_matches_workspace(sizes):
     lib = _lib.load()
