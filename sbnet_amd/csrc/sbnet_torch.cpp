@@ -142,8 +142,13 @@ struct Workspace {
     std::recursive_mutex* busy = nullptr;
 };
 
+// (While the stream is being captured the scratch is a tensor of the graph's own pool: the graph keeps its address, and the
+// kept buffer may grow or be released before a replay, or be in use by the stream's own calls during one.)
 Workspace workspace(const at::Device& device, int64_t bytes)
 {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(device.index()).stream(), &capture) != hipSuccess) (void)hipGetLastError();
+    if (capture == hipStreamCaptureStatusActive) return {at::detail::empty_cuda({bytes}, at::kByte, device, c10::nullopt), nullptr};
     Scratch& s = stream_scratch(device.index());
     if (!s.buffer.defined() || s.buffer.numel() < bytes)
         s.buffer = at::detail::empty_cuda({bytes < (1 << 16) ? (1 << 16) : bytes}, at::kByte, device, c10::nullopt);

@@ -1328,6 +1328,43 @@ def test_reduce_mask_around_the_scan(N, H, W, bsize, bstride, boffset, avgpool):
     check_reduce(mask, bcount_covering(H, W, bstride, boffset), bsize, bstride, boffset, 0.2, avgpool)
 
 
+def test_captured_ops_own_their_scratch():
+    """A graph's block maps lie in the graph's own memory: the stream's scratch may be released, or grow, before a replay."""
+    rng = np.random.default_rng(3)
+    shape, geom = (2, 60, 70, 8), ([12, 12], [8, 8], [-1, -1])
+    idx = torch.from_numpy(np.array([[n, i, j] for n in range(2) for i in range(0, 7, 2) for j in range(8)], np.int16)).to(DEV)
+    q = torch.from_numpy(rng.standard_normal((len(idx), 12, 12, 8)).astype(np.float32)).to(DEV)
+    base = torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(DEV)
+    mask = torch.from_numpy((rng.random(shape[:3]) < 0.01).astype(np.float32)).to(DEV)
+
+    def step(numbers):
+        g = [numbers(v) for v in geom]
+        return [sbnet_amd.reduce_mask(mask, numbers([8, 9]), *g, tol=0.5, sync=False).bin_counts,
+                sbnet_amd.sparse_scatter(q, [len(idx)], idx, base, *g, add=False),
+                sbnet_amd.sparse_scatter(q, [len(idx)], idx, base, *g, add=True, atomic=True),
+                ops.gather_backward(q, [len(idx)], idx, shape, *g)]
+
+    for numbers in (list, lambda v: np.asarray(v, np.int32)):   # the extension module, the general wrappers
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        want = step(numbers)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            step(numbers)
+        torch.cuda.synchronize()
+        ops.release_workspaces()
+        with torch.cuda.graph(graph, stream=side):
+            got = step(numbers)
+        assert not ops._load_native().has_workspaces()
+        held = [torch.full((1 << 18,), 7.0, device=DEV) for _ in range(8)]
+        for _ in range(3):
+            for t in got:
+                t.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert all(bool((h == 7.0).all()) for h in held)
+
+
 def test_two_threads_on_one_stream_share_its_scratch_call_by_call():
     """Overlapping adds and writes, masks and gradients of two geometries, each call of several launches over the one scratch
     buffer of the stream: what a thread gets is what it gets alone.  One thread's parameters go the general wrappers' way."""
