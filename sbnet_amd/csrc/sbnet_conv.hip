@@ -23,8 +23,11 @@ namespace sbnet {
 // lane ends with four consecutive channels of one pixel: 16-byte stores into NHWC memory.  Both operands go from memory
 // straight to registers: with the instruction's k index spread as (lane / 16) * 4 + step, a lane's four pixel values
 // are one 16-byte load, and 4 lanes read the 64 bytes of a pixel that 16 k need.  The fp32 matrix rate is low enough
-// (a 2x2 wave tile multiplies for 512 cycles per 16 k, for which it reads 4 KB) that L1 feeds it, and without LDS
+// that the caches feed it (with FN = 2 a wave multiplies for 256 cycles per 16 k, for which it reads 1 KB of pixels and
+// 2 KB of weights: 48 bytes a cycle for the four waves of a CU), and without LDS
 // tiles there are no barriers: the problems are small (a few thousand pixels) and their time is a chain of latencies.
+// Large products run at 80-95 TFLOP/s (of 153), with single-float loads at 35-40; from where the library is faster at
+// them is a rule of the caller (sbnet_torch.cpp).
 // CONV_DEPTH sets of operands are in flight per wave.
 //
 // Measured (MI355X, kernel trace): 85 blocks of 17x17x48, 3x3 to 48 channels (19 000 pixels, 0.8 GFLOP; 5.2 us at the
@@ -546,7 +549,9 @@ hipError_t launch_block_conv_next(const ConvArgs& c, const ConvArgs& next, hipSt
     a.K2 = next.K;
     a.w2Bytes = (uint32_t)(next.C * next.K * 4);
     // A wave per 16 pixels and all channels: with fewer of them than SIMDs to fill, two launches that split further are
-    // faster (2350 pixels, 128 channels in between: 22.2 against 28 us, four waves to 16 pixels).
+    // faster.  us a block, in one launch / in two, by the channels in between and at 993, 2025, 6807 waves: 24: 19.7 / 21.1,
+    // 26.2 / 27.6, 50.7 / 55.4; 48: 31.5 / 31.4, 41.0 / 45.1, 103 / 116; 64: 44.1 / 44.5, 62.4 / 74.2, 170 / 215; 128: 128 / 125,
+    // 191 / 230, 623 / 813; and at 307: 15.1 / 14.3, 23.3 / 19.0, 33.0 / 24.6, 104 / 50.  (16 channels gain at any size.)
     if ((a.rows + 15) / 16 < 1536) return hipSuccess;
     done = true;
     switch ((c.K + 15) / 16) {

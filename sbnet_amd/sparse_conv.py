@@ -7,8 +7,8 @@ sbnet_tensorflow/benchmark/sparse_conv_lib.py: `convert_mask_to_indices_custom` 
 `convert_mask_to_indices` (279-318), `upsample_indices` (249-276), `convert_mask_to_block_indices` (321-340),
 `sparse_conv2d` (462-523) and `sparse_conv2d_matmul` (827-888), which the reference computes with TensorFlow's
 gather_nd / scatter_nd and which here run on the same block ops.  The three block ops
-run the HIP kernels of this package; the dense convolutions, batch norm and ReLU between gather and
-scatter are PyTorch's (MIOpen on this hardware), exactly where the reference calls cuDNN.
+run the HIP kernels of this package; so do, where that is the faster way (below), the convolutions, batch norm and ReLU
+between gather and scatter.  Elsewhere these are PyTorch's (MIOpen on this hardware), where the reference calls cuDNN.
 
 Conventions follow the reference: activations are NHWC tensors, kernels are [kh, kw, cin, cout],
 `strides` and `bsize` are 4-element lists, `data_format='NCHW'` means the block stack is gathered
@@ -17,10 +17,11 @@ transpose.  Everything is differentiable through torch.autograd (the block ops t
 sbnet_amd.autograd).
 
 Where no gradient is asked for, `sparse_conv2d_custom` and `sparse_res_block_bottleneck` (in inference) run this
-package's own convolution kernels instead (sbnet_amd/csrc/sbnet_conv.hip), which read the active blocks straight from x
-and keep what lies between two convolutions of a residual block in NHWC stacks; the stack's layout is then nobody's to
-see, and `transpose` / `data_format` select nothing.  The gradients of a residual block's training step on planar stacks
-are in own kernels, too (sbnet_block_grad.hip).
+package's own convolution kernels (sbnet_amd/csrc/sbnet_conv.hip), which read the active blocks straight from x
+and keep what lies between two convolutions of a residual block in NHWC stacks; large 3x3 products, and products of
+channels that are no multiple of four beyond small ones, go to the library.  The gradients of a residual block's training
+step are in own kernels, too (sbnet_block_grad.hip), up to a size.  The stack's layout is nobody's to see, and
+`transpose` / `data_format` decide it only where nothing else does.
 """
 import collections
 import ctypes
@@ -75,7 +76,7 @@ def sparse_conv2d_custom(x, w, indices, block_params, strides, use_var=False, tr
         # The stack's layout is nobody's to see, and from 16 channels on the library is the faster on planar ones: up to
         # twice as fast for 3x3 products on most block counts (256 channels, 484 blocks of 24x24: 2635 against 5824 us),
         # 8 % slower on some; with fewer channels it pays for its layout copies (3 channels, 465 000 pixels: 57 against 44).
-        transpose = transpose or (x.dim() == 4 and x.shape[3] >= 16 and
+        transpose = transpose or (all(isinstance(t, torch.Tensor) and t.dim() == 4 for t in (x, w)) and x.shape[3] >= 16 and
                                   not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
         p = ops.sparse_gather(x, indices.bin_counts, indices.active_block_indices, block_params.bsize,
                               block_params.bstrides, block_params.boffset, transpose=transpose)
