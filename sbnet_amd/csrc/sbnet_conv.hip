@@ -252,14 +252,10 @@ __global__ __launch_bounds__(256) void k_block_conv(ConvKernelArgs a)
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    if (PRE)
-        for (uint32_t c = tid; c < cPad; c += 64 * WAVES) {
-            float mean = 0.f, scale = 0.f, beta = 0.f;
-            if (c < C) bn_read(a.c.pre, c, mean, scale, beta);
-            preMean[c] = mean;
-            preScale[c] = scale;
-            preBeta[c] = beta;
-        }
+    if (PRE) {
+        for (uint32_t c = tid; c < C; c += 64 * WAVES) bn_read(a.c.pre, c, preMean[c], preScale[c], preBeta[c]);
+        if (tid < cPad - C) preMean[C + tid] = preScale[C + tid] = preBeta[C + tid] = 0.f;
+    }
     if constexpr (GRAD) {
         for (uint32_t i = tid; i < (uint32_t)TN; i += 64 * WAVES) {
             const uint32_t n = min(n0 + i, K - 1);

@@ -339,10 +339,10 @@ def res_block_bottleneck(x, params, strides, is_training, data_format="NHWC", w_
 def _block_bottleneck(x, params, indices, block_params, no_activation, in_place):
     """The residual function of the active blocks in inference: added to x (returns x) or as an NHWC stack; None where
     only the composed path applies."""
-    norms = [[None] * 4 if no_activation and not i else [b.gamma, b.beta, b.moving_mean, b.moving_var]
-             for i, b in enumerate(params.bn)]
+    norms = [t for b in params.bn
+             for t in ((None,) * 4 if b is None else (b.gamma, b.beta, b.moving_mean, b.moving_var))]
     return (ops._native or ops._load_native()).block_bottleneck(
-        x, params.w, sum(norms, []), indices.bin_counts, indices.active_block_indices, block_params.bsize,
+        x, params.w, norms, indices.bin_counts, indices.active_block_indices, block_params.bsize,
         block_params.bstrides, block_params.boffset, block_params.bsize_out, BN_EPS, no_activation, in_place)
 
 
