@@ -92,12 +92,12 @@ size_t scatter_owner_workspace_bytes(const Geom& g, int numActive);
 hipError_t launch_scatter_owned(const float* x, float* y, const int16_t* idx, int numActive, const Geom& g,
                                 bool transpose, void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done);
 
-// y = copy of ybase with the blocks written ("=") or added ("+=", non-overlapping) on top, moving every byte once.
-// Blocks that do not overlap: an inverse map (cell of the block grid -> list position) in the scratch, then one
-// streaming kernel over y that reads ybase where the result needs it, the stack where a block covers the pixel,
-// and writes y once (planar stacks of geometries the kernel does not stage: a pass that copies the uncovered
-// pixels, then the scatter kernels, which read ybase where they add).  Overlapping plain writes: the owner map of
-// the ordered scatter as coverage record, a copy of the uncovered pixels, then the ordered scatter.  Needs scratch
+// y = copy of ybase with the blocks written ("=") or added ("+=", non-overlapping) on top, moving every byte once: one
+// streaming kernel over y that reads ybase where the result needs it, the stack where a block covers the pixel, and writes
+// y once (planar stacks of geometries the kernel does not stage: tiles of the blocks and strips that copy the rest, in one
+// launch).  Which block lies where is read from the list by every workgroup, or from an inverse map (cell of the block grid
+// -> list position) in the scratch.  Plain writes under more than 2x2 blocks: the owner map of the ordered scatter as
+// coverage record, a copy of the uncovered pixels, then the ordered scatter.  Needs scratch
 // of scatter_cover_workspace_bytes() / scatter_owner_workspace_bytes(); `done` is false when the method does not
 // apply (no scratch, atomic mode, too little coverage to pay for the extra launches) and nothing was launched:
 // the caller then copies ybase and scatters in place.

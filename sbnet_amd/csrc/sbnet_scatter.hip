@@ -4,6 +4,8 @@
 // Reference semantics: sbnet_tensorflow/sbnet_ops/sparse_gather.cc:103-130, 135-142, 338-346.
 #include "sbnet_device.h"
 
+#include <type_traits>
+
 namespace sbnet {
 
 constexpr int NHWC_RANK_ROWS = 1;  // list rows per thread that the NHWC kernel fetches at once when it ranks its block
@@ -702,7 +704,7 @@ __global__ __launch_bounds__(256) void k_pull_map(const int16_t* __restrict__ id
     if (ib >= numActive || (a.g.countDev && ib >= *a.g.countDev)) return;
     const int64_t slot = pull_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
     if (slot < 0) return;  // this block cannot touch the image
-    if (atomicCAS(map + slot, -1, ib) != -1) *dup = 1;
+    if (atomicMax(map + slot, ib) != -1) *dup = 1;
 }
 
 // Both steps by one workgroup, for maps and lists small enough that one workgroup is done in the time a second
@@ -720,7 +722,7 @@ __global__ __launch_bounds__(1024) void k_pull_map_small(const int16_t* __restri
     if (a.g.countDev) count = min(count, max(*a.g.countDev, 0));
     for (int ib = tid; ib < count; ib += 1024) {
         const int64_t slot = pull_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
-        if (slot >= 0 && atomicCAS(map + slot, -1, ib) != -1) *dup = 1;
+        if (slot >= 0 && atomicMax(map + slot, ib) != -1) *dup = 1;
     }
 }
 
@@ -1494,27 +1496,42 @@ hipError_t launch_zero(float* y, size_t count, hipStream_t stream)
 // top (sparse_gather.cc:338-346 copies the whole base, then scatters).  Copy-then-scatter moves every covered
 // pixel twice more than needed.
 //
-// Blocks that do not overlap (bstride >= bsize on both axes, which add without atomics requires anyway,
-// sparse_gather.cc:322-326): the plane divides into cells of bstride[0] x bstride[1] pixels, cell (bh, bw)
-// holds block (bh, bw) in its first bsize rows and columns, and a pixel can only be written by the block of its
-// own cell.  With an inverse map "cell -> list position" (k_pull_fill, k_cell_map) ONE streaming kernel
-// (k_scatter_strip) walks the output in row order: a workgroup takes a strip of 4 image rows of one row of
-// cells, 256 channel vectors wide; a lane looks its cell up once, reads the base where the result needs it (all
-// of it for an add, the uncovered pixels for a plain write), reads the block stack where a block covers the
-// pixel, and writes the output once.  No flag bytes, no second pass over the covered pixels.
+// The plane divides into cells of bstride[0] x bstride[1] pixels.  Blocks that do not overlap (bstride >= bsize on both
+// axes, which add without atomics requires anyway, sparse_gather.cc:322-326): cell (bh, bw) holds block (bh, bw) in its
+// first bsize rows and columns, and a pixel can only be written by the block of its own cell.  Plain writes with at most
+// 2x2 blocks over a pixel: a pixel of cell (bh, bw) can also lie under the blocks (bh - 1, bw), (bh, bw - 1) and
+// (bh - 1, bw - 1), and the one listed last wins.  ONE streaming kernel (k_scatter_strip) walks the output in row order: a
+// workgroup takes a strip of 4 image rows of one row of cells, 256 channel vectors wide; a lane looks its cell up once,
+// reads the base where the result needs it (all of it for an add, the uncovered pixels for a plain write), reads the
+// block stack where a block covers the pixel, and writes the output once.
 //
-// Overlapping plain writes keep the owner map of the ordered scatter as their coverage record (k_copy_uncovered,
-// then the ordinary scatter kernels, which read the base where they add).
+// Which block lies where: with LIST every workgroup reads the block list itself and enters the rows that lie over its
+// strip into LDS, so that the whole op is one launch (STRIP_LIST_MAX); for longer lists an inverse map "cell -> list
+// position" is made first (k_pull_fill, k_cell_map).
+//
+// Planar stacks whose geometry the strips do not stage are moved by the tile kernel, along their planes, in the same launch
+// as strips that copy what no block covers (k_scatter_tiles_and_rest).  Plain writes under more than 2x2 blocks, or of lists
+// too long to be ranked, keep the owner map of the ordered scatter as their coverage record (k_copy_uncovered, then the
+// ordinary scatter kernels).
+//
+// Bound by memory where the tensor is large, by launches while it is small.  us of all launches, back to back, before (flat
+// copy and scatter, or owner map, copy of the uncovered pixels and scatter) / now, MI355X: overlapping plain writes on
+// 64x64x16, 32 10x10 blocks 8.5 / 5.9; [4,256,256,64], 231 18x18 blocks 27.9 / 23.8, planar 29.8 / 22.4; 300x480x256, 176
+// blocks 55.5 / 46.4 (6.6 TB/s), planar 59.5 / 52 (5.9 TB/s); planar with gaps, [4,256,256,64] 28.8 / 21.9.
+// Tiles before strips of 4 rows are as fast as any: spread among the strips 51.3 alone and 64.8 inside a training step
+// against 53.2 and 64.0 (300x480x256), with strips of 8 rows 52.2 and 69.3.
 
 struct StripArgs {
     Geom g;
     int bhMin, bwMin, nBH, nBW;  // cells that touch the image: bh in [bhMin, bhMin + nBH), likewise bw
+    int ovH, ovW;                // 1 where blocks reach into the next cell: the map has a row, a column more in front
+    uint32_t blocks;             // capacity of the block list
     uint32_t kPerBand;           // strips per row of cells: ceil(U / STRIP_ROWS)
     uint32_t CV;                 // channel vectors per pixel
     uint32_t CVT;                // channel vectors per pixel that one strip moves (a chunk of the channels)
     uint32_t CT;                 // the same in floats
     uint32_t nCC;                // channel chunks: ceil(CV / CVT)
-    uint32_t PX;                 // pixels per strip: 256 / CVT
+    uint32_t PX;                 // pixels per strip: threads / CVT
     uint32_t imgBytes;
     int64_t imgFloats;
     uint32_t swzMask;            // LDS staging of a planar stack: see strip_lds_index
@@ -1530,28 +1547,38 @@ struct StripArgs {
 __device__ __forceinline__ int64_t cell_slot(const StripArgs& a, int n, int bh, int bw)
 {
     if ((unsigned)n >= (unsigned)a.g.N) return -1;
-    const int ih = bh - a.bhMin, iw = bw - a.bwMin;
-    if ((unsigned)ih >= (unsigned)a.nBH || (unsigned)iw >= (unsigned)a.nBW) return -1;
-    return ((int64_t)n * a.nBH + ih) * a.nBW + iw;
+    const int ih = bh - a.bhMin + a.ovH, iw = bw - a.bwMin + a.ovW;
+    if ((unsigned)ih >= (unsigned)(a.nBH + a.ovH) || (unsigned)iw >= (unsigned)(a.nBW + a.ovW)) return -1;
+    return ((int64_t)n * (a.nBH + a.ovH) + ih) * (a.nBW + a.ovW) + iw;
 }
 
-// One thread per list row: the row's position goes into its cell.  A cell named by several rows keeps them as a
-// linked list (the map holds the row that arrived last, chain[row] the one it displaced) and raises `dup`; the
-// main kernel then walks the lists, so that a plain write still takes the row listed last and an add still sums
-// in list order, as the sequential CPU functor does (sparse_gather.cc:105-129).
-__global__ __launch_bounds__(256) void k_cell_map(const int16_t* __restrict__ idx, int numActive, StripArgs a,
-                                                   int32_t* __restrict__ map, int32_t* __restrict__ chain,
-                                                   int32_t* __restrict__ dup)
+// One thread per list row: the row's position goes into its cell.  A cell named by several rows takes the one listed last
+// for plain writes.  For an add (`chain`) it keeps them as a linked list (the map holds the row that arrived last,
+// chain[row] the one it displaced) and raises `dup`; the main kernel then walks the lists and sums in list order, as
+// the sequential CPU functor does (sparse_gather.cc:105-129).
+__device__ __forceinline__ void cell_enter(const int16_t* __restrict__ idx, int ib, const StripArgs& a, int32_t* map,
+                                           int32_t* chain, int32_t* dup)
 {
-    const int ib = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (ib >= numActive || (a.g.countDev && ib >= *a.g.countDev)) return;
     const int64_t slot = cell_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
+    if (!chain) {
+        if (slot >= 0) atomicMax(map + slot, ib);
+        return;
+    }
     int32_t prev = -1;
     if (slot >= 0) {
         prev = atomicExch(map + slot, ib);
         if (prev >= 0) *dup = 1;
     }
     chain[ib] = prev;
+}
+
+__global__ __launch_bounds__(256) void k_cell_map(const int16_t* __restrict__ idx, int numActive, StripArgs a,
+                                                   int32_t* __restrict__ map, int32_t* __restrict__ chain,
+                                                   int32_t* __restrict__ dup)
+{
+    const int ib = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (ib >= numActive || (a.g.countDev && ib >= *a.g.countDev)) return;
+    cell_enter(idx, ib, a, map, chain, dup);
 }
 
 // The cleared map and the list's rows in it by one workgroup, for maps and lists small enough that one workgroup
@@ -1566,15 +1593,53 @@ __global__ __launch_bounds__(1024) void k_cell_map_small(const int16_t* __restri
     __syncthreads();  // (the stores above are complete, and visible to this workgroup's atomics, beyond this point)
     int count = numActive;
     if (a.g.countDev) count = min(count, max(*a.g.countDev, 0));
-    for (int ib = tid; ib < count; ib += 1024) {
-        const int64_t slot = cell_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
-        int32_t prev = -1;
-        if (slot >= 0) {
-            prev = atomicExch(map + slot, ib);
-            if (prev >= 0) *dup = 1;
+    for (int ib = tid; ib < count; ib += 1024) cell_enter(idx, ib, a, map, chain, dup);
+}
+
+// The listed blocks over one strip's cells, entered into LDS by the strip's own workgroup: `cur` those of the strip's row of
+// cells, `up` those of the row above, entry 0 the cell left of the strip's first pixel's (or that one, where blocks
+// reach into no other cell).  Each entry is the position of the row listed last that names the block, -1 where none does.
+// Lists are read whole by every workgroup: 3 KB at 512 rows, from L2, beside the 16 to 32 KB that a strip moves.
+template <int CELLS>
+struct StripCells {
+    int32_t cur[CELLS], up[CELLS];
+    int32_t several;   // some block of the strip's row of cells is named by more than one row
+};
+
+constexpr int LIST_ROWS = 4;   // rows of the list in flight per thread
+
+template <int CELLS>
+__device__ __forceinline__ void strip_cells_of_list(StripCells<CELLS>& q, const int16_t* __restrict__ idx, const StripArgs& a,
+                                                    uint32_t n, int bh, int bw0)
+{
+    const uint32_t tid = threadIdx.x, nthr = blockDim.x;
+    const uint32_t count = list_count(a.g, a.blocks);
+    const ListRows lr = list_rows(idx, count);
+    for (uint32_t i = tid; i < (uint32_t)CELLS; i += nthr) q.cur[i] = q.up[i] = -1;
+    if (tid == 0) q.several = 0;
+    lds_barrier();
+    for (uint32_t j0 = 0; j0 < count; j0 += LIST_ROWS * nthr) {
+        ListRow rows[LIST_ROWS];
+#pragma unroll
+        for (int k = 0; k < LIST_ROWS; ++k) {
+            const uint32_t j = j0 + (uint32_t)k * nthr + tid;
+            rows[k] = list_row_load(lr, j, j < count);
         }
-        chain[ib] = prev;
+#pragma unroll
+        for (int k = 0; k < LIST_ROWS; ++k) {
+            const uint32_t j = j0 + (uint32_t)k * nthr + tid;
+            int n2, bh2, bw2;
+            list_row_unpack(rows[k], n2, bh2, bw2);
+            const uint32_t e = (uint32_t)(bw2 - bw0);
+            if (j >= count || n2 != (int)n || e >= (uint32_t)CELLS) continue;
+            if (bh2 == bh) {
+                if (atomicMax(&q.cur[e], (int)j) >= 0) q.several = 1;
+            } else if (a.ovH && bh2 == bh - 1) {
+                atomicMax(&q.up[e], (int)j);
+            }
+        }
     }
+    lds_barrier();
 }
 
 // VEC channels of block ib at block pixel (r, s), channel vector cv.
@@ -1611,9 +1676,9 @@ __device__ __forceinline__ uint32_t strip_lds_index(const StripArgs& a, uint32_t
 
 constexpr int STRIP_SLOTS = 4;  // 16-byte slots per thread: 256 threads x 4 x 16 B = the strip's 16 KB
 
-__device__ __forceinline__ void strip_stage_planar(const float* __restrict__ x, const int32_t* __restrict__ mapRow,
-                                                   const StripArgs& a, float* lds, uint32_t pc, uint32_t c0, int r0,
-                                                   int hTop)
+// strip: the entries of the strip's cells, the first one's first.
+__device__ __forceinline__ void strip_stage_planar(const float* __restrict__ x, const int32_t* strip, const StripArgs& a,
+                                                   float* lds, uint32_t pc, uint32_t c0, int r0, int hTop)
 {
     const uint32_t C = (uint32_t)a.g.C, S = (uint32_t)a.g.S;
     const int64_t plane = (int64_t)a.g.R * a.g.S;
@@ -1636,7 +1701,7 @@ __device__ __forceinline__ void strip_stage_planar(const float* __restrict__ x, 
         const int r = r0 + (int)uu[k];
         use[k] = cell < a.cellsPerStrip && iw0 + cell < (uint32_t)a.nBW && c0 + cl[k] < C && r < a.g.R &&
                  (unsigned)(hTop + (int)uu[k]) < (unsigned)a.g.H && pc * a.PX + px[k] < (uint32_t)a.g.W;
-        ib[k] = use[k] ? mapRow[iw0 + cell] : -1;
+        ib[k] = use[k] ? strip[cell] : -1;
     }
     f4 val[STRIP_SLOTS];
 #pragma unroll
@@ -1659,57 +1724,71 @@ __device__ __forceinline__ void strip_stage_planar(const float* __restrict__ x, 
     }
 }
 
-// sparse_gather.cc:103-130 on top of a copy of ybase (sparse_gather.cc:338-346), non-overlapping blocks.
+// Which strip: channel chunk, pixel chunk, strip of the row of cells, row of cells, image, the first fastest:
+// neighbouring workgroups write neighbouring pieces of the same image rows.
+struct StripId {
+    uint32_t cc, pc, band, n;
+    int r0, hTop;   // first row of the strip, of a block and of the image
+};
+
+__device__ __forceinline__ StripId decode_strip(const StripArgs& a, uint32_t strip)
+{
+    StripId id;
+    uint32_t l = strip, t = fdiv(l, a.dCC);
+    id.cc = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * a.nCC));
+    l = t; t = fdiv(l, a.dPC);
+    id.pc = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * a.nPC));
+    l = t; t = fdiv(l, a.dK);
+    id.r0 = __builtin_amdgcn_readfirstlane((int)(l - t * a.kPerBand)) * STRIP_ROWS;
+    l = t; t = fdiv(l, a.dBH);
+    id.band = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * (uint32_t)a.nBH));
+    id.n = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+    id.hTop = a.g.oh + ((int)id.band + a.bhMin) * a.g.U + id.r0;
+    return id;
+}
+
+// Entries of a strip's row of cells and of the row above it in the map, cell iw0's first.
+template <bool OVER>
+__device__ __forceinline__ void strip_cells_of_map(const StripArgs& a, const int32_t* __restrict__ map, const StripId& id, uint32_t iw0,
+                                                   const int32_t*& cur, const int32_t*& up)
+{
+    const uint32_t cols = (uint32_t)(a.nBW + (OVER ? a.ovW : 0)), rows = (uint32_t)(a.nBH + (OVER ? a.ovH : 0));
+    cur = map + ((int64_t)id.n * rows + id.band + (OVER ? a.ovH : 0)) * cols + iw0 + (OVER ? a.ovW : 0);
+    up = cur - cols;
+}
+
+// sparse_gather.cc:103-130 on top of a copy of ybase (sparse_gather.cc:338-346).
 // OP: STRIP_ASSIGN / STRIP_ADD write the whole output; STRIP_COPY writes only the pixels that no block covers and
-// leaves the covered ones to a scatter kernel that follows (planar stacks whose geometry the staging above does
-// not take).
+// leaves the covered ones to the tiles of the same launch.  OVER: blocks overlap (plain writes, NHWC stack).
 constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2;
 
-template <int VEC, int OP, bool PLANAR>
-__global__ __launch_bounds__(256) void k_scatter_strip(const float* __restrict__ x, const float* __restrict__ ybase,
-                                                       float* __restrict__ y, const int32_t* __restrict__ map,
-                                                       const int32_t* __restrict__ chain,
-                                                       const int32_t* __restrict__ dup, StripArgs a)
+template <int VEC, int OP, bool PLANAR, bool LIST, bool OVER, int CELLS>
+__device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const float* __restrict__ ybase,
+                                              float* __restrict__ y, const int16_t* __restrict__ idx,
+                                              const int32_t* __restrict__ map, const int32_t* __restrict__ chain,
+                                              const int32_t* __restrict__ dup, const StripArgs& a, float* lds,
+                                              StripCells<CELLS>* cells, uint32_t strip)
 {
     typedef typename Vec<VEC>::type vec;
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
     constexpr bool ADD = OP == STRIP_ADD;
     const uint32_t tid = threadIdx.x;
-    // Which strip: channel chunk, pixel chunk, strip of the row of cells, row of cells, image, the first fastest:
-    // neighbouring workgroups write neighbouring pieces of the same image rows.
-    uint32_t l = blockIdx.x;
-    uint32_t t = fdiv(l, a.dCC);
-    const uint32_t cc = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * a.nCC));
-    l = t; t = fdiv(l, a.dPC);
-    const uint32_t pc = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * a.nPC));
-    l = t; t = fdiv(l, a.dK);
-    const int r0 = __builtin_amdgcn_readfirstlane((int)(l - t * a.kPerBand)) * STRIP_ROWS;  // first block row of the strip
-    l = t; t = fdiv(l, a.dBH);
-    const uint32_t band = (uint32_t)__builtin_amdgcn_readfirstlane((int)(l - t * (uint32_t)a.nBH));
-    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
-    const int hTop = a.g.oh + ((int)band + a.bhMin) * a.g.U + r0;  // the strip's first image row
+    const StripId id = decode_strip(a, strip);
+    const uint32_t cc = id.cc, pc = id.pc, band = id.band, n = id.n;
+    const int r0 = id.r0, hTop = id.hTop;
 
     const uint32_t wl = fdiv(tid, a.dCVT), cvl = tid - wl * a.CVT;
     const uint32_t cv = cc * a.CVT + cvl;
     const uint32_t w = pc * a.PX + wl;
     const bool live = wl < a.PX && w < (uint32_t)a.g.W && cv < a.CV;
 
-    // the lane's cell: one look-up for the strip's rows (they lie in one row of cells)
-    const int32_t* __restrict__ mapRow = map + ((int64_t)n * a.nBH + band) * a.nBW;
-    const uint32_t dw = w - (uint32_t)(a.g.ow + a.bwMin * a.g.V);  // >= 0 for every pixel of the image
-    const uint32_t iw = fdiv(dw, a.dV), s = dw - iw * (uint32_t)a.g.V;
-    int ib = -1;
-    if (live && s < (uint32_t)a.g.S && r0 < a.g.R) ib = mapRow[iw];
-
     const rsrc_t br = make_rsrc(ybase + (int64_t)n * a.imgFloats, a.imgBytes);
     const rsrc_t yr = make_rsrc(y + (int64_t)n * a.imgFloats, a.imgBytes);
     uint32_t off[STRIP_ROWS];
-    bool inBlock[STRIP_ROWS];  // (the same for the whole workgroup)
 #pragma unroll
     for (int u = 0; u < STRIP_ROWS; ++u) {
         const int h = hTop + u;
         const bool rowLive = r0 + u < a.g.U && (unsigned)h < (unsigned)a.g.H;
-        inBlock[u] = r0 + u < a.g.R;
         off[u] = live && rowLive ? (((uint32_t)h * (uint32_t)a.g.W + w) * a.CV + cv) * (uint32_t)(VEC * 4) : BUF_OOB;
     }
     vec b[STRIP_ROWS], v[STRIP_ROWS];
@@ -1718,32 +1797,65 @@ __global__ __launch_bounds__(256) void k_scatter_strip(const float* __restrict__
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) b[u] = buf_load<VEC>(br, off[u]);
     }
+
+    // the lane's cell: one look-up for the strip's rows (they lie in one row of cells)
+    const uint32_t pixel0 = (uint32_t)(a.g.ow + a.bwMin * a.g.V);   // (w - pixel0 >= 0 for every pixel of the image)
+    const uint32_t iw = fdiv(w - pixel0, a.dV), s = w - pixel0 - iw * (uint32_t)a.g.V;
+    const uint32_t iw0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)fdiv(pc * a.PX - pixel0, a.dV));
+    const int32_t *cur, *up;   // entries of the strip's cells, iw0's first
+    if constexpr (LIST) {
+        strip_cells_of_list(*cells, idx, a, n, (int)band + a.bhMin, (int)iw0 + a.bwMin - (OVER ? a.ovW : 0));
+        cur = cells->cur + (OVER ? a.ovW : 0);
+        up = cells->up + (OVER ? a.ovW : 0);
+    } else {
+        strip_cells_of_map<OVER>(a, map, id, iw0, cur, up);
+    }
+    int ib = -1, ibUp = -1;   // the block that wins the lane's pixels among those of this row of cells, of the one above
+    uint32_t sIb = s, sUp = s;
+    if (live && r0 < a.g.R) {
+        if (s < (uint32_t)a.g.S) ib = cur[iw - iw0];
+        if constexpr (OVER) {
+            const bool left = s + (uint32_t)a.g.V < (uint32_t)a.g.S, above = r0 + a.g.U < a.g.R;
+            int ibL = -1, upL = -1;
+            if (left) ibL = cur[(int)(iw - iw0) - 1];
+            if (above && s < (uint32_t)a.g.S) ibUp = up[iw - iw0];
+            if (above && left) upL = up[(int)(iw - iw0) - 1];
+            if (ibL > ib) { ib = ibL; sIb = s + (uint32_t)a.g.V; }
+            if (upL > ibUp) { ibUp = upL; sUp = s + (uint32_t)a.g.V; }
+        }
+    }
+    int at[STRIP_ROWS];   // the block whose value row u takes, -1: the base's
+#pragma unroll
+    for (int u = 0; u < STRIP_ROWS; ++u) {
+        const int r = r0 + u;
+        at[u] = r < a.g.R ? ib : -1;
+        if (OVER && r + a.g.U < a.g.R) at[u] = max(at[u], ibUp);
+        if (off[u] == BUF_OOB) at[u] = -1;
+    }
     if (OP == STRIP_COPY) {
-        // covered pixels (whichever rows of the list cover them) belong to the scatter kernel that follows
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) {
-            if (ib >= 0 && inBlock[u]) off[u] = BUF_OOB;
+            if (at[u] >= 0) off[u] = BUF_OOB;
             b[u] = buf_load<VEC>(br, off[u]);
         }
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
         return;
     }
-    const bool dups = *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0;
-    if (!dups) {
-        const bool cov = ib >= 0;
+    bool several = false;
+    if (ADD) several = LIST ? cells->several != 0 : *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0;
+    if (!several) {
         if (!ADD) {
 #pragma unroll
-            for (int u = 0; u < STRIP_ROWS; ++u) b[u] = buf_load<VEC>(br, cov && inBlock[u] ? BUF_OOB : off[u]);  // covered pixels are not read
+            for (int u = 0; u < STRIP_ROWS; ++u) b[u] = buf_load<VEC>(br, at[u] >= 0 ? BUF_OOB : off[u]);  // covered pixels are not read
         }
         if (PLANAR && r0 < a.g.R) {
-            extern __shared__ __attribute__((aligned(16))) float lds[];
-            strip_stage_planar(x, mapRow, a, lds, pc, cc * a.CT, r0, hTop);
+            strip_stage_planar(x, cur, a, lds, pc, cc * a.CT, r0, hTop);
             lds_barrier();
 #pragma unroll
             for (int u = 0; u < STRIP_ROWS; ++u) {
                 v[u] = vzero<VEC>();
-                if (cov && inBlock[u] && off[u] != BUF_OOB) {
+                if (at[u] >= 0) {
                     if (VEC == 4) {
                         const f4 q = lds_read4(lds + strip_lds_index(a, (uint32_t)u, wl, cvl * 4u));
 #pragma unroll
@@ -1757,56 +1869,161 @@ __global__ __launch_bounds__(256) void k_scatter_strip(const float* __restrict__
         } else {
 #pragma unroll
             for (int u = 0; u < STRIP_ROWS; ++u) {
+                const bool fromUp = OVER && at[u] > ib;   // (positions differ: at[u] is the larger of the two)
                 v[u] = vzero<VEC>();
-                if (cov && inBlock[u] && off[u] != BUF_OOB) v[u] = strip_stack_load<VEC, false>(x, ib, r0 + u, s, cv, a);
+                if (at[u] >= 0)
+                    v[u] = strip_stack_load<VEC, false>(x, at[u], r0 + u + (fromUp ? a.g.U : 0), fromUp ? sUp : sIb, cv, a);
             }
         }
 #pragma unroll
-        for (int u = 0; u < STRIP_ROWS; ++u) {
-            const bool hit = cov && inBlock[u];
-            buf_store<BUF_NT>(yr, off[u], hit ? (ADD ? vadd(b[u], v[u]) : v[u]) : b[u]);
-        }
+        for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], at[u] >= 0 ? (ADD ? vadd(b[u], v[u]) : v[u]) : b[u]);
         return;
     }
-    // Some cell is named by several rows of the list (rare; reduce_mask never produces such a list): the rows of a
-    // cell form a linked list.  A plain write takes the row listed last; an add sums the rows in list order.
-    if (!ADD) {
-        for (int c = ib; c >= 0; c = chain[c]) ib = max(ib, c);
+    // An add, and some cell is named by several rows of the list (rare; reduce_mask never produces such a list): the sum of
+    // the rows in list order.
+    auto add_row = [&](int row) {
 #pragma unroll
-        for (int u = 0; u < STRIP_ROWS; ++u) {
-            const bool hit = ib >= 0 && inBlock[u];
-            vec out;
-            if (hit && off[u] != BUF_OOB) out = strip_stack_load<VEC, PLANAR>(x, ib, r0 + u, s, cv, a);
-            else out = buf_load<VEC>(br, hit ? BUF_OOB : off[u]);
-            buf_store<BUF_NT>(yr, off[u], out);
+        for (int u = 0; u < STRIP_ROWS; ++u)
+            if (at[u] >= 0) b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, row, r0 + u, s, cv, a));
+    };
+    if constexpr (LIST) {
+        const uint32_t count = list_count(a.g, a.blocks);
+        for (uint32_t j = 0; j < count; ++j) {
+            const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
+            if (o.n == (int)n && o.bh == (int)band + a.bhMin && o.bw == (int)iw + a.bwMin) add_row((int)j);
         }
-    } else {
+    } else {   // (the rows of a cell form a linked list)
         int prev = -1;
         while (ib >= 0) {
-            int cur = 0x7fffffff;
+            int next = 0x7fffffff;
             for (int c = ib; c >= 0; c = chain[c])
-                if (c > prev && c < cur) cur = c;
-            if (cur == 0x7fffffff) break;
-#pragma unroll
-            for (int u = 0; u < STRIP_ROWS; ++u)
-                if (inBlock[u] && off[u] != BUF_OOB) b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, cur, r0 + u, s, cv, a));
-            prev = cur;
+                if (c > prev && c < next) next = c;
+            if (next == 0x7fffffff) break;
+            add_row(next);
+            prev = next;
         }
+    }
 #pragma unroll
-        for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+    for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+}
+
+constexpr int STRIP_THREADS = 256, STRIP_CELLS = STRIP_THREADS + 2;   // a pixel a thread, one-pixel cells, one to the left
+
+template <int VEC, int OP, bool PLANAR, bool LIST, bool OVER>
+__global__ __launch_bounds__(STRIP_THREADS) void k_scatter_strip(const float* __restrict__ x, const float* __restrict__ ybase,
+                                                                 float* __restrict__ y, const int16_t* __restrict__ idx,
+                                                                 const int32_t* __restrict__ map,
+                                                                 const int32_t* __restrict__ chain,
+                                                                 const int32_t* __restrict__ dup, StripArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ StripCells<LIST ? STRIP_CELLS : 1> cells;
+    scatter_strip<VEC, OP, PLANAR, LIST, OVER>(x, ybase, y, idx, map, chain, dup, a, lds, &cells, blockIdx.x);
+}
+
+// STRIP_COPY where the channels make no 16-byte vectors: a lane takes four consecutive floats of the image row, whatever
+// pixels they belong to (gfx950 moves misaligned dwordx4 at the speed of aligned ones), and moves them one by one where
+// a block covers some of them or the row ends.  [3,301,203,15], 781 planar 9x9 blocks, tiles included: 9.7 us; 12.5 with a
+// float a lane, 10.3 as a flat copy and a scatter.
+template <bool LIST, bool OVER, int CELLS>
+__device__ __forceinline__ void copy_strip_flat(const float* __restrict__ ybase, float* __restrict__ y,
+                                                const int16_t* __restrict__ idx, const int32_t* __restrict__ map, const StripArgs& a,
+                                                StripCells<CELLS>* cells, uint32_t strip)
+{
+    const StripId id = decode_strip(a, strip);
+    const uint32_t rowF = (uint32_t)a.g.W * a.CT, f0 = (id.pc * blockDim.x + threadIdx.x) * 4u;   // (CT: all channels)
+    const uint32_t pixel0 = (uint32_t)(a.g.ow + a.bwMin * a.g.V);
+    const uint32_t iw0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)fdiv(fdiv(id.pc * blockDim.x * 4u, a.dCT) - pixel0, a.dV));
+    const int32_t *cur, *up;
+    if constexpr (LIST) {
+        strip_cells_of_list(*cells, idx, a, id.n, (int)id.band + a.bhMin, (int)iw0 + a.bwMin - (OVER ? a.ovW : 0));
+        cur = cells->cur + (OVER ? a.ovW : 0);
+        up = cells->up + (OVER ? a.ovW : 0);
+    } else {
+        strip_cells_of_map<OVER>(a, map, id, iw0, cur, up);
+    }
+    // Which of the four floats are covered (or past the row), in rows under this row of cells, under the row above.
+    uint32_t here = 0u, above = 0u, dead = 0u;
+    uint32_t w = fdiv(f0, a.dCT), c = f0 - w * a.CT;
+    bool h = false, ab = false, fresh = true;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        const bool in = f0 + k < rowF;
+        if (in && fresh) {
+            const uint32_t iw = fdiv(w - pixel0, a.dV), s = w - pixel0 - iw * (uint32_t)a.g.V;
+            const int e = (int)(iw - iw0);
+            const bool own = s < (uint32_t)a.g.S, left = OVER && s + (uint32_t)a.g.V < (uint32_t)a.g.S;
+            h = (own && cur[e] >= 0) || (left && cur[e - 1] >= 0);
+            if (OVER && id.r0 + a.g.U < a.g.R) ab = (own && up[e] >= 0) || (left && up[e - 1] >= 0);
+        }
+        here |= (uint32_t)(in && h) << k;
+        above |= (uint32_t)(in && ab) << k;
+        dead |= (uint32_t)!in << k;
+        fresh = ++c == a.CT;
+        c = fresh ? 0u : c;
+        w += fresh ? 1u : 0u;
+    }
+    const rsrc_t br = make_rsrc(ybase + (int64_t)id.n * a.imgFloats, a.imgBytes);
+    const rsrc_t yr = make_rsrc(y + (int64_t)id.n * a.imgFloats, a.imgBytes);
+    uint32_t off[STRIP_ROWS], skip[STRIP_ROWS], some = 0u;
+    f4 v[STRIP_ROWS];
+#pragma unroll
+    for (int u = 0; u < STRIP_ROWS; ++u) {
+        const int r = id.r0 + u, row = id.hTop + u;
+        const bool rowLive = r < a.g.U && (unsigned)row < (unsigned)a.g.H;
+        skip[u] = rowLive ? dead | (r < a.g.R ? here : 0u) | (OVER && r + a.g.U < a.g.R ? above : 0u) : 15u;
+        off[u] = ((uint32_t)row * rowF + f0) * 4u;
+        some |= (uint32_t)(skip[u] != 0u && skip[u] != 15u);
+        v[u] = buf_load<4>(br, skip[u] ? BUF_OOB : off[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, skip[u] ? BUF_OOB : off[u], v[u]);
+    if (!some) return;
+    float t[STRIP_ROWS][4];
+#pragma unroll
+    for (int u = 0; u < STRIP_ROWS; ++u)
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) t[u][k] = buf_load<1>(br, skip[u] && !((skip[u] >> k) & 1u) ? off[u] + 4u * k : BUF_OOB);
+#pragma unroll
+    for (int u = 0; u < STRIP_ROWS; ++u)
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) buf_store<BUF_NT>(yr, skip[u] && !((skip[u] >> k) & 1u) ? off[u] + 4u * k : BUF_OOB, t[u][k]);
+}
+
+// Planar stack of a geometry that the strips do not stage (18x18 blocks at an odd offset: 72-byte pieces at 8-byte
+// alignment): the tiles of the listed blocks, which read the stack along its planes, and strips that copy what no block
+// covers, in one launch.  MODE: of the tiles; SCATTER_RANKED_INLINE where blocks overlap.
+constexpr int REST_CELLS = 512 + 2;
+
+template <int VEC, int MODE, bool LIST>
+__global__ __launch_bounds__(512) void k_scatter_tiles_and_rest(const float* __restrict__ x, const float* __restrict__ ybase,
+                                                                float* __restrict__ y, const int16_t* __restrict__ idx,
+                                                                const int32_t* __restrict__ map, TileArgs a, ColorArgs col,
+                                                                StripArgs s)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ uint32_t waveBits[8];
+    __shared__ StripCells<LIST ? REST_CELLS : 1> cells;
+    if (blockIdx.x < a.total) {
+        const uint32_t ib = fdiv(blockIdx.x, a.dTpb);
+        scatter_planar_tile<VEC, MODE, TileRt>(x, y, ybase, idx, a, col, lds, waveBits, ib, blockIdx.x - ib * a.tpb);
+    } else if constexpr (VEC < 4) {
+        copy_strip_flat<LIST, MODE == SCATTER_RANKED_INLINE>(ybase, y, idx, map, s, &cells, blockIdx.x - a.total);
+    } else {
+        scatter_strip<VEC, STRIP_COPY, false, LIST, MODE == SCATTER_RANKED_INLINE>(x, ybase, y, idx, map, nullptr, nullptr, s, lds,
+                                                                                   &cells, blockIdx.x - a.total);
     }
 }
 
 // ---- planar stack, blocks that tile the plane (bsize == bstride): one launch over the cells --------------------
 //
-// A planar stack whose rows the strips above cannot stage (18x18 blocks at an odd offset: 72-byte pieces at 8-byte
-// alignment) wants to be read along its planes, by the tile kernel.  With bsize == bstride a cell is exactly its
-// block, so the launch runs over the CELLS of the grid instead of the list: a workgroup looks its cell up in the
-// map; an active cell is scattered as one tile of scatter_planar_tile (which reads the base where it adds), an
-// empty cell is copied from the base, tile number `rem` of its `tpb` taking every tpb-th part of the cell's row
-// segments.  Every byte of the output is written once and nothing is read twice.  A cell that several rows of the
-// list name (rare) is built element by element: the row listed last for a plain write, every row in list order
-// for an add (sparse_gather.cc:105-129).
+// The stack is read along its planes, by the tile kernel.  With bsize == bstride a cell is exactly its
+// block, so the launch runs over the CELLS of the grid instead of the list: a workgroup looks its cell up, in the list
+// itself (LIST) or in the map; an active cell is scattered as one tile of scatter_planar_tile (which reads the base
+// where it adds), an empty cell is copied from the base, tile number `rem` of its `tpb` taking every tpb-th part of the
+// cell's row segments.  Every byte of the output is written once and nothing is read twice.  A cell that several rows of
+// the list name takes the one listed last for a plain write; an add builds it element by element, from every row in list
+// order (sparse_gather.cc:105-129; rare).
 struct CellArgs {
     int bhMin, bwMin, nBH, nBW;
     uint32_t CV;  // channel vectors per pixel
@@ -1815,18 +2032,16 @@ struct CellArgs {
 
 constexpr int CELL_UNR = 4;
 
-template <int VEC, int MODE>
+// head: -1, or the cell's row of the list that `chain` goes on from (chain == nullptr: the whole list is searched).
+template <int VEC>
 __device__ __forceinline__ void cell_by_elements(const float* __restrict__ x, const float* __restrict__ ybase,
-                                                 float* __restrict__ y, const int32_t* __restrict__ chain,
-                                                 const TileArgs& a, const CellArgs& c, int head, uint32_t cell,
-                                                 uint32_t rem)
+                                                 float* __restrict__ y, const int16_t* __restrict__ idx,
+                                                 const int32_t* __restrict__ chain, const TileArgs& a, const CellArgs& c,
+                                                 int head, uint32_t n, int bh, int bw, uint32_t rem)
 {
     typedef typename Vec<VEC>::type vec;
     const Geom& g = a.g;
-    const uint32_t n = fdiv(cell, c.dBHW);
-    const uint32_t inImg = cell - n * (uint32_t)(c.nBH * c.nBW);
-    const uint32_t ih = fdiv(inImg, c.dBW), iw = inImg - ih * (uint32_t)c.nBW;
-    const int h0 = g.oh + ((int)ih + c.bhMin) * g.U, w0 = g.ow + ((int)iw + c.bwMin) * g.V;
+    const int h0 = g.oh + bh * g.U, w0 = g.ow + bw * g.V;
     const int hlo = max(0, h0), hhi = min(g.H, h0 + g.U), wlo = max(0, w0), whi = min(g.W, w0 + g.V);
     if (hhi <= hlo || whi <= wlo) return;
     const uint32_t segV = (uint32_t)(whi - wlo) * c.CV;  // vectors per row segment: contiguous in the tensor
@@ -1851,39 +2066,36 @@ __device__ __forceinline__ void cell_by_elements(const float* __restrict__ x, co
         }
         return;
     }
-    // several rows of the list name this cell
+    // an add, and several rows of the list name this cell
     const int64_t plane = (int64_t)g.R * g.S;
-    int last = head;
-    for (int q = head; q >= 0; q = chain[q]) last = max(last, q);
+    const int count = (int)list_count(g, a.blocks);
     for (uint32_t e = rem * nthr + threadIdx.x; e < total; e += stride) {
         const uint32_t r = e / segV, j = e - r * segV;
         const uint32_t px = j / c.CV, cv = j - px * c.CV;
         const uint32_t off = ((((uint32_t)hlo + r) * (uint32_t)g.W + (uint32_t)wlo) * c.CV + j) * (uint32_t)(VEC * 4);
         const int64_t at = ((int64_t)hlo + r - h0) * g.S + ((int64_t)wlo + px - w0);  // the pixel inside the block's plane
-        vec out;
-        if (MODE == SCATTER_ADD) {
-            out = buf_load<VEC>(br, off);
-            int prev = -1;
-            for (;;) {
-                int cur = 0x7fffffff;
+        vec out = buf_load<VEC>(br, off);
+        int prev = -1;
+        for (;;) {
+            int cur = 0x7fffffff;
+            if (chain) {
                 for (int q = head; q >= 0; q = chain[q])
                     if (q > prev && q < cur) cur = q;
-                if (cur == 0x7fffffff) break;
-                const float* __restrict__ src = x + ((int64_t)cur * g.C + cv * VEC) * plane + at;
-#pragma unroll
-                for (int k = 0; k < VEC; ++k) vset(out, k, vget(out, k) + src[k * plane]);
-                prev = cur;
+            } else {
+                for (int q = prev + 1; q < count && cur == 0x7fffffff; ++q)
+                    if (idx[(size_t)q * 3] == (int)n && idx[(size_t)q * 3 + 1] == bh && idx[(size_t)q * 3 + 2] == bw) cur = q;
             }
-        } else {
-            const float* __restrict__ src = x + ((int64_t)last * g.C + cv * VEC) * plane + at;
+            if (cur == 0x7fffffff) break;
+            const float* __restrict__ src = x + ((int64_t)cur * g.C + cv * VEC) * plane + at;
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) vset(out, k, src[k * plane]);
+            for (int k = 0; k < VEC; ++k) vset(out, k, vget(out, k) + src[k * plane]);
+            prev = cur;
         }
         buf_store<BUF_NT>(yr, off, out);
     }
 }
 
-template <int VEC, int MODE>
+template <int VEC, int MODE, bool LIST>
 __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__ x, const float* ybase, float* y,
                                                        const int16_t* __restrict__ idx,
                                                        const int32_t* __restrict__ map,
@@ -1893,6 +2105,7 @@ __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ uint32_t waveBits[8];
+    __shared__ int32_t found[2];   // LIST: the cell's row listed last, number of its rows
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
     uint32_t cell, rem;
     if (a.grid2d) {
@@ -1902,16 +2115,50 @@ __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__
         cell = blockIdx.x / a.tpb;
         rem = blockIdx.x - cell * a.tpb;
     }
-    // (scalar loads: the map was written by an earlier launch and is not written here)
-    const int head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(map)))[cell];
-    const bool dups = *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0;
+    const uint32_t n = fdiv(cell, c.dBHW), inImg = cell - n * (uint32_t)(c.nBH * c.nBW), ih = fdiv(inImg, c.dBW);
+    const int bh = (int)ih + c.bhMin, bw = (int)(inImg - ih * (uint32_t)c.nBW) + c.bwMin;
+    int head;
     bool several = false;
-    if (dups && head >= 0) several = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(chain)))[head] >= 0;
+    if constexpr (LIST) {
+        const uint32_t tid = threadIdx.x, nthr = blockDim.x, count = list_count(a.g, a.blocks);
+        const ListRows lr = list_rows(idx, count);
+        if (tid == 0) {
+            found[0] = -1;
+            found[1] = 0;
+        }
+        lds_barrier();
+        for (uint32_t j0 = 0; j0 < count; j0 += LIST_ROWS * nthr) {
+            ListRow rows[LIST_ROWS];
+#pragma unroll
+            for (int k = 0; k < LIST_ROWS; ++k) {
+                const uint32_t j = j0 + (uint32_t)k * nthr + tid;
+                rows[k] = list_row_load(lr, j, j < count);
+            }
+#pragma unroll
+            for (int k = 0; k < LIST_ROWS; ++k) {
+                const uint32_t j = j0 + (uint32_t)k * nthr + tid;
+                int n2, bh2, bw2;
+                list_row_unpack(rows[k], n2, bh2, bw2);
+                if (j < count && n2 == (int)n && bh2 == bh && bw2 == bw) {
+                    atomicMax(&found[0], (int)j);
+                    atomicAdd(&found[1], 1);
+                }
+            }
+        }
+        lds_barrier();
+        head = __builtin_amdgcn_readfirstlane(found[0]);
+        if (MODE == SCATTER_ADD) several = __builtin_amdgcn_readfirstlane(found[1]) > 1;
+    } else {
+        // (scalar loads: the map was written by an earlier launch and is not written here)
+        head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(map)))[cell];
+        if (MODE == SCATTER_ADD && head >= 0 && *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0)
+            several = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(chain)))[head] >= 0;
+    }
     if (head >= 0 && !several) {
         scatter_planar_tile<VEC, MODE, TileRt>(x, y, ybase, idx, a, col, lds, waveBits, (uint32_t)head, rem);
         return;
     }
-    cell_by_elements<VEC, MODE>(x, ybase, y, chain, a, c, head, cell, rem);
+    cell_by_elements<VEC>(x, ybase, y, idx, LIST ? nullptr : chain, a, c, head, n, bh, bw, rem);
 }
 
 struct CoverArgs {
@@ -1978,12 +2225,19 @@ __global__ __launch_bounds__(256) void k_copy_uncovered(const float* __restrict_
     for (int u = 0; u < COVER_UNR; ++u) buf_store<BUF_NT>(dr, off[u], v[u]);
 }
 
-// Cells that touch the image and the strip geometry; false where k_scatter_strip does not apply.
+// Cells that touch the image and the strip geometry; false where the strips do not apply.
 // `planar`: the strips also stage a planar stack through LDS (strip_stage_planar); false where that does not apply.
-static bool make_strip_args(const Geom& g, int vec, bool planar, const float* x, StripArgs& a, int64_t& mapN)
+// `rest`: threads of a workgroup whose strips only copy, and may split a pixel's channels; 0: STRIP_THREADS, they may not.
+static bool make_strip_args(const Geom& g, int numActive, int vec, bool planar, const float* x, StripArgs& a, int64_t& mapN,
+                            int rest = 0)
 {
-    if (g.U < g.R || g.V < g.S) return false;  // overlapping blocks: a pixel may belong to several
+    const uint32_t threads = rest ? (uint32_t)rest : (uint32_t)STRIP_THREADS;
+    a.ovH = g.U < g.R ? 1 : 0;
+    a.ovW = g.V < g.S ? 1 : 0;
+    if (g.R > 2 * (int64_t)g.U || g.S > 2 * (int64_t)g.V) return false;  // more than 2x2 blocks over a pixel
+    if (planar && (a.ovH || a.ovW)) return false;
     a.g = g;
+    a.blocks = (uint32_t)numActive;
     a.imgFloats = (int64_t)g.H * g.W * g.C;
     if (a.imgFloats >= (1ll << 30)) return false;  // 32-bit byte offsets inside one image
     if ((int64_t)g.R * g.S >= (1ll << 31)) return false;
@@ -1994,7 +2248,7 @@ static bool make_strip_args(const Geom& g, int vec, bool planar, const float* x,
     if (bhMin < -(1ll << 30) || bwMin < -(1ll << 30) || bhMax > (1ll << 30) || bwMax > (1ll << 30)) return false;
     a.bhMin = (int)bhMin; a.bwMin = (int)bwMin;
     a.nBH = (int)(bhMax - bhMin + 1); a.nBW = (int)(bwMax - bwMin + 1);
-    mapN = (int64_t)g.N * a.nBH * a.nBW;
+    mapN = (int64_t)g.N * (a.nBH + a.ovH) * (a.nBW + a.ovW);
     if (mapN >= (1ll << 31)) return false;
     if ((int64_t)g.ow + (int64_t)a.bwMin * g.V < -(1ll << 31)) return false;
     a.kPerBand = (uint32_t)((g.U + STRIP_ROWS - 1) / STRIP_ROWS);
@@ -2002,12 +2256,21 @@ static bool make_strip_args(const Geom& g, int vec, bool planar, const float* x,
     // NHWC stack: all channels of a pixel in one strip (both sides move whole pixels).  Planar stack: chunks of 32
     // channels, so that a strip is wide enough in pixels to take whole cells.
     a.CVT = planar && a.CV * (uint32_t)vec > 32u ? 32u / (uint32_t)vec : a.CV;
-    if (a.CVT > 256u) return false;
+    if (a.CVT > threads) {
+        if (!rest) return false;
+        a.CVT = threads;
+    }
     a.CT = a.CVT * (uint32_t)vec;
     a.nCC = (a.CV + a.CVT - 1u) / a.CVT;
-    a.PX = 256u / a.CVT;
+    a.PX = threads / a.CVT;
     a.imgBytes = (uint32_t)(a.imgFloats * 4);
     a.nPC = ((uint32_t)g.W + a.PX - 1u) / a.PX;
+    if (rest && vec < 4) {   // (copy_strip_flat)
+        a.CT = (uint32_t)g.C;
+        a.nCC = 1;
+        a.nPC = ((uint32_t)g.W * a.CT + 4u * threads - 1u) / (4u * threads);
+        if (4ll * threads / ((int64_t)g.C * g.V) + 4 > REST_CELLS) return false;   // more cells than LDS entries
+    }
     const int64_t tiles = (int64_t)g.N * a.nBH * a.kPerBand * a.nPC * a.nCC;
     if (tiles >= (1ll << 31)) return false;
     a.tiles = (uint32_t)tiles;
@@ -2043,7 +2306,7 @@ size_t scatter_cover_workspace_bytes(const Geom& g, int numActive)
     StripArgs a;
     int64_t mapN = 0;
     // (with the widest channel vectors C allows; a call whose pointers force narrower ones checks again)
-    if (make_strip_args(g, g.C % 4 == 0 ? 4 : (g.C % 2 == 0 ? 2 : 1), false, nullptr, a, mapN))
+    if (make_strip_args(g, numActive, g.C % 4 == 0 ? 4 : (g.C % 2 == 0 ? 2 : 1), false, nullptr, a, mapN))
         return (size_t)mapN * 4 + 16 + (size_t)numActive * 4 + 16;
     return 0;
 }
@@ -2245,55 +2508,98 @@ hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* id
     return hipGetLastError();
 }
 
+// What the one-pass kernels look cells up in: the list itself, or a map that earlier launches made of it.
+struct CellMap {
+    bool list;
+    const int32_t *map, *chain, *dup;
+};
+
 template <int VEC>
-static void launch_strip(const float* x, const float* ybase, float* y, bool planar, int op, const int32_t* map,
-                         const int32_t* chain, const int32_t* dup, const StripArgs& a, hipStream_t stream)
+static void launch_strip(const float* x, const float* ybase, float* y, const int16_t* idx, bool planar, bool add, const CellMap& m,
+                         const StripArgs& a, hipStream_t stream)
 {
     const dim3 grid(a.tiles);
     const size_t lds = planar ? (size_t)STRIP_ROWS * a.PX * a.CT * sizeof(float) : 0;  // 16 KB with 16-byte vectors
-#define SBNET_STRIP(OP, PL) \
-    hipLaunchKernelGGL((k_scatter_strip<VEC, OP, PL>), grid, dim3(256), lds, stream, x, ybase, y, map, chain, dup, a)
-    if (op == STRIP_COPY) SBNET_STRIP(STRIP_COPY, false);
-    else if (op == STRIP_ADD && planar) SBNET_STRIP(STRIP_ADD, true);
-    else if (op == STRIP_ADD) SBNET_STRIP(STRIP_ADD, false);
-    else if (planar) SBNET_STRIP(STRIP_ASSIGN, true);
-    else SBNET_STRIP(STRIP_ASSIGN, false);
-#undef SBNET_STRIP
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(STRIP_THREADS), lds, stream, x, ybase, y, idx, m.map, m.chain, m.dup, a); };
+    const bool over = a.ovH || a.ovW;
+    if (add && planar) m.list ? go(k_scatter_strip<VEC, STRIP_ADD, true, true, false>) : go(k_scatter_strip<VEC, STRIP_ADD, true, false, false>);
+    else if (add) m.list ? go(k_scatter_strip<VEC, STRIP_ADD, false, true, false>) : go(k_scatter_strip<VEC, STRIP_ADD, false, false, false>);
+    else if (planar) m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, true, true, false>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, true, false, false>);
+    else if (over) m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, false, true, true>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, false, false, true>);
+    else m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, false, true, false>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, false, false, false>);
 }
 
-// The copying scatter of a planar stack as one launch over the cells (k_scatter_cells); false, with nothing
-// launched, where that does not apply: blocks that do not tile the plane, cells too small to be copied one by one.
-template <int VEC>
-static bool launch_cells(const float* x, const float* ybase, float* y, const int16_t* idx, int numActive, const Geom& g,
-                         ScatterMode mode, const StripArgs& sa, int64_t mapN, const int32_t* map, const int32_t* chain,
-                         const int32_t* dup, hipStream_t stream, bool dry)
+// The copying scatter of a planar stack as one launch over the cells (k_scatter_cells); false where that does not apply:
+// blocks that do not tile the plane, cells too small to be copied one by one.
+struct CellsPlan {
+    TileArgs a;
+    CellArgs c;
+    int threads;
+    size_t lds;
+    dim3 grid;
+};
+
+static bool plan_cells(const Geom& g, int numActive, int vec, const StripArgs& sa, int64_t mapN, CellsPlan& p)
 {
     if (g.R != g.U || g.S != g.V || (int64_t)g.R * g.S < 4) return false;
     if ((int64_t)g.U * g.V * g.C * 4 < 4096 || mapN > 0x7fffffffll) return false;
-    TileArgs a;
-    int threads;
-    size_t lds;
     unsigned grid;
-    if (!scatter_tile_args(g, (int)mapN, VEC, a, threads, lds, grid)) return false;
-    if (mapN * (int64_t)a.tpb >= (1ll << 31)) return false;
-    if (dry) return true;
-    a.grid2d = mapN <= GRID_Y_MAX;
-    CellArgs c;
-    c.bhMin = sa.bhMin; c.bwMin = sa.bwMin; c.nBH = sa.nBH; c.nBW = sa.nBW;
-    c.CV = (uint32_t)(g.C / VEC);
-    c.dBW = make_fastdiv((uint32_t)sa.nBW);
-    c.dBHW = make_fastdiv((uint32_t)(sa.nBH * sa.nBW));
-    const ColorArgs aux{1, 1, 0, nullptr, nullptr, nullptr, 0, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0};
-    const dim3 gr = a.grid2d ? dim3(a.tpb, (unsigned)mapN) : dim3((unsigned)(mapN * a.tpb));
-    (void)numActive;
-    if (mode == SCATTER_ADD)
-        hipLaunchKernelGGL((k_scatter_cells<VEC, SCATTER_ADD>), gr, dim3(threads), lds, stream, x, ybase, y, idx, map, chain,
-                           dup, a, aux, c);
-    else
-        hipLaunchKernelGGL((k_scatter_cells<VEC, SCATTER_ASSIGN>), gr, dim3(threads), lds, stream, x, ybase, y, idx, map,
-                           chain, dup, a, aux, c);
+    if (!scatter_tile_args(g, (int)mapN, vec, p.a, p.threads, p.lds, grid)) return false;
+    if (mapN * (int64_t)p.a.tpb >= (1ll << 31)) return false;
+    p.a.grid2d = mapN <= GRID_Y_MAX;
+    p.a.blocks = (uint32_t)numActive;
+    p.c.bhMin = sa.bhMin; p.c.bwMin = sa.bwMin; p.c.nBH = sa.nBH; p.c.nBW = sa.nBW;
+    p.c.CV = (uint32_t)(g.C / vec);
+    p.c.dBW = make_fastdiv((uint32_t)sa.nBW);
+    p.c.dBHW = make_fastdiv((uint32_t)(sa.nBH * sa.nBW));
+    p.grid = p.a.grid2d ? dim3(p.a.tpb, (unsigned)mapN) : dim3((unsigned)(mapN * p.a.tpb));
     return true;
 }
+
+static const ColorArgs NO_ORDER{1, 1, 0, nullptr, nullptr, nullptr, 0, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0};
+
+template <int VEC>
+static void launch_cells(const float* x, const float* ybase, float* y, const int16_t* idx, bool add, const CellMap& m,
+                         const CellsPlan& p, hipStream_t stream)
+{
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, p.grid, dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, m.chain, m.dup, p.a, NO_ORDER, p.c); };
+    if (add) m.list ? go(k_scatter_cells<VEC, SCATTER_ADD, true>) : go(k_scatter_cells<VEC, SCATTER_ADD, false>);
+    else m.list ? go(k_scatter_cells<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_cells<VEC, SCATTER_ASSIGN, false>);
+}
+
+// Tiles of the listed blocks and strips of what they leave, in one launch (k_scatter_tiles_and_rest).
+struct RestPlan {
+    TileArgs a;
+    StripArgs s;
+    int threads;
+    size_t lds;
+};
+
+static bool plan_rest(const Geom& g, int numActive, int vec, RestPlan& p, int64_t& mapN)
+{
+    unsigned grid;
+    if ((int64_t)g.R * g.S < 4 || !scatter_tile_args(g, numActive, vec, p.a, p.threads, p.lds, grid)) return false;
+    if ((g.U < g.R || g.V < g.S) && !rank_inline_applies(g, numActive, true, vec)) return false;
+    p.threads = p.threads < 128 ? 128 : p.threads;   // (for the strips)
+    return make_strip_args(g, numActive, vec, false, nullptr, p.s, mapN, p.threads) &&
+           (uint64_t)p.a.total + p.s.tiles < (1ull << 31);
+}
+
+template <int VEC>
+static void launch_rest(const float* x, const float* ybase, float* y, const int16_t* idx, bool add, const CellMap& m,
+                        const RestPlan& p, hipStream_t stream)
+{
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.a.total + p.s.tiles), dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, p.a, NO_ORDER, p.s); };
+    if (add) m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD, false>);
+    else if (p.s.ovH || p.s.ovW) m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_RANKED_INLINE, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_RANKED_INLINE, false>);
+    else m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN, false>);
+}
+
+// Lists up to here are read by every workgroup of the one-pass kernels; longer ones go through a map, one or two launches
+// more.  us with the map / with the list, MI355X: 512x512x64, add, 102 rows 27.0 / 24.8, 512: 30.2 / 27.7, 921: 34.8 / 31.7;
+// [4,256,256,64], 1351 rows of 8x8: 29.2 / 26.8, as cells 28.9 / 26.8; eight images, 2703 rows: 57.7 / 55.4, as cells 55.3 /
+// 66.4; 16 images, 5406: 110 / 120.
+constexpr int STRIP_LIST_MAX = 1536;
 
 hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y, const int16_t* idx, int numActive,
                                     const Geom& g, bool transpose, ScatterMode mode, void* workspace,
@@ -2303,56 +2609,54 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
     if (mode == SCATTER_ATOMIC || numActive <= 0) return hipSuccess;
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 3)) return hipSuccess;
 
-    // Blocks that do not overlap: one streaming pass over the output (k_scatter_strip).  A planar stack whose
-    // geometry the strips do not stage is scattered by the tile kernel after a pass that copies the rest.
-    {
-        StripArgs a;
-        int64_t mapN = 0;
+    // One pass over the output: strips (NHWC stacks, planar ones that they can stage), cells, or tiles and strips.
+    if (mode == SCATTER_ASSIGN || !(g.U < g.R || g.V < g.S)) {
+        const bool add = mode == SCATTER_ADD;
         const int vb = pick_vec(g, ybase, y), vx = pick_vec(g, transpose ? nullptr : x, nullptr);
         const int vec = vb < vx ? vb : vx;
-        const size_t need = scatter_cover_workspace_bytes(g, numActive);
-        bool planar = transpose;
-        bool ok = need != 0 && workspaceBytes >= need;
-        bool cells = false;  // one launch over the cells of the block grid instead of the strips
-        if (ok && !make_strip_args(g, vec, planar, x, a, mapN)) {
-            planar = false;
-            ok = transpose && make_strip_args(g, vec, false, x, a, mapN);
-            if (ok) {
-                cells = vec == 4 ? launch_cells<4>(x, ybase, y, idx, numActive, g, mode, a, mapN, nullptr, nullptr, nullptr, stream, true)
-                      : vec == 2 ? launch_cells<2>(x, ybase, y, idx, numActive, g, mode, a, mapN, nullptr, nullptr, nullptr, stream, true)
-                                 : launch_cells<1>(x, ybase, y, idx, numActive, g, mode, a, mapN, nullptr, nullptr, nullptr, stream, true);
-                // (else two passes and four launches: worth it once the blocks cover enough of the tensor)
-                if (!cells) ok = (int64_t)numActive * g.R * g.S * g.C * 4 >= (16ll << 20);
-            }
+        const bool list = numActive <= STRIP_LIST_MAX;
+        StripArgs a;
+        CellsPlan cells;
+        RestPlan rest;
+        int64_t mapN = 0;
+        enum { NONE, STRIPS, CELLS, REST } how = NONE;
+        if (make_strip_args(g, numActive, vec, transpose, x, a, mapN)) {
+            how = STRIPS;
+        } else if (transpose) {
+            if (make_strip_args(g, numActive, vec, false, x, a, mapN) && plan_cells(g, numActive, vec, a, mapN, cells)) how = CELLS;
+            // (with a map two more launches: worth it once the blocks cover enough of the tensor)
+            else if ((list || (int64_t)numActive * g.R * g.S * g.C * 4 >= (16ll << 20)) && plan_rest(g, numActive, vec, rest, mapN)) how = REST;
         }
-        if (ok) {
-            a.g = g;
-            int32_t* map = static_cast<int32_t*>(workspace);
-            int32_t* dup = map + mapN;
-            int32_t* chain = dup + 4;
-            if (mapN <= BLOCK_MAP_ONE_WG && numActive <= BLOCK_MAP_ONE_WG) {
-                hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN,
-                                   chain, dup);
-            } else {
-                int64_t fillWgs = (mapN + 255) / 256;
-                if (fillWgs > 4096) fillWgs = 4096;
-                hipLaunchKernelGGL(k_pull_fill, dim3((unsigned)fillWgs), dim3(256), 0, stream, map, mapN, dup);
-                hipLaunchKernelGGL(k_cell_map, dim3((unsigned)((numActive + 255) / 256)), dim3(256), 0, stream, idx,
-                                   numActive, a, map, chain, dup);
+        if (how == REST) a = rest.s;
+        if (!list && workspaceBytes < (size_t)mapN * 4 + 16 + (size_t)numActive * 4 + 16) how = NONE;
+        if (how != NONE) {
+            CellMap m{list, nullptr, nullptr, nullptr};
+            if (!list) {
+                int32_t* map = static_cast<int32_t*>(workspace);
+                int32_t* dup = map + mapN;
+                int32_t* chain = add ? dup + 4 : nullptr;
+                if (mapN <= BLOCK_MAP_ONE_WG && numActive <= BLOCK_MAP_ONE_WG) {
+                    hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN,
+                                       chain, dup);
+                } else {
+                    int64_t fillWgs = (mapN + 255) / 256;
+                    if (fillWgs > 4096) fillWgs = 4096;
+                    hipLaunchKernelGGL(k_pull_fill, dim3((unsigned)fillWgs), dim3(256), 0, stream, map, mapN, dup);
+                    hipLaunchKernelGGL(k_cell_map, dim3((unsigned)((numActive + 255) / 256)), dim3(256), 0, stream, idx,
+                                       numActive, a, map, chain, dup);
+                }
+                m.map = map; m.chain = chain; m.dup = dup;
             }
-            if (cells) {
-                if (vec == 4) launch_cells<4>(x, ybase, y, idx, numActive, g, mode, a, mapN, map, chain, dup, stream, false);
-                else if (vec == 2) launch_cells<2>(x, ybase, y, idx, numActive, g, mode, a, mapN, map, chain, dup, stream, false);
-                else launch_cells<1>(x, ybase, y, idx, numActive, g, mode, a, mapN, map, chain, dup, stream, false);
-                done = true;
-                return hipGetLastError();
-            }
-            const int op = transpose && !planar ? STRIP_COPY : (mode == SCATTER_ADD ? STRIP_ADD : STRIP_ASSIGN);
-            if (vec == 4) launch_strip<4>(x, ybase, y, planar, op, map, chain, dup, a, stream);
-            else if (vec == 2) launch_strip<2>(x, ybase, y, planar, op, map, chain, dup, a, stream);
-            else launch_strip<1>(x, ybase, y, planar, op, map, chain, dup, a, stream);
+            auto go = [&](auto width) {
+                constexpr int VEC = decltype(width)::value;
+                if (how == STRIPS) launch_strip<VEC>(x, ybase, y, idx, transpose, add, m, a, stream);
+                else if (how == CELLS) launch_cells<VEC>(x, ybase, y, idx, add, m, cells, stream);
+                else launch_rest<VEC>(x, ybase, y, idx, add, m, rest, stream);
+            };
+            if (vec == 4) go(std::integral_constant<int, 4>());
+            else if (vec == 2) go(std::integral_constant<int, 2>());
+            else go(std::integral_constant<int, 1>());
             done = true;
-            if (op == STRIP_COPY) return scatter_from(x, y, ybase, idx, numActive, g, transpose, mode, stream);
             return hipGetLastError();
         }
     }

@@ -1,0 +1,70 @@
+"""The copying scatter's one-pass kernels against the oracle, on both sides of the length up to which their workgroups
+read the block list themselves (1536 rows) and from which on a map is made of it first."""
+import numpy as np
+import pytest
+import torch
+
+import sbnet_amd
+from oracle import sbnet_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+@pytest.mark.parametrize("M", [1, 1536, 1537])
+@pytest.mark.parametrize("shape,bs,bst,bo", [
+    ((8, 66, 80, 8), (6, 7), (4, 5), (-1, -2)),      # overlap in both directions: 16-byte vectors
+    ((8, 66, 80, 6), (6, 4), (4, 4), (-1, 0)),       # in rows only
+    ((8, 67, 81, 3), (4, 7), (4, 5), (-2, -3)),      # in columns only; floats of a vector in different pixels
+    ((8, 70, 97, 1), (3, 4), (4, 5), (-1, -1)),      # gaps; up to four pixels in a vector, rows that end inside one
+    ((8, 70, 97, 18), (3, 4), (4, 6), (2, -1)),
+    ((8, 65, 66, 4), (4, 4), (4, 4), (0, 0)),        # planar stack staged in strips
+    ((8, 130, 135, 18), (8, 8), (8, 8), (-3, -5)),   # planar stack by cells
+    ((8, 140, 135, 130), (4, 5), (6, 7), (0, 0)),    # more channel vectors than a strip that only copies is wide
+], ids=lambda v: "x".join(map(str, v)))
+def test_copying_scatter_reads_lists_and_maps(shape, bs, bst, bo, M):
+    N, H, W, C = shape
+    rng = np.random.default_rng(M + C)
+    bc = [1 + (H - bo[0] - 1) // bst[0], 1 + (W - bo[1] - 1) // bst[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(-1, bc[0] + 1) for j in range(-1, bc[1])], np.int16)
+    idx = cells[rng.permutation(len(cells))[:M]]     # some of them reach over the border, some lie outside
+    assert len(idx) == M
+    idx_d, base = dev(idx), rng.standard_normal(shape).astype(np.float32)
+    base_d = dev(base)
+    flat = torch.empty(base_d.numel() + 1, device=DEV)
+    mis = flat[1:].view(base_d.shape)                # aligned to 4 bytes only
+    mis.copy_(base_d)
+    overlap = bs[0] > bst[0] or bs[1] > bst[1]
+    for transpose in (False, True):
+        stack = rng.standard_normal((M, C, *bs) if transpose else (M, *bs, C)).astype(np.float32)
+        stack_d = dev(stack)
+        for add in ((False,) if overlap else (False, True)):
+            for count in (M, max(1, M - 3)):         # on the host; on the device, with rows past it
+                cnt = torch.tensor([count], dtype=torch.int32, device="cpu" if count == M else DEV)
+                want = orc.sparse_scatter(stack, [count], idx, base, bs, bst, bo, add=add, transpose=transpose)
+                for b in (base_d, mis):
+                    y = sbnet_amd.sparse_scatter(stack_d, cnt, idx_d, b, bs, bst, bo, add=add, transpose=transpose)
+                    np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="transpose %s add %s count %d" % (transpose, add, count))
+
+
+@pytest.mark.parametrize("shape,bs,bo", [((2, 40, 56, 32), (4, 4), (0, 0)), ((2, 50, 41, 24), (13, 15), (0, -1))],
+                         ids=["strips", "cells"])
+def test_long_lists_that_name_blocks_several_times(shape, bs, bo):
+    """Rows that name the same block through the map: the one listed last wins, an add takes all in list order."""
+    N, H, W, C = shape
+    rng = np.random.default_rng(H)
+    bc = [1 + (H - bo[0] - 1) // bs[0], 1 + (W - bo[1] - 1) // bs[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(bc[0]) for j in range(bc[1])], np.int16)
+    idx = cells[rng.integers(len(cells), size=1600)]
+    base = rng.standard_normal(shape).astype(np.float32)
+    for transpose in (False, True):
+        stack = rng.standard_normal((1600, C, *bs) if transpose else (1600, *bs, C)).astype(np.float32)
+        for add in (False, True):
+            want = orc.sparse_scatter(stack, [1600], idx, base, bs, bs, bo, add=add, transpose=transpose)
+            y = sbnet_amd.sparse_scatter(dev(stack), [1600], dev(idx), dev(base), bs, bs, bo, add=add, transpose=transpose)
+            np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="transpose %s add %s" % (transpose, add))
