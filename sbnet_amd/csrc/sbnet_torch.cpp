@@ -17,7 +17,9 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <map>
 #include <mutex>
@@ -27,7 +29,8 @@
 
 namespace {
 
-PyObject* g_check = nullptr;   // ops._check: raises the exception of a status
+PyObject* g_check = nullptr;      // ops._check: raises the exception of a status
+PyObject* g_by_layers = nullptr;  // sparse_conv._residual_by_layers: a residual function's gradients through its layers
 
 struct Pair {
     int32_t v[2];
@@ -182,6 +185,20 @@ bool call(F f, std::recursive_mutex* busy = nullptr)
     return false;
 }
 
+[[noreturn]] void raise_pending()
+{
+    python_error e;
+    e.persist();
+    throw e;
+}
+
+// The same for code that C++ calls: throws what was raised.
+template <typename F>
+void run(F f, std::recursive_mutex* busy = nullptr)
+{
+    if (!call(f, busy)) raise_pending();
+}
+
 // A function of the module: N arguments, of which those after the first FEWEST may be missing (None), and no C++ exception
 // through the interpreter's frames.
 template <PyObject* (*F)(PyObject* const*), Py_ssize_t N, Py_ssize_t FEWEST = N>
@@ -249,36 +266,75 @@ PyObject* reduce_mask(PyObject* const* a)
     return t;
 }
 
+struct Gather {
+    const at::Tensor* x;
+    Blocks b;
+    Pair bs, bt, bo;
+    int transpose;
+};
+
+// x, bin_counts, active_block_indices, bsize, bstride, boffset, transpose; false where the general wrapper has to see to them.
+bool gather_of(PyObject* const* a, Gather& g)
+{
+    g.x = dev_f32(a[0]);
+    if (!g.x || g.x->dim() != 4 || !blocks_of(a[1], a[2], g.b) || g.b.idx->device() != g.x->device() || !pair_of(a[3], g.bs) ||
+        !pair_of(a[4], g.bt) || !pair_of(a[5], g.bo) || g.bs.v[0] <= 0 || g.bs.v[1] <= 0)
+        return false;
+    g.transpose = PyObject_IsTrue(a[6]);
+    return g.transpose >= 0;
+}
+
+at::Tensor run_gather(const Gather& g, const at::Tensor* out)
+{
+    const Blocks& b = g.b;
+    c10::DeviceGuard guard(g.x->device());
+    at::Tensor y = out ? *out : empty_stack(b.M, g.x->size(3), g.bs, g.transpose, *g.x);
+    const float* const xp = static_cast<const float*>(g.x->data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
+    float* const yp = static_cast<float*>(y.data_ptr());
+    const int64_t* const dims = g.x->sizes().data();
+    void* const stream = stream_of(*g.x);
+    run([&] {
+        return b.count ? sbnet_sparse_gather_device_count(xp, dims, 4, b.count, b.M, ip, g.bs.v, 2, g.bt.v, 2, g.bo.v, 2,
+                                                          g.transpose, yp, stream)
+                       : sbnet_sparse_gather(xp, dims, 4, b.M, ip, g.bs.v, 2, g.bt.v, 2, g.bo.v, 2, g.transpose, yp, stream);
+    });
+    return y;
+}
+
 // gather(x, bin_counts, active_block_indices, bsize, bstride, boffset, transpose, out) -> stack
 PyObject* gather(PyObject* const* a)
 {
-    const at::Tensor* x = dev_f32(a[0]);
-    Blocks b;
-    Pair bs, bt, bo;
-    if (!x || x->dim() != 4 || !blocks_of(a[1], a[2], b) || b.idx->device() != x->device() || !pair_of(a[3], bs) ||
-        !pair_of(a[4], bt) || !pair_of(a[5], bo) || bs.v[0] <= 0 || bs.v[1] <= 0)
+    Gather g;
+    if (!gather_of(a, g)) {
+        if (PyErr_Occurred()) return nullptr;
         Py_RETURN_NONE;
-    const int transpose = PyObject_IsTrue(a[6]);
-    if (transpose < 0) return nullptr;
+    }
     const at::Tensor* out = nullptr;
     if (a[7] != Py_None) {
         out = dev_f32(a[7]);
-        if (!out || out->device() != x->device() || !is_stack(*out, b.M, x->size(3), bs, transpose)) Py_RETURN_NONE;
+        if (!out || out->device() != g.x->device() || !is_stack(*out, g.b.M, g.x->size(3), g.bs, g.transpose)) Py_RETURN_NONE;
     }
-    c10::DeviceGuard guard(x->device());
-    at::Tensor y = out ? *out : empty_stack(b.M, x->size(3), bs, transpose, *x);
-    const float* const xp = static_cast<const float*>(x->data_ptr());
-    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-    float* const yp = static_cast<float*>(y.data_ptr());
-    const int64_t* const dims = x->sizes().data();
-    void* const stream = stream_of(*x);
-    if (!call([&] {
-            return b.count ? sbnet_sparse_gather_device_count(xp, dims, 4, b.count, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2,
-                                                              transpose, yp, stream)
-                           : sbnet_sparse_gather(xp, dims, 4, b.M, ip, bs.v, 2, bt.v, 2, bo.v, 2, transpose, yp, stream);
-        }))
-        return nullptr;
-    return THPVariable_Wrap(std::move(y));
+    return THPVariable_Wrap(run_gather(g, out));
+}
+
+at::Tensor run_gather_grad(const at::Tensor& g, const at::Tensor& idx, int32_t M, const int64_t* dims, const Pair& bs, const Pair& bt,
+                           const Pair& bo, int transpose)
+{
+    c10::DeviceGuard guard(g.device());
+    at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, g);
+    const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
+    const Workspace scratch = need ? workspace(g.device(), need) : Workspace();
+    const at::Tensor& ws = scratch.buffer;
+    const float* const gp = static_cast<const float*>(g.data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(idx.data_ptr());
+    float* const dp = static_cast<float*>(dx.data_ptr());
+    void* const stream = stream_of(g);
+    run([&] {
+        return sbnet_sparse_gather_grad(gp, M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
+                                        need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
+    }, scratch.busy);
+    return dx;
 }
 
 // gather_grad(grad, bin_counts, active_block_indices, x_shape, bsize, bstride, boffset, transpose) -> dx
@@ -299,68 +355,98 @@ PyObject* gather_grad(PyObject* const* a)
     const int transpose = PyObject_IsTrue(a[7]);
     if (transpose < 0) return nullptr;
     if (!is_stack(*g, b.M, dims[3], bs, transpose)) Py_RETURN_NONE;
-    c10::DeviceGuard guard(g->device());
-    at::Tensor dx = empty_f32({dims[0], dims[1], dims[2], dims[3]}, *g);
-    const int64_t need = (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2);
-    const Workspace scratch = need ? workspace(g->device(), need) : Workspace();
+    return THPVariable_Wrap(run_gather_grad(*g, *b.idx, b.M, dims, bs, bt, bo, transpose));
+}
+
+struct Scatter {
+    const at::Tensor *x, *base;
+    Blocks b;
+    Pair bs, bt, bo;
+    int add, atomic, transpose;
+};
+
+// x, bin_counts, active_block_indices, ybase, bsize, bstride, boffset, add, atomic, transpose
+bool scatter_of(PyObject* const* a, Scatter& q)
+{
+    q.x = dev_f32(a[0]);
+    q.base = dev_f32(a[3]);
+    if (!q.x || !q.base || q.base->dim() != 4 || !blocks_of(a[1], a[2], q.b) || q.b.idx->device() != q.base->device() ||
+        q.x->device() != q.base->device() || !pair_of(a[4], q.bs) || !pair_of(a[5], q.bt) || !pair_of(a[6], q.bo))
+        return false;
+    q.add = PyObject_IsTrue(a[7]);
+    q.atomic = PyObject_IsTrue(a[8]);
+    q.transpose = PyObject_IsTrue(a[9]);
+    if (q.add < 0 || q.atomic < 0 || q.transpose < 0) return false;
+    if (q.b.count && q.x->dim() > 0 && q.x->size(0) < q.b.M) q.b.M = (int32_t)q.x->size(0);
+    return is_stack(*q.x, q.b.M, q.base->size(3), q.bs, q.transpose);
+}
+
+at::Tensor run_scatter(const Scatter& q, bool in_place)
+{
+    const Blocks& b = q.b;
+    const Pair &bs = q.bs, &bt = q.bt, &bo = q.bo;
+    const bool overlap = bt.v[0] < bs.v[0] || bt.v[1] < bs.v[1];
+    c10::DeviceGuard guard(q.base->device());
+    const int64_t* const dims = q.base->sizes().data();
+    const bool wants = (q.add && q.atomic) || !in_place || (!q.add && overlap);
+    const int64_t need = wants ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
+    const Workspace scratch = need ? workspace(q.base->device(), need) : Workspace();
     const at::Tensor& ws = scratch.buffer;
-    const float* const gp = static_cast<const float*>(g->data_ptr());
+    void* const wp = need ? ws.data_ptr() : nullptr;
+    const size_t wn = need ? (size_t)ws.numel() : 0;
+    at::Tensor y = in_place ? *q.base : empty_f32(q.base->sizes(), *q.base);
+    const float *const xp = static_cast<const float*>(q.x->data_ptr()), *const bp = static_cast<const float*>(q.base->data_ptr());
     const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-    float* const dp = static_cast<float*>(dx.data_ptr());
-    void* const stream = stream_of(*g);
-    if (!call([&] {
-            return sbnet_sparse_gather_grad(gp, b.M, ip, dp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, transpose,
-                                            need ? ws.data_ptr() : nullptr, need ? (size_t)ws.numel() : 0, stream);
-        }, scratch.busy))
-        return nullptr;
-    return THPVariable_Wrap(std::move(dx));
+    float* const yp = static_cast<float*>(y.data_ptr());
+    void* const stream = stream_of(*q.base);
+    run([&] {
+        if (in_place)
+            return b.count ? sbnet_sparse_scatter_var_device_count(xp, b.count, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2,
+                                                                   bo.v, 2, q.add, q.atomic, q.transpose, wp, wn, stream)
+                           : sbnet_sparse_scatter_var(xp, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, q.add, q.atomic,
+                                                      q.transpose, wp, wn, stream);
+        return b.count ? sbnet_sparse_scatter_device_count(xp, b.count, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2,
+                                                           q.add, q.atomic, q.transpose, yp, wp, wn, stream)
+                       : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, q.add, q.atomic,
+                                              q.transpose, yp, wp, wn, stream);
+    }, scratch.busy);
+    return y;
 }
 
 // scatter(x, bin_counts, active_block_indices, ybase, bsize, bstride, boffset, add, atomic, transpose, use_var) -> y
 PyObject* scatter(PyObject* const* a)
 {
-    const at::Tensor *x = dev_f32(a[0]), *base = dev_f32(a[3]);
-    Blocks b;
-    Pair bs, bt, bo;
-    if (!x || !base || base->dim() != 4 || !blocks_of(a[1], a[2], b) || b.idx->device() != base->device() ||
-        x->device() != base->device() || !pair_of(a[4], bs) || !pair_of(a[5], bt) || !pair_of(a[6], bo))
+    Scatter q;
+    if (!scatter_of(a, q)) {
+        if (PyErr_Occurred()) return nullptr;
         Py_RETURN_NONE;
-    const int add = PyObject_IsTrue(a[7]), atomic = PyObject_IsTrue(a[8]), transpose = PyObject_IsTrue(a[9]),
-              in_place = PyObject_IsTrue(a[10]);
-    if (add < 0 || atomic < 0 || transpose < 0 || in_place < 0) return nullptr;
-    if (b.count && x->dim() > 0 && x->size(0) < b.M) b.M = (int32_t)x->size(0);
-    if (!is_stack(*x, b.M, base->size(3), bs, transpose)) Py_RETURN_NONE;
-    const bool overlap = bt.v[0] < bs.v[0] || bt.v[1] < bs.v[1];
-    c10::DeviceGuard guard(base->device());
-    const int64_t* const dims = base->sizes().data();
-    const bool wants = (add && atomic) || !in_place || (!add && overlap);
-    const int64_t need = wants ? (int64_t)sbnet_sparse_scatter_workspace_bytes(b.M, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2) : 0;
-    const Workspace scratch = need ? workspace(base->device(), need) : Workspace();
-    const at::Tensor& ws = scratch.buffer;
-    void* const wp = need ? ws.data_ptr() : nullptr;
-    const size_t wn = need ? (size_t)ws.numel() : 0;
-    at::Tensor y = in_place ? *base : empty_f32(base->sizes(), *base);
-    const float *const xp = static_cast<const float*>(x->data_ptr()), *const bp = static_cast<const float*>(base->data_ptr());
-    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-    float* const yp = static_cast<float*>(y.data_ptr());
-    void* const stream = stream_of(*base);
-    if (!call([&] {
-            if (in_place)
-                return b.count ? sbnet_sparse_scatter_var_device_count(xp, b.count, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2,
-                                                                       bo.v, 2, add, atomic, transpose, wp, wn, stream)
-                               : sbnet_sparse_scatter_var(xp, b.M, ip, yp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
-                                                          transpose, wp, wn, stream);
-            return b.count ? sbnet_sparse_scatter_device_count(xp, b.count, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2,
-                                                               add, atomic, transpose, yp, wp, wn, stream)
-                           : sbnet_sparse_scatter(xp, b.M, ip, bp, dims, 4, bs.v, 2, bt.v, 2, bo.v, 2, add, atomic,
-                                                  transpose, yp, wp, wn, stream);
-        }, scratch.busy))
-        return nullptr;
+    }
+    const int in_place = PyObject_IsTrue(a[10]);
+    if (in_place < 0) return nullptr;
+    at::Tensor y = run_scatter(q, in_place);
     if (in_place) {
         Py_INCREF(a[3]);   // the caller's own tensor object, as the Python wrapper returns it
         return a[3];
     }
     return THPVariable_Wrap(std::move(y));
+}
+
+// The gradient of the base of plain writes; an undefined tensor for a geometry that the one pass does not take.
+at::Tensor run_base_grad(const at::Tensor& g, const at::Tensor& idx, int32_t M, const Pair& bs, const Pair& bt, const Pair& bo)
+{
+    if (reinterpret_cast<uintptr_t>(g.data_ptr()) & 15) return at::Tensor();
+    const int64_t* const dims = g.sizes().data();
+    const size_t need = sbnet_sparse_scatter_base_grad_workspace_bytes(M, dims, bs.v, bt.v, bo.v);
+    if (!need) return at::Tensor();
+    c10::DeviceGuard guard(g.device());
+    at::Tensor d = empty_f32(g.sizes(), g);
+    at::Tensor ws = own_scratch(g, need);
+    const float* const gp = static_cast<const float*>(g.data_ptr());
+    const int16_t* const ip = static_cast<const int16_t*>(idx.data_ptr());
+    float* const dp = static_cast<float*>(d.data_ptr());
+    void *const wp = ws.data_ptr(), *const stream = stream_of(g);
+    run([&] { return sbnet_sparse_scatter_base_grad(gp, M, ip, dp, dims, bs.v, bt.v, bo.v, wp, need, stream); });
+    return d;
 }
 
 // scatter_base_grad(grad, bin_counts, active_block_indices, bsize, bstride, boffset) -> gradient of the base of plain writes
@@ -369,21 +455,11 @@ PyObject* scatter_base_grad(PyObject* const* a)
     const at::Tensor* g = dev_f32(a[0]);
     Blocks b;
     Pair bs, bt, bo;
-    if (!g || g->dim() != 4 || reinterpret_cast<uintptr_t>(g->data_ptr()) & 15 || !blocks_of(a[1], a[2], b) || b.count ||
-        b.idx->device() != g->device() || !pair_of(a[3], bs) || !pair_of(a[4], bt) || !pair_of(a[5], bo))
+    if (!g || g->dim() != 4 || !blocks_of(a[1], a[2], b) || b.count || b.idx->device() != g->device() || !pair_of(a[3], bs) ||
+        !pair_of(a[4], bt) || !pair_of(a[5], bo))
         Py_RETURN_NONE;
-    const int64_t* const dims = g->sizes().data();
-    const size_t need = sbnet_sparse_scatter_base_grad_workspace_bytes(b.M, dims, bs.v, bt.v, bo.v);
-    if (!need) Py_RETURN_NONE;
-    c10::DeviceGuard guard(g->device());
-    at::Tensor d = empty_f32(g->sizes(), *g);
-    at::Tensor ws = own_scratch(*g, need);
-    const float* const gp = static_cast<const float*>(g->data_ptr());
-    const int16_t* const ip = static_cast<const int16_t*>(b.idx->data_ptr());
-    float* const dp = static_cast<float*>(d.data_ptr());
-    void *const wp = ws.data_ptr(), *const stream = stream_of(*g);
-    if (!call([&] { return sbnet_sparse_scatter_base_grad(gp, b.M, ip, dp, dims, bs.v, bt.v, bo.v, wp, need, stream); }))
-        return nullptr;
+    at::Tensor d = run_base_grad(*g, *b.idx, b.M, bs, bt, bo);
+    if (!d.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(d));
 }
 
@@ -511,27 +587,19 @@ PyObject* block_bottleneck(PyObject* const* a)
     return THPVariable_Wrap(std::move(q));
 }
 
-// bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3, wanted) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1,
-// ...), on planar stacks, or None where the kernels do not take the sizes.  wanted: a tuple with the truth of each of the
-// ten, those not wanted are None; all where it is missing.
-PyObject* bottleneck_grad(PyObject* const* a)
+// The gradients of a residual function on planar stacks: dp, dw1-3, (dgamma, dbeta)1-3, undefined what is not wanted.  saved:
+// [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3.  False where the kernels do not take the sizes.
+bool run_bottleneck_grad(const at::Tensor* dq, const at::Tensor* const* t, const bool* wanted, at::Tensor* res)
 {
-    const at::Tensor* dq = dev_f32(a[0]);
-    if (!dq || dq->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 18) Py_RETURN_NONE;
-    bool wanted[10];
-    if (a[2] != Py_None && (!PyTuple_CheckExact(a[2]) || PyTuple_GET_SIZE(a[2]) != 10)) Py_RETURN_NONE;
-    for (int i = 0; i < 10; ++i) wanted[i] = a[2] == Py_None || PyTuple_GET_ITEM(a[2], i) == Py_True;
-    const at::Tensor* t[18];
     const float* ptr[6][3];
     for (int i = 0; i < 18; ++i) {
-        t[i] = dev_f32(PyList_GET_ITEM(a[1], i));
-        if (!t[i] || t[i]->device() != dq->device()) Py_RETURN_NONE;
+        if (!t[i] || t[i]->device() != dq->device()) return false;
         ptr[i % 6][i / 6] = static_cast<const float*>(t[i]->data_ptr());
     }
-    if (t[0]->dim() != 4 || t[0]->size(0) > INT32_MAX) Py_RETURN_NONE;
+    if (t[0]->dim() != 4 || t[0]->size(0) > INT32_MAX) return false;
     const int64_t M = t[0]->size(0);
     int64_t C = t[0]->size(1), R = t[0]->size(2), S = t[0]->size(3);
-    if (M <= 0 || C <= 0 || R <= 0 || S <= 0 || R > INT32_MAX || S > INT32_MAX) Py_RETURN_NONE;
+    if (M <= 0 || C <= 0 || R <= 0 || S <= 0 || R > INT32_MAX || S > INT32_MAX) return false;
     const int32_t bs[2] = {(int32_t)R, (int32_t)S};
     int32_t wd[12];
     for (int i = 0; i < 3; ++i) {
@@ -540,7 +608,7 @@ PyObject* bottleneck_grad(PyObject* const* a)
         if (q[0]->dim() != 4 || q[0]->sizes() != at::IntArrayRef({M, C, R, S}) || q[1]->sizes() != q[0]->sizes() ||
             q[0]->numel() >= 2 * CONV_MOST || q[2]->numel() != C || q[3]->numel() != C || q[5]->numel() != C || w->dim() != 4 ||
             w->size(1) != C || w->size(2) > R || w->size(3) > S || w->numel() <= 0 || w->numel() >= CONV_MOST)
-            Py_RETURN_NONE;
+            return false;
         wd[4 * i] = (int32_t)w->size(2);
         wd[4 * i + 1] = (int32_t)w->size(3);
         wd[4 * i + 2] = (int32_t)C;
@@ -549,11 +617,10 @@ PyObject* bottleneck_grad(PyObject* const* a)
         S -= w->size(3) - 1;
         C = w->size(0);
     }
-    if (dq->sizes() != at::IntArrayRef({M, C, R, S}) || dq->numel() >= 2 * CONV_MOST) Py_RETURN_NONE;
+    if (dq->sizes() != at::IntArrayRef({M, C, R, S}) || dq->numel() >= 2 * CONV_MOST) return false;
     const size_t need = sbnet_bottleneck_grad_workspace_bytes((int32_t)M, bs, wd);
-    if (!need) Py_RETURN_NONE;
+    if (!need) return false;
     c10::DeviceGuard guard(dq->device());
-    at::Tensor res[10];
     float *out[10];
     if (wanted[0]) res[0] = empty_f32(t[0]->sizes(), *dq);
     for (int i = 0; i < 3; ++i) {
@@ -567,18 +634,277 @@ PyObject* bottleneck_grad(PyObject* const* a)
     at::Tensor ws = own_scratch(*dq, need);
     const float* const dqp = static_cast<const float*>(dq->data_ptr());
     void *const wp = ws.data_ptr(), *const stream = stream_of(*dq);
-    if (!call([&] {
-            return sbnet_bottleneck_grad(dqp, (int32_t)M, bs, ptr[0], ptr[1], ptr[2], ptr[3], ptr[5], ptr[4], wd, out[0],
-                                         out + 1, dgamma, dbeta, wp, need, stream);
-        }))
-        return nullptr;
+    run([&] {
+        return sbnet_bottleneck_grad(dqp, (int32_t)M, bs, ptr[0], ptr[1], ptr[2], ptr[3], ptr[5], ptr[4], wd, out[0],
+                                     out + 1, dgamma, dbeta, wp, need, stream);
+    });
+    return true;
+}
+
+PyObject* or_none(at::Tensor&& t)
+{
+    if (t.defined()) return THPVariable_Wrap(std::move(t));
+    Py_RETURN_NONE;
+}
+
+// bottleneck_grad(dq, [z, act, mean, inv, kernel [K,C,kh,kw], gamma] * 3, wanted) -> (dp, dw1, dw2, dw3, dgamma1, dbeta1,
+// ...), on planar stacks, or None where the kernels do not take the sizes.  wanted: a tuple with the truth of each of the
+// ten, those not wanted are None; all where it is missing.
+PyObject* bottleneck_grad(PyObject* const* a)
+{
+    const at::Tensor* dq = dev_f32(a[0]);
+    if (!dq || dq->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 18) Py_RETURN_NONE;
+    bool wanted[10];
+    if (a[2] != Py_None && (!PyTuple_CheckExact(a[2]) || PyTuple_GET_SIZE(a[2]) != 10)) Py_RETURN_NONE;
+    for (int i = 0; i < 10; ++i) wanted[i] = a[2] == Py_None || PyTuple_GET_ITEM(a[2], i) == Py_True;
+    const at::Tensor* t[18];
+    for (int i = 0; i < 18; ++i) t[i] = dev_f32(PyList_GET_ITEM(a[1], i));
+    at::Tensor res[10];
+    if (!run_bottleneck_grad(dq, t, wanted, res)) Py_RETURN_NONE;
     PyObject* r = PyTuple_New(10);
     if (!r) return nullptr;
-    for (int i = 0; i < 10; ++i) {
-        PyObject* const o = wanted[i] ? THPVariable_Wrap(std::move(res[i])) : (Py_INCREF(Py_None), Py_None);
-        PyTuple_SET_ITEM(r, i, o);
-    }
+    for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(r, i, or_none(std::move(res[i])));
     return r;
+}
+
+// ---- the differentiable ops -------------------------------------------------------------------------------
+//
+// torch::autograd functions of the same steps as the ones in autograd.py and sparse_conv.py, for plain tensors: an autograd
+// function in Python costs about 35 us of host time a call forward and 10-15 backward, and these steps are bound by that
+// wherever the tensors are not large (a training step of a residual block spent 490 us in the host for 260 on the GPU).
+// What looks on or transforms (dispatch and functorch modes, forward-mode tangents, tracing) is left to those.
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// A backward pass's hold of the interpreter, which guards the scratch table and takes the errors.
+struct Gil {
+    PyGILState_STATE state = PyGILState_Ensure();
+    ~Gil() { PyGILState_Release(state); }
+};
+
+// A gradient as the kernels take it; an error as the general wrappers raise for tensors without memory of their own.
+at::Tensor plain_grad(const at::Tensor& grad)
+{
+    at::Tensor g = grad.contiguous();
+    TORCH_CHECK(g.has_storage() && g.is_cuda() && g.scalar_type() == at::kFloat && (g.numel() == 0 || g.const_data_ptr()),
+                "grad must be a float32 tensor on the GPU");
+    return g;
+}
+
+at::Tensor plain_list(const at::Tensor& idx)
+{
+    at::Tensor t = idx.contiguous();
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kShort, "active_block_indices must be an int16 tensor on the GPU");
+    return t;
+}
+
+// Sizes that a function keeps: one entry of its context.
+std::vector<int64_t> sizes_of(int32_t M, const Pair& bs, const Pair& bt, const Pair& bo, const at::Tensor& t, int flags)
+{
+    return {M, bs.v[0], bs.v[1], bt.v[0], bt.v[1], bo.v[0], bo.v[1], t.size(0), t.size(1), t.size(2), t.size(3), flags};
+}
+
+Pair pair_at(const std::vector<int64_t>& v, int i) { return {{(int32_t)v[i], (int32_t)v[i + 1]}}; }
+
+struct GatherFunction : torch::autograd::Function<GatherFunction> {
+    static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const Gather* g)
+    {
+        ctx->save_for_backward({*g->b.idx});
+        ctx->saved_data["sizes"] = sizes_of(g->b.M, g->bs, g->bt, g->bo, x, g->transpose);
+        return run_gather(*g, nullptr);
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const Gil gil;
+        const at::Tensor idx = plain_list(ctx->get_saved_variables()[0]), g = plain_grad(grads[0]);
+        const std::vector<int64_t> v = ctx->saved_data["sizes"].toIntVector();
+        return {run_gather_grad(g, idx, (int32_t)v[0], v.data() + 7, pair_at(v, 1), pair_at(v, 3), pair_at(v, 5), (int)v[11]), at::Tensor()};
+    }
+};
+
+struct ScatterFunction : torch::autograd::Function<ScatterFunction> {
+    static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& base, const Scatter* q)
+    {
+        ctx->save_for_backward({*q->b.idx});
+        std::vector<int64_t> v = sizes_of(q->b.M, q->bs, q->bt, q->bo, base, q->transpose | q->add << 1);
+        v.push_back(x.size(0));
+        ctx->saved_data["sizes"] = std::move(v);
+        return run_scatter(*q, false);
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const Gil gil;
+        const at::Tensor idx = plain_list(ctx->get_saved_variables()[0]), grad = plain_grad(grads[0]);
+        const std::vector<int64_t> v = ctx->saved_data["sizes"].toIntVector();
+        const int32_t M = (int32_t)v[0];
+        const Pair bs = pair_at(v, 1), bt = pair_at(v, 3), bo = pair_at(v, 5);
+        const int transpose = v[11] & 1, add = (v[11] >> 1) & 1;
+        at::Tensor blocks, base;
+        if (ctx->needs_input_grad(0)) blocks = run_gather({&grad, {&idx, M, nullptr}, bs, bt, bo, transpose}, nullptr);
+        if (ctx->needs_input_grad(1)) {
+            if (add) base = grad;
+            else if (!(at::GradMode::is_enabled() && grad.requires_grad())) base = run_base_grad(grad, idx, M, bs, bt, bo);
+            if (!base.defined()) {   // a graph of the gradients is asked for, or a geometry that the one pass does not take
+                at::Tensor stamp;
+                {
+                    at::AutoGradMode off(false);
+                    stamp = at::ones_like(grad);
+                    const int64_t C = v[10], R = bs.v[0], S = bs.v[1];
+                    const at::Tensor zeros = transpose ? at::zeros({v[12], C, R, S}, grad.options()) : at::zeros({v[12], R, S, C}, grad.options());
+                    run_scatter({&zeros, &stamp, {&idx, M, nullptr}, bs, bt, bo, 0, 0, transpose}, true);
+                }
+                base = grad * stamp;
+            }
+        }
+        return {blocks, base, at::Tensor()};
+    }
+};
+
+// Nobody transforms or looks on at what torch does.
+bool plain_autograd()
+{
+    return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+// gather_autograd(x, bin_counts, active_block_indices, bsize, bstride, boffset, transpose) -> stack with a gradient
+PyObject* gather_autograd(PyObject* const* a)
+{
+    Gather g;
+    if (!plain_autograd() || !gather_of(a, g) || g.b.count) {
+        if (PyErr_Occurred()) return nullptr;
+        Py_RETURN_NONE;
+    }
+    return THPVariable_Wrap(GatherFunction::apply(*g.x, (const Gather*)&g));
+}
+
+// scatter_autograd(x, bin_counts, active_block_indices, ybase, bsize, bstride, boffset, add, atomic, transpose) -> y
+PyObject* scatter_autograd(PyObject* const* a)
+{
+    Scatter q;
+    if (!plain_autograd() || !scatter_of(a, q) || q.b.count) {
+        if (PyErr_Occurred()) return nullptr;
+        Py_RETURN_NONE;
+    }
+    return THPVariable_Wrap(ScatterFunction::apply(*q.x, *q.base, (const Scatter*)&q));
+}
+
+// A residual function's running statistics and the batch norms' numbers.
+struct Residual {
+    at::Tensor mean[3], var[3];   // undefined: none
+    double momentum, eps;
+};
+
+struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
+    // The library's calls, one by one, as the layers make them.
+    static at::Tensor forward(AutogradContext* ctx, const at::Tensor& p, const at::Tensor& w1, const at::Tensor& g1, const at::Tensor& b1,
+                              const at::Tensor& w2, const at::Tensor& g2, const at::Tensor& b2, const at::Tensor& w3,
+                              const at::Tensor& g3, const at::Tensor& b3, const Residual* r)
+    {
+        const at::Tensor *const w[3] = {&w1, &w2, &w3}, *const gamma[3] = {&g1, &g2, &g3}, *const beta[3] = {&b1, &b2, &b3};
+        at::Tensor z = p;
+        variable_list saved;
+        for (int i = 0; i < 3; ++i) {
+            auto bn = at::_batch_norm_impl_index(z, *gamma[i], *beta[i], r->mean[i], r->var[i], true, r->momentum, r->eps,
+                                                 at::globalContext().userEnabledCuDNN());
+            at::Tensor& act = std::get<0>(bn);
+            act.relu_();
+            const at::Tensor kernel = w[i]->permute({3, 2, 0, 1}).contiguous();
+            saved.insert(saved.end(), {z, act, std::get<1>(bn), std::get<2>(bn), kernel, *gamma[i]});
+            z = at::conv2d(act, kernel, {}, at::IntArrayRef({1, 1}));
+        }
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["layers"] = std::vector<at::Tensor>{w1, b1, w2, b2, w3, b3};   // for a graph of the gradients alone
+        return z;
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        const Gil gil;
+        const variable_list saved = ctx->get_saved_variables();
+        // of p and, per layer, kernel, gamma and beta, as the inputs are; the kernels' gradients stand first in what comes back
+        bool needs[10], wanted[10];
+        for (int i = 0; i < 10; ++i) needs[i] = ctx->needs_input_grad(i);
+        constexpr int AT[10] = {0, 1, 4, 5, 2, 6, 7, 3, 8, 9};   // where input i's gradient is
+        for (int i = 0; i < 10; ++i) wanted[AT[i]] = needs[i];
+        variable_list out(11);
+        const bool graph = at::GradMode::is_enabled();
+        if (!graph) {
+            const at::Tensor dq = plain_grad(grads[0]);
+            const at::Tensor* t[18];
+            bool plain = dq.dim() == 4;
+            for (int i = 0; i < 18; ++i) {
+                t[i] = &saved[i];
+                plain = plain && saved[i].is_cuda() && saved[i].scalar_type() == at::kFloat && saved[i].is_contiguous() && saved[i].has_storage();
+            }
+            at::Tensor res[10];
+            if (plain && run_bottleneck_grad(&dq, t, wanted, res)) {
+                for (int i = 0; i < 10; ++i) out[i] = res[AT[i]];
+                return out;
+            }
+        }
+        // a graph of the gradients is asked for, or sizes that the kernels do not take: through the layers one by one
+        const std::vector<at::Tensor> layers = ctx->saved_data["layers"].toTensorVector();
+        THPObjectPtr list(PyList_New(18)), pairs(PyList_New(6)), need(PyTuple_New(10)), dq(THPVariable_Wrap(grads[0]));
+        if (!list || !pairs || !need || !dq) raise_pending();
+        for (int i = 0; i < 18; ++i) PyList_SET_ITEM(list.get(), i, THPVariable_Wrap(saved[i]));
+        for (int i = 0; i < 6; ++i) PyList_SET_ITEM(pairs.get(), i, THPVariable_Wrap(layers[i]));
+        for (int i = 0; i < 10; ++i) PyTuple_SET_ITEM(need.get(), i, PyBool_FromLong(needs[i]));
+        THPObjectPtr got(PyObject_CallFunctionObjArgs(g_by_layers, list.get(), pairs.get(), need.get(), dq.get(), graph ? Py_True : Py_False, nullptr));
+        if (!got) raise_pending();
+        TORCH_CHECK(PyList_CheckExact(got.get()) && PyList_GET_SIZE(got.get()) == 10, "gradients of ten inputs");
+        for (int i = 0; i < 10; ++i) {
+            PyObject* const o = PyList_GET_ITEM(got.get(), i);
+            if (o != Py_None) out[i] = THPVariable_Unpack(o);
+        }
+        return out;
+    }
+};
+
+// residual(p, [moving mean, moving variance] * 3, [kernel, gamma, beta] * 3, momentum, eps) -> the residual function of a planar
+// stack with batch statistics, with own gradients
+PyObject* residual(PyObject* const* a)
+{
+    const at::Tensor* p = dev_f32(a[0]);
+    if (!plain_autograd() || !p || p->dim() != 4 || !PyList_CheckExact(a[1]) || PyList_GET_SIZE(a[1]) != 6 || !PyList_CheckExact(a[2]) ||
+        PyList_GET_SIZE(a[2]) != 9 || !PyFloat_CheckExact(a[3]) || !PyFloat_CheckExact(a[4]))
+        Py_RETURN_NONE;
+    Residual r;
+    r.momentum = PyFloat_AS_DOUBLE(a[3]);
+    r.eps = PyFloat_AS_DOUBLE(a[4]);
+    for (int i = 0; i < 6; ++i) {
+        PyObject* const o = PyList_GET_ITEM(a[1], i);
+        if (o == Py_None) continue;
+        const at::Tensor* t = dev_f32(o);
+        if (!t) Py_RETURN_NONE;
+        (i & 1 ? r.var : r.mean)[i / 2] = *t;
+    }
+    const at::Tensor* t[9];
+    for (int i = 0; i < 9; ++i) {
+        t[i] = dev_f32(PyList_GET_ITEM(a[2], i));
+        if (!t[i] || t[i]->dim() != (i % 3 ? 1 : 4)) Py_RETURN_NONE;
+    }
+    at::Tensor q;
+    {
+        const pybind11::gil_scoped_release free;   // (the library's calls may compile)
+        q = ResidualFunction::apply(*p, *t[0], *t[1], *t[2], *t[3], *t[4], *t[5], *t[6], *t[7], *t[8], (const Residual*)&r);
+    }
+    return THPVariable_Wrap(std::move(q));
+}
+
+// all_plain(tensors) -> whether all are float32 tensors on the GPU, one behind the other in memory
+PyObject* all_plain(PyObject* const* a)
+{
+    if (!PyList_CheckExact(a[0])) Py_RETURN_FALSE;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); ++i) {
+        PyObject* const o = PyList_GET_ITEM(a[0], i);
+        if (!THPVariable_Check(o)) Py_RETURN_FALSE;
+        const at::Tensor& t = THPVariable_Unpack(o);
+        if (!t.is_cuda() || t.scalar_type() != at::kFloat || t.layout() != at::kStrided || !t.is_contiguous()) Py_RETURN_FALSE;
+    }
+    Py_RETURN_TRUE;
 }
 
 // workspace(device index, bytes) -> uint8 tensor: the scratch of the current stream, for the wrappers in Python
@@ -636,6 +962,13 @@ PyObject* set_check(PyObject*, PyObject* f)
     Py_RETURN_NONE;
 }
 
+PyObject* set_by_layers(PyObject*, PyObject* f)
+{
+    Py_INCREF(f);
+    Py_XSETREF(g_by_layers, f);
+    Py_RETURN_NONE;
+}
+
 template <typename F>
 PyCFunction fast(F f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)); }
 
@@ -648,12 +981,17 @@ PyMethodDef methods[] = {
     {"block_conv", fast(op_entry<block_conv, 7>), METH_FASTCALL, nullptr},
     {"block_bottleneck", fast(op_entry<block_bottleneck, 12>), METH_FASTCALL, nullptr},
     {"bottleneck_grad", fast(op_entry<bottleneck_grad, 3, 2>), METH_FASTCALL, nullptr},
+    {"gather_autograd", fast(op_entry<gather_autograd, 7>), METH_FASTCALL, nullptr},
+    {"scatter_autograd", fast(op_entry<scatter_autograd, 10>), METH_FASTCALL, nullptr},
+    {"residual", fast(op_entry<residual, 5>), METH_FASTCALL, nullptr},
+    {"all_plain", fast(entry<all_plain, 1>), METH_FASTCALL, nullptr},
     {"workspace", fast(entry<workspace_py, 2>), METH_FASTCALL, nullptr},
     {"lock_workspace", fast(entry<lock_workspace, 1>), METH_FASTCALL, nullptr},
     {"unlock_workspace", fast(entry<unlock_workspace, 1>), METH_FASTCALL, nullptr},
     {"release_workspaces", release_workspaces, METH_NOARGS, nullptr},
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},
     {"set_check", set_check, METH_O, nullptr},
+    {"set_by_layers", set_by_layers, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -14,6 +14,7 @@ import ctypes
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -50,6 +51,12 @@ def _load_native():
     module.set_check(_check)
     _native = module
     return module
+
+
+def _plain_autograd():
+    """No forward-mode tangents and no tracing, which the native functions know nothing of (of the dispatcher's modes and of
+    functorch's transforms they do)."""
+    return forward_ad._current_level < 0 and not torch.jit.is_tracing()
 
 
 def _pair(v):
@@ -227,6 +234,11 @@ def sparse_gather(x, bin_counts, active_block_indices, dynamic_bsize=None, dynam
     if torch.is_grad_enabled() and isinstance(x, torch.Tensor) and x.requires_grad:
         if out is not None:
             raise ValueError("out= cannot be combined with a differentiable input")
+        if _plain_autograd():
+            y = (_native or _load_native()).gather_autograd(x, bin_counts, active_block_indices, dynamic_bsize, dynamic_bstride,
+                                                            dynamic_boffset, transpose)
+            if y is not None:
+                return y
         from .autograd import SparseGatherFunction
         return SparseGatherFunction.apply(x, bin_counts, active_block_indices, dynamic_bsize, dynamic_bstride,
                                           dynamic_boffset, bool(transpose))
@@ -387,6 +399,11 @@ def sparse_scatter(x, bin_counts, active_block_indices, ybase, dynamic_bsize=Non
         raise TypeError("sparse_scatter: add is required (the op attribute has no default, sparse_gather.cc:258)")
     if torch.is_grad_enabled() and ((isinstance(x, torch.Tensor) and x.requires_grad) or
                                     (isinstance(ybase, torch.Tensor) and ybase.requires_grad)):
+        if _plain_autograd():
+            y = (_native or _load_native()).scatter_autograd(x, bin_counts, active_block_indices, ybase, dynamic_bsize,
+                                                             dynamic_bstride, dynamic_boffset, add, atomic, transpose)
+            if y is not None:
+                return y
         from .autograd import SparseScatterFunction
         return SparseScatterFunction.apply(x, bin_counts, active_block_indices, ybase, dynamic_bsize,
                                            dynamic_bstride, dynamic_boffset, bool(add), bool(atomic),

@@ -412,42 +412,61 @@ class _ResidualInTraining(torch.autograd.Function):
             if grads is not None:
                 dp, dw1, dw2, dw3, *norms = grads
                 return dp, None, dw1, norms[0], norms[1], dw2, norms[2], norms[3], dw3, norms[4], norms[5]
-        # a graph of the gradients is asked for, or sizes that the kernels do not take: through the layers one by one
-        wanted = [ctx.needs_input_grad[0], *ctx.needs_input_grad[2:]]
-        with torch.enable_grad():
-            inputs = [saved[0]]
-            for i, (w, beta) in enumerate(ctx.layers):
-                inputs += [w, saved[6 * i + 5], beta]
-            if not create_graph:
-                inputs = [t.detach().requires_grad_() for t in inputs]
-            q = inputs[0]
-            for i in range(3):
-                w, gamma, beta = inputs[1 + 3 * i:4 + 3 * i]
-                y = _batch_norm(q, BatchNormParams(gamma, beta, None, None), True, True)
-                w_ = _AsItWas.apply(_hwio_to_oihw(w), saved[6 * i + 4])
-                q = F.conv2d(_ReluAsItWas.apply(y, saved[6 * i + 1]), w_)
-            found = iter(torch.autograd.grad(q, [t for t, n in zip(inputs, wanted) if n], dq, create_graph=create_graph))
-        grads = [next(found) if n else None for n in wanted]
+        layers = [t for pair in ctx.layers for t in pair]
+        grads = _residual_by_layers(saved, layers, [ctx.needs_input_grad[0], *ctx.needs_input_grad[2:]], dq, create_graph)
         return (grads[0], None, *grads[1:])
+
+
+def _residual_by_layers(saved, layers, wanted, dq, create_graph):
+    """Gradients of p and of each layer's kernel, gamma and beta through the layers one by one: where a graph of the gradients
+    is asked for, or for sizes that the kernels do not take.  layers: kernel and beta of each, as they are now."""
+    with torch.enable_grad():
+        inputs = [saved[0]]
+        for i in range(3):
+            inputs += [layers[2 * i], saved[6 * i + 5], layers[2 * i + 1]]
+        if not create_graph:
+            inputs = [t.detach().requires_grad_() for t in inputs]
+        q = inputs[0]
+        for i in range(3):
+            w, gamma, beta = inputs[1 + 3 * i:4 + 3 * i]
+            y = _batch_norm(q, BatchNormParams(gamma, beta, None, None), True, True)
+            w_ = _AsItWas.apply(_hwio_to_oihw(w), saved[6 * i + 4])
+            q = F.conv2d(_ReluAsItWas.apply(y, saved[6 * i + 1]), w_)
+        found = iter(torch.autograd.grad(q, [t for t, n in zip(inputs, wanted) if n], dq, create_graph=create_graph))
+    return [next(found) if n else None for n in wanted]
+
+
+def _residual_in_training(p, params):
+    """_ResidualInTraining in native code, for plain tensors."""
+    native = ops._native or ops._load_native()
+    native.set_by_layers(_residual_by_layers)
+    moving = [t for b in params.bn for t in (b.moving_mean, b.moving_var)]
+    tensors = [t for w, b in zip(params.w, params.bn) for t in (w, b.gamma, b.beta)]
+    q = native.residual(p, moving, tensors, 1.0 - BN_DECAY, BN_EPS) if ops._plain_autograd() else None
+    return q if q is not None else _ResidualInTraining.apply(p, list(zip(moving[::2], moving[1::2])), *tensors)
 
 
 def _own_residual_gradient(p, params):
     """Whether _ResidualInTraining applies: not under forward-mode or functorch transforms, autocast, or where deterministic
     algorithms are asked for (its batch norm sums are added up with atomics, in double), and up to the size where the
     library's gradients become the faster ones."""
-    tensors = [p, *params.w, *(t for b in params.bn for t in (b.gamma, b.beta))]
-    stats = [t for b in params.bn for t in (b.moving_mean, b.moving_var) if t is not None]
-    return (torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
+    w, bn = params.w, params.bn
+    stats = [t for b in bn for t in (b.moving_mean, b.moving_var) if t is not None]
+    tensors = [p, *w]
+    for b in bn:
+        tensors += b.gamma, b.beta
+    if not (torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
             torch._C._functorch.peek_interpreter_stack() is None and not torch.is_autocast_enabled("cuda") and
             not torch.are_deterministic_algorithms_enabled() and len(tensors) == 10 and
-            all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32 and t.is_contiguous()
-                for t in tensors + stats) and
-            all(w.dim() == 4 and w.shape[2] % 4 == 0 and w.shape[3] % 4 == 0 for w in params.w) and
-            not any(t.requires_grad for t in stats) and
-            2 * p.shape[0] * p.shape[2] * p.shape[3] * sum(w.numel() for w in params.w) <=
-            (OWN_GRADIENT_MOST if any(w.requires_grad for w in params.w) else OWN_GRADIENT_MOST_FROZEN) and
-            p.shape[0] * (p.shape[2] - sum(w.shape[0] - 1 for w in params.w[:2])) *
-            (p.shape[3] - sum(w.shape[1] - 1 for w in params.w[:2])) >= 2)
+            (ops._native or ops._load_native()).all_plain(tensors + stats)):
+        return False
+    (a0, b0, c0, k0), (a1, b1, c1, k1), (_, _, c2, k2) = [t.shape for t in w] if all(t.dim() == 4 for t in w) else [(0,) * 4] * 3
+    if a0 == 0 or c0 % 4 or k0 % 4 or c1 % 4 or k1 % 4 or c2 % 4 or k2 % 4 or any(t.requires_grad for t in stats):
+        return False
+    M, _, R, S = p.shape
+    most = OWN_GRADIENT_MOST if any(t.requires_grad for t in w) else OWN_GRADIENT_MOST_FROZEN
+    return (2 * M * R * S * sum(t.numel() for t in w) <= most and
+            M * (R - a0 - a1 + 2) * (S - b0 - b1 + 2) >= 2)
 
 
 def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_training, data_format="NHWC",
@@ -474,8 +493,7 @@ def sparse_res_block_bottleneck(x, params, indices, block_params, strides, is_tr
         x = _conv_layer(x, w_project, strides[2], "SAME", False)
     if (is_training and transpose and not no_activation and strides[1] == strides[2] == 1 and
             _own_residual_gradient(p, params)):
-        q = _ResidualInTraining.apply(p, [(b.moving_mean, b.moving_var) for b in params.bn],
-                                      *(t for w, b in zip(params.w, params.bn) for t in (w, b.gamma, b.beta)))
+        q = _residual_in_training(p, params)
     else:
         q = _bottleneck_residual(p, params, strides, "VALID", is_training, "NCHW" if transpose else "NHWC", no_activation)
     q = q.contiguous()

@@ -1,0 +1,116 @@
+"""The differentiable ops in native code against the autograd functions in Python whose place they take, and what still goes to
+those."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+from torch.utils._python_dispatch import TorchDispatchMode
+
+import sbnet_amd
+from sbnet_amd import SparseGatherFunction, SparseScatterFunction, ops
+
+DEV = "cuda:0"
+BS, BT, BO = [6, 6], [4, 5], [-1, -2]
+
+
+def make(C=12, M=5, transpose=False, seed=0, device=DEV):
+    g = torch.Generator(device=device).manual_seed(seed)
+    idx = torch.tensor([(0, i, (2 * i) % 3) for i in range(M)], dtype=torch.int16, device=device)
+    x = torch.randn(1, 24, 20, C, device=device, generator=g)
+    q = torch.randn(*((M, C, *BS) if transpose else (M, *BS, C)), device=device, generator=g)
+    return x, q, idx, torch.tensor([M], dtype=torch.int32)
+
+
+def test_tensors_that_are_not_plain_are_left_alone():
+    x, q, idx, cnt = make(device="cpu")
+    native = ops._load_native()
+    x.requires_grad_()
+    assert native.gather_autograd(x, cnt, idx, BS, BT, BO, False) is None
+    assert native.scatter_autograd(q, cnt, idx, x, BS, BT, BO, False, False, False) is None
+    assert native.residual(q, [None] * 6, [q] * 9, 0.1, 1e-3) is None
+    assert not native.all_plain([x, q])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("wanted", ["x", "q", "xq"])
+def test_gradients_are_those_of_the_functions_in_python(wanted, transpose, add):
+    x, q, idx, cnt = make(transpose=transpose)
+    x.requires_grad_("x" in wanted)
+    q.requires_grad_("q" in wanted)
+    leaves = [t for t in (x, q) if t.requires_grad]
+    results = []
+    for python in (False, True):
+        if python:
+            p = SparseGatherFunction.apply(x, cnt, idx, BS, BT, BO, transpose)
+            y = SparseScatterFunction.apply(q, cnt, idx, x, BS, BT, BO, add, True, transpose)
+        else:
+            p = sbnet_amd.sparse_gather(x, cnt, idx, BS, BT, BO, transpose=transpose)
+            y = sbnet_amd.sparse_scatter(q, cnt, idx, x, BS, BT, BO, add=add, atomic=True, transpose=transpose)
+            assert "Function" in y.grad_fn.name() and "Sparse" not in y.grad_fn.name()
+        assert p.requires_grad == x.requires_grad and y.requires_grad
+        # gradients that are not contiguous; an unused output; twice, with the graph kept
+        dy = torch.linspace(-1, 1, y.shape[3], device=DEV).expand(y.shape)
+        grads = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+        grads += torch.autograd.grad([y] + [p] * p.requires_grad, leaves, [dy] + [p.detach()] * p.requires_grad)
+        results.append((p.detach(), y.detach(), *grads))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("add", [False, True])
+def test_gradient_of_the_bases_gradient(add):
+    x, q, idx, cnt = make()
+    results = []
+    for op in (sbnet_amd.sparse_scatter, SparseScatterFunction.apply):
+        base, dy = x.clone().requires_grad_(), torch.cos(x).requires_grad_()
+        y = op(q, cnt, idx, base, BS, BT, BO, add, True, False)
+        g, = torch.autograd.grad(y, base, dy, create_graph=True)
+        results.append((g.detach(), torch.autograd.grad(g, dy, x)[0]))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_hooks_of_saved_tensors_see_the_list():
+    x, q, idx, cnt = make()
+    x.requires_grad_()
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t.cpu(), lambda t: t.to(DEV)):
+        p = sbnet_amd.sparse_gather(x, cnt, idx, BS, BT, BO)
+        y = sbnet_amd.sparse_scatter(q, cnt, idx, x, BS, BT, BO, add=True, atomic=True)
+    assert seen == [idx.shape, idx.shape]
+    got, = torch.autograd.grad([p, y], x, [p.detach(), y.detach()])
+    want, = torch.autograd.grad([sbnet_amd.sparse_gather(x, cnt, idx, BS, BT, BO)], x, [p.detach()])
+    assert torch.equal(got, want + y.detach())
+
+
+@pytest.mark.gpu
+def test_what_looks_on_or_transforms_goes_to_the_functions_in_python():
+    x, q, idx, cnt = make()
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x.requires_grad_()
+    with Mode():
+        assert "SparseGatherFunction" in sbnet_amd.sparse_gather(x, cnt, idx, BS, BT, BO).grad_fn.name()
+        assert "SparseScatterFunction" in sbnet_amd.sparse_scatter(q, cnt, idx, x, BS, BT, BO, add=True, atomic=True).grad_fn.name()
+    with forward_ad.dual_level(), pytest.raises(RuntimeError):   # (no rule for forward mode: refused, not dropped)
+        sbnet_amd.sparse_gather(forward_ad.make_dual(x, torch.ones_like(x)), cnt, idx, BS, BT, BO)
+    with pytest.raises(RuntimeError):                             # (functorch wants setup_context)
+        torch.func.grad(lambda t: sbnet_amd.sparse_gather(t, cnt, idx, BS, BT, BO).sum())(x.detach())
+    # a count on the device
+    y = sbnet_amd.sparse_gather(x, cnt.to(DEV), idx, BS, BT, BO)
+    assert "SparseGatherFunction" in y.grad_fn.name()
+
+
+@pytest.mark.gpu
+def test_a_changed_list_is_noticed():
+    x, _, idx, cnt = make()
+    y = sbnet_amd.sparse_gather(x.requires_grad_(), cnt, idx, BS, BT, BO)
+    idx.add_(0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y.sum(), x)
