@@ -362,6 +362,10 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
                           float* const* dw, float* const* dgamma, float* const* dbeta, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* Up to three convolution kernels from [kh,kw,C,K] (w_dims[4 * i ...] = kh, kw, C, K) to the [K,C,kh,kw] that the library's
+   convolutions and sbnet_bottleneck_grad take, in one launch. */
+int sbnet_kernels_oihw(const float* const* weights, const int32_t* w_dims, float* const* out, int count, void* stream);
+
 /* Library-managed device scratch for callers that have no allocator at hand (the functor level of the reference
    passes none down, sparse_gather.h:45-66): returns a buffer of at least `bytes` bytes on the current device.  One
    grow-only buffer is kept per (device, stream); calls on one stream run in order, so consecutive calls of ONE

@@ -15,7 +15,9 @@ typedef float acc_t __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------------------------
 //
 // Four channels per thread, `cols` threads side by side, `tall` rows at a time; a workgroup takes as many rows as leave
-// about 512 workgroups.  Two tensors in, one out, once each.
+// about 512 workgroups.  Two tensors in, one out, once each.  The channels' coefficients are worked out once per
+// workgroup, a channel a thread (four of them in every thread, 32 loads ahead of the first row, took 22.9 us for the three
+// launches of a step on 85 blocks of 11x11, 256-64-64 channels; 15.2 this way).
 
 struct ChannelArgs {
     uint32_t rows, C;
@@ -39,29 +41,32 @@ static ChannelArgs channel_args(uint32_t rows, int C, dim3& grid)
 __global__ __launch_bounds__(256) void k_norm_grad(float* __restrict__ g, NormGradArgs norm, ChannelArgs a,
                                                    float* __restrict__ dgamma, float* __restrict__ dbeta)
 {
+    __shared__ __attribute__((aligned(16))) float coef[4][256];   // mean, scale and the two means, of the workgroup's channels
     const uint32_t tid = threadIdx.x, ty = tid / a.cols, tx = tid - ty * a.cols;
-    const uint32_t c = (blockIdx.y * a.cols + tx) * 4u;
-    if (ty >= a.tall || c >= a.C) return;
-    float mean[4], scale[4], c1[4], c2[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    const uint32_t first = blockIdx.y * a.cols * 4u, mine = first + tid;
+    if (tid < a.cols * 4u && mine < a.C) {
         double s1 = 0.0, s2 = 0.0;
 #pragma unroll
         for (int i = 0; i < GRAD_SLOTS; ++i) {
-            const double2 t = *reinterpret_cast<const double2*>(norm.sums + ((size_t)i * a.C + c + j) * 2);
+            const double2 t = *reinterpret_cast<const double2*>(norm.sums + ((size_t)i * a.C + mine) * 2);
             s1 += t.x;
             s2 += t.y;
         }
-        const float inv = norm.inv[c + j];
-        mean[j] = norm.mean[c + j];
-        scale[j] = inv * norm.gamma[c + j];
-        c1[j] = (float)(s1 / a.rows);
-        c2[j] = (float)(s2 / a.rows * inv);
-        if (blockIdx.x == 0 && ty == 0) {
-            if (dgamma) dgamma[c + j] = (float)s2;
-            if (dbeta) dbeta[c + j] = (float)s1;
+        const float inv = norm.inv[mine];
+        coef[0][tid] = norm.mean[mine];
+        coef[1][tid] = inv * norm.gamma[mine];
+        coef[2][tid] = (float)(s1 / a.rows);
+        coef[3][tid] = (float)(s2 / a.rows * inv);
+        if (blockIdx.x == 0) {
+            if (dgamma) dgamma[mine] = (float)s2;
+            if (dbeta) dbeta[mine] = (float)s1;
         }
     }
+    lds_barrier();
+    const uint32_t c = first + tx * 4u;
+    if (ty >= a.tall || c >= a.C) return;
+    const f4 mean = lds_read4(coef[0] + tx * 4u), scale = lds_read4(coef[1] + tx * 4u), c1 = lds_read4(coef[2] + tx * 4u),
+             c2 = lds_read4(coef[3] + tx * 4u);
     const float* const z = norm.z;
     const uint32_t end = min((blockIdx.x + 1) * a.rowsPerWg, a.rows);
 #pragma unroll 4
@@ -151,6 +156,71 @@ hipError_t launch_transposes(const TransposeArgs* t, int count, hipStream_t stre
 }
 
 // ---------------------------------------------------------------------------------------------
+// k_kernels: [taps][C][K] -> [K][C][taps], the three kernels of a residual function in one launch
+// ---------------------------------------------------------------------------------------------
+//
+// In the order of the results; what is read lies K floats apart, in the caches: the kernels are small.  (Three copies of
+// permuted views through the library: 11 us on the GPU and 24 in the host for 256-64-64-256 channels; 4 and 5 this way.)
+
+struct KernelsProblem {
+    const float* from;
+    float* to;
+    uint32_t count, K, C, taps, firstWg;
+    FastDiv dRow, dTaps;   // by C * taps, by taps
+};
+
+struct KernelsArgs {
+    KernelsProblem p[3];
+    int count;
+};
+
+constexpr uint32_t KERNELS_UNR = 4;
+
+__global__ __launch_bounds__(256) void k_kernels(KernelsArgs a)
+{
+    int i = 0;
+    while (i + 1 < a.count && blockIdx.x >= a.p[i + 1].firstWg) ++i;
+    const KernelsProblem& q = a.p[i];
+    const uint32_t o0 = (blockIdx.x - q.firstWg) * (256u * KERNELS_UNR) + threadIdx.x;
+    float v[KERNELS_UNR];
+#pragma unroll
+    for (uint32_t u = 0; u < KERNELS_UNR; ++u) {
+        const uint32_t o = min(o0 + 256u * u, q.count - 1u);
+        const uint32_t k = fdiv(o, q.dRow), r = o - k * (q.C * q.taps), c = fdiv(r, q.dTaps), t = r - c * q.taps;
+        v[u] = q.from[(size_t)(t * q.C + c) * q.K + k];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < KERNELS_UNR; ++u)
+        if (o0 + 256u * u < q.count) q.to[o0 + 256u * u] = v[u];
+}
+
+hipError_t launch_kernels(const float* const* from, const int32_t* dims, float* const* to, int count, hipStream_t stream)
+{
+    if (count < 1 || count > 3) return hipErrorInvalidValue;
+    KernelsArgs a;
+    uint64_t wgs = 0;
+    for (int i = 0; i < count; ++i) {
+        const int32_t* d = dims + 4 * i;
+        const uint64_t n = (uint64_t)d[0] * d[1] * d[2] * d[3];
+        if (n == 0 || n >= (1ull << 30)) return hipErrorInvalidValue;
+        KernelsProblem& q = a.p[i];
+        q.from = from[i];
+        q.to = to[i];
+        q.count = (uint32_t)n;
+        q.taps = (uint32_t)(d[0] * d[1]);
+        q.C = (uint32_t)d[2];
+        q.K = (uint32_t)d[3];
+        q.firstWg = (uint32_t)wgs;
+        q.dRow = make_fastdiv(q.C * q.taps);
+        q.dTaps = make_fastdiv(q.taps);
+        wgs += (n + 256u * KERNELS_UNR - 1) / (256u * KERNELS_UNR);
+    }
+    a.count = count;
+    hipLaunchKernelGGL(k_kernels, dim3((unsigned)wgs), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
 // k_wgrad: dw[m, n] = sum over output pixels p of act[p + tap, c] * dz[p, n], m = (tap, c)
 // ---------------------------------------------------------------------------------------------
 //
@@ -163,9 +233,9 @@ hipError_t launch_transposes(const TransposeArgs* t, int count, hipStream_t stre
 // of its pixel feeds four fragments (fragment i has rows 4 * l + i), so 4 pixels x 64 x 64 products cost two 16-byte loads
 // and 16 matrix instructions per lane, straight from memory.
 //
-// Measured (MI355X, kernel trace; 256-64-64-256 channels on about 85 active 11x11 blocks of [1,100,175,256]): 17.8 us for the
-// three products and 17.6 for the sum of the partial tiles, where the library took 77 us and six transposes of its operands
-// (23 us).  The whole gradient: 127 us in 12 launches; 190 us in 27 with the library's passes.
+// Measured (MI355X, kernel trace; 256-64-64-256 channels on about 85 active 11x11 blocks of [1,100,175,256]): 18.5 us for the
+// three products and 5.2 for the sum of the partial tiles, where the library took 77 us and six transposes of its operands
+// (23 us).  The whole gradient: 105 us in 12 launches; 190 us in 27 with the library's passes.
 
 struct WgradProblem {
     WgradArgs w;
@@ -287,11 +357,16 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradKernelArgs a)
     }
 }
 
-// Adds the partial tiles, in double, and writes the gradients.
-__global__ __launch_bounds__(256) void k_wgrad_sum(WgradKernelArgs a)
+// Adds the partial tiles, in double, and writes the gradients.  The results are few and the splits many: a workgroup takes
+// 64 pieces of 16 bytes, its waves every eighth split of them.  (A thread for all splits of a piece: 17.6 us for 642 partial
+// tiles of 16 KB, from 68 workgroups that wait for one round of loads after the other; 5.2 this way.)
+constexpr int SUM_WAVES = 8;
+
+__global__ __launch_bounds__(64 * SUM_WAVES) void k_wgrad_sum(WgradKernelArgs a)
 {
-    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
-    if (id >= a.sums) return;
+    __shared__ double part[SUM_WAVES][4][64];
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t id = blockIdx.x * 64u + (threadIdx.x & 63u);   // (a.sums is a multiple of 64)
     int k = 0;
     while (k + 1 < a.count && id >= a.p[k + 1].firstSum) ++k;
     const WgradProblem& q = a.p[k];
@@ -303,19 +378,21 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(WgradKernelArgs a)
     const size_t step = (size_t)q.tiles * frags * 256;
     double s[4] = {};
 #pragma unroll 8
-    for (uint32_t i = 0; i < q.splits; ++i) {
+    for (uint32_t i = wave; i < q.splits; i += SUM_WAVES) {
         const f4 v = *reinterpret_cast<const f4*>(p + i * step);
 #pragma unroll
         for (int j = 0; j < 4; ++j) s[j] += (double)v[j];
     }
-    const uint32_t i = frag / (uint32_t)q.jb, j = frag - i * (uint32_t)q.jb;
-    const uint32_t n = (tn * 16u + l16) * (uint32_t)q.jb + j;
-    if (n >= (uint32_t)q.w.K) return;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t m = tm * 64u + (quad * 4u + r) * 4u + i;
-        if (m < q.mTot) q.w.dw[(size_t)m * q.w.K + n] = (float)s[r];
-    }
+    for (int r = 0; r < 4; ++r) part[wave][r][lane] = s[r];
+    lds_barrier();
+    if (wave >= 4u) return;   // (wave r has the r-th float of each piece)
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < SUM_WAVES; ++w) sum += part[w][wave][lane];
+    const uint32_t i = frag / (uint32_t)q.jb, j = frag - i * (uint32_t)q.jb;
+    const uint32_t n = (tn * 16u + l16) * (uint32_t)q.jb + j, m = tm * 64u + (quad * 4u + wave) * 4u + i;
+    if (n < (uint32_t)q.w.K && m < q.mTot) q.w.dw[(size_t)m * q.w.K + n] = (float)sum;
 }
 
 // About 640 workgroups in all, each of at least 64 pixels, the pixels' ranges of all problems equally long.
@@ -379,7 +456,7 @@ hipError_t launch_wgrad(const WgradArgs* w, int count, void* workspace, hipStrea
     const WgradProblem& last = a.p[count - 1];
     const uint32_t wgs = last.firstWg + last.splits * last.tiles;
     hipLaunchKernelGGL(k_wgrad, dim3(wgs), dim3(256), 65536, stream, a);
-    hipLaunchKernelGGL(k_wgrad_sum, dim3((a.sums + 255) / 256), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(k_wgrad_sum, dim3(a.sums / 64), dim3(64 * SUM_WAVES), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -867,6 +867,20 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
     return SBNET_OK;
 }
 
+int sbnet_kernels_oihw(const float* const* weights, const int32_t* w_dims, float* const* out, int count, void* stream)
+{
+    if (!weights || !w_dims || !out || count < 1 || count > 3) return SBNET_EINVAL_ARG;
+    for (int i = 0; i < count; ++i) {
+        const int32_t* d = w_dims + 4 * i;
+        if (!weights[i] || !out[i] || d[0] <= 0 || d[1] <= 0 || d[2] <= 0 || d[3] <= 0 ||
+            (int64_t)d[0] * d[1] >= (1ll << 30) || (int64_t)d[0] * d[1] * d[2] >= (1ll << 30) ||
+            (int64_t)d[0] * d[1] * d[2] * d[3] >= (1ll << 30))
+            return SBNET_EINVAL_ARG;
+    }
+    SBNET_HIP(sbnet::launch_kernels(weights, w_dims, out, count, static_cast<hipStream_t>(stream)));
+    return SBNET_OK;
+}
+
 int sbnet_sparse_scatter_functor(const float* x, int N, int H, int W, int C, float* y, int bOffsH0,
                                  int bOffsW0, int bSzH, int bSzW, int bStrH, int bStrW, int numActive,
                                  const int16_t* activeBlockIndices, int add, int transpose, int atomic,

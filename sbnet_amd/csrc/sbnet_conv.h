@@ -76,6 +76,9 @@ struct WgradArgs {
 size_t wgrad_workspace_bytes(const WgradArgs* w, int count);
 hipError_t launch_wgrad(const WgradArgs* w, int count, void* workspace, hipStream_t stream);
 
+// Up to three kernels [kh,kw,C,K] (dims: four each) to [K,C,kh,kw] in one launch.
+hipError_t launch_kernels(const float* const* from, const int32_t* dims, float* const* to, int count, hipStream_t stream);
+
 // Up to ten matrix transposes [M][A][B] -> [M][B][A] in one launch (block stacks from planar to NHWC and back).
 struct TransposeArgs {
     const float* from;

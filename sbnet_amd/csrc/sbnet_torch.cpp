@@ -797,6 +797,31 @@ struct Residual {
     double momentum, eps;
 };
 
+// Kernels [kh,kw,C,K] as the library takes them, [K,C,kh,kw].
+void kernels_of(const at::Tensor* const* w, at::Tensor* out)
+{
+    const float* from[3];
+    float* to[3];
+    int32_t dims[12];
+    bool own = true;
+    for (int i = 0; i < 3; ++i) {
+        own = own && w[i]->numel() > 0 && w[i]->numel() < CONV_MOST && w[i]->device() == w[0]->device();
+        for (int j = 0; j < 4 && own; ++j) dims[4 * i + j] = (int32_t)w[i]->size(j);
+    }
+    if (!own) {
+        for (int i = 0; i < 3; ++i) out[i] = w[i]->permute({3, 2, 0, 1}).contiguous();
+        return;
+    }
+    c10::DeviceGuard guard(w[0]->device());
+    for (int i = 0; i < 3; ++i) {
+        out[i] = empty_f32({dims[4 * i + 3], dims[4 * i + 2], dims[4 * i], dims[4 * i + 1]}, *w[0]);
+        from[i] = static_cast<const float*>(w[i]->const_data_ptr());
+        to[i] = static_cast<float*>(out[i].data_ptr());
+    }
+    const int status = sbnet_kernels_oihw(from, dims, to, 3, stream_of(*w[0]));
+    TORCH_CHECK(status == SBNET_OK, sbnet_status_string(status), " (hipError_t ", sbnet_last_hip_error(), ")");
+}
+
 struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
     // The library's calls, one by one, as the layers make them.
     static at::Tensor forward(AutogradContext* ctx, const at::Tensor& p, const at::Tensor& w1, const at::Tensor& g1, const at::Tensor& b1,
@@ -804,16 +829,16 @@ struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
                               const at::Tensor& g3, const at::Tensor& b3, const Residual* r)
     {
         const at::Tensor *const w[3] = {&w1, &w2, &w3}, *const gamma[3] = {&g1, &g2, &g3}, *const beta[3] = {&b1, &b2, &b3};
-        at::Tensor z = p;
+        at::Tensor z = p, kernels[3];
+        kernels_of(w, kernels);
         variable_list saved;
         for (int i = 0; i < 3; ++i) {
             auto bn = at::_batch_norm_impl_index(z, *gamma[i], *beta[i], r->mean[i], r->var[i], true, r->momentum, r->eps,
                                                  at::globalContext().userEnabledCuDNN());
             at::Tensor& act = std::get<0>(bn);
             act.relu_();
-            const at::Tensor kernel = w[i]->permute({3, 2, 0, 1}).contiguous();
-            saved.insert(saved.end(), {z, act, std::get<1>(bn), std::get<2>(bn), kernel, *gamma[i]});
-            z = at::conv2d(act, kernel, {}, at::IntArrayRef({1, 1}));
+            saved.insert(saved.end(), {z, act, std::get<1>(bn), std::get<2>(bn), kernels[i], *gamma[i]});
+            z = at::conv2d(act, kernels[i], {}, at::IntArrayRef({1, 1}));
         }
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["layers"] = std::vector<at::Tensor>{w1, b1, w2, b2, w3, b3};   // for a graph of the gradients alone

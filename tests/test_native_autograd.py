@@ -114,3 +114,23 @@ def test_a_changed_list_is_noticed():
     idx.add_(0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(y.sum(), x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [[(1, 1, 4, 4)], [(3, 3, 20, 12), (1, 5, 7, 3)], [(1, 1, 256, 64), (3, 3, 64, 64), (7, 7, 1, 33)]],
+                         ids=str)
+def test_kernels_in_the_librarys_order(shapes):
+    import ctypes
+    import numpy as np
+    from sbnet_amd import _lib
+    w = [torch.randn(*s, device=DEV) for s in shapes]
+    out = [torch.empty(s[3], s[2], s[0], s[1], device=DEV) for s in shapes]
+    n = len(w)
+    pointers = lambda ts: ctypes.cast((ctypes.c_void_p * 4)(*(t.data_ptr() for t in ts)), ctypes.c_void_p)
+    fn = _lib.load().sbnet_kernels_oihw
+    call = lambda d, k: fn(pointers(w), ops._pair(d.reshape(-1))[1], pointers(out), k, ops._stream())
+    dims = np.array(shapes, np.int32)
+    assert call(dims, n) == 0
+    for a, b in zip(out, w):
+        assert torch.equal(a, b.permute(3, 2, 0, 1))
+    assert call(dims, 4) == call(dims, 0) == call(dims * 0, n) == _lib.SBNET_EINVAL_ARG
