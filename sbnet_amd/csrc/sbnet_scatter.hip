@@ -1267,12 +1267,6 @@ static void launch_fill_zero(float* y, size_t count, hipStream_t stream)
 // channel vectors wide, as in k_scatter_strip; a pixel of cell (bh, bw) can be covered by the blocks (bh, bw),
 // (bh, bw-1), (bh-1, bw) and (bh-1, bw-1).  When the list names a block twice the passes fall back to hardware
 // atomics, which need zeros everywhere: then every pixel is cleared.
-//
-// FROM: the same map applied to a tensor, y = src * (0 where a block covers the pixel, 1 elsewhere): the gradient of the
-// plain-write scatter with respect to its base.  A product, so that infinities and NaN under a block become NaN, as they
-// do in the product with a stamped-out mask that this replaces (fill with ones, fill a stack with zeros, scatter it,
-// multiply: 125 us at 300x480x256 with 30 % of the 18x18 blocks, 443 MB of them the product's).  This pass moves 295 MB: 46 us
-// there, 6.4 TB/s.
 struct FillArgs {
     Geom g;
     int bhMin, bwMin, nBH, nBW;  // extent of the inverse block map
@@ -1291,10 +1285,9 @@ __device__ __forceinline__ bool fill_block_active(const FillArgs& a, const int32
     return map[((int64_t)n * a.nBH + ih) * a.nBW + iw] >= 0;
 }
 
-template <int VEC, bool FROM>
+template <int VEC>
 __global__ __launch_bounds__(256) void k_fill_uncovered(float* __restrict__ y, const int32_t* __restrict__ map,
-                                                        const int32_t* __restrict__ dup, const float* __restrict__ src,
-                                                        FillArgs a)
+                                                        const int32_t* __restrict__ dup, FillArgs a)
 {
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
     const uint32_t tid = threadIdx.x;
@@ -1315,17 +1308,7 @@ __global__ __launch_bounds__(256) void k_fill_uncovered(float* __restrict__ y, c
     const uint32_t iw = fdiv(dw, a.dV);
     const int sc = (int)(dw - iw * (uint32_t)a.g.V), bw = (int)iw + a.cellW0;
 
-    typename Vec<VEC>::type v[STRIP_ROWS];
-    if constexpr (FROM) {   // (ahead of the map, which the products wait for)
-        const rsrc_t sr = make_rsrc(src + (int64_t)n * a.imgFloats, a.imgBytes);
-#pragma unroll
-        for (int u = 0; u < STRIP_ROWS; ++u) {
-            const int h = hTop + u;
-            const bool read = live && r0 + u < a.g.U && (unsigned)h < (unsigned)a.g.H;
-            v[u] = buf_load<VEC>(sr, read ? (((uint32_t)h * (uint32_t)a.g.W + w) * a.CV + cv) * (uint32_t)(VEC * 4) : BUF_OOB);
-        }
-    }
-    const bool all = !FROM && *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0;
+    const bool all = *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0;
     // the block of the pixel's own cell and of the cell to its left, in this row of cells and in the one above
     const bool left = sc + a.g.V < a.g.S, here = sc < a.g.S;
     bool cur = false, up = false;
@@ -1339,10 +1322,9 @@ __global__ __launch_bounds__(256) void k_fill_uncovered(float* __restrict__ y, c
     for (int u = 0; u < STRIP_ROWS; ++u) {
         const int r = r0 + u, h = hTop + u;
         const bool covered = (cur && r < a.g.R) || (up && r + a.g.U < a.g.R);
-        const bool write = live && r < a.g.U && (unsigned)h < (unsigned)a.g.H && (FROM || !covered);
+        const bool write = live && r < a.g.U && (unsigned)h < (unsigned)a.g.H && !covered;
         const uint32_t off = write ? (((uint32_t)h * (uint32_t)a.g.W + w) * a.CV + cv) * (uint32_t)(VEC * 4) : BUF_OOB;
-        if constexpr (FROM) buf_store<BUF_NT>(yr, off, v[u] * (covered ? 0.f : 1.f));
-        else buf_store<BUF_NT>(yr, off, vzero<VEC>());
+        buf_store<BUF_NT>(yr, off, vzero<VEC>());
     }
 }
 
@@ -1374,39 +1356,6 @@ static bool make_fill_args(const Geom& g, int vec, const PullArgs& pa, FillArgs&
     a.dPC = make_fastdiv(a.nPC);
     a.dBands = make_fastdiv((uint32_t)a.nBands);
     return true;
-}
-
-size_t scatter_base_grad_workspace_bytes(const Geom& g, int numActive)
-{
-    PullArgs pa;
-    FillArgs fa;
-    int64_t mapN = 0;
-    unsigned grid;
-    if (numActive <= 0 || !make_map_args(g, pa, mapN) || !make_fill_args(g, pick_vec(g, nullptr, nullptr), pa, fa, grid)) return 0;
-    return (size_t)mapN * 4 + 16;
-}
-
-hipError_t launch_scatter_base_grad(const float* dy, float* dbase, const int16_t* idx, int numActive, const Geom& g,
-                                    void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done)
-{
-    done = false;
-    const size_t need = scatter_base_grad_workspace_bytes(g, numActive);
-    if (!need || !workspace || workspaceBytes < need || (reinterpret_cast<uintptr_t>(workspace) & 3)) return hipSuccess;
-    PullArgs pa;
-    FillArgs fa;
-    int64_t mapN = 0;
-    unsigned grid = 0;
-    const int vec = pick_vec(g, dbase, dy);
-    if (!make_map_args(g, pa, mapN) || !make_fill_args(g, vec, pa, fa, grid)) return hipSuccess;
-    int32_t* map = static_cast<int32_t*>(workspace);
-    const int32_t* cmap = map;
-    const int32_t* dup = map + mapN;
-    launch_block_map(idx, numActive, pa, map, mapN, map + mapN, stream);
-    if (vec == 4) hipLaunchKernelGGL((k_fill_uncovered<4, true>), dim3(grid), dim3(256), 0, stream, dbase, cmap, dup, dy, fa);
-    else if (vec == 2) hipLaunchKernelGGL((k_fill_uncovered<2, true>), dim3(grid), dim3(256), 0, stream, dbase, cmap, dup, dy, fa);
-    else hipLaunchKernelGGL((k_fill_uncovered<1, true>), dim3(grid), dim3(256), 0, stream, dbase, cmap, dup, dy, fa);
-    done = true;
-    return hipGetLastError();
 }
 
 // ontoZeros: y holds nothing yet and the result is "zeros, plus the blocks" (the gradient of sparse_gather,
@@ -1469,9 +1418,9 @@ hipError_t launch_scatter_colored(const float* x, float* y, const int16_t* idx, 
         col.first = 1;
         const int32_t* cmap = map;
         const int32_t* cdup = dup;
-        if (vec == 4) hipLaunchKernelGGL((k_fill_uncovered<4, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
-        else if (vec == 2) hipLaunchKernelGGL((k_fill_uncovered<2, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
-        else hipLaunchKernelGGL((k_fill_uncovered<1, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
+        if (vec == 4) hipLaunchKernelGGL((k_fill_uncovered<4>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
+        else if (vec == 2) hipLaunchKernelGGL((k_fill_uncovered<2>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
+        else hipLaunchKernelGGL((k_fill_uncovered<1>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
     } else if (ontoZeros) {
         launch_fill_zero(y, (size_t)g.N * g.H * g.W * g.C, stream);
     }
@@ -1760,7 +1709,11 @@ __device__ __forceinline__ void strip_cells_of_map(const StripArgs& a, const int
 // sparse_gather.cc:103-130 on top of a copy of ybase (sparse_gather.cc:338-346).
 // OP: STRIP_ASSIGN / STRIP_ADD write the whole output; STRIP_COPY writes only the pixels that no block covers and
 // leaves the covered ones to the tiles of the same launch.  OVER: blocks overlap (plain writes, NHWC stack).
-constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2;
+// STRIP_MASK: y = base * (0 where a block covers the pixel, 1 elsewhere), the gradient of plain writes with respect to their
+// base.  A product, so that infinities and NaN under a block become NaN, as they do in the product with a stamped-out mask that
+// this replaces (fill with ones, fill a stack with zeros, scatter it, multiply: 125 us at 300x480x256 with 30 % of the 18x18
+// blocks, 443 MB of them the product's).  This pass moves 295 MB: 46 us there, 6.4 TB/s.
+constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2, STRIP_MASK = 3;
 
 template <int VEC, int OP, bool PLANAR, bool LIST, bool OVER, int CELLS>
 __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const float* __restrict__ ybase,
@@ -1792,8 +1745,8 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         off[u] = live && rowLive ? (((uint32_t)h * (uint32_t)a.g.W + w) * a.CV + cv) * (uint32_t)(VEC * 4) : BUF_OOB;
     }
     vec b[STRIP_ROWS], v[STRIP_ROWS];
-    if (ADD) {
-        // an add reads the base everywhere: these loads do not wait for the look-up
+    if (ADD || OP == STRIP_MASK) {
+        // the base is read everywhere: these loads do not wait for the look-up
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) b[u] = buf_load<VEC>(br, off[u]);
     }
@@ -1840,6 +1793,11 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         }
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+        return;
+    }
+    if (OP == STRIP_MASK) {
+#pragma unroll
+        for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u] * (at[u] >= 0 ? 0.f : 1.f));
         return;
     }
     bool several = false;
@@ -2493,9 +2451,9 @@ hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* id
     launch_block_map(idx, numActive, pa, map, mapN, dup, stream);
     const int32_t* cmap = map;
     const int32_t* cdup = dup;
-    if (vec == 4) hipLaunchKernelGGL((k_fill_uncovered<4, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
-    else if (vec == 2) hipLaunchKernelGGL((k_fill_uncovered<2, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
-    else hipLaunchKernelGGL((k_fill_uncovered<1, false>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, (const float*)nullptr, fa);
+    if (vec == 4) hipLaunchKernelGGL((k_fill_uncovered<4>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
+    else if (vec == 2) hipLaunchKernelGGL((k_fill_uncovered<2>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
+    else hipLaunchKernelGGL((k_fill_uncovered<1>), dim3(fillGrid), dim3(256), 0, stream, y, cmap, cdup, fa);
     ColorArgs col;
     col.kh = 2; col.kw = 2; col.pass = 0;  // (unused by this mode, like the fields of the other orders)
     col.dup = cdup; col.owner = nullptr; col.rank = nullptr; col.first = 0; col.map = cmap;
@@ -2508,6 +2466,21 @@ hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* id
     return hipGetLastError();
 }
 
+// The map of the cells, in one launch or two.
+static void launch_cell_map(const int16_t* idx, int numActive, const StripArgs& a, int32_t* map, int64_t mapN, int32_t* chain,
+                            int32_t* dup, hipStream_t stream)
+{
+    if (mapN <= BLOCK_MAP_ONE_WG && numActive <= BLOCK_MAP_ONE_WG) {
+        hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN, chain, dup);
+        return;
+    }
+    int64_t fillWgs = (mapN + 255) / 256;
+    if (fillWgs > 4096) fillWgs = 4096;
+    hipLaunchKernelGGL(k_pull_fill, dim3((unsigned)fillWgs), dim3(256), 0, stream, map, mapN, dup);
+    hipLaunchKernelGGL(k_cell_map, dim3((unsigned)((numActive + 255) / 256)), dim3(256), 0, stream, idx, numActive, a, map,
+                       chain, dup);
+}
+
 // What the one-pass kernels look cells up in: the list itself, or a map that earlier launches made of it.
 struct CellMap {
     bool list;
@@ -2516,7 +2489,7 @@ struct CellMap {
 
 template <int VEC>
 static void launch_strip(const float* x, const float* ybase, float* y, const int16_t* idx, bool planar, bool add, const CellMap& m,
-                         const StripArgs& a, hipStream_t stream)
+                         const StripArgs& a, hipStream_t stream, bool mask = false)
 {
     const dim3 grid(a.tiles);
     const size_t lds = planar ? (size_t)STRIP_ROWS * a.PX * a.CT * sizeof(float) : 0;  // 16 KB with 16-byte vectors
@@ -2525,6 +2498,7 @@ static void launch_strip(const float* x, const float* ybase, float* y, const int
     if (add && planar) m.list ? go(k_scatter_strip<VEC, STRIP_ADD, true, true, false>) : go(k_scatter_strip<VEC, STRIP_ADD, true, false, false>);
     else if (add) m.list ? go(k_scatter_strip<VEC, STRIP_ADD, false, true, false>) : go(k_scatter_strip<VEC, STRIP_ADD, false, false, false>);
     else if (planar) m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, true, true, false>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, true, false, false>);
+    else if (mask) m.list ? go(k_scatter_strip<VEC, STRIP_MASK, false, true, true>) : go(k_scatter_strip<VEC, STRIP_MASK, false, false, true>);
     else if (over) m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, false, true, true>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, false, false, true>);
     else m.list ? go(k_scatter_strip<VEC, STRIP_ASSIGN, false, true, false>) : go(k_scatter_strip<VEC, STRIP_ASSIGN, false, false, false>);
 }
@@ -2599,7 +2573,13 @@ static void launch_rest(const float* x, const float* ybase, float* y, const int1
 // more.  us with the map / with the list, MI355X: 512x512x64, add, 102 rows 27.0 / 24.8, 512: 30.2 / 27.7, 921: 34.8 / 31.7;
 // [4,256,256,64], 1351 rows of 8x8: 29.2 / 26.8, as cells 28.9 / 26.8; eight images, 2703 rows: 57.7 / 55.4, as cells 55.3 /
 // 66.4; 16 images, 5406: 110 / 120.
+// Where a workgroup can do nothing before it has looked its cell up, and there are many of them, the list costs more than the
+// launches.  Cells: 242 of 20x20x128, 3000 workgroups 17.8 / 16.2; 2312 of 16x16x64, 9000: 49.8 / 50.8; 2116 of 24x24x64, 21 000:
+// 86 / 97.  Tiles and the rest, by strips times rows: 0.3 M 18.1 / 16.5, 1.4 M 104.4 / 99.9, 3.8 M 108 / 112, 4.5 M 120 / 112, 6.1 M
+// 121.6 / 125.5, 6.3 M 104 / 112, 10.6 M 103 / 107.  Strips, which move the most, gain at every size measured.
 constexpr int STRIP_LIST_MAX = 1536;
+constexpr uint32_t CELLS_LIST_MAX_WGS = 6144;
+constexpr int64_t REST_LIST_MAX = 3500000;   // strips times rows
 
 hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y, const int16_t* idx, int numActive,
                                     const Geom& g, bool transpose, ScatterMode mode, void* workspace,
@@ -2614,7 +2594,7 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
         const bool add = mode == SCATTER_ADD;
         const int vb = pick_vec(g, ybase, y), vx = pick_vec(g, transpose ? nullptr : x, nullptr);
         const int vec = vb < vx ? vb : vx;
-        const bool list = numActive <= STRIP_LIST_MAX;
+        bool list = numActive <= STRIP_LIST_MAX;
         StripArgs a;
         CellsPlan cells;
         RestPlan rest;
@@ -2624,8 +2604,11 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
             how = STRIPS;
         } else if (transpose) {
             if (make_strip_args(g, numActive, vec, false, x, a, mapN) && plan_cells(g, numActive, vec, a, mapN, cells)) how = CELLS;
+            else if (plan_rest(g, numActive, vec, rest, mapN)) how = REST;
+            if (how == CELLS) list = list && (uint32_t)mapN * cells.a.tpb <= CELLS_LIST_MAX_WGS;
+            if (how == REST) list = list && (int64_t)rest.s.tiles * numActive <= REST_LIST_MAX;
             // (with a map two more launches: worth it once the blocks cover enough of the tensor)
-            else if ((list || (int64_t)numActive * g.R * g.S * g.C * 4 >= (16ll << 20)) && plan_rest(g, numActive, vec, rest, mapN)) how = REST;
+            if (how == REST && !list && (int64_t)numActive * g.R * g.S * g.C * 4 < (16ll << 20)) how = NONE;
         }
         if (how == REST) a = rest.s;
         if (!list && workspaceBytes < (size_t)mapN * 4 + 16 + (size_t)numActive * 4 + 16) how = NONE;
@@ -2635,16 +2618,7 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
                 int32_t* map = static_cast<int32_t*>(workspace);
                 int32_t* dup = map + mapN;
                 int32_t* chain = add ? dup + 4 : nullptr;
-                if (mapN <= BLOCK_MAP_ONE_WG && numActive <= BLOCK_MAP_ONE_WG) {
-                    hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN,
-                                       chain, dup);
-                } else {
-                    int64_t fillWgs = (mapN + 255) / 256;
-                    if (fillWgs > 4096) fillWgs = 4096;
-                    hipLaunchKernelGGL(k_pull_fill, dim3((unsigned)fillWgs), dim3(256), 0, stream, map, mapN, dup);
-                    hipLaunchKernelGGL(k_cell_map, dim3((unsigned)((numActive + 255) / 256)), dim3(256), 0, stream, idx,
-                                       numActive, a, map, chain, dup);
-                }
+                launch_cell_map(idx, numActive, a, map, mapN, chain, dup, stream);
                 m.map = map; m.chain = chain; m.dup = dup;
             }
             auto go = [&](auto width) {
@@ -2678,6 +2652,37 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
     else hipLaunchKernelGGL((k_copy_uncovered<1>), grid, dim3(256), 0, stream, ybase, y, owner, c);
     done = true;
     return scatter_from(x, y, ybase, idx, numActive, g, transpose, mode, stream, owner);
+}
+
+size_t scatter_base_grad_workspace_bytes(const Geom& g, int numActive)
+{
+    StripArgs a;
+    int64_t mapN = 0;
+    if (numActive <= 0 || !make_strip_args(g, numActive, pick_vec(g, nullptr, nullptr), false, nullptr, a, mapN)) return 0;
+    return (size_t)mapN * 4 + 16;
+}
+
+hipError_t launch_scatter_base_grad(const float* dy, float* dbase, const int16_t* idx, int numActive, const Geom& g,
+                                    void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done)
+{
+    done = false;
+    const size_t need = scatter_base_grad_workspace_bytes(g, numActive);
+    if (!need || !workspace || workspaceBytes < need || (reinterpret_cast<uintptr_t>(workspace) & 3)) return hipSuccess;
+    StripArgs a;
+    int64_t mapN = 0;
+    const int vec = pick_vec(g, dbase, dy);
+    if (!make_strip_args(g, numActive, vec, false, nullptr, a, mapN)) return hipSuccess;
+    CellMap m{numActive <= STRIP_LIST_MAX, nullptr, nullptr, nullptr};
+    if (!m.list) {
+        int32_t* map = static_cast<int32_t*>(workspace);
+        launch_cell_map(idx, numActive, a, map, mapN, nullptr, map + mapN, stream);
+        m.map = map;
+    }
+    if (vec == 4) launch_strip<4>(nullptr, dy, dbase, idx, false, false, m, a, stream, true);
+    else if (vec == 2) launch_strip<2>(nullptr, dy, dbase, idx, false, false, m, a, stream, true);
+    else launch_strip<1>(nullptr, dy, dbase, idx, false, false, m, a, stream, true);
+    done = true;
+    return hipGetLastError();
 }
 
 hipError_t launch_copy(float* dst, const float* src, size_t count, hipStream_t stream)
