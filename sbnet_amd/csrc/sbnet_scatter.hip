@@ -979,6 +979,13 @@ static bool launch_fixed_scatter(const float* x, float* y, const float* ysrc, co
     return false;
 }
 
+// Whether launch_fixed_scatter has an instance of the tile.
+static bool fixed_tile(const TileArgs& a, int threads)
+{
+    return tile_match<TileFixed<27, 27, 128, 124, 512>>(a, threads) || tile_match<TileFixed<27, 27, 128, 184, 512>>(a, threads) ||
+           tile_match<TileFixed<16, 16, 64, 128, 512>>(a, threads);
+}
+
 // The scatter's half of the tile_choice test hook (kind 2): same `out` fields.
 int scatter_tile_choice(const Geom& g, int numActive, int vec, int32_t* out)
 {
@@ -997,9 +1004,7 @@ int scatter_tile_choice(const Geom& g, int numActive, int vec, int32_t* out)
     out[7] = items > slots ? items : slots;
     out[8] = TILE_LD;
     out[9] = RS - (a.psplit - 1) * a.P;
-    out[10] = vec == 4 &&
-              (tile_match<TileFixed<27, 27, 128, 124, 512>>(a, threads) || tile_match<TileFixed<27, 27, 128, 184, 512>>(a, threads) ||
-               tile_match<TileFixed<16, 16, 64, 128, 512>>(a, threads));
+    out[10] = vec == 4 && fixed_tile(a, threads);
     return 1;
 }
 
@@ -1510,7 +1515,7 @@ __device__ __forceinline__ void cell_enter(const int16_t* __restrict__ idx, int 
 {
     const int64_t slot = cell_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
     if (!chain) {
-        if (slot >= 0) atomicMax(map + slot, ib);
+        if (slot >= 0 && atomicMax(map + slot, ib) >= 0) *dup = 1;
         return;
     }
     int32_t prev = -1;
@@ -1552,7 +1557,7 @@ __global__ __launch_bounds__(1024) void k_cell_map_small(const int16_t* __restri
 template <int CELLS>
 struct StripCells {
     int32_t cur[CELLS], up[CELLS];
-    int32_t several;   // some block of the strip's row of cells is named by more than one row
+    int32_t several;   // some block over the strip is named by more than one row
 };
 
 constexpr int LIST_ROWS = 4;   // rows of the list in flight per thread
@@ -1584,7 +1589,7 @@ __device__ __forceinline__ void strip_cells_of_list(StripCells<CELLS>& q, const 
             if (bh2 == bh) {
                 if (atomicMax(&q.cur[e], (int)j) >= 0) q.several = 1;
             } else if (a.ovH && bh2 == bh - 1) {
-                atomicMax(&q.up[e], (int)j);
+                if (atomicMax(&q.up[e], (int)j) >= 0) q.several = 1;
             }
         }
     }
@@ -1713,7 +1718,31 @@ __device__ __forceinline__ void strip_cells_of_map(const StripArgs& a, const int
 // base.  A product, so that infinities and NaN under a block become NaN, as they do in the product with a stamped-out mask that
 // this replaces (fill with ones, fill a stack with zeros, scatter it, multiply: 125 us at 300x480x256 with 30 % of the 18x18
 // blocks, 443 MB of them the product's).  This pass moves 295 MB: 46 us there, 6.4 TB/s.
-constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2, STRIP_MASK = 3;
+// STRIP_SUM: y = 0 + the blocks over a pixel, in list order, without a base: the gradient of the gather (NHWC stack).
+// STRIP_ZERO: zeros where no block lies, and nothing else; the tiles of the same launch sum up the rest, unless the list names
+// a block twice, which they cannot: then the strips sum up everything (stack of either layout).
+constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2, STRIP_MASK = 3, STRIP_SUM = 4, STRIP_ZERO = 5;
+
+// 0 + the values in ascending order of their list positions, those with position -1 being +0 (sum_of_pixel, for four).
+template <typename T>
+__device__ __forceinline__ T sum_of_four(int32_t p0, T a, int32_t p1, T b, int32_t p2, T c, int32_t p3, T d, const T& zero)
+{
+    if ((int)(p0 >= 0) + (int)(p1 >= 0) + (int)(p2 >= 0) + (int)(p3 >= 0) >= 2) {
+        auto cx = [](int32_t& p, T& x, int32_t& q, T& y) {
+            const bool sw = p > q;
+            const int32_t t0 = sw ? q : p, t1 = sw ? p : q;
+            const T x0 = sw ? y : x, y0 = sw ? x : y;
+            p = t0; q = t1; x = x0; y = y0;
+        };
+        cx(p0, a, p1, b);
+        cx(p2, c, p3, d);
+        cx(p0, a, p2, c);
+        cx(p1, b, p3, d);
+        cx(p1, b, p2, c);
+        return vadd(vadd(vadd(vadd(zero, a), b), c), d);
+    }
+    return vadd(vadd(vadd(a, b), c), d);
+}
 
 template <int VEC, int OP, bool PLANAR, bool LIST, bool OVER, int CELLS>
 __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const float* __restrict__ ybase,
@@ -1735,7 +1764,8 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
     const uint32_t w = pc * a.PX + wl;
     const bool live = wl < a.PX && w < (uint32_t)a.g.W && cv < a.CV;
 
-    const rsrc_t br = make_rsrc(ybase + (int64_t)n * a.imgFloats, a.imgBytes);
+    constexpr bool SUM = OP == STRIP_SUM || OP == STRIP_ZERO;   // (without a base)
+    const rsrc_t br = make_rsrc(SUM ? ybase : ybase + (int64_t)n * a.imgFloats, SUM ? 0u : a.imgBytes);
     const rsrc_t yr = make_rsrc(y + (int64_t)n * a.imgFloats, a.imgBytes);
     uint32_t off[STRIP_ROWS];
 #pragma unroll
@@ -1764,6 +1794,7 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         strip_cells_of_map<OVER>(a, map, id, iw0, cur, up);
     }
     int ib = -1, ibUp = -1;   // the block that wins the lane's pixels among those of this row of cells, of the one above
+    int own = -1, left1 = -1, up0 = -1, up1 = -1;   // the four blocks themselves
     uint32_t sIb = s, sUp = s;
     if (live && r0 < a.g.R) {
         if (s < (uint32_t)a.g.S) ib = cur[iw - iw0];
@@ -1773,6 +1804,7 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
             if (left) ibL = cur[(int)(iw - iw0) - 1];
             if (above && s < (uint32_t)a.g.S) ibUp = up[iw - iw0];
             if (above && left) upL = up[(int)(iw - iw0) - 1];
+            own = ib; left1 = ibL; up0 = ibUp; up1 = upL;
             if (ibL > ib) { ib = ibL; sIb = s + (uint32_t)a.g.V; }
             if (upL > ibUp) { ibUp = upL; sUp = s + (uint32_t)a.g.V; }
         }
@@ -1793,6 +1825,55 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         }
 #pragma unroll
         for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+        return;
+    }
+    if constexpr (SUM) {
+        if (LIST ? cells->several != 0 : *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0) {
+            // the list names a block twice (rare): the whole list, row by row
+#pragma unroll
+            for (int u = 0; u < STRIP_ROWS; ++u) b[u] = vzero<VEC>();
+            const uint32_t count = list_count(a.g, a.blocks);
+            for (uint32_t j = 0; j < count; ++j) {
+                const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
+                const int ss = (int)w - o.w0;
+                if (o.n != (int)n || (unsigned)ss >= (unsigned)a.g.S) continue;
+#pragma unroll
+                for (int u = 0; u < STRIP_ROWS; ++u) {
+                    const int rr = hTop + u - o.h0;
+                    if (off[u] != BUF_OOB && (unsigned)rr < (unsigned)a.g.R)
+                        b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, (int)j, rr, (uint32_t)ss, cv, a));
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+            return;
+        }
+        if constexpr (OP == STRIP_ZERO) {
+#pragma unroll
+            for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, at[u] >= 0 ? BUF_OOB : off[u], vzero<VEC>());
+        } else {
+            vec q[STRIP_ROWS][4];
+            int pos[STRIP_ROWS][4];
+#pragma unroll
+            for (int u = 0; u < STRIP_ROWS; ++u) {
+                const int r = r0 + u;
+                const bool in = off[u] != BUF_OOB, here = in && r < a.g.R, above = in && r + a.g.U < a.g.R;
+                pos[u][0] = here ? own : -1;
+                pos[u][1] = here ? left1 : -1;
+                pos[u][2] = above ? up0 : -1;
+                pos[u][3] = above ? up1 : -1;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {   // (under branches: a wave without such pixels skips the load)
+                    q[u][k] = vzero<VEC>();
+                    if (pos[u][k] >= 0)
+                        q[u][k] = strip_stack_load<VEC, false>(x, pos[u][k], r + (k >= 2 ? a.g.U : 0), s + (k & 1 ? (uint32_t)a.g.V : 0u), cv, a);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < STRIP_ROWS; ++u)
+                buf_store<BUF_NT>(yr, off[u], sum_of_four(pos[u][0], q[u][0], pos[u][1], q[u][1], pos[u][2], q[u][2], pos[u][3], q[u][3],
+                                                          vzero<VEC>()));
+        }
         return;
     }
     if (OP == STRIP_MASK) {
@@ -1970,6 +2051,24 @@ __global__ __launch_bounds__(512) void k_scatter_tiles_and_rest(const float* __r
     } else {
         scatter_strip<VEC, STRIP_COPY, false, LIST, MODE == SCATTER_RANKED_INLINE>(x, ybase, y, idx, map, nullptr, nullptr, s, lds,
                                                                                    &cells, blockIdx.x - a.total);
+    }
+}
+
+// The gather's gradient from a planar stack: tiles that store every covered pixel once (SCATTER_SUM) and strips of zeros, in
+// one launch behind the one that makes the map.
+template <int VEC>
+__global__ __launch_bounds__(512) void k_sum_tiles_and_zeros(const float* __restrict__ x, float* __restrict__ y,
+                                                             const int16_t* __restrict__ idx, TileArgs a, ColorArgs col, StripArgs s)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ uint32_t waveBits[8];
+    __shared__ StripCells<1> cells;
+    if (blockIdx.x < a.total) {
+        if (list_has_repeats(col)) return;
+        const uint32_t ib = fdiv(blockIdx.x, a.dTpb);
+        scatter_planar_tile<VEC, SCATTER_SUM, TileRt>(x, y, y, idx, a, col, lds, waveBits, ib, blockIdx.x - ib * a.tpb);
+    } else {
+        scatter_strip<VEC, STRIP_ZERO, true, false, true>(x, nullptr, y, idx, col.map, nullptr, col.dup, s, lds, &cells, blockIdx.x - a.total);
     }
 }
 
@@ -2185,9 +2284,10 @@ __global__ __launch_bounds__(256) void k_copy_uncovered(const float* __restrict_
 
 // Cells that touch the image and the strip geometry; false where the strips do not apply.
 // `planar`: the strips also stage a planar stack through LDS (strip_stage_planar); false where that does not apply.
-// `rest`: threads of a workgroup whose strips only copy, and may split a pixel's channels; 0: STRIP_THREADS, they may not.
+// `rest`: threads of a workgroup whose strips share the launch with tiles, and may split a pixel's channels; 0: STRIP_THREADS,
+// they may not.  `flat`: for copy_strip_flat.
 static bool make_strip_args(const Geom& g, int numActive, int vec, bool planar, const float* x, StripArgs& a, int64_t& mapN,
-                            int rest = 0)
+                            int rest = 0, bool flat = false)
 {
     const uint32_t threads = rest ? (uint32_t)rest : (uint32_t)STRIP_THREADS;
     a.ovH = g.U < g.R ? 1 : 0;
@@ -2223,7 +2323,7 @@ static bool make_strip_args(const Geom& g, int numActive, int vec, bool planar, 
     a.PX = threads / a.CVT;
     a.imgBytes = (uint32_t)(a.imgFloats * 4);
     a.nPC = ((uint32_t)g.W + a.PX - 1u) / a.PX;
-    if (rest && vec < 4) {   // (copy_strip_flat)
+    if (flat) {
         a.CT = (uint32_t)g.C;
         a.nCC = 1;
         a.nPC = ((uint32_t)g.W * a.CT + 4u * threads - 1u) / (4u * threads);
@@ -2396,6 +2496,9 @@ hipError_t launch_scatter_owned(const float* x, float* y, const int16_t* idx, in
     return scatter_from(x, y, y, idx, numActive, g, transpose, SCATTER_ASSIGN, stream, owner);
 }
 
+static void launch_sum_by_strips(const float* x, float* y, const int16_t* idx, int numActive, const Geom& g, bool transpose,
+                                 void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done);
+
 // y = zeros, plus the sum of the blocks (the gradient of sparse_gather), for overlapping blocks of which at most 2x2
 // cover a pixel, in one pass over the stack: zeros where no block lies (k_fill_uncovered), then SCATTER_SUM.
 // `done` is false, and nothing launched, where this does not apply; the caller then takes the colour passes.
@@ -2424,7 +2527,10 @@ hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* id
                                      bool transpose, void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done)
 {
     done = false;
-    if (numActive <= 0 || numActive > SUM_MAX_BLOCKS || g.countDev || !(g.U < g.R || g.V < g.S)) return hipSuccess;
+    if (numActive <= 0 || numActive > SUM_MAX_BLOCKS || g.countDev) return hipSuccess;
+    launch_sum_by_strips(x, y, idx, numActive, g, transpose, workspace, workspaceBytes, stream, done);
+    if (done) return hipGetLastError();
+    if (!(g.U < g.R || g.V < g.S)) return hipSuccess;
     // (the other blocks' values are read through one buffer over the whole stack: 32-bit byte offsets)
     if ((int64_t)numActive * g.C * g.R * g.S * 4 >= (1ll << 32) - 16) return hipSuccess;
     const size_t need = scatter_color_workspace_bytes(g, numActive);  // (the map and the flag are its first part)
@@ -2555,7 +2661,7 @@ static bool plan_rest(const Geom& g, int numActive, int vec, RestPlan& p, int64_
     if ((int64_t)g.R * g.S < 4 || !scatter_tile_args(g, numActive, vec, p.a, p.threads, p.lds, grid)) return false;
     if ((g.U < g.R || g.V < g.S) && !rank_inline_applies(g, numActive, true, vec)) return false;
     p.threads = p.threads < 128 ? 128 : p.threads;   // (for the strips)
-    return make_strip_args(g, numActive, vec, false, nullptr, p.s, mapN, p.threads) &&
+    return make_strip_args(g, numActive, vec, false, nullptr, p.s, mapN, p.threads, vec < 4) &&
            (uint64_t)p.a.total + p.s.tiles < (1ull << 31);
 }
 
@@ -2652,6 +2758,64 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
     else hipLaunchKernelGGL((k_copy_uncovered<1>), grid, dim3(256), 0, stream, ybase, y, owner, c);
     done = true;
     return scatter_from(x, y, ybase, idx, numActive, g, transpose, mode, stream, owner);
+}
+
+// The gather's gradient with at most 2x2 blocks over a pixel, for lists short enough that one which names a block twice may be
+// walked row by row: an NHWC stack by strips that read the list, in one launch; a planar one by tiles and strips behind a map.
+// us of all launches, before (map, zeros, sums) / now, MI355X: planar [4,64,64,16] 13.0 / 8.0, [1,100,175,256] 15.6 / 10.2,
+// [4,256,256,64] 25.9 / 20.7, 300x480x256 48.9 / 45.8, 16 images 111.7 / 107.2 (27x27x128, which has a tile of fixed size, 90 /
+// 105: stays); NHWC [4,64,64,16] 12.9 / 5.6, [1,100,175,256] 15.2 / 9.5, 33.6 MB 16.7 / 14.1, 41 MB 18.1 / 16.8; 46 MB 16.6 / 17.1,
+// 50 MB 20.7 / 23.2, 236 MB 74 / 85: in a large tensor the block-driven sums stream better than strips that wait for their
+// look-up.  With vectors of 8 or 4 bytes the strips are the faster at any size: 30 channels, 31 MB 36.2 / 15.7, 126 MB 124 / 55; 15:
+// 19.4 / 11.0; 129, 68 MB 74.6 / 72.0.
+constexpr int64_t SUM_STRIPS_MOST = 40ll << 20;
+
+static void launch_sum_by_strips(const float* x, float* y, const int16_t* idx, int numActive, const Geom& g, bool transpose,
+                                 void* workspace, size_t workspaceBytes, hipStream_t stream, bool& done)
+{
+    done = false;
+    if (numActive > STRIP_LIST_MAX) return;
+    const int vec = pick_vec(g, y, transpose ? nullptr : x);
+    int64_t mapN = 0;
+    auto width = [&](auto go) {
+        if (vec == 4) go(std::integral_constant<int, 4>());
+        else if (vec == 2) go(std::integral_constant<int, 2>());
+        else go(std::integral_constant<int, 1>());
+        done = true;
+    };
+    if (!transpose) {
+        StripArgs a;
+        if ((vec == 4 && (int64_t)g.N * g.H * g.W * g.C * 4 > SUM_STRIPS_MOST) || !make_strip_args(g, numActive, vec, false, nullptr, a, mapN)) return;
+        width([&](auto w) {
+            hipLaunchKernelGGL((k_scatter_strip<decltype(w)::value, STRIP_SUM, false, true, true>), dim3(a.tiles), dim3(STRIP_THREADS), 0,
+                               stream, x, (const float*)nullptr, y, idx, (const int32_t*)nullptr, (const int32_t*)nullptr,
+                               (const int32_t*)nullptr, a);
+        });
+        return;
+    }
+    // (the other blocks' values are read through one buffer over the whole stack: 32-bit byte offsets)
+    if ((int64_t)numActive * g.C * g.R * g.S * 4 >= (1ll << 32) - 16 || (int64_t)g.R * g.S < 4) return;
+    TileArgs a;
+    StripArgs s;
+    int threads;
+    size_t lds;
+    unsigned grid;
+    if (!scatter_tile_args(g, numActive, vec, a, threads, lds, grid) || (vec == 4 && fixed_tile(a, threads))) return;
+    threads = threads < 128 ? 128 : threads;
+    if (!make_strip_args(g, numActive, vec, false, nullptr, s, mapN, threads)) return;
+    if (!workspace || workspaceBytes < (size_t)mapN * 4 + 16 || (reinterpret_cast<uintptr_t>(workspace) & 3) ||
+        (uint64_t)a.total + s.tiles >= (1ull << 31))
+        return;
+    int32_t* map = static_cast<int32_t*>(workspace);
+    launch_cell_map(idx, numActive, s, map, mapN, nullptr, map + mapN, stream);
+    ColorArgs col = NO_ORDER;
+    col.dup = map + mapN;
+    col.map = map;
+    col.bhMin = s.bhMin - s.ovH; col.bwMin = s.bwMin - s.ovW; col.nBH = s.nBH + s.ovH; col.nBW = s.nBW + s.ovW;
+    width([&](auto w) {
+        hipLaunchKernelGGL((k_sum_tiles_and_zeros<decltype(w)::value>), dim3(a.total + s.tiles), dim3(threads), lds, stream, x, y, idx, a,
+                           col, s);
+    });
 }
 
 size_t scatter_base_grad_workspace_bytes(const Geom& g, int numActive)

@@ -68,3 +68,34 @@ def test_long_lists_that_name_blocks_several_times(shape, bs, bo):
             want = orc.sparse_scatter(stack, [1600], idx, base, bs, bs, bo, add=add, transpose=transpose)
             y = sbnet_amd.sparse_scatter(dev(stack), [1600], dev(idx), dev(base), bs, bs, bo, add=add, transpose=transpose)
             np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="transpose %s add %s" % (transpose, add))
+
+
+@pytest.mark.parametrize("M", [1, 1536, 1537])
+@pytest.mark.parametrize("shape,bs,bst,bo", [
+    ((8, 66, 80, 8), (6, 7), (4, 5), (-1, -2)),       # overlap in both directions
+    ((8, 66, 80, 6), (6, 4), (4, 4), (-1, 0)),        # in rows only; 8-byte vectors
+    ((8, 67, 81, 3), (4, 7), (4, 5), (-2, -3)),       # in columns only
+    ((8, 70, 97, 1), (3, 4), (4, 5), (-1, -1)),       # gaps
+    ((8, 140, 135, 132), (4, 5), (6, 7), (0, 0)),     # more channel vectors than a strip of zeros is wide; too large for sums by strips
+], ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("twice", [False, True])
+def test_gather_gradient_by_strips(shape, bs, bst, bo, M, twice):
+    """The sums in list order, with zeros of either sign, exactly; lists that name blocks twice included up to 1536 rows."""
+    from sbnet_amd import ops
+    N, H, W, C = shape
+    rng = np.random.default_rng(M + C)
+    bc = [1 + (H - bo[0] - 1) // bst[0], 1 + (W - bo[1] - 1) // bst[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(-1, bc[0] + 1) for j in range(-1, bc[1])], np.int16)
+    idx = cells[rng.permutation(len(cells))[:M]]
+    if twice:
+        idx[-1] = idx[M // 2]
+    for transpose in (False, True):
+        g = rng.standard_normal((M, C, *bs) if transpose else (M, *bs, C)).astype(np.float32)
+        g.reshape(-1)[::5] = -0.0
+        want = orc.sparse_scatter(g, [M], idx, np.zeros(shape, np.float32), bs, bst, bo, add=True, atomic=True,
+                                  transpose=transpose)
+        got = ops.gather_backward(dev(g), [M], dev(idx), shape, list(bs), list(bst), list(bo), transpose).cpu().numpy()
+        if twice and M > 1536:     # hardware atomics: five terms below 5 in any order, 2 * 4 * 2^-24 * 25
+            np.testing.assert_allclose(got, want, rtol=0, atol=1.2e-5)
+        else:
+            np.testing.assert_array_equal(got.view(np.int32), want.view(np.int32), err_msg="transpose %s" % transpose)
