@@ -362,6 +362,9 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
                           float* const* dw, float* const* dgamma, float* const* dbeta, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* max(x, 0) in place, NaN kept; x 16-byte aligned. */
+int sbnet_relu(float* x, int64_t count, void* stream);
+
 /* Up to three convolution kernels from [kh,kw,C,K] (w_dims[4 * i ...] = kh, kw, C, K) to the [K,C,kh,kw] that the library's
    convolutions and sbnet_bottleneck_grad take, in one launch. */
 int sbnet_kernels_oihw(const float* const* weights, const int32_t* w_dims, float* const* out, int count, void* stream);

@@ -70,6 +70,7 @@ SIGNATURES = {
     "sbnet_bottleneck_grad_workspace_bytes": (_sz, [_i32, _i32p, _i32p]),
     "sbnet_bottleneck_grad": (_int, [_vp, _i32, _i32p, _vp, _vp, _vp, _vp, _vp, _vp, _i32p, _vp, _vp, _vp, _vp, _vp, _sz,
                                      _vp]),
+    "sbnet_relu": (_int, [_vp, ctypes.c_int64, _vp]),
     "sbnet_kernels_oihw": (_int, [_vp, _i32p, _vp, _int, _vp]),
     "sbnet_scratch_acquire": (_vp, [_sz, _vp]),
     "sbnet_shutdown": (_int, []),

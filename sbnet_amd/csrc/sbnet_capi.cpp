@@ -840,8 +840,7 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
         if (needs[i]) t[n++] = sbnet::TransposeArgs{weights[i], at(b.kernel[i]), 1, (uint32_t)c.C, C * (uint32_t)(c.kh * c.kw)};
     }
     t[n++] = sbnet::TransposeArgs{dq, at(b.dz[3]), (uint32_t)num_blocks, (uint32_t)b.c[2].C, (uint32_t)(b.c[2].H * b.c[2].W)};
-    if (needs[2]) SBNET_HIP(sbnet::launch_zero(at(0), b.sumBytes / sizeof(float), s));
-    SBNET_HIP(sbnet::launch_transposes(t, n, s));
+    SBNET_HIP(sbnet::launch_transposes(t, n, s, at(0), needs[2] ? (uint32_t)(b.sumBytes / sizeof(float)) : 0u));
     for (int i = 2; i >= 0 && needs[i]; --i) {
         sbnet::ConvArgs& c = b.c[i];
         c.a = at(b.dz[i + 1]);
@@ -864,6 +863,13 @@ int sbnet_bottleneck_grad(const float* dq, int32_t num_blocks, const int32_t* bs
     if (!dp) return SBNET_OK;
     t[0] = sbnet::TransposeArgs{at(b.dz[0]), dp, (uint32_t)num_blocks, (uint32_t)(b.c[0].Ro * b.c[0].So), (uint32_t)b.c[0].K};
     SBNET_HIP(sbnet::launch_transposes(t, 1, s));
+    return SBNET_OK;
+}
+
+int sbnet_relu(float* x, int64_t count, void* stream)
+{
+    if (count < 0 || (count > 0 && (!x || (reinterpret_cast<uintptr_t>(x) & 15)))) return SBNET_EINVAL_ARG;
+    SBNET_HIP(sbnet::launch_relu(x, (size_t)count, static_cast<hipStream_t>(stream)));
     return SBNET_OK;
 }
 

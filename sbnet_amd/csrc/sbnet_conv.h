@@ -76,15 +76,19 @@ struct WgradArgs {
 size_t wgrad_workspace_bytes(const WgradArgs* w, int count);
 hipError_t launch_wgrad(const WgradArgs* w, int count, void* workspace, hipStream_t stream);
 
+// A ReLU in place; x 16-byte aligned.
+hipError_t launch_relu(float* x, size_t count, hipStream_t stream);
+
 // Up to three kernels [kh,kw,C,K] (dims: four each) to [K,C,kh,kw] in one launch.
 hipError_t launch_kernels(const float* const* from, const int32_t* dims, float* const* to, int count, hipStream_t stream);
 
-// Up to ten matrix transposes [M][A][B] -> [M][B][A] in one launch (block stacks from planar to NHWC and back).
+// Up to ten matrix transposes [M][A][B] -> [M][B][A] in one launch (block stacks from planar to NHWC and back), which clears
+// zeroCount floats besides.
 struct TransposeArgs {
     const float* from;
     float* to;
     uint32_t M, A, B;
 };
-hipError_t launch_transposes(const TransposeArgs* t, int count, hipStream_t stream);
+hipError_t launch_transposes(const TransposeArgs* t, int count, hipStream_t stream, float* zeros = nullptr, uint32_t zeroCount = 0);
 
 }  // namespace sbnet

@@ -797,6 +797,12 @@ struct Residual {
     double momentum, eps;
 };
 
+// The status of a call that is made without the interpreter.
+void checked(int status)
+{
+    TORCH_CHECK(status == SBNET_OK, sbnet_status_string(status), " (hipError_t ", sbnet_last_hip_error(), ")");
+}
+
 // Kernels [kh,kw,C,K] as the library takes them, [K,C,kh,kw].
 void kernels_of(const at::Tensor* const* w, at::Tensor* out)
 {
@@ -818,8 +824,17 @@ void kernels_of(const at::Tensor* const* w, at::Tensor* out)
         from[i] = static_cast<const float*>(w[i]->const_data_ptr());
         to[i] = static_cast<float*>(out[i].data_ptr());
     }
-    const int status = sbnet_kernels_oihw(from, dims, to, 3, stream_of(*w[0]));
-    TORCH_CHECK(status == SBNET_OK, sbnet_status_string(status), " (hipError_t ", sbnet_last_hip_error(), ")");
+    checked(sbnet_kernels_oihw(from, dims, to, 3, stream_of(*w[0])));
+}
+
+void relu(at::Tensor& t)
+{
+    if (!t.is_contiguous() || (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15)) {
+        t.relu_();
+        return;
+    }
+    c10::DeviceGuard guard(t.device());
+    checked(sbnet_relu(static_cast<float*>(t.data_ptr()), t.numel(), stream_of(t)));
 }
 
 struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
@@ -836,7 +851,7 @@ struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
             auto bn = at::_batch_norm_impl_index(z, *gamma[i], *beta[i], r->mean[i], r->var[i], true, r->momentum, r->eps,
                                                  at::globalContext().userEnabledCuDNN());
             at::Tensor& act = std::get<0>(bn);
-            act.relu_();
+            relu(act);
             saved.insert(saved.end(), {z, act, std::get<1>(bn), std::get<2>(bn), kernels[i], *gamma[i]});
             z = at::conv2d(act, kernels[i], {}, at::IntArrayRef({1, 1}));
         }

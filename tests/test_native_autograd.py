@@ -134,3 +134,17 @@ def test_kernels_in_the_librarys_order(shapes):
     for a, b in zip(out, w):
         assert torch.equal(a, b.permute(3, 2, 0, 1))
     assert call(dims, 4) == call(dims, 0) == call(dims * 0, n) == _lib.SBNET_EINVAL_ARG
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 4096, 4099, 100001])
+def test_relu_is_the_librarys(n):
+    from sbnet_amd import _lib
+    x = torch.randn(n, device=DEV)
+    special = torch.tensor([float("nan"), -0.0, 0.0, float("inf"), -float("inf"), -1e-45, 1e-45], device=DEV)[:n]
+    x[n - len(special):] = special
+    want = torch.relu(x)
+    fn = _lib.load().sbnet_relu
+    assert fn(x.data_ptr(), n, ops._stream()) == 0
+    assert torch.equal(x.view(torch.int32), want.view(torch.int32))
+    assert fn(x.data_ptr() + 4, 1, ops._stream()) == _lib.SBNET_EINVAL_ARG
