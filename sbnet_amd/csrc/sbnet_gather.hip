@@ -89,7 +89,12 @@ __global__ __launch_bounds__(256) void k_gather_nhwc(const float* __restrict__ x
 }
 
 // sparse_gather.cc:67-88 with transpose == true: y[ib, c, r, s] = x[n, h0+r, w0+s, c] or 0.
-template <int VEC>
+// RAGGED: 16-byte vectors of a tensor whose channels, four or more, or address make none: gfx950 loads misaligned dwordx4 at the
+// speed of aligned ones, and the vector that would reach past a pixel's last channel starts earlier instead (what it holds twice
+// is written twice).  us, 60 MB tensors, 40 % of the blocks, one float (two with 18 and 30 channels) a lane / this way,
+// MI355X: 14x14 blocks, 5 channels 29.7 / 14.3, 15: 21.0 / 12.6, 18: 18.2 / 13.3, 30: 13.4 / 11.7, 63: 18.0 / 14.2, 129: 14.9 / 11.5; 6x6:
+// 15: 36.0 / 20.3, 63: 33.4 / 20.8; 27x27: 15: 16.8 / 11.9, 129: 12.9 / 10.8.
+template <int VEC, bool RAGGED>
 __device__ __forceinline__ void gather_planar_tile(const float* __restrict__ x, float* __restrict__ y,
                                                    const int16_t* __restrict__ idx, const TileArgs& a, float* lds,
                                                    uint32_t ib, uint32_t rem)
@@ -107,20 +112,21 @@ __device__ __forceinline__ void gather_planar_tile(const float* __restrict__ x, 
 
     vec v[TILE_LD];
     uint32_t pls[TILE_LD];
+    const uint32_t c0l = (tid & ((1u << a.lppLog) - 1u)) * VEC;
+    const uint32_t back = RAGGED ? (uint32_t)max(0, t.c0 + (int)c0l + VEC - a.g.C) : 0u;   // channels that the vector starts earlier
     nhwc_walk<VEC, TileRt>(a, t, o, tid, nthr, [&](int u, uint32_t pl, uint32_t off, uint32_t, uint32_t, uint32_t) {
-        v[u] = buf_load<VEC>(xr, off);
+        v[u] = buf_load<VEC>(xr, !RAGGED || off == BUF_OOB ? off : off - 4u * back);
         pls[u] = pl;
     });
 
     // registers -> LDS, transposing: this thread's VEC channels go to VEC rows, pixel pl to column pl
-    const uint32_t c0l = (tid & ((1u << a.lppLog) - 1u)) * VEC;
 #pragma unroll
     for (int u = 0; u < TILE_LD; ++u) {
-        if (pls[u] < (uint32_t)t.Pn) {
+        if (pls[u] < (uint32_t)t.Pn && (!RAGGED || back < (uint32_t)VEC)) {   // (vectors past the last channel hold nothing)
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
-                const uint32_t c = c0l + k;
-                lds[c * a.Pp + (pls[u] ^ lds_swz(c))] = vget(v[u], k);
+                const uint32_t c = c0l + k - back;
+                if (!RAGGED || (int)c >= 0) lds[c * a.Pp + (pls[u] ^ lds_swz(c))] = vget(v[u], k);
             }
         }
     }
@@ -157,13 +163,13 @@ __device__ __forceinline__ void gather_planar_tile(const float* __restrict__ x, 
     }
 }
 
-template <int VEC>
+template <int VEC, bool RAGGED>
 __global__ __launch_bounds__(512) void k_gather_planar(const float* __restrict__ x, float* __restrict__ y,
                                                        const int16_t* __restrict__ idx, TileArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     for_each_block_of_workgroup(a, a.tpb, [&](uint32_t ib, uint32_t rem) {
-        gather_planar_tile<VEC>(x, y, idx, a, lds, ib, rem);
+        gather_planar_tile<VEC, RAGGED>(x, y, idx, a, lds, ib, rem);
     });
 }
 
@@ -588,15 +594,20 @@ static void gather_dispatch(const float* x, float* y, const int16_t* idx, const 
         }
         // 32 KB tiles: 46.5 us against 52.7 us with 16 KB tiles on the 800x800x128 workload.
         // Planes of fewer than 4 pixels and images or blocks beyond 32-bit byte offsets take the generic kernel.
-        if ((int64_t)g.R * g.S < 4 || !make_tile_args(g, numActive, VEC, a, threads, lds, grid, 32 * 1024)) {
+        const bool ragged = VEC < 4 && g.C >= 4;
+        if ((int64_t)g.R * g.S < 4 || !make_tile_args(g, numActive, ragged ? 4 : VEC, a, threads, lds, grid, 32 * 1024)) {
             const int64_t total = (int64_t)numActive * g.C * g.R * g.S;
             const int64_t wgs = (total + 255) / 256;
             hipLaunchKernelGGL((k_planar_small<SCATTER_ASSIGN, true>), dim3((unsigned)(wgs > 65536 ? 65536 : wgs)),
                                dim3(256), 0, stream, x, y, (const float*)y, idx, g, total, (const int32_t*)nullptr);
             return;
         }
-        hipLaunchKernelGGL(k_gather_planar<VEC>, tile_grid(a.grid2d, a.tpb, numActive, a.total, a.g), dim3(threads), lds,
-                           stream, x, y, idx, a);
+        if (ragged)
+            hipLaunchKernelGGL((k_gather_planar<4, true>), tile_grid(a.grid2d, a.tpb, numActive, a.total, a.g), dim3(threads), lds,
+                               stream, x, y, idx, a);
+        else
+            hipLaunchKernelGGL((k_gather_planar<VEC, false>), tile_grid(a.grid2d, a.tpb, numActive, a.total, a.g), dim3(threads), lds,
+                               stream, x, y, idx, a);
     }
 }
 
