@@ -612,7 +612,7 @@ static void gather_dispatch(const float* x, float* y, const int16_t* idx, const 
 }
 
 // Test hook (sbnet_test_tile_choice): the tile the planar kernels would use for a geometry, without launching.
-// kind 0: k_gather_lines, 1: k_gather_planar, 2: k_scatter_planar.  out = {threads, ldsBytes, P, Pp, psplit, Ct,
+// kind 0: k_gather_lines, 1: k_gather_planar with vectors of vec floats (its ragged launches have 4), 2: k_scatter_planar.  out = {threads, ldsBytes, P, Pp, psplit, Ct,
 // cchunks, vectors or slots per thread needed, vectors or slots per thread available, last split's pixels, fixed
 // instance available}.  Returns 0 when that kernel does not apply to the geometry.
 int tile_choice(int kind, const Geom& g, int numActive, int vec, int yAlignedTo, int32_t* out)
