@@ -31,6 +31,8 @@ namespace {
 
 PyObject* g_check = nullptr;      // ops._check: raises the exception of a status
 PyObject* g_by_layers = nullptr;  // sparse_conv._residual_by_layers: a residual function's gradients through its layers
+PyObject* g_gather_gradient = nullptr;    // autograd.gather_gradient, autograd.scatter_gradients: the gradients by the general
+PyObject* g_scatter_gradients = nullptr;  // wrappers
 
 struct Pair {
     int32_t v[2];
@@ -56,13 +58,18 @@ bool pair_of(PyObject* o, Pair& p)
     return false;
 }
 
+bool has_memory(const at::Tensor& t, at::ScalarType type)
+{
+    return t.defined() && t.scalar_type() == type && t.layout() == at::kStrided && t.has_storage() &&
+           (t.numel() == 0 || t.const_data_ptr());
+}
+
 // A tensor (or parameter) with memory behind it: no subclass and no wrapper of a transform (vmap, grad, fake tensors).
 const at::Tensor* plain_tensor(PyObject* o, at::ScalarType type)
 {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(o);
-    if (!t.defined() || t.scalar_type() != type || t.layout() != at::kStrided || !t.has_storage()) return nullptr;
-    return t.numel() == 0 || t.const_data_ptr() ? &t : nullptr;
+    return has_memory(t, type) ? &t : nullptr;
 }
 
 // A contiguous one on the GPU.
@@ -70,6 +77,12 @@ const at::Tensor* dev_tensor(PyObject* o, at::ScalarType type)
 {
     const at::Tensor* t = plain_tensor(o, type);
     return t && t->is_cuda() && t->is_contiguous() ? t : nullptr;
+}
+
+// The same of a tensor that comes from the autograd engine: a gradient, or what a saved-tensor hook handed back.
+bool is_dev(const at::Tensor& t, at::ScalarType type)
+{
+    return t.defined() && !t.key_set().has(c10::DispatchKey::Python) && has_memory(t, type) && t.is_cuda() && t.is_contiguous();
 }
 
 const at::Tensor* dev_f32(PyObject* o) { return dev_tensor(o, at::kFloat); }
@@ -81,10 +94,12 @@ struct Blocks {
     const int32_t* count;
 };
 
+bool is_list(const at::Tensor& idx) { return idx.dim() == 2 && idx.size(1) == 3 && idx.size(0) <= INT32_MAX; }
+
 bool blocks_of(PyObject* counts, PyObject* list, Blocks& b)
 {
     b.idx = dev_tensor(list, at::kShort);
-    if (!b.idx || b.idx->dim() != 2 || b.idx->size(1) != 3 || b.idx->size(0) > INT32_MAX) return false;
+    if (!b.idx || !is_list(*b.idx)) return false;
     b.count = nullptr;
     if (THPVariable_Check(counts)) {
         const at::Tensor* c = plain_tensor(counts, at::kInt);
@@ -683,19 +698,27 @@ struct Gil {
     ~Gil() { PyGILState_Release(state); }
 };
 
-// A gradient as the kernels take it; an error as the general wrappers raise for tensors without memory of their own.
-at::Tensor plain_grad(const at::Tensor& grad)
+// Whether a backward pass may hand the list it saved to the kernels beside a gradient: what comes back from a saved-tensor
+// hook is whatever the hook made, and a gradient may be a transform's (a batch of them).  Anything else, and anything
+// while modes look on, goes to the general wrappers, which convert, check and raise.
+bool plain_list(const at::Tensor& idx, int32_t M, const at::Tensor& grad)
 {
-    at::Tensor g = grad.contiguous();
-    TORCH_CHECK(g.has_storage() && g.is_cuda() && g.scalar_type() == at::kFloat && (g.numel() == 0 || g.const_data_ptr()),
-                "grad must be a float32 tensor on the GPU");
-    return g;
+    return !c10::impl::TorchDispatchModeTLS::any_modes_set() && is_dev(idx, at::kShort) && is_list(idx) && M <= idx.size(0) &&
+           is_dev(grad, at::kFloat) && grad.dim() == 4 && idx.device() == grad.device();
 }
 
-at::Tensor plain_list(const at::Tensor& idx)
+PyObject* tuple_of(at::IntArrayRef v)
 {
-    at::Tensor t = idx.contiguous();
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kShort, "active_block_indices must be an int16 tensor on the GPU");
+    PyObject* t = PyTuple_New((Py_ssize_t)v.size());
+    if (!t) raise_pending();
+    for (size_t i = 0; i < v.size(); ++i) {
+        PyObject* const o = PyLong_FromLongLong(v[i]);
+        if (!o) {
+            Py_DECREF(t);
+            raise_pending();
+        }
+        PyTuple_SET_ITEM(t, (Py_ssize_t)i, o);
+    }
     return t;
 }
 
@@ -718,9 +741,18 @@ struct GatherFunction : torch::autograd::Function<GatherFunction> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const Gil gil;
-        const at::Tensor idx = plain_list(ctx->get_saved_variables()[0]), g = plain_grad(grads[0]);
+        const at::Tensor idx = ctx->get_saved_variables()[0], g = grads[0].contiguous();
         const std::vector<int64_t> v = ctx->saved_data["sizes"].toIntVector();
-        return {run_gather_grad(g, idx, (int32_t)v[0], v.data() + 7, pair_at(v, 1), pair_at(v, 3), pair_at(v, 5), (int)v[11]), at::Tensor()};
+        const int32_t M = (int32_t)v[0];
+        const Pair bs = pair_at(v, 1);
+        if (plain_list(idx, M, g) && is_stack(g, M, v[10], bs, v[11]))
+            return {run_gather_grad(g, idx, M, v.data() + 7, bs, pair_at(v, 3), pair_at(v, 5), (int)v[11]), at::Tensor()};
+        THPObjectPtr grad(THPVariable_Wrap(g)), list(THPVariable_Wrap(idx)), sizes(tuple_of(v));
+        if (!grad || !list) raise_pending();
+        THPObjectPtr got(PyObject_CallFunctionObjArgs(g_gather_gradient, grad.get(), list.get(), sizes.get(), nullptr));
+        if (!got) raise_pending();
+        TORCH_CHECK(THPVariable_Check(got.get()), "a gradient");
+        return {THPVariable_Unpack(got.get()), at::Tensor()};
     }
 };
 
@@ -737,29 +769,35 @@ struct ScatterFunction : torch::autograd::Function<ScatterFunction> {
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         const Gil gil;
-        const at::Tensor idx = plain_list(ctx->get_saved_variables()[0]), grad = plain_grad(grads[0]);
+        const at::Tensor idx = ctx->get_saved_variables()[0], grad = grads[0].contiguous();
         const std::vector<int64_t> v = ctx->saved_data["sizes"].toIntVector();
         const int32_t M = (int32_t)v[0];
         const Pair bs = pair_at(v, 1), bt = pair_at(v, 3), bo = pair_at(v, 5);
-        const int transpose = v[11] & 1, add = (v[11] >> 1) & 1;
-        at::Tensor blocks, base;
-        if (ctx->needs_input_grad(0)) blocks = run_gather({&grad, {&idx, M, nullptr}, bs, bt, bo, transpose}, nullptr);
-        if (ctx->needs_input_grad(1)) {
-            if (add) base = grad;
-            else if (!(at::GradMode::is_enabled() && grad.requires_grad())) base = run_base_grad(grad, idx, M, bs, bt, bo);
-            if (!base.defined()) {   // a graph of the gradients is asked for, or a geometry that the one pass does not take
-                at::Tensor stamp;
-                {
-                    at::AutoGradMode off(false);
-                    stamp = at::ones_like(grad);
-                    const int64_t C = v[10], R = bs.v[0], S = bs.v[1];
-                    const at::Tensor zeros = transpose ? at::zeros({v[12], C, R, S}, grad.options()) : at::zeros({v[12], R, S, C}, grad.options());
-                    run_scatter({&zeros, &stamp, {&idx, M, nullptr}, bs, bt, bo, 0, 0, transpose}, true);
-                }
-                base = grad * stamp;
+        const bool transpose = v[11] & 1, add = v[11] & 2;
+        const bool blocks = ctx->needs_input_grad(0), base = ctx->needs_input_grad(1);
+        if (plain_list(idx, M, grad) && grad.sizes() == at::IntArrayRef(v.data() + 7, 4)) {
+            at::Tensor dbase;
+            if (base && add) dbase = grad;
+            else if (base && !(at::GradMode::is_enabled() && grad.requires_grad())) dbase = run_base_grad(grad, idx, M, bs, bt, bo);
+            if (!base || dbase.defined()) {
+                at::Tensor dblocks;
+                if (blocks) dblocks = run_gather({&grad, {&idx, M, nullptr}, bs, bt, bo, transpose}, nullptr);
+                return {dblocks, dbase, at::Tensor()};
             }
         }
-        return {blocks, base, at::Tensor()};
+        // besides: a graph of the gradients is asked for, or a geometry that the one pass does not take
+        THPObjectPtr g(THPVariable_Wrap(grad)), list(THPVariable_Wrap(idx)), sizes(tuple_of(v));
+        if (!g || !list) raise_pending();
+        THPObjectPtr got(PyObject_CallFunctionObjArgs(g_scatter_gradients, g.get(), list.get(), sizes.get(), blocks ? Py_True : Py_False,
+                                                      base ? Py_True : Py_False, nullptr));
+        if (!got) raise_pending();
+        TORCH_CHECK(PyTuple_CheckExact(got.get()) && PyTuple_GET_SIZE(got.get()) == 2, "gradients of two inputs");
+        variable_list out(3);
+        for (int i = 0; i < 2; ++i) {
+            PyObject* const o = PyTuple_GET_ITEM(got.get(), i);
+            if (o != Py_None) out[i] = THPVariable_Unpack(o);
+        }
+        return out;
     }
 };
 
@@ -872,12 +910,12 @@ struct ResidualFunction : torch::autograd::Function<ResidualFunction> {
         variable_list out(11);
         const bool graph = at::GradMode::is_enabled();
         if (!graph) {
-            const at::Tensor dq = plain_grad(grads[0]);
+            const at::Tensor dq = grads[0].contiguous();
             const at::Tensor* t[18];
-            bool plain = dq.dim() == 4;
+            bool plain = !c10::impl::TorchDispatchModeTLS::any_modes_set() && is_dev(dq, at::kFloat) && dq.dim() == 4;
             for (int i = 0; i < 18; ++i) {
                 t[i] = &saved[i];
-                plain = plain && saved[i].is_cuda() && saved[i].scalar_type() == at::kFloat && saved[i].is_contiguous() && saved[i].has_storage();
+                plain = plain && is_dev(saved[i], at::kFloat);
             }
             at::Tensor res[10];
             if (plain && run_bottleneck_grad(&dq, t, wanted, res)) {
@@ -1009,6 +1047,17 @@ PyObject* set_by_layers(PyObject*, PyObject* f)
     Py_RETURN_NONE;
 }
 
+// set_gradients(gather_gradient, scatter_gradients)
+PyObject* set_gradients(PyObject* const* a)
+{
+    PyObject** const at[2] = {&g_gather_gradient, &g_scatter_gradients};
+    for (int i = 0; i < 2; ++i) {
+        Py_INCREF(a[i]);
+        Py_XSETREF(*at[i], a[i]);
+    }
+    Py_RETURN_NONE;
+}
+
 template <typename F>
 PyCFunction fast(F f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)); }
 
@@ -1032,6 +1081,7 @@ PyMethodDef methods[] = {
     {"has_workspaces", has_workspaces, METH_NOARGS, nullptr},
     {"set_check", set_check, METH_O, nullptr},
     {"set_by_layers", set_by_layers, METH_O, nullptr},
+    {"set_gradients", fast(entry<set_gradients, 2>), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

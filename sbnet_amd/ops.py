@@ -47,8 +47,10 @@ _native = None
 
 def _load_native():
     global _native
+    from . import autograd
     module = _lib.native()
     module.set_check(_check)
+    module.set_gradients(autograd.gather_gradient, autograd.scatter_gradients)
     _native = module
     return module
 

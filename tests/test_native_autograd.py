@@ -86,6 +86,74 @@ def test_hooks_of_saved_tensors_see_the_list():
     assert torch.equal(got, want + y.detach())
 
 
+def scatter_native(x, q, idx, cnt, add=True):
+    return sbnet_amd.sparse_scatter(q, cnt, idx, x, BS, BT, BO, add=add, atomic=True)
+
+
+def scatter_python(x, q, idx, cnt, add=True):
+    return SparseScatterFunction.apply(q, cnt, idx, x, BS, BT, BO, add, True, False)
+
+
+def gather_native(x, q, idx, cnt):
+    return sbnet_amd.sparse_gather(x, cnt, idx, BS, BT, BO)
+
+
+def gather_python(x, q, idx, cnt):
+    return SparseGatherFunction.apply(x, cnt, idx, BS, BT, BO, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [gather_native, gather_python, scatter_native, scatter_python])
+@pytest.mark.parametrize("change,error,text", [
+    (lambda t: t[:3].clone(), ops.InvalidArgument, "outside the block list of 3 rows"),
+    (lambda t: t[:, :2].clone(), ops.InvalidArgument, "must have shape"),
+    (lambda t: t.view(-1), ops.InvalidArgument, "must have shape"),
+    (lambda t: t.int(), TypeError, "int16 tensor on the GPU"),
+    (lambda t: t.cpu(), TypeError, "int16 tensor on the GPU"),
+], ids=["shorter", "narrower", "flat", "int32", "cpu"])
+def test_a_list_that_a_hook_hands_back_otherwise_is_refused(op, change, error, text):
+    x, q, idx, cnt = make()
+    q.requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, change):
+        y = op(x.requires_grad_(), q, idx, cnt)
+    with pytest.raises(error, match=text):
+        torch.autograd.grad(y.sum(), [x] if "gather" in op.__name__ else [x, q])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [scatter_native, scatter_python])
+def test_a_batch_of_gradients_passes_through_an_adds_base(op):
+    """The base's gradient of an add is the gradient itself, whatever tensor that is."""
+    x, q, idx, cnt = make()
+    y = op(x.requires_grad_(), q, idx, cnt)
+    dy = torch.randn(3, *y.shape, device=DEV)
+    got, = torch.autograd.grad(y, x, dy, is_grads_batched=True)
+    assert torch.equal(got, dy)
+
+
+@pytest.mark.gpu
+def test_modes_of_the_backward_pass_look_on():
+    """What runs under a mode is left to the general wrappers, whose results are the same."""
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    x, q, idx, cnt = make()
+    x.requires_grad_()
+    q.requires_grad_()
+    for op, leaves in ((gather_native, [x]), (scatter_native, [x, q]), (lambda *a: scatter_native(*a, add=False), [x, q])):
+        y = op(x, q, idx, cnt)
+        want = torch.autograd.grad(y, leaves, y.detach(), retain_graph=True)
+        with Mode():
+            got = torch.autograd.grad(y, leaves, y.detach())
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    assert torch.ops.aten.empty.memory_format in seen   # (the general wrapper's own results)
+
+
 @pytest.mark.gpu
 def test_what_looks_on_or_transforms_goes_to_the_functions_in_python():
     x, q, idx, cnt = make()
