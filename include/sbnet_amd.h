@@ -246,24 +246,28 @@ size_t sbnet_sparse_scatter_workspace_bytes(int32_t num_active, const int64_t* y
  *               those are comes from one small extra launch that compares the blocks of the list pairwise (at
  *               most 2x2 blocks over a pixel and at most 4096 blocks; in-place op), or else from an owner map
  *               (one int32 per pixel: the last listed block that covers it) built by two extra launches.
- *               (1) sbnet_sparse_scatter with atomic=0 and blocks that do not overlap (bstride >= bsize): y is
- *               built in one pass over its bytes instead of "copy ybase, scatter on top".  One or two small
- *               launches put an inverse map (block position -> list position) into the scratch; one streaming kernel
- *               then walks y in row order, reads ybase where the result needs it (all of it for an add, the
+ *               (1) sbnet_sparse_scatter with atomic=0 and at most 2x2 blocks over a pixel: y is
+ *               built in one pass over its bytes instead of "copy ybase, scatter on top": one streaming kernel
+ *               walks y in row order, reads ybase where the result needs it (all of it for an add, the
  *               uncovered pixels for a plain write), reads the block stack where a block covers the pixel and
- *               writes y once.  Same y, every byte moved once.  A list that names a block several times gets
- *               the CPU functor's result here as well (the last of the rows wins a plain write, an add sums
- *               all of them in list order).  A planar stack (transpose=1) is staged through LDS by the same
+ *               writes y once.  Which block lies where its workgroups read from the list itself, or, for longer lists
+ *               (1536 blocks) and some large launches, from an inverse map (block position -> list position) that one or
+ *               two small launches put into the scratch first.  A list that names a block several times gets
+ *               the CPU functor's result (the last of the rows wins a plain write, an add sums
+ *               all of them in list order).  A planar stack (transpose=1) of blocks that do not overlap is staged
+ *               through LDS by the same
  *               kernel when bsize[1] and bstride[1] are multiples of 4, bstride[1] divides the kernel's strip
  *               width (256 channel vectors, i.e. 32 pixels at 32 channels or more) and boffset[1] is a
  *               multiple of bstride[1]; other planar geometries whose blocks tile the plane (bsize == bstride,
  *               cells of 4 KB or more) are built by one launch over the cells of the block grid (a cell with a
- *               block from the stack, an empty cell from ybase; exact for repeated rows as well); the remaining
- *               planar geometries take two passes once the blocks cover 16 MB (copy of the uncovered pixels,
- *               then the scatter kernel, which reads ybase where it adds), and copy-then-scatter below that:
- *               in these two cases rows that name the same block race as they do in the reference's GPU
- *               kernels.  Overlapping plain writes (add=0, bstride < bsize) from
- *               16 MB of blocks on use the owner map of (0) as their coverage record in the same way.
+ *               block from the stack, an empty cell from ybase); the remaining
+ *               planar geometries by one launch that scatters the blocks as tiles, each pixel by one
+ *               of the list's rows, and copies what no block covers in strips; all of these are exact for repeated rows.
+ *               Left to copy-then-scatter, where rows that name the same block race as they do in the reference's GPU
+ *               kernels: NHWC stacks of more than 256 channel vectors a pixel, images of 2^30 floats and more, planar
+ *               blocks of fewer than 4 pixels, and, of those remaining planar geometries, blocks of less
+ *               than 16 MB where the map would be needed.  Overlapping plain writes (add=0, bstride < bsize) that the one
+ *               pass does not take use, from 16 MB of blocks on, the owner map of (0) as their coverage record.
  *               (2) add=1, atomic=1: with it the overlapping adds need no atomics:
  *               - transpose=0 and at most 2x2 blocks per pixel: each pixel is summed by one owner in ascending
  *                 block-list order, bit-identical to the reference's sequential CPU functor;

@@ -246,6 +246,14 @@ constexpr int RANK_ROWS_PER_THREAD = 2;   // rows of the list fetched per thread
 // adds all of its pixels with hardware atomics onto zeros (k_fill_uncovered clears everything in that case).
 constexpr int SCATTER_SUM = 7;  // kernel-side mode of sbnet_sparse_gather_grad
 
+// Tiles of blocks that do not overlap, written onto a copy of the base that the same launch makes: every pixel is written by
+// one workgroup, so a block that several rows of the list name is one row's to write.  A workgroup finds the other rows by
+// comparing its own with the list while the tile's loads are in flight (LISTED), or by the map of the cells (MAPPED).  Plain
+// writes: the row listed last.  Adds: the row listed last, or the head of the cell's chain, sums up all rows of the block in
+// list order (sparse_gather.cc:105-129).
+constexpr int SCATTER_ASSIGN_LISTED = 8, SCATTER_ADD_LISTED = 9;    // kernel-side modes of the copying scatter
+constexpr int SCATTER_ASSIGN_MAPPED = 10, SCATTER_ADD_MAPPED = 11;
+
 struct ColorArgs {
     int kh, kw, pass;
     const int32_t* dup;
@@ -265,6 +273,7 @@ struct ColorArgs {
     const int32_t* perm;
     const int32_t* counts;
     int permStride;
+    const int32_t* chain;  // SCATTER_ADD_MAPPED: see k_cell_map
 };
 
 // Position `pos` of a colour pass's launch -> position in the block list, false when the pass has no such block.
@@ -411,6 +420,31 @@ __device__ __forceinline__ bool list_has_repeats(const ColorArgs& col)
 {
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
     return *(const_i32_ptr)(reinterpret_cast<uintptr_t>(col.dup)) != 0;
+}
+
+// The map's entry for the block's cell, -1 for a block that lies over no cell of the image.
+__device__ __forceinline__ int32_t cell_head(const ColorArgs& col, const BlockOrigin& o)
+{
+    typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
+    const int ih = o.bh - col.bhMin, iw = o.bw - col.bwMin;
+    if (!o.valid || (unsigned)ih >= (unsigned)col.nBH || (unsigned)iw >= (unsigned)col.nBW) return -1;
+    return ((const_i32_ptr)(reinterpret_cast<uintptr_t>(col.map)))[((int64_t)o.n * col.nBH + ih) * col.nBW + iw];
+}
+
+// The row that follows in a cell's chain, -1 at its end (scalar loads: an earlier launch made the chains).
+__device__ __forceinline__ int32_t chain_next(const int32_t* chain, int32_t row)
+{
+    typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
+    return ((const_i32_ptr)(reinterpret_cast<uintptr_t>(chain)))[row];
+}
+
+// The smallest row of a cell's chain behind `prev`, 0x7fffffff where there is none.
+__device__ __forceinline__ int32_t next_in_chain(const int32_t* chain, int32_t head, int32_t prev)
+{
+    int32_t next = 0x7fffffff;
+    for (int32_t q = head; q >= 0; q = chain_next(chain, q))
+        if (q > prev && q < next) next = q;
+    return next;
 }
 
 // True when this launch has nothing to do for the block; `atomics` tells how to add otherwise.
@@ -645,6 +679,28 @@ __device__ __forceinline__ void list_row_unpack(const ListRow& row, int& n, int&
     n = (int)(int16_t)(nb & 0xffffu);
     bh = (int)(int16_t)(nb >> 16);
     bw = (int)(int16_t)(row.shift ? row.w.y >> 16 : row.w.y & 0xffffu);
+}
+
+// f(j) for the rows j of the list that `is(n, bh, bw)` holds for, in list order; for whole waves, each of which walks the
+// list by itself: 256 rows at a time, four a lane.
+template <typename IS, typename F>
+__device__ __forceinline__ void for_rows_of_list(const int16_t* idx, uint32_t count, IS is, F f)
+{
+    constexpr uint32_t UNR = 4;
+    const uint32_t lane = threadIdx.x & 63u;
+    const ListRows lr = list_rows(idx, count);
+    for (uint32_t j0 = 0; j0 < count; j0 += 64u * UNR) {
+        ListRow rows[UNR];
+#pragma unroll
+        for (uint32_t u = 0; u < UNR; ++u) rows[u] = list_row_load(lr, j0 + u * 64u + lane, j0 + u * 64u + lane < count);
+#pragma unroll
+        for (uint32_t u = 0; u < UNR; ++u) {
+            int n, bh, bw;
+            list_row_unpack(rows[u], n, bh, bw);
+            uint64_t found = __ballot(j0 + u * 64u + lane < count && is(n, bh, bw));
+            for (; found != 0ull; found &= found - 1ull) f(j0 + u * 64u + (uint32_t)__builtin_ctzll(found));
+        }
+    }
 }
 
 template <int AUX> __device__ __forceinline__ void buf_store(rsrc_t r, uint32_t off, const f4& v)

@@ -290,6 +290,12 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     const uint32_t slots = (uint32_t)t.ctEff * vpr;
     // SCATTER_RANKED_INLINE: the rows listed after this block, RANK_ROWS_PER_THREAD per thread, fetched behind the
     // tile's own loads (loads return in order, so they are there when the tile's data is)
+    // (SCATTER_ADD_LISTED: all rows)
+    const uint32_t firstRow = MODE == SCATTER_ADD_LISTED ? 0u : t.ib + 1u;
+    constexpr bool LISTED = MODE == SCATTER_ASSIGN_LISTED || MODE == SCATTER_ADD_LISTED;
+    constexpr bool MAPPED = MODE == SCATTER_ASSIGN_MAPPED || MODE == SCATTER_ADD_MAPPED;
+    constexpr bool ADD_ONCE = MODE == SCATTER_ADD_LISTED || MODE == SCATTER_ADD_MAPPED;
+    int32_t head = -1;   // of the block's cell, by the map
     ListRow rows[RANK_ROWS_PER_THREAD];
     uint32_t listCount = 0;
     ListRows lr;
@@ -352,12 +358,13 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     };
     auto fetch_rows = [&]() {
         fetch_neighbours();
-        if (MODE != SCATTER_RANKED_INLINE) return;
+        if (MAPPED) head = cell_head(col, origin_of(raw, a.g));
+        if (MODE != SCATTER_RANKED_INLINE && !LISTED) return;
         listCount = list_count(a.g, a.blocks);
         lr = list_rows(idx, listCount);
 #pragma unroll
         for (int u = 0; u < RANK_ROWS_PER_THREAD; ++u) {
-            const uint32_t j = t.ib + 1u + (uint32_t)u * nthr + tid;
+            const uint32_t j = firstRow + (uint32_t)u * nthr + tid;
             rows[u] = list_row_load(lr, j, j < listCount);
         }
     };
@@ -445,7 +452,7 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
         });
     };
     // An add's reads of the base do not depend on the tile: they go out before the barrier, behind the tile's loads.
-    constexpr bool EARLY = MODE == SCATTER_ADD || MODE == SCATTER_COLOR;
+    constexpr bool EARLY = MODE == SCATTER_ADD || ADD_ONCE || MODE == SCATTER_COLOR;
     if (EARLY) {
         walk();
         if (!atomics) {
@@ -453,12 +460,43 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
             for (int u = 0; u < TILE_LD; ++u) cur[u] = buf_load<VEC>(sr, MODE == SCATTER_COLOR && !rmw[u] ? BUF_OOB : offs[u]);
         }
     }
+    bool several = false;   // ADD_ONCE: other rows name the block, and this one sums them up
+    if (MAPPED) {
+        if (head != (int32_t)t.ib) return;   // (the whole workgroup)
+        if (ADD_ONCE && list_has_repeats(col)) several = chain_next(col.chain, head) >= 0;
+    }
+    if (LISTED) {
+        uint32_t bits = 0u;   // 1: a later row names the block, 2: an earlier one
+        auto compare = [&](const ListRow& row, uint32_t j) {
+            int n2, bh2, bw2;
+            list_row_unpack(row, n2, bh2, bw2);
+            if (j < listCount && j != t.ib && n2 == o.n && bh2 == o.bh && bw2 == o.bw) bits |= j > t.ib ? 1u : 2u;
+        };
+#pragma unroll
+        for (int u = 0; u < RANK_ROWS_PER_THREAD; ++u) compare(rows[u], firstRow + (uint32_t)u * nthr + tid);
+        constexpr int AHEAD = 4;
+        for (uint32_t j = firstRow + (uint32_t)RANK_ROWS_PER_THREAD * nthr + tid; j < listCount; j += AHEAD * nthr) {
+            ListRow more[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) more[u] = list_row_load(lr, j + (uint32_t)u * nthr, j + (uint32_t)u * nthr < listCount);
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) compare(more[u], j + (uint32_t)u * nthr);
+        }
+        const uint32_t later = __ballot(bits & 1u) != 0ull ? 1u : 0u, earlier = __ballot(bits & 2u) != 0ull ? 2u : 0u;
+        if ((tid & 63u) == 0u) waveBits[tid >> 6] = later | earlier;
+    }
     lds_barrier();
     if (!EARLY) {
         if (MODE == SCATTER_RANKED_INLINE) {
             for (uint32_t wv = 0; wv < (nthr >> 6); ++wv) rbits |= waveBits[wv];
         }
         if (!summed) walk();
+    }
+    if (LISTED) {
+        uint32_t bits = 0u;
+        for (uint32_t wv = 0; wv < (nthr >> 6); ++wv) bits |= waveBits[wv];
+        if (bits & 1u) return;   // (the whole workgroup)
+        several = (bits & 2u) != 0u;
     }
 #pragma unroll
     for (int u = 0; u < TILE_LD; ++u) {
@@ -474,10 +512,31 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     if (MODE == SCATTER_OWNED) {
 #pragma unroll
         for (int u = 0; u < TILE_LD; ++u) buf_store<BUF_NT>(yr, own[u] == (int32_t)t.ib ? offs[u] : BUF_OOB, w[u]);
-    } else if (MODE == SCATTER_ASSIGN || MODE == SCATTER_RANKED || MODE == SCATTER_RANKED_INLINE) {
+    } else if (MODE == SCATTER_ASSIGN || MODE == SCATTER_RANKED || MODE == SCATTER_RANKED_INLINE || MODE == SCATTER_ASSIGN_LISTED ||
+               MODE == SCATTER_ASSIGN_MAPPED) {
 #pragma unroll
         for (int u = 0; u < TILE_LD; ++u) buf_store<BUF_NT>(yr, offs[u], w[u]);
-    } else if (MODE == SCATTER_ADD || (MODE == SCATTER_COLOR && !atomics)) {
+    } else if (ADD_ONCE && several) {
+        // (rare) the base plus the block's rows, one after the other
+        auto add_row = [&](uint32_t j) {
+            const float* __restrict__ src = x + ((int64_t)j * G::C(a) + t.c0 + c0l) * RS + t.p0;
+#pragma unroll
+            for (int u = 0; u < TILE_LD; ++u) {
+                if (offs[u] == BUF_OOB) continue;
+#pragma unroll
+                for (int k = 0; k < VEC; ++k) vset(cur[u], k, vget(cur[u], k) + src[(int64_t)k * RS + pls[u]]);
+                __builtin_amdgcn_sched_barrier(0);   // (one pixel's loads at a time: registers that this rare way would cost all tiles)
+            }
+        };
+        if (LISTED) {
+            for_rows_of_list(idx, listCount, [&](int n2, int bh2, int bw2) { return n2 == o.n && bh2 == o.bh && bw2 == o.bw; }, add_row);
+        } else {
+            for (int32_t j = next_in_chain(col.chain, (int32_t)t.ib, -1); j != 0x7fffffff; j = next_in_chain(col.chain, (int32_t)t.ib, j))
+                add_row((uint32_t)j);
+        }
+#pragma unroll
+        for (int u = 0; u < TILE_LD; ++u) buf_store<BUF_NT>(yr, offs[u], cur[u]);
+    } else if (MODE == SCATTER_ADD || ADD_ONCE || (MODE == SCATTER_COLOR && !atomics)) {
 #pragma unroll
         for (int u = 0; u < TILE_LD; ++u) buf_store<BUF_NT>(yr, offs[u], vadd(cur[u], w[u]));
     } else if (MODE == SCATTER_SUM && !atomics) {
@@ -2031,7 +2090,8 @@ __device__ __forceinline__ void copy_strip_flat(const float* __restrict__ ybase,
 
 // Planar stack of a geometry that the strips do not stage (18x18 blocks at an odd offset: 72-byte pieces at 8-byte
 // alignment): the tiles of the listed blocks, which read the stack along its planes, and strips that copy what no block
-// covers, in one launch.  MODE: of the tiles; SCATTER_RANKED_INLINE where blocks overlap.
+// covers, in one launch.  MODE: of the tiles, which write every pixel once whatever the list names: SCATTER_RANKED_INLINE
+// where blocks overlap, else SCATTER_ASSIGN_LISTED / SCATTER_ADD_LISTED, or with a map SCATTER_ASSIGN_MAPPED / SCATTER_ADD_MAPPED.
 constexpr int REST_CELLS = 512 + 2;
 
 template <int VEC, int MODE, bool LIST>
@@ -2636,7 +2696,18 @@ static bool plan_cells(const Geom& g, int numActive, int vec, const StripArgs& s
     return true;
 }
 
-static const ColorArgs NO_ORDER{1, 1, 0, nullptr, nullptr, nullptr, 0, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0};
+static const ColorArgs NO_ORDER{1, 1, 0, nullptr, nullptr, nullptr, 0, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0, nullptr};
+
+// The same with the cells' map, and the chains of rows that name one cell.
+static ColorArgs order_by_map(const StripArgs& s, const int32_t* map, const int32_t* chain, const int32_t* dup)
+{
+    ColorArgs col = NO_ORDER;
+    col.dup = dup;
+    col.map = map;
+    col.chain = chain;
+    col.bhMin = s.bhMin - s.ovH; col.bwMin = s.bwMin - s.ovW; col.nBH = s.nBH + s.ovH; col.nBW = s.nBW + s.ovW;
+    return col;
+}
 
 template <int VEC>
 static void launch_cells(const float* x, const float* ybase, float* y, const int16_t* idx, bool add, const CellMap& m,
@@ -2647,7 +2718,10 @@ static void launch_cells(const float* x, const float* ybase, float* y, const int
     else m.list ? go(k_scatter_cells<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_cells<VEC, SCATTER_ASSIGN, false>);
 }
 
-// Tiles of the listed blocks and strips of what they leave, in one launch (k_scatter_tiles_and_rest).
+// Tiles of the listed blocks and strips of what they leave, in one launch (k_scatter_tiles_and_rest).  That every tile of
+// blocks with gaps looks for other rows of its block costs 0.3 us at 300x480x256 (49.3 / 49.5), 1 at [4,400,400,128] with
+// 1400 or 2000 blocks (119.6 / 120.5), nothing where the blocks are added (58.8 / 58.4, 147 / 147, 162 / 162), and 0.5 of 10 us
+// where the tiles are small: [3,301,203,15], 781 blocks.
 struct RestPlan {
     TileArgs a;
     StripArgs s;
@@ -2669,10 +2743,11 @@ template <int VEC>
 static void launch_rest(const float* x, const float* ybase, float* y, const int16_t* idx, bool add, const CellMap& m,
                         const RestPlan& p, hipStream_t stream)
 {
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.a.total + p.s.tiles), dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, p.a, NO_ORDER, p.s); };
-    if (add) m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD, false>);
+    const ColorArgs col = m.list ? NO_ORDER : order_by_map(p.s, m.map, m.chain, m.dup);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.a.total + p.s.tiles), dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, p.a, col, p.s); };
+    if (add) m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD_LISTED, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ADD_MAPPED, false>);
     else if (p.s.ovH || p.s.ovW) m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_RANKED_INLINE, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_RANKED_INLINE, false>);
-    else m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN, false>);
+    else m.list ? go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN_LISTED, true>) : go(k_scatter_tiles_and_rest<VEC, SCATTER_ASSIGN_MAPPED, false>);
 }
 
 // Lists up to here are read by every workgroup of the one-pass kernels; longer ones go through a map, one or two launches
@@ -2808,10 +2883,7 @@ static void launch_sum_by_strips(const float* x, float* y, const int16_t* idx, i
         return;
     int32_t* map = static_cast<int32_t*>(workspace);
     launch_cell_map(idx, numActive, s, map, mapN, nullptr, map + mapN, stream);
-    ColorArgs col = NO_ORDER;
-    col.dup = map + mapN;
-    col.map = map;
-    col.bhMin = s.bhMin - s.ovH; col.bwMin = s.bwMin - s.ovW; col.nBH = s.nBH + s.ovH; col.nBW = s.nBW + s.ovW;
+    const ColorArgs col = order_by_map(s, map, nullptr, map + mapN);
     width([&](auto w) {
         hipLaunchKernelGGL((k_sum_tiles_and_zeros<decltype(w)::value>), dim3(a.total + s.tiles), dim3(threads), lds, stream, x, y, idx, a,
                            col, s);

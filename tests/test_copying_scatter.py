@@ -70,6 +70,38 @@ def test_long_lists_that_name_blocks_several_times(shape, bs, bo):
             np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="transpose %s add %s" % (transpose, add))
 
 
+@pytest.mark.parametrize("shape,bs,bst,bo", [
+    ((3, 41, 38, 32), (5, 6), (6, 7), (-1, -2)),       # 16-byte vectors; a list that the workgroups read
+    ((3, 41, 38, 6), (5, 6), (5, 7), (-1, 0)),
+    ((3, 41, 38, 15), (9, 5), (10, 6), (-3, -2)),
+    ((1, 70, 70, 130), (18, 18), (19, 21), (-1, -1)),  # several tiles a block
+    ((4, 116, 119, 112), (5, 5), (6, 6), (-2, 0)),     # 1600 rows or more: a map, and chains of rows
+    ((4, 116, 119, 110), (5, 5), (6, 6), (-2, 0)),
+], ids=lambda v: "x".join(map(str, v)))
+def test_repeated_rows_of_planar_blocks_with_gaps(shape, bs, bst, bo):
+    """Tiles beside strips that copy the rest: the row listed last wins, an add takes all in list order, exactly."""
+    N, H, W, C = shape
+    rng = np.random.default_rng(C)
+    bc = [1 + (H - bo[0] - 1) // bst[0], 1 + (W - bo[1] - 1) // bst[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(-1, bc[0] + 1) for j in range(-1, bc[1])], np.int16)
+    long = N * H * W * C > 4e6
+    M = 1600 if long else len(cells) // 2
+    idx = cells[rng.integers(len(cells), size=M)]
+    idx[0] = idx[1] = idx[M // 2] = idx[-1] = cells[len(cells) // 2]
+    base = rng.standard_normal(shape).astype(np.float32)
+    stack = rng.standard_normal((M, C, *bs)).astype(np.float32)
+    flat = torch.empty(base.size + 1, device=DEV)
+    mis = flat[1:].view(base.shape)
+    mis.copy_(dev(base))
+    for add in (False, True):
+        for count in (M, M - 3):
+            cnt = torch.tensor([count], dtype=torch.int32, device="cpu" if count == M else DEV)
+            want = orc.sparse_scatter(stack, [count], idx, base, bs, bst, bo, add=add, transpose=True)
+            for b in (dev(base), mis):
+                y = sbnet_amd.sparse_scatter(dev(stack), cnt, dev(idx), b, bs, bst, bo, add=add, transpose=True)
+                np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="add %s count %d" % (add, count))
+
+
 @pytest.mark.parametrize("M", [1, 1536, 1537])
 @pytest.mark.parametrize("shape,bs,bst,bo", [
     ((8, 66, 80, 8), (6, 7), (4, 5), (-1, -2)),       # overlap in both directions
