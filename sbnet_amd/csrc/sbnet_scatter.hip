@@ -266,11 +266,12 @@ __global__ __launch_bounds__(256) void k_scatter_nhwc(const float* __restrict__ 
 }
 
 // sparse_gather.cc:103-130 with transpose == true: the block stack is [blocks, C, R, S].
-template <int VEC, int MODE, typename G>
+// KNOWN: the caller has looked for other rows of the block (`several`), and found this one to be the row that writes it.
+template <int VEC, int MODE, typename G, bool KNOWN = false>
 __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x, float* y, const float* ysrc,
                                                     const int16_t* __restrict__ idx, const TileArgs& a,
                                                     const ColorArgs& col, float* lds, uint32_t* waveBits,
-                                                    uint32_t ib, uint32_t rem)
+                                                    uint32_t ib, uint32_t rem, bool several = false)
 {
     typedef typename Vec<VEC>::type vec;
     const uint32_t tid = threadIdx.x, nthr = G::nthr(a);
@@ -292,8 +293,8 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     // tile's own loads (loads return in order, so they are there when the tile's data is)
     // (SCATTER_ADD_LISTED: all rows)
     const uint32_t firstRow = MODE == SCATTER_ADD_LISTED ? 0u : t.ib + 1u;
-    constexpr bool LISTED = MODE == SCATTER_ASSIGN_LISTED || MODE == SCATTER_ADD_LISTED;
-    constexpr bool MAPPED = MODE == SCATTER_ASSIGN_MAPPED || MODE == SCATTER_ADD_MAPPED;
+    constexpr bool LISTED = !KNOWN && (MODE == SCATTER_ASSIGN_LISTED || MODE == SCATTER_ADD_LISTED);
+    constexpr bool MAPPED = !KNOWN && (MODE == SCATTER_ASSIGN_MAPPED || MODE == SCATTER_ADD_MAPPED);
     constexpr bool ADD_ONCE = MODE == SCATTER_ADD_LISTED || MODE == SCATTER_ADD_MAPPED;
     int32_t head = -1;   // of the block's cell, by the map
     ListRow rows[RANK_ROWS_PER_THREAD];
@@ -460,7 +461,7 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
             for (int u = 0; u < TILE_LD; ++u) cur[u] = buf_load<VEC>(sr, MODE == SCATTER_COLOR && !rmw[u] ? BUF_OOB : offs[u]);
         }
     }
-    bool several = false;   // ADD_ONCE: other rows name the block, and this one sums them up
+    // (ADD_ONCE: `several` when other rows name the block, and this one sums them up)
     if (MAPPED) {
         if (head != (int32_t)t.ib) return;   // (the whole workgroup)
         if (ADD_ONCE && list_has_repeats(col)) several = chain_next(col.chain, head) >= 0;
@@ -528,8 +529,8 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
                 __builtin_amdgcn_sched_barrier(0);   // (one pixel's loads at a time: registers that this rare way would cost all tiles)
             }
         };
-        if (LISTED) {
-            for_rows_of_list(idx, listCount, [&](int n2, int bh2, int bw2) { return n2 == o.n && bh2 == o.bh && bw2 == o.bw; }, add_row);
+        if (MODE == SCATTER_ADD_LISTED) {
+            for_rows_of_list(idx, list_count(a.g, a.blocks), [&](int n2, int bh2, int bw2) { return n2 == o.n && bh2 == o.bh && bw2 == o.bw; }, add_row);
         } else {
             for (int32_t j = next_in_chain(col.chain, (int32_t)t.ib, -1); j != 0x7fffffff; j = next_in_chain(col.chain, (int32_t)t.ib, j))
                 add_row((uint32_t)j);
@@ -2139,8 +2140,9 @@ __global__ __launch_bounds__(512) void k_sum_tiles_and_zeros(const float* __rest
 // itself (LIST) or in the map; an active cell is scattered as one tile of scatter_planar_tile (which reads the base
 // where it adds), an empty cell is copied from the base, tile number `rem` of its `tpb` taking every tpb-th part of the
 // cell's row segments.  Every byte of the output is written once and nothing is read twice.  A cell that several rows of
-// the list name takes the one listed last for a plain write; an add builds it element by element, from every row in list
-// order (sparse_gather.cc:105-129; rare).
+// the list name takes the one listed last for a plain write; an add sums them in list order, with that row's tile
+// (sparse_gather.cc:105-129).  us, adds of 204 blocks of 17x17x64 to [4,256,256,64], MI355X: 26.2, with a block named twice 26.4
+// (69.7 where every channel vector searched the list for its rows).
 struct CellArgs {
     int bhMin, bwMin, nBH, nBW;
     uint32_t CV;  // channel vectors per pixel
@@ -2149,12 +2151,9 @@ struct CellArgs {
 
 constexpr int CELL_UNR = 4;
 
-// head: -1, or the cell's row of the list that `chain` goes on from (chain == nullptr: the whole list is searched).
 template <int VEC>
-__device__ __forceinline__ void cell_by_elements(const float* __restrict__ x, const float* __restrict__ ybase,
-                                                 float* __restrict__ y, const int16_t* __restrict__ idx,
-                                                 const int32_t* __restrict__ chain, const TileArgs& a, const CellArgs& c,
-                                                 int head, uint32_t n, int bh, int bw, uint32_t rem)
+__device__ __forceinline__ void copy_cell(const float* __restrict__ ybase, float* __restrict__ y, const TileArgs& a, const CellArgs& c,
+                                          uint32_t n, int bh, int bw, uint32_t rem)
 {
     typedef typename Vec<VEC>::type vec;
     const Geom& g = a.g;
@@ -2166,64 +2165,32 @@ __device__ __forceinline__ void cell_by_elements(const float* __restrict__ x, co
     const uint32_t nthr = blockDim.x, stride = a.tpb * nthr;
     const rsrc_t br = make_rsrc(ybase + (int64_t)n * a.imgFloats, a.imgBytes);
     const rsrc_t yr = make_rsrc(y + (int64_t)n * a.imgFloats, a.imgBytes);
-    if (head < 0) {
-        for (uint32_t e0 = rem * nthr + threadIdx.x; e0 < total; e0 += CELL_UNR * stride) {
-            uint32_t off[CELL_UNR];
-            vec v[CELL_UNR];
+    for (uint32_t e0 = rem * nthr + threadIdx.x; e0 < total; e0 += CELL_UNR * stride) {
+        uint32_t off[CELL_UNR];
+        vec v[CELL_UNR];
 #pragma unroll
-            for (int u = 0; u < CELL_UNR; ++u) {
-                const uint32_t e = e0 + (uint32_t)u * stride;
-                const uint32_t r = e / segV, j = e - r * segV;
-                off[u] = e < total ? ((((uint32_t)hlo + r) * (uint32_t)g.W + (uint32_t)wlo) * c.CV + j) * (uint32_t)(VEC * 4)
-                                   : BUF_OOB;
-                v[u] = buf_load<VEC>(br, off[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < CELL_UNR; ++u) buf_store<BUF_NT>(yr, off[u], v[u]);
+        for (int u = 0; u < CELL_UNR; ++u) {
+            const uint32_t e = e0 + (uint32_t)u * stride;
+            const uint32_t r = e / segV, j = e - r * segV;
+            off[u] = e < total ? ((((uint32_t)hlo + r) * (uint32_t)g.W + (uint32_t)wlo) * c.CV + j) * (uint32_t)(VEC * 4)
+                               : BUF_OOB;
+            v[u] = buf_load<VEC>(br, off[u]);
         }
-        return;
-    }
-    // an add, and several rows of the list name this cell
-    const int64_t plane = (int64_t)g.R * g.S;
-    const int count = (int)list_count(g, a.blocks);
-    for (uint32_t e = rem * nthr + threadIdx.x; e < total; e += stride) {
-        const uint32_t r = e / segV, j = e - r * segV;
-        const uint32_t px = j / c.CV, cv = j - px * c.CV;
-        const uint32_t off = ((((uint32_t)hlo + r) * (uint32_t)g.W + (uint32_t)wlo) * c.CV + j) * (uint32_t)(VEC * 4);
-        const int64_t at = ((int64_t)hlo + r - h0) * g.S + ((int64_t)wlo + px - w0);  // the pixel inside the block's plane
-        vec out = buf_load<VEC>(br, off);
-        int prev = -1;
-        for (;;) {
-            int cur = 0x7fffffff;
-            if (chain) {
-                for (int q = head; q >= 0; q = chain[q])
-                    if (q > prev && q < cur) cur = q;
-            } else {
-                for (int q = prev + 1; q < count && cur == 0x7fffffff; ++q)
-                    if (idx[(size_t)q * 3] == (int)n && idx[(size_t)q * 3 + 1] == bh && idx[(size_t)q * 3 + 2] == bw) cur = q;
-            }
-            if (cur == 0x7fffffff) break;
-            const float* __restrict__ src = x + ((int64_t)cur * g.C + cv * VEC) * plane + at;
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) vset(out, k, vget(out, k) + src[k * plane]);
-            prev = cur;
-        }
-        buf_store<BUF_NT>(yr, off, out);
+        for (int u = 0; u < CELL_UNR; ++u) buf_store<BUF_NT>(yr, off[u], v[u]);
     }
 }
 
 template <int VEC, int MODE, bool LIST>
 __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__ x, const float* ybase, float* y,
-                                                       const int16_t* __restrict__ idx,
-                                                       const int32_t* __restrict__ map,
-                                                       const int32_t* __restrict__ chain,
-                                                       const int32_t* __restrict__ dup, TileArgs a, ColorArgs col,
+                                                       const int16_t* __restrict__ idx, TileArgs a, ColorArgs col,
                                                        CellArgs c)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ uint32_t waveBits[8];
     __shared__ int32_t found[2];   // LIST: the cell's row listed last, number of its rows
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
+    constexpr bool ADD = MODE == SCATTER_ADD_LISTED || MODE == SCATTER_ADD_MAPPED;
     uint32_t cell, rem;
     if (a.grid2d) {
         cell = blockIdx.y;
@@ -2264,18 +2231,14 @@ __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__
         }
         lds_barrier();
         head = __builtin_amdgcn_readfirstlane(found[0]);
-        if (MODE == SCATTER_ADD) several = __builtin_amdgcn_readfirstlane(found[1]) > 1;
+        if (ADD) several = __builtin_amdgcn_readfirstlane(found[1]) > 1;
     } else {
         // (scalar loads: the map was written by an earlier launch and is not written here)
-        head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(map)))[cell];
-        if (MODE == SCATTER_ADD && head >= 0 && *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0)
-            several = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(chain)))[head] >= 0;
+        head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(col.map)))[cell];
+        if (ADD && head >= 0 && list_has_repeats(col)) several = chain_next(col.chain, head) >= 0;
     }
-    if (head >= 0 && !several) {
-        scatter_planar_tile<VEC, MODE, TileRt>(x, y, ybase, idx, a, col, lds, waveBits, (uint32_t)head, rem);
-        return;
-    }
-    cell_by_elements<VEC>(x, ybase, y, idx, LIST ? nullptr : chain, a, c, head, n, bh, bw, rem);
+    if (head >= 0) scatter_planar_tile<VEC, MODE, TileRt, true>(x, y, ybase, idx, a, col, lds, waveBits, (uint32_t)head, rem, several);
+    else copy_cell<VEC>(ybase, y, a, c, n, bh, bw, rem);
 }
 
 struct CoverArgs {
@@ -2713,8 +2676,10 @@ template <int VEC>
 static void launch_cells(const float* x, const float* ybase, float* y, const int16_t* idx, bool add, const CellMap& m,
                          const CellsPlan& p, hipStream_t stream)
 {
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, p.grid, dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, m.chain, m.dup, p.a, NO_ORDER, p.c); };
-    if (add) m.list ? go(k_scatter_cells<VEC, SCATTER_ADD, true>) : go(k_scatter_cells<VEC, SCATTER_ADD, false>);
+    ColorArgs col = NO_ORDER;
+    col.map = m.map; col.chain = m.chain; col.dup = m.dup;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, p.grid, dim3(p.threads), p.lds, stream, x, ybase, y, idx, p.a, col, p.c); };
+    if (add) m.list ? go(k_scatter_cells<VEC, SCATTER_ADD_LISTED, true>) : go(k_scatter_cells<VEC, SCATTER_ADD_MAPPED, false>);
     else m.list ? go(k_scatter_cells<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_cells<VEC, SCATTER_ASSIGN, false>);
 }
 
