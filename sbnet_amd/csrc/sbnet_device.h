@@ -682,24 +682,17 @@ __device__ __forceinline__ void list_row_unpack(const ListRow& row, int& n, int&
 }
 
 // f(j) for the rows j of the list that `is(n, bh, bw)` holds for, in list order; for whole waves, each of which walks the
-// list by itself: 256 rows at a time, four a lane.
+// list by itself, a row a lane.  (For rare ways out of kernels: more rows in flight would cost all of the kernel registers.)
 template <typename IS, typename F>
 __device__ __forceinline__ void for_rows_of_list(const int16_t* idx, uint32_t count, IS is, F f)
 {
-    constexpr uint32_t UNR = 4;
     const uint32_t lane = threadIdx.x & 63u;
     const ListRows lr = list_rows(idx, count);
-    for (uint32_t j0 = 0; j0 < count; j0 += 64u * UNR) {
-        ListRow rows[UNR];
-#pragma unroll
-        for (uint32_t u = 0; u < UNR; ++u) rows[u] = list_row_load(lr, j0 + u * 64u + lane, j0 + u * 64u + lane < count);
-#pragma unroll
-        for (uint32_t u = 0; u < UNR; ++u) {
-            int n, bh, bw;
-            list_row_unpack(rows[u], n, bh, bw);
-            uint64_t found = __ballot(j0 + u * 64u + lane < count && is(n, bh, bw));
-            for (; found != 0ull; found &= found - 1ull) f(j0 + u * 64u + (uint32_t)__builtin_ctzll(found));
-        }
+    for (uint32_t j0 = 0; j0 < count; j0 += 64u) {
+        int n, bh, bw;
+        list_row_unpack(list_row_load(lr, j0 + lane, j0 + lane < count), n, bh, bw);
+        uint64_t found = __ballot(j0 + lane < count && is(n, bh, bw));
+        for (; found != 0ull; found &= found - 1ull) f(j0 + (uint32_t)__builtin_ctzll(found));
     }
 }
 

@@ -1617,14 +1617,14 @@ __global__ __launch_bounds__(1024) void k_cell_map_small(const int16_t* __restri
 template <int CELLS>
 struct StripCells {
     int32_t cur[CELLS], up[CELLS];
-    int32_t several;   // some block over the strip is named by more than one row
+    int32_t several;   // some block among the strip's first `most` cells is named by more than one row
 };
 
 constexpr int LIST_ROWS = 4;   // rows of the list in flight per thread
 
 template <int CELLS>
 __device__ __forceinline__ void strip_cells_of_list(StripCells<CELLS>& q, const int16_t* __restrict__ idx, const StripArgs& a,
-                                                    uint32_t n, int bh, int bw0)
+                                                    uint32_t n, int bh, int bw0, uint32_t most)
 {
     const uint32_t tid = threadIdx.x, nthr = blockDim.x;
     const uint32_t count = list_count(a.g, a.blocks);
@@ -1647,9 +1647,9 @@ __device__ __forceinline__ void strip_cells_of_list(StripCells<CELLS>& q, const 
             const uint32_t e = (uint32_t)(bw2 - bw0);
             if (j >= count || n2 != (int)n || e >= (uint32_t)CELLS) continue;
             if (bh2 == bh) {
-                if (atomicMax(&q.cur[e], (int)j) >= 0) q.several = 1;
+                if (atomicMax(&q.cur[e], (int)j) >= 0 && e < most) q.several = 1;
             } else if (a.ovH && bh2 == bh - 1) {
-                if (atomicMax(&q.up[e], (int)j) >= 0) q.several = 1;
+                if (atomicMax(&q.up[e], (int)j) >= 0 && e < most) q.several = 1;
             }
         }
     }
@@ -1846,8 +1846,11 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
     const uint32_t iw = fdiv(w - pixel0, a.dV), s = w - pixel0 - iw * (uint32_t)a.g.V;
     const uint32_t iw0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)fdiv(pc * a.PX - pixel0, a.dV));
     const int32_t *cur, *up;   // entries of the strip's cells, iw0's first
+    const int bh = (int)band + a.bhMin, bw0 = (int)iw0 + a.bwMin - (OVER ? a.ovW : 0);
+    uint32_t cellCount = 0u;   // (LIST) of the strip, the one on the left included
     if constexpr (LIST) {
-        strip_cells_of_list(*cells, idx, a, n, (int)band + a.bhMin, (int)iw0 + a.bwMin - (OVER ? a.ovW : 0));
+        if (ADD || SUM) cellCount = (uint32_t)((int)fdiv(min(pc * a.PX + a.PX, (uint32_t)a.g.W) - 1u - pixel0, a.dV) + a.bwMin - bw0) + 1u;
+        strip_cells_of_list(*cells, idx, a, n, bh, bw0, cellCount);
         cur = cells->cur + (OVER ? a.ovW : 0);
         up = cells->up + (OVER ? a.ovW : 0);
     } else {
@@ -1889,21 +1892,24 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
     }
     if constexpr (SUM) {
         if (LIST ? cells->several != 0 : *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0) {
-            // the list names a block twice (rare): the whole list, row by row
+            // the list names a block twice (rare): the rows of blocks over the strip, one after the other.  us with no block
+            // named twice / one / eight, 1400 blocks of 10x10x32 on [4,256,256,32]: 17.5 / 23.9 / 23.7
 #pragma unroll
             for (int u = 0; u < STRIP_ROWS; ++u) b[u] = vzero<VEC>();
-            const uint32_t count = list_count(a.g, a.blocks);
-            for (uint32_t j = 0; j < count; ++j) {
+            auto over = [&](int n2, int bh2, int bw2) {
+                return n2 == (int)n && (bh2 == bh || (a.ovH && bh2 == bh - 1)) && (!LIST || (uint32_t)(bw2 - bw0) < cellCount);
+            };
+            for_rows_of_list(idx, list_count(a.g, a.blocks), over, [&](uint32_t j) {
                 const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
                 const int ss = (int)w - o.w0;
-                if (o.n != (int)n || (unsigned)ss >= (unsigned)a.g.S) continue;
+                if ((unsigned)ss >= (unsigned)a.g.S) return;
 #pragma unroll
                 for (int u = 0; u < STRIP_ROWS; ++u) {
                     const int rr = hTop + u - o.h0;
                     if (off[u] != BUF_OOB && (unsigned)rr < (unsigned)a.g.R)
                         b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, (int)j, rr, (uint32_t)ss, cv, a));
                 }
-            }
+            });
 #pragma unroll
             for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
             return;
@@ -1979,18 +1985,19 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         return;
     }
     // An add, and some cell is named by several rows of the list (rare; reduce_mask never produces such a list): the sum of
-    // the rows in list order.
+    // the rows in list order.  us with no block named twice / one / eight, 1400 blocks of 8x8x64 on [4,256,256,64]: 28.0 / 32.6 / 32.6.
     auto add_row = [&](int row) {
 #pragma unroll
-        for (int u = 0; u < STRIP_ROWS; ++u)
+        for (int u = 0; u < STRIP_ROWS; ++u) {
             if (at[u] >= 0) b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, row, r0 + u, s, cv, a));
+            __builtin_amdgcn_sched_barrier(0);   // (one load at a time: registers that this rare way would cost all strips)
+        }
     };
     if constexpr (LIST) {
-        const uint32_t count = list_count(a.g, a.blocks);
-        for (uint32_t j = 0; j < count; ++j) {
-            const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
-            if (o.n == (int)n && o.bh == (int)band + a.bhMin && o.bw == (int)iw + a.bwMin) add_row((int)j);
-        }
+        auto over = [&](int n2, int bh2, int bw2) { return n2 == (int)n && bh2 == bh && (uint32_t)(bw2 - bw0) < cellCount; };
+        for_rows_of_list(idx, list_count(a.g, a.blocks), over, [&](uint32_t j) {
+            if (origin_of(load_triple(idx, j), a.g).bw == (int)iw + a.bwMin) add_row((int)j);
+        });
     } else {   // (the rows of a cell form a linked list)
         int prev = -1;
         while (ib >= 0) {
@@ -2035,7 +2042,7 @@ __device__ __forceinline__ void copy_strip_flat(const float* __restrict__ ybase,
     const uint32_t iw0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)fdiv(fdiv(id.pc * blockDim.x * 4u, a.dCT) - pixel0, a.dV));
     const int32_t *cur, *up;
     if constexpr (LIST) {
-        strip_cells_of_list(*cells, idx, a, id.n, (int)id.band + a.bhMin, (int)iw0 + a.bwMin - (OVER ? a.ovW : 0));
+        strip_cells_of_list(*cells, idx, a, id.n, (int)id.band + a.bhMin, (int)iw0 + a.bwMin - (OVER ? a.ovW : 0), 0u);
         cur = cells->cur + (OVER ? a.ovW : 0);
         up = cells->up + (OVER ? a.ovW : 0);
     } else {
@@ -2684,9 +2691,9 @@ static void launch_cells(const float* x, const float* ybase, float* y, const int
 }
 
 // Tiles of the listed blocks and strips of what they leave, in one launch (k_scatter_tiles_and_rest).  That every tile of
-// blocks with gaps looks for other rows of its block costs 0.3 us at 300x480x256 (49.3 / 49.5), 1 at [4,400,400,128] with
-// 1400 or 2000 blocks (119.6 / 120.5), nothing where the blocks are added (58.8 / 58.4, 147 / 147, 162 / 162), and 0.5 of 10 us
-// where the tiles are small: [3,301,203,15], 781 blocks.
+// blocks with gaps looks for other rows of its block costs little.  us without / with it: [3,301,203,15], 781 blocks of 9x9 10.4 /
+// 10.4; 300x480x256 49.3 / 49.2, add 59.0 / 58.5; [4,400,400,128], 1400 blocks 119.8 / 119.7, add 147.3 / 146.9; by the map, 2000
+// blocks, 119.8 / 121.0, add 162 / 162.
 struct RestPlan {
     TileArgs a;
     StripArgs s;
