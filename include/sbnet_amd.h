@@ -196,8 +196,8 @@ int sbnet_sparse_gather_functor(const float* x, int N, int H, int W, int C, floa
    are written only to the pixels that no block covers, and one pass over the stack writes every other pixel once:
    the block listed last over a pixel fetches the other blocks' values of it and stores 0 + their sum in list order
    + its own.  No atomics: the result is the sequential CPU functor's (sparse_gather.cc:105-129), bit for bit, also
-   for real-valued data and signed zeros, and the same on every call.  A list that names a block twice falls back
-   to hardware atomics onto zeros; deeper overlaps take ceil(R/U)*ceil(S/V) passes of mutually non-overlapping
+   for real-valued data and signed zeros, and the same on every call.  A list of more
+   than 1536 blocks that names one twice falls back to hardware atomics onto zeros; deeper overlaps take ceil(R/U)*ceil(S/V) passes of mutually non-overlapping
    blocks (reproducible, equal to the composition up to fp32 reassociation); without workspace dx is cleared and
    the atomic scatter-add runs on it.  Checks and status codes as sbnet_sparse_scatter_var. */
 int sbnet_sparse_gather_grad(const float* dy, int32_t num_active, const int16_t* active_block_indices, float* dx,

@@ -238,13 +238,16 @@ constexpr int SCATTER_RANKED_INLINE = 6;  // kernel-side mode; callers ask for S
 constexpr int RANK_ROWS_PER_THREAD = 2;   // rows of the list fetched per thread ahead of the tile's LDS phase
 
 // "Zeros plus the sum of the blocks" (the gradient of sparse_gather) in one pass over the stack, for at most 2x2
-// blocks over a pixel: k_fill_uncovered has written zeros where no block lies; every covered pixel is written once,
+// blocks over a pixel: something else writes zeros where no block lies; every covered pixel is written once,
 // by the block listed last among those that cover it (the owner, as in SCATTER_RANKED), which fetches the other
 // blocks' values of that pixel from the stack and adds them up in list order, its own last: 0 + a + b + own, the
 // sequential CPU functor's sum (sparse_gather.cc:105-129), bit for bit, without atomics.  The neighbours' list
-// positions come from the inverse block map.  A list that names a block twice has no such map: every block then
-// adds all of its pixels with hardware atomics onto zeros (k_fill_uncovered clears everything in that case).
-constexpr int SCATTER_SUM = 7;  // kernel-side mode of sbnet_sparse_gather_grad
+// positions come from the inverse block map, which has one row for a block.  Lists that name a block twice:
+// SCATTER_SUM, behind k_fill_uncovered: every block adds all of its pixels with hardware atomics onto zeros
+// (k_fill_uncovered clears everything in that case).  SCATTER_SUM_MARKED, beside strips (STRIP_ZERO): the cells' map holds
+// CELL_REPEATED for such a block, which counts as listed after every row; the strips sum up its pixels, the tiles all others.
+constexpr int SCATTER_SUM = 7, SCATTER_SUM_MARKED = 12;  // kernel-side modes of sbnet_sparse_gather_grad
+constexpr int32_t CELL_REPEATED = 0x40000000;
 
 // Tiles of blocks that do not overlap, written onto a copy of the base that the same launch makes: every pixel is written by
 // one workgroup, so a block that several rows of the list name is one row's to write.  A workgroup finds the other rows by
@@ -376,14 +379,16 @@ __device__ __forceinline__ NeighbourPos neighbour_positions(const ColorArgs& col
     for (int q = 0; q < 9; ++q) {  // (independent loads; a neighbour beyond the map reads the first entry and is masked)
         const int dh = q / 3 - 1, dw = q % 3 - 1;
         const int ih = o.bh + dh - col.bhMin, iw = o.bw + dw - col.bwMin;
-        in[q] = q != 4 && (unsigned)ih < (unsigned)col.nBH && (unsigned)iw < (unsigned)col.nBW;
+        in[q] = (unsigned)ih < (unsigned)col.nBH && (unsigned)iw < (unsigned)col.nBW;
         const int64_t slot = in[q] ? ((int64_t)o.n * col.nBH + ih) * col.nBW + iw : 0;
         other[q] = *(const_i32_ptr)(reinterpret_cast<uintptr_t>(col.map + slot));
     }
     NeighbourPos nb;
-    nb.later = 0u;
+    nb.later = in[4] && other[4] == CELL_REPEATED ? 0x1ffu : 0u;
+    nb.pos[4] = -1;
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
+        if (q == 4) continue;
         const int dh = q / 3 - 1, dw = q % 3 - 1;
         const bool active = in[q] && other[q] >= 0;
         if (active && (uint32_t)other[q] > ib) {

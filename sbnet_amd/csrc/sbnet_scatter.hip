@@ -303,7 +303,8 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     // SCATTER_SUM: the other blocks' values of the pixels that this block sums (three per pixel at most) are fetched
     // behind the tile's own loads as well: the neighbours' list positions (scalar loads), the walk over the tile's
     // pixels, then the loads, all before the first wait for the tile's data.
-    constexpr int NSUM = MODE == SCATTER_SUM ? TILE_LD : 1;
+    constexpr bool SUM = MODE == SCATTER_SUM || MODE == SCATTER_SUM_MARKED;
+    constexpr int NSUM = SUM ? TILE_LD : 1;
     typename Vec<VEC>::type nv[NSUM][3];
     PixelNeighbours pn[NSUM];
     uint32_t offs[TILE_LD], pls[TILE_LD];
@@ -312,9 +313,9 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     bool summed = false;  // offs / pls / pn / nv are set
     const uint32_t c0l = (tid & ((1u << G::lppLog(a)) - 1u)) * VEC;
     auto fetch_neighbours = [&]() {
-        if (MODE != SCATTER_SUM) return;
+        if (!SUM) return;
         const BlockOrigin o = origin_of(raw, a.g);
-        atomics = list_has_repeats(col);
+        atomics = MODE == SCATTER_SUM && list_has_repeats(col);
         if (!o.valid || atomics) return;
         nb = neighbour_positions(col, o, t.ib);
         summed = true;
@@ -328,7 +329,7 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
             if (ranked_out(nb.later, r, sc, a.g)) off = BUF_OOB;  // (a block listed later owns the pixel)
             offs[u] = off;
             pls[u] = pl;
-            const int v = MODE == SCATTER_SUM ? u : 0;
+            const int v = SUM ? u : 0;
             pn[v].pv = pn[v].ph = pn[v].pd = -1;
             nv[v][0] = nv[v][1] = nv[v][2] = vzero<VEC>();
             if (!(anyV || anyH || anyD)) return;
@@ -540,11 +541,11 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
     } else if (MODE == SCATTER_ADD || ADD_ONCE || (MODE == SCATTER_COLOR && !atomics)) {
 #pragma unroll
         for (int u = 0; u < TILE_LD; ++u) buf_store<BUF_NT>(yr, offs[u], vadd(cur[u], w[u]));
-    } else if (MODE == SCATTER_SUM && !atomics) {
+    } else if (SUM && !atomics) {
         // the owner's sum: 0 + the blocks listed before this one, in list order, + its own value
 #pragma unroll
         for (int u = 0; u < TILE_LD; ++u) {
-            const int v = MODE == SCATTER_SUM ? u : 0;
+            const int v = SUM ? u : 0;
             buf_store<BUF_NT>(yr, offs[u], sum_of_pixel(pn[v].pv, nv[v][0], pn[v].ph, nv[v][1], pn[v].pd, nv[v][2], w[u],
                                                        vzero<VEC>()));
         }
@@ -1567,15 +1568,18 @@ __device__ __forceinline__ int64_t cell_slot(const StripArgs& a, int n, int bh, 
 }
 
 // One thread per list row: the row's position goes into its cell.  A cell named by several rows takes the one listed last
-// for plain writes.  For an add (`chain`) it keeps them as a linked list (the map holds the row that arrived last,
+// for plain writes, or a mark (`mark`).  For an add (`chain`) it keeps them as a linked list (the map holds the row that arrived last,
 // chain[row] the one it displaced) and raises `dup`; the main kernel then walks the lists and sums in list order, as
 // the sequential CPU functor does (sparse_gather.cc:105-129).
 __device__ __forceinline__ void cell_enter(const int16_t* __restrict__ idx, int ib, const StripArgs& a, int32_t* map,
-                                           int32_t* chain, int32_t* dup)
+                                           int32_t* chain, int32_t* dup, bool mark)
 {
     const int64_t slot = cell_slot(a, idx[(size_t)ib * 3], idx[(size_t)ib * 3 + 1], idx[(size_t)ib * 3 + 2]);
     if (!chain) {
-        if (slot >= 0 && atomicMax(map + slot, ib) >= 0) *dup = 1;
+        if (slot >= 0 && atomicMax(map + slot, ib) >= 0) {
+            *dup = 1;
+            if (mark) atomicMax(map + slot, CELL_REPEATED);
+        }
         return;
     }
     int32_t prev = -1;
@@ -1588,18 +1592,18 @@ __device__ __forceinline__ void cell_enter(const int16_t* __restrict__ idx, int 
 
 __global__ __launch_bounds__(256) void k_cell_map(const int16_t* __restrict__ idx, int numActive, StripArgs a,
                                                    int32_t* __restrict__ map, int32_t* __restrict__ chain,
-                                                   int32_t* __restrict__ dup)
+                                                   int32_t* __restrict__ dup, bool mark)
 {
     const int ib = (int)(blockIdx.x * 256 + threadIdx.x);
     if (ib >= numActive || (a.g.countDev && ib >= *a.g.countDev)) return;
-    cell_enter(idx, ib, a, map, chain, dup);
+    cell_enter(idx, ib, a, map, chain, dup, mark);
 }
 
 // The cleared map and the list's rows in it by one workgroup, for maps and lists small enough that one workgroup
 // is done in the time a second launch takes to start.
 __global__ __launch_bounds__(1024) void k_cell_map_small(const int16_t* __restrict__ idx, int numActive, StripArgs a,
                                                           int32_t* __restrict__ map, int mapN,
-                                                          int32_t* __restrict__ chain, int32_t* __restrict__ dup)
+                                                          int32_t* __restrict__ chain, int32_t* __restrict__ dup, bool mark)
 {
     const int tid = (int)threadIdx.x;
     for (int i = tid; i < mapN; i += 1024) map[i] = -1;
@@ -1607,7 +1611,7 @@ __global__ __launch_bounds__(1024) void k_cell_map_small(const int16_t* __restri
     __syncthreads();  // (the stores above are complete, and visible to this workgroup's atomics, beyond this point)
     int count = numActive;
     if (a.g.countDev) count = min(count, max(*a.g.countDev, 0));
-    for (int ib = tid; ib < count; ib += 1024) cell_enter(idx, ib, a, map, chain, dup);
+    for (int ib = tid; ib < count; ib += 1024) cell_enter(idx, ib, a, map, chain, dup, mark);
 }
 
 // The listed blocks over one strip's cells, entered into LDS by the strip's own workgroup: `cur` those of the strip's row of
@@ -1779,8 +1783,8 @@ __device__ __forceinline__ void strip_cells_of_map(const StripArgs& a, const int
 // this replaces (fill with ones, fill a stack with zeros, scatter it, multiply: 125 us at 300x480x256 with 30 % of the 18x18
 // blocks, 443 MB of them the product's).  This pass moves 295 MB: 46 us there, 6.4 TB/s.
 // STRIP_SUM: y = 0 + the blocks over a pixel, in list order, without a base: the gradient of the gather (NHWC stack).
-// STRIP_ZERO: zeros where no block lies, and nothing else; the tiles of the same launch sum up the rest, unless the list names
-// a block twice, which they cannot: then the strips sum up everything (stack of either layout).
+// STRIP_ZERO: zeros where no block lies, and sums in list order where one lies that several rows name (planar stack); the
+// tiles of the same launch sum up the rest.
 constexpr int STRIP_ASSIGN = 0, STRIP_ADD = 1, STRIP_COPY = 2, STRIP_MASK = 3, STRIP_SUM = 4, STRIP_ZERO = 5;
 
 // 0 + the values in ascending order of their list positions, those with position -1 being +0 (sum_of_pixel, for four).
@@ -1891,33 +1895,65 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
         return;
     }
     if constexpr (SUM) {
-        if (LIST ? cells->several != 0 : *(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0) {
-            // the list names a block twice (rare): the rows of blocks over the strip, one after the other.  us with no block
-            // named twice / one / eight, 1400 blocks of 10x10x32 on [4,256,256,32]: 17.5 / 23.9 / 23.7
-#pragma unroll
-            for (int u = 0; u < STRIP_ROWS; ++u) b[u] = vzero<VEC>();
-            auto over = [&](int n2, int bh2, int bw2) {
-                return n2 == (int)n && (bh2 == bh || (a.ovH && bh2 == bh - 1)) && (!LIST || (uint32_t)(bw2 - bw0) < cellCount);
-            };
-            for_rows_of_list(idx, list_count(a.g, a.blocks), over, [&](uint32_t j) {
-                const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
-                const int ss = (int)w - o.w0;
-                if ((unsigned)ss >= (unsigned)a.g.S) return;
+        if constexpr (OP == STRIP_ZERO) {
+            if (*(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0) {   // (rare)
+                int heads[4] = {own, left1, up0, up1};
+                int wRare = (int)w, nRare = (int)n;
+                // (keeps the compiler from working any of this out ahead of the branch: 46.0 us at 300x480x256, 45.0 this way)
+                asm volatile("" : "+v"(wRare), "+s"(nRare), "+v"(heads[0]), "+v"(heads[1]), "+v"(heads[2]), "+v"(heads[3]));
+                const bool here = heads[0] == CELL_REPEATED || heads[1] == CELL_REPEATED,
+                           above = heads[2] == CELL_REPEATED || heads[3] == CELL_REPEATED;
+                uint32_t to[STRIP_ROWS];
 #pragma unroll
                 for (int u = 0; u < STRIP_ROWS; ++u) {
-                    const int rr = hTop + u - o.h0;
-                    if (off[u] != BUF_OOB && (unsigned)rr < (unsigned)a.g.R)
-                        b[u] = vadd(b[u], strip_stack_load<VEC, PLANAR>(x, (int)j, rr, (uint32_t)ss, cv, a));
+                    const int r = r0 + u;
+                    to[u] = (here && r < a.g.R) || (above && r + a.g.U < a.g.R) ? off[u] : BUF_OOB;
+                    b[u] = vzero<VEC>();
                 }
-            });
+                if (__ballot(here || above) != 0ull) {
+                    auto over = [&](int n2, int bh2, int) { return n2 == nRare && (bh2 == bh || (a.ovH && bh2 == bh - 1)); };
+                    for_rows_of_list(idx, list_count(a.g, a.blocks), over, [&](uint32_t j) {
+                        const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
+                        const int ss = wRare - o.w0;
+                        if ((unsigned)ss >= (unsigned)a.g.S) return;
 #pragma unroll
-            for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
-            return;
-        }
-        if constexpr (OP == STRIP_ZERO) {
+                        for (int u = 0; u < STRIP_ROWS; ++u) {
+                            const int rr = hTop + u - o.h0;
+                            if (to[u] != BUF_OOB && (unsigned)rr < (unsigned)a.g.R)
+                                b[u] = vadd(b[u], strip_stack_load<VEC, true>(x, (int)j, rr, (uint32_t)ss, cv, a));
+                        }
+                    });
+                }
+#pragma unroll
+                for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, at[u] >= 0 ? to[u] : off[u], b[u]);
+                return;
+            }
 #pragma unroll
             for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, at[u] >= 0 ? BUF_OOB : off[u], vzero<VEC>());
         } else {
+            if (cells->several != 0) {
+                // the list names a block twice (rare): the rows of blocks over the strip, one after the other.  us with no block
+                // named twice / one / eight, 1400 blocks of 10x10x32 on [4,256,256,32]: 17.5 / 23.9 / 23.7
+#pragma unroll
+                for (int u = 0; u < STRIP_ROWS; ++u) b[u] = vzero<VEC>();
+                auto over = [&](int n2, int bh2, int bw2) {
+                    return n2 == (int)n && (bh2 == bh || (a.ovH && bh2 == bh - 1)) && (uint32_t)(bw2 - bw0) < cellCount;
+                };
+                for_rows_of_list(idx, list_count(a.g, a.blocks), over, [&](uint32_t j) {
+                    const BlockOrigin o = origin_of(load_triple(idx, j), a.g);
+                    const int ss = (int)w - o.w0;
+                    if ((unsigned)ss >= (unsigned)a.g.S) return;
+#pragma unroll
+                    for (int u = 0; u < STRIP_ROWS; ++u) {
+                        const int rr = hTop + u - o.h0;
+                        if (off[u] != BUF_OOB && (unsigned)rr < (unsigned)a.g.R)
+                            b[u] = vadd(b[u], strip_stack_load<VEC, false>(x, (int)j, rr, (uint32_t)ss, cv, a));
+                    }
+                });
+#pragma unroll
+                for (int u = 0; u < STRIP_ROWS; ++u) buf_store<BUF_NT>(yr, off[u], b[u]);
+                return;
+            }
             vec q[STRIP_ROWS][4];
             int pos[STRIP_ROWS][4];
 #pragma unroll
@@ -2122,8 +2158,9 @@ __global__ __launch_bounds__(512) void k_scatter_tiles_and_rest(const float* __r
     }
 }
 
-// The gather's gradient from a planar stack: tiles that store every covered pixel once (SCATTER_SUM) and strips of zeros, in
-// one launch behind the one that makes the map.
+// The gather's gradient from a planar stack: tiles that store every covered pixel once (SCATTER_SUM_MARKED) and strips of zeros,
+// in one launch behind the one that makes the map.  us with no block named twice / one / eight: 300x480x256, 176 blocks of 18x18 45.0 / 79 /
+// 122; [4,256,256,64], 231 of 18x18 21 / 31 / 34; [16,256,256,64], 1080 of 20x20 108.4 / 115 / 125.
 template <int VEC>
 __global__ __launch_bounds__(512) void k_sum_tiles_and_zeros(const float* __restrict__ x, float* __restrict__ y,
                                                              const int16_t* __restrict__ idx, TileArgs a, ColorArgs col, StripArgs s)
@@ -2132,9 +2169,8 @@ __global__ __launch_bounds__(512) void k_sum_tiles_and_zeros(const float* __rest
     __shared__ uint32_t waveBits[8];
     __shared__ StripCells<1> cells;
     if (blockIdx.x < a.total) {
-        if (list_has_repeats(col)) return;
         const uint32_t ib = fdiv(blockIdx.x, a.dTpb);
-        scatter_planar_tile<VEC, SCATTER_SUM, TileRt>(x, y, y, idx, a, col, lds, waveBits, ib, blockIdx.x - ib * a.tpb);
+        scatter_planar_tile<VEC, SCATTER_SUM_MARKED, TileRt>(x, y, y, idx, a, col, lds, waveBits, ib, blockIdx.x - ib * a.tpb);
     } else {
         scatter_strip<VEC, STRIP_ZERO, true, false, true>(x, nullptr, y, idx, col.map, nullptr, col.dup, s, lds, &cells, blockIdx.x - a.total);
     }
@@ -2604,17 +2640,17 @@ hipError_t launch_scatter_onto_zeros(const float* x, float* y, const int16_t* id
 
 // The map of the cells, in one launch or two.
 static void launch_cell_map(const int16_t* idx, int numActive, const StripArgs& a, int32_t* map, int64_t mapN, int32_t* chain,
-                            int32_t* dup, hipStream_t stream)
+                            int32_t* dup, hipStream_t stream, bool mark = false)
 {
     if (mapN <= BLOCK_MAP_ONE_WG && numActive <= BLOCK_MAP_ONE_WG) {
-        hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN, chain, dup);
+        hipLaunchKernelGGL(k_cell_map_small, dim3(1), dim3(1024), 0, stream, idx, numActive, a, map, (int)mapN, chain, dup, mark);
         return;
     }
     int64_t fillWgs = (mapN + 255) / 256;
     if (fillWgs > 4096) fillWgs = 4096;
     hipLaunchKernelGGL(k_pull_fill, dim3((unsigned)fillWgs), dim3(256), 0, stream, map, mapN, dup);
     hipLaunchKernelGGL(k_cell_map, dim3((unsigned)((numActive + 255) / 256)), dim3(256), 0, stream, idx, numActive, a, map,
-                       chain, dup);
+                       chain, dup, mark);
 }
 
 // What the one-pass kernels look cells up in: the list itself, or a map that earlier launches made of it.
@@ -2854,7 +2890,7 @@ static void launch_sum_by_strips(const float* x, float* y, const int16_t* idx, i
         (uint64_t)a.total + s.tiles >= (1ull << 31))
         return;
     int32_t* map = static_cast<int32_t*>(workspace);
-    launch_cell_map(idx, numActive, s, map, mapN, nullptr, map + mapN, stream);
+    launch_cell_map(idx, numActive, s, map, mapN, nullptr, map + mapN, stream, true);
     const ColorArgs col = order_by_map(s, map, nullptr, map + mapN);
     width([&](auto w) {
         hipLaunchKernelGGL((k_sum_tiles_and_zeros<decltype(w)::value>), dim3(a.total + s.tiles), dim3(threads), lds, stream, x, y, idx, a,

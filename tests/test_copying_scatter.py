@@ -131,3 +131,30 @@ def test_gather_gradient_by_strips(shape, bs, bst, bo, M, twice):
             np.testing.assert_allclose(got, want, rtol=0, atol=1.2e-5)
         else:
             np.testing.assert_array_equal(got.view(np.int32), want.view(np.int32), err_msg="transpose %s" % transpose)
+
+
+@pytest.mark.parametrize("shape,bs,bst,bo", [
+    ((3, 45, 43, 32), (6, 7), (4, 5), (-1, -2)),       # overlap in both directions
+    ((3, 45, 43, 6), (6, 4), (4, 4), (-1, 0)),         # in rows only
+    ((3, 45, 43, 15), (4, 7), (4, 5), (-2, -3)),       # in columns only
+    ((3, 45, 43, 8), (5, 6), (6, 6), (0, -1)),         # in none
+    ((1, 60, 62, 132), (12, 13), (6, 7), (-1, -1)),    # every pixel under four blocks
+], ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("few", [True, False])
+def test_gather_gradient_of_lists_with_many_repeats(shape, bs, bst, bo, few):
+    """The sums in list order, exactly, with blocks that one, two and more rows name side by side."""
+    from sbnet_amd import ops
+    N, H, W, C = shape
+    rng = np.random.default_rng(C)
+    bc = [1 + (H - bo[0] - 1) // bst[0], 1 + (W - bo[1] - 1) // bst[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(-1, bc[0] + 1) for j in range(-1, bc[1])], np.int16)
+    M = len(cells) * 3 // 4
+    idx = cells[rng.permutation(len(cells))[:M]] if few else cells[rng.integers(len(cells), size=M)]
+    idx[:3] = idx[-1] = cells[len(cells) // 2]         # one block by four rows, first and last ones among them
+    for transpose in (False, True):
+        g = rng.standard_normal((M, C, *bs) if transpose else (M, *bs, C)).astype(np.float32)
+        g.reshape(-1)[::5] = -0.0
+        want = orc.sparse_scatter(g, [M], idx, np.zeros(shape, np.float32), bs, bst, bo, add=True, atomic=True,
+                                  transpose=transpose)
+        got = ops.gather_backward(dev(g), [M], dev(idx), shape, list(bs), list(bst), list(bo), transpose).cpu().numpy()
+        np.testing.assert_array_equal(got.view(np.int32), want.view(np.int32), err_msg="transpose %s" % transpose)
