@@ -560,6 +560,10 @@ static bool launch_fixed_lines(const float* x, float* y, const int16_t* idx, con
            launch_fixed_lines_one<LinesFixed<18, 18, 256, 2, 512>>(x, y, idx, a, threads, ld, lds, numActive, stream);
 }
 
+// Channels per vector of the planar gather, vec being what channels and address allow: from four channels on vectors of four,
+// ragged where they make none (see gather_planar_tile).
+static int planar_gather_vec(const Geom& g, int vec) { return g.C >= 4 ? 4 : vec; }
+
 template <int VEC>
 static void gather_dispatch(const float* x, float* y, const int16_t* idx, const Geom& g, int numActive,
                             bool transpose, hipStream_t stream, hipError_t& err)
@@ -594,15 +598,15 @@ static void gather_dispatch(const float* x, float* y, const int16_t* idx, const 
         }
         // 32 KB tiles: 46.5 us against 52.7 us with 16 KB tiles on the 800x800x128 workload.
         // Planes of fewer than 4 pixels and images or blocks beyond 32-bit byte offsets take the generic kernel.
-        const bool ragged = VEC < 4 && g.C >= 4;
-        if ((int64_t)g.R * g.S < 4 || !make_tile_args(g, numActive, ragged ? 4 : VEC, a, threads, lds, grid, 32 * 1024)) {
+        const int vec = planar_gather_vec(g, VEC);
+        if ((int64_t)g.R * g.S < 4 || !make_tile_args(g, numActive, vec, a, threads, lds, grid, 32 * 1024)) {
             const int64_t total = (int64_t)numActive * g.C * g.R * g.S;
             const int64_t wgs = (total + 255) / 256;
             hipLaunchKernelGGL((k_planar_small<SCATTER_ASSIGN, true>), dim3((unsigned)(wgs > 65536 ? 65536 : wgs)),
                                dim3(256), 0, stream, x, y, (const float*)y, idx, g, total, (const int32_t*)nullptr);
             return;
         }
-        if (ragged)
+        if (vec != VEC)
             hipLaunchKernelGGL((k_gather_planar<4, true>), tile_grid(a.grid2d, a.tpb, numActive, a.total, a.g), dim3(threads), lds,
                                stream, x, y, idx, a);
         else
@@ -612,7 +616,7 @@ static void gather_dispatch(const float* x, float* y, const int16_t* idx, const 
 }
 
 // Test hook (sbnet_test_tile_choice): the tile the planar kernels would use for a geometry, without launching.
-// kind 0: k_gather_lines, 1: k_gather_planar with vectors of vec floats (its ragged launches have 4), 2: k_scatter_planar.  out = {threads, ldsBytes, P, Pp, psplit, Ct,
+// kind 0: k_gather_lines, 1: k_gather_planar, 2: k_scatter_planar; vec: floats per vector that channels and addresses allow.  out = {threads, ldsBytes, P, Pp, psplit, Ct,
 // cchunks, vectors or slots per thread needed, vectors or slots per thread available, last split's pixels, fixed
 // instance available}.  Returns 0 when that kernel does not apply to the geometry.
 int tile_choice(int kind, const Geom& g, int numActive, int vec, int yAlignedTo, int32_t* out)
@@ -639,7 +643,7 @@ int tile_choice(int kind, const Geom& g, int numActive, int vec, int yAlignedTo,
     }
     if (kind == 2) return scatter_tile_choice(g, numActive, vec, out);
     TileArgs a;
-    if (RS < 4 || !make_tile_args(g, numActive, vec, a, threads, lds, grid, 32 * 1024)) return 0;
+    if (RS < 4 || !make_tile_args(g, numActive, planar_gather_vec(g, vec), a, threads, lds, grid, 32 * 1024)) return 0;
     const int lpp = 1 << a.lppLog;
     out[0] = threads; out[1] = (int32_t)lds; out[2] = a.P; out[3] = a.Pp; out[4] = a.psplit; out[5] = a.Ct;
     out[6] = a.cchunks;

@@ -54,7 +54,19 @@ def test_tiles_fit_the_kernels(kind):
                     short_tails += t["last"] < 4
     # last splits of fewer than 4 pixels do occur (63x63 with 32 channels ...): the scatter kernel moves those float
     # by float (tests/test_hip_parity.py::test_planar_scatter_short_last_split runs them on the GPU)
-    assert short_tails > 0
+    assert short_tails > 0 or kind == GATHER_PLANAR   # (the gather's tiles of 16-byte vectors leave none at these sizes)
+
+
+def test_gathers_of_any_width_take_the_tiles_of_16_byte_vectors():
+    """From four channels on the planar gather moves 16-byte vectors, whatever channels and address make."""
+    for R, S, C in itertools.product((2, 9, 14, 27, 63), (3, 14, 65), (4, 5, 6, 15, 17, 30, 33, 63, 130, 257)):
+        for num_active in (3, 5000):
+            want = choice(GATHER_PLANAR, R, S, C, num_active, 4)
+            assert want["Ct"] % 4 == 0 and want["cchunks"] * want["Ct"] >= C > (want["cchunks"] - 1) * want["Ct"]
+            assert want["need"] <= want["have"] and want["lds"] == want["Ct"] * want["Pp"] * 4 <= 32 * 1024, want
+            for vec in (1, 2):
+                assert choice(GATHER_PLANAR, R, S, C, num_active, vec) == want, (R, S, C, vec)
+    assert choice(GATHER_PLANAR, 9, 14, 3, 5000, 1)["Ct"] == 4 and choice(GATHER_PLANAR, 9, 14, 2, 5000, 2)["Ct"] == 2
 
 
 LINE = 16  # floats per unit of ownership of the line-owning gather: 64 bytes
