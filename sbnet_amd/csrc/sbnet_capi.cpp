@@ -1003,6 +1003,17 @@ int sbnet_test_tile_choice(int kind, int N, int H, int W, int C, int R, int S, i
     return sbnet::tile_choice(kind, make_geom(N, H, W, C, bsize, bstride, boffset), num_active, vec, y_aligned_to, out);
 }
 
+// Test hook, not part of the public header: the copying scatter's route.  dims, geometry: four and six ints (bsize, bstride,
+// boffset); out must hold 5 int32; see sbnet::scatter_route.
+int sbnet_test_scatter_route(const int32_t* dims, const int32_t* geometry, int num_active, int transpose, int add, int y_aligned_to,
+                             int32_t* out)
+{
+    if (!dims || !geometry || !out || num_active <= 0 || !geom_ok(dims[0], dims[1], dims[2], dims[3], geometry, geometry + 2)) return -1;
+    sbnet::scatter_route(make_geom(dims[0], dims[1], dims[2], dims[3], geometry, geometry + 2, geometry + 4), num_active, transpose != 0,
+                         add != 0, y_aligned_to, out);
+    return 0;
+}
+
 int sbnet_copy_tensor(float* dst, const float* src, size_t count, void* stream)
 {
     if (count && (!dst || !src)) return SBNET_EINVAL_ARG;

@@ -47,6 +47,8 @@ hipError_t static_scratch(void** ptr);
 
 // Test hook: see tile_choice in sbnet_gather.hip.
 int tile_choice(int kind, const Geom& g, int numActive, int vec, int yAlignedTo, int32_t* out);
+// Test hook: see scatter_route in sbnet_scatter.hip.
+void scatter_route(const Geom& g, int numActive, bool transpose, bool add, int yAlignedTo, int32_t* out);
 
 hipError_t launch_gather(const float* x, float* y, const int16_t* idx, int numActive,
                          const Geom& g, bool transpose, hipStream_t stream);

@@ -2770,6 +2770,59 @@ constexpr int STRIP_LIST_MAX = 1536;
 constexpr uint32_t CELLS_LIST_MAX_WGS = 6144;
 constexpr int64_t REST_LIST_MAX = 3500000;   // strips times rows
 
+// How the copying scatter goes: in one pass over the output, by strips (NHWC stacks, planar ones that they can stage), by cells,
+// or by tiles and strips; ROUTE_NONE: not in one pass.
+enum OverRoute { ROUTE_NONE = 0, ROUTE_STRIPS = 1, ROUTE_CELLS = 2, ROUTE_REST = 3 };
+
+struct OverPlan {
+    OverRoute how;
+    bool list;   // the workgroups read the list themselves
+    int vec;
+    StripArgs a;
+    CellsPlan cells;
+    RestPlan rest;
+    int64_t mapN;
+};
+
+static void plan_over(const float* x, const float* ybase, const float* y, int numActive, const Geom& g, bool transpose, bool add,
+                      size_t workspaceBytes, OverPlan& p)
+{
+    p.how = ROUTE_NONE;
+    p.list = numActive <= STRIP_LIST_MAX;
+    p.mapN = 0;
+    const int vb = pick_vec(g, ybase, y), vx = pick_vec(g, transpose ? nullptr : x, nullptr);
+    p.vec = vb < vx ? vb : vx;
+    if (add && (g.U < g.R || g.V < g.S)) return;
+    if (make_strip_args(g, numActive, p.vec, transpose, x, p.a, p.mapN)) {
+        p.how = ROUTE_STRIPS;
+    } else if (transpose) {
+        if (make_strip_args(g, numActive, p.vec, false, x, p.a, p.mapN) && plan_cells(g, numActive, p.vec, p.a, p.mapN, p.cells)) {
+            p.how = ROUTE_CELLS;
+            p.list = p.list && (uint32_t)p.mapN * p.cells.a.tpb <= CELLS_LIST_MAX_WGS;
+        } else if (plan_rest(g, numActive, p.vec, p.rest, p.mapN)) {
+            p.how = ROUTE_REST;
+            p.a = p.rest.s;
+            p.list = p.list && (int64_t)p.rest.s.tiles * numActive <= REST_LIST_MAX;
+            // (with a map two more launches: worth it once the blocks cover enough of the tensor)
+            if (!p.list && (int64_t)numActive * g.R * g.S * g.C * 4 < (16ll << 20)) p.how = ROUTE_NONE;
+        }
+    }
+    if (!p.list && workspaceBytes < (size_t)p.mapN * 4 + 16 + (size_t)numActive * 4 + 16) p.how = ROUTE_NONE;
+}
+
+// Test hook (sbnet_test_scatter_route): the route for a geometry and addresses aligned to yAlignedTo bytes (0: 16 and more),
+// without launching.  out = {route, by the list, vector width, workgroups, strips among them}.
+void scatter_route(const Geom& g, int numActive, bool transpose, bool add, int yAlignedTo, int32_t* out)
+{
+    const float* const y = reinterpret_cast<const float*>((uintptr_t)0x10000 + (uintptr_t)yAlignedTo);   // (never dereferenced)
+    OverPlan p;
+    plan_over(nullptr, y, y, numActive, g, transpose, add, (size_t)-1, p);
+    out[0] = p.how; out[1] = p.list; out[2] = p.vec;
+    out[3] = p.how == ROUTE_CELLS ? (int32_t)((uint32_t)p.mapN * p.cells.a.tpb) : p.how == ROUTE_REST ? (int32_t)(p.rest.a.total + p.rest.s.tiles)
+           : p.how == ROUTE_STRIPS ? (int32_t)p.a.tiles : 0;
+    out[4] = p.how == ROUTE_REST ? (int32_t)p.rest.s.tiles : p.how == ROUTE_STRIPS ? out[3] : 0;
+}
+
 hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y, const int16_t* idx, int numActive,
                                     const Geom& g, bool transpose, ScatterMode mode, void* workspace,
                                     size_t workspaceBytes, hipStream_t stream, bool& done)
@@ -2778,50 +2831,29 @@ hipError_t launch_scatter_over_base(const float* x, const float* ybase, float* y
     if (mode == SCATTER_ATOMIC || numActive <= 0) return hipSuccess;
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 3)) return hipSuccess;
 
-    // One pass over the output: strips (NHWC stacks, planar ones that they can stage), cells, or tiles and strips.
-    if (mode == SCATTER_ASSIGN || !(g.U < g.R || g.V < g.S)) {
-        const bool add = mode == SCATTER_ADD;
-        const int vb = pick_vec(g, ybase, y), vx = pick_vec(g, transpose ? nullptr : x, nullptr);
-        const int vec = vb < vx ? vb : vx;
-        bool list = numActive <= STRIP_LIST_MAX;
-        StripArgs a;
-        CellsPlan cells;
-        RestPlan rest;
-        int64_t mapN = 0;
-        enum { NONE, STRIPS, CELLS, REST } how = NONE;
-        if (make_strip_args(g, numActive, vec, transpose, x, a, mapN)) {
-            how = STRIPS;
-        } else if (transpose) {
-            if (make_strip_args(g, numActive, vec, false, x, a, mapN) && plan_cells(g, numActive, vec, a, mapN, cells)) how = CELLS;
-            else if (plan_rest(g, numActive, vec, rest, mapN)) how = REST;
-            if (how == CELLS) list = list && (uint32_t)mapN * cells.a.tpb <= CELLS_LIST_MAX_WGS;
-            if (how == REST) list = list && (int64_t)rest.s.tiles * numActive <= REST_LIST_MAX;
-            // (with a map two more launches: worth it once the blocks cover enough of the tensor)
-            if (how == REST && !list && (int64_t)numActive * g.R * g.S * g.C * 4 < (16ll << 20)) how = NONE;
+    const bool add = mode == SCATTER_ADD;
+    OverPlan p;
+    plan_over(x, ybase, y, numActive, g, transpose, add, workspaceBytes, p);
+    if (p.how != ROUTE_NONE) {
+        CellMap m{p.list, nullptr, nullptr, nullptr};
+        if (!p.list) {
+            int32_t* map = static_cast<int32_t*>(workspace);
+            int32_t* dup = map + p.mapN;
+            int32_t* chain = add ? dup + 4 : nullptr;
+            launch_cell_map(idx, numActive, p.a, map, p.mapN, chain, dup, stream);
+            m.map = map; m.chain = chain; m.dup = dup;
         }
-        if (how == REST) a = rest.s;
-        if (!list && workspaceBytes < (size_t)mapN * 4 + 16 + (size_t)numActive * 4 + 16) how = NONE;
-        if (how != NONE) {
-            CellMap m{list, nullptr, nullptr, nullptr};
-            if (!list) {
-                int32_t* map = static_cast<int32_t*>(workspace);
-                int32_t* dup = map + mapN;
-                int32_t* chain = add ? dup + 4 : nullptr;
-                launch_cell_map(idx, numActive, a, map, mapN, chain, dup, stream);
-                m.map = map; m.chain = chain; m.dup = dup;
-            }
-            auto go = [&](auto width) {
-                constexpr int VEC = decltype(width)::value;
-                if (how == STRIPS) launch_strip<VEC>(x, ybase, y, idx, transpose, add, m, a, stream);
-                else if (how == CELLS) launch_cells<VEC>(x, ybase, y, idx, add, m, cells, stream);
-                else launch_rest<VEC>(x, ybase, y, idx, add, m, rest, stream);
-            };
-            if (vec == 4) go(std::integral_constant<int, 4>());
-            else if (vec == 2) go(std::integral_constant<int, 2>());
-            else go(std::integral_constant<int, 1>());
-            done = true;
-            return hipGetLastError();
-        }
+        auto go = [&](auto width) {
+            constexpr int VEC = decltype(width)::value;
+            if (p.how == ROUTE_STRIPS) launch_strip<VEC>(x, ybase, y, idx, transpose, add, m, p.a, stream);
+            else if (p.how == ROUTE_CELLS) launch_cells<VEC>(x, ybase, y, idx, add, m, p.cells, stream);
+            else launch_rest<VEC>(x, ybase, y, idx, add, m, p.rest, stream);
+        };
+        if (p.vec == 4) go(std::integral_constant<int, 4>());
+        else if (p.vec == 2) go(std::integral_constant<int, 2>());
+        else go(std::integral_constant<int, 1>());
+        done = true;
+        return hipGetLastError();
     }
 
     // Plain writes of overlapping blocks: the owner map of the ordered scatter also tells which pixels are covered.
