@@ -1813,7 +1813,7 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
                                               float* __restrict__ y, const int16_t* __restrict__ idx,
                                               const int32_t* __restrict__ map, const int32_t* __restrict__ chain,
                                               const int32_t* __restrict__ dup, const StripArgs& a, float* lds,
-                                              StripCells<CELLS>* cells, uint32_t strip)
+                                              StripCells<CELLS>* cells, uint32_t strip, bool repeats = false)
 {
     typedef typename Vec<VEC>::type vec;
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
@@ -1896,7 +1896,7 @@ __device__ __forceinline__ void scatter_strip(const float* __restrict__ x, const
     }
     if constexpr (SUM) {
         if constexpr (OP == STRIP_ZERO) {
-            if (*(const_i32_ptr)(reinterpret_cast<uintptr_t>(dup)) != 0) {   // (rare)
+            if (repeats) {   // (rare)
                 int heads[4] = {own, left1, up0, up1};
                 int wRare = (int)w, nRare = (int)n;
                 // (keeps the compiler from working any of this out ahead of the branch: 46.0 us at 300x480x256, 45.0 this way)
@@ -2172,7 +2172,8 @@ __global__ __launch_bounds__(512) void k_sum_tiles_and_zeros(const float* __rest
         const uint32_t ib = fdiv(blockIdx.x, a.dTpb);
         scatter_planar_tile<VEC, SCATTER_SUM_MARKED, TileRt>(x, y, y, idx, a, col, lds, waveBits, ib, blockIdx.x - ib * a.tpb);
     } else {
-        scatter_strip<VEC, STRIP_ZERO, true, false, true>(x, nullptr, y, idx, col.map, nullptr, col.dup, s, lds, &cells, blockIdx.x - a.total);
+        const bool repeats = list_has_repeats(col);   // (ahead of the strip's own loads)
+        scatter_strip<VEC, STRIP_ZERO, true, false, true>(x, nullptr, y, idx, col.map, nullptr, nullptr, s, lds, &cells, blockIdx.x - a.total, repeats);
     }
 }
 
@@ -2226,7 +2227,8 @@ __device__ __forceinline__ void copy_cell(const float* __restrict__ ybase, float
 
 template <int VEC, int MODE, bool LIST>
 __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__ x, const float* ybase, float* y,
-                                                       const int16_t* __restrict__ idx, TileArgs a, ColorArgs col,
+                                                       const int16_t* __restrict__ idx,
+                                                       const int32_t* __restrict__ map, TileArgs a, ColorArgs col,
                                                        CellArgs c)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -2277,7 +2279,7 @@ __global__ __launch_bounds__(512) void k_scatter_cells(const float* __restrict__
         if (ADD) several = __builtin_amdgcn_readfirstlane(found[1]) > 1;
     } else {
         // (scalar loads: the map was written by an earlier launch and is not written here)
-        head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(col.map)))[cell];
+        head = ((const_i32_ptr)(reinterpret_cast<uintptr_t>(map)))[cell];
         if (ADD && head >= 0 && list_has_repeats(col)) several = chain_next(col.chain, head) >= 0;
     }
     if (head >= 0) scatter_planar_tile<VEC, MODE, TileRt, true>(x, y, ybase, idx, a, col, lds, waveBits, (uint32_t)head, rem, several);
@@ -2720,8 +2722,8 @@ static void launch_cells(const float* x, const float* ybase, float* y, const int
                          const CellsPlan& p, hipStream_t stream)
 {
     ColorArgs col = NO_ORDER;
-    col.map = m.map; col.chain = m.chain; col.dup = m.dup;
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, p.grid, dim3(p.threads), p.lds, stream, x, ybase, y, idx, p.a, col, p.c); };
+    col.chain = m.chain; col.dup = m.dup;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, p.grid, dim3(p.threads), p.lds, stream, x, ybase, y, idx, m.map, p.a, col, p.c); };
     if (add) m.list ? go(k_scatter_cells<VEC, SCATTER_ADD_LISTED, true>) : go(k_scatter_cells<VEC, SCATTER_ADD_MAPPED, false>);
     else m.list ? go(k_scatter_cells<VEC, SCATTER_ASSIGN, true>) : go(k_scatter_cells<VEC, SCATTER_ASSIGN, false>);
 }
@@ -2762,13 +2764,21 @@ static void launch_rest(const float* x, const float* ybase, float* y, const int1
 // more.  us with the map / with the list, MI355X: 512x512x64, add, 102 rows 27.0 / 24.8, 512: 30.2 / 27.7, 921: 34.8 / 31.7;
 // [4,256,256,64], 1351 rows of 8x8: 29.2 / 26.8, as cells 28.9 / 26.8; eight images, 2703 rows: 57.7 / 55.4, as cells 55.3 /
 // 66.4; 16 images, 5406: 110 / 120.
-// Where a workgroup can do nothing before it has looked its cell up, and there are many of them, the list costs more than the
-// launches.  Cells: 242 of 20x20x128, 3000 workgroups 17.8 / 16.2; 2312 of 16x16x64, 9000: 49.8 / 50.8; 2116 of 24x24x64, 21 000:
-// 86 / 97.  Tiles and the rest, by strips times rows: 0.3 M 18.1 / 16.5, 1.4 M 104.4 / 99.9, 3.8 M 108 / 112, 4.5 M 120 / 112, 6.1 M
-// 121.6 / 125.5, 6.3 M 104 / 112, 10.6 M 103 / 107.  Strips, which move the most, gain at every size measured.
+// Where there are very many workgroups the list costs more than the launches.  Cells, where a workgroup can do nothing before it
+// has looked its cell up; its wait counts, the length of the list hardly does.  Workgroups and rows: 4050, 400 and 1500 rows of
+// 9x9x32 17.2 / 15.1 and 17.7 / 15.6; 5408, 400 and 1500 of 10x10x64 21.6 / 20.0 and 23.1 / 21.2; 6724, 400 and 1500 of 20x20x32 32.3 /
+// 30.5 and 33.5 / 33.2; 10816, 400 of 16x16x64 52.6 / 59.1; 11016, 100 of 18x18x256 50.1 / 58.5; 21780, 400 of 25x25x128 110.5 / 120.3.
+// Tiles and the rest: every tile compares its row with the list (tiles; map / list): 7200 of 27x27x128, 121.3 / 115.5; 8800 of 14x14x128,
+// gaps, 122.3 / 120.4; 9600 of 18x18x256 58.8 / 59.3, gaps 60.1 / 61.4; 12000 of 14x14x128 121.7 / 127.0; 16800 of 27x27x128 128.1 / 136.2,
+// gaps 120.5 / 130.5.  Every strip enters it (strips times rows, few tiles): 1.9 M 28.4 / 26.4, 6.0 M 26.6 / 23.8, 8.3 M 27.9 / 24.9,
+// 11.1 M 122.9 / 115.7; 12.3 M 46.5 / 47.6, 16.7 M 46.2 / 48.8, but 15.1 M 123.6 / 116.5.  The tiles of 27x27x128 and 16x16x64, for
+// which the other scatters have kernels of fixed size, are in step with them: 27x27x128 with gaps, 84, 252 and 504 blocks, copy and
+// fixed tiles in two launches / this one 118.7 / 118.5, 118.7 / 115.6, 116.0 / 117.0; 16x16x64, 102 and 307 blocks 27.0 / 21.5, 25.5 / 22.0.
+// Strips, which move the most, gain at every size measured.
 constexpr int STRIP_LIST_MAX = 1536;
 constexpr uint32_t CELLS_LIST_MAX_WGS = 6144;
-constexpr int64_t REST_LIST_MAX = 3500000;   // strips times rows
+constexpr uint32_t REST_LIST_MAX_TILES = 9000;
+constexpr int64_t REST_LIST_MAX = 12000000;   // strips times rows
 
 // How the copying scatter goes: in one pass over the output, by strips (NHWC stacks, planar ones that they can stage), by cells,
 // or by tiles and strips; ROUTE_NONE: not in one pass.
@@ -2802,7 +2812,7 @@ static void plan_over(const float* x, const float* ybase, const float* y, int nu
         } else if (plan_rest(g, numActive, p.vec, p.rest, p.mapN)) {
             p.how = ROUTE_REST;
             p.a = p.rest.s;
-            p.list = p.list && (int64_t)p.rest.s.tiles * numActive <= REST_LIST_MAX;
+            p.list = p.list && p.rest.a.total <= REST_LIST_MAX_TILES && (int64_t)p.rest.s.tiles * numActive <= REST_LIST_MAX;
             // (with a map two more launches: worth it once the blocks cover enough of the tensor)
             if (!p.list && (int64_t)numActive * g.R * g.S * g.C * 4 < (16ll << 20)) p.how = ROUTE_NONE;
         }
