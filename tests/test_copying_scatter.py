@@ -1,11 +1,14 @@
-"""The copying scatter's one-pass kernels against the oracle, on both sides of the length up to which their workgroups
-read the block list themselves (1536 rows) and from which on a map is made of it first."""
+"""The copying scatter's one-pass kernels against the oracle, by the list, which their workgroups read themselves up to 1536
+rows, and by the map that is made of it first for longer ones and some large launches; the gather's gradient by the same kernels."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import sbnet_amd
 from oracle import sbnet_oracle as orc
+from sbnet_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -16,7 +19,18 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
 
 
-@pytest.mark.parametrize("M", [1, 1536, 1537])
+NONE, STRIPS, CELLS, REST = range(4)
+
+
+def route(shape, bs, bst, bo, M, transpose, add, aligned_to=0):
+    """How the library goes about a copying scatter: the kernel, whether by the list, the vector width."""
+    out = (ctypes.c_int32 * 5)()
+    assert _lib.load().sbnet_test_scatter_route((ctypes.c_int32 * 4)(*shape), (ctypes.c_int32 * 6)(*bs, *bst, *bo), M, int(transpose),
+                                                int(add), aligned_to, out) == 0
+    return tuple(out[:3])
+
+
+@pytest.mark.parametrize("M", [1, 700, 1536, 1537])
 @pytest.mark.parametrize("shape,bs,bst,bo", [
     ((8, 66, 80, 8), (6, 7), (4, 5), (-1, -2)),      # overlap in both directions: 16-byte vectors
     ((8, 66, 80, 6), (6, 4), (4, 4), (-1, 0)),       # in rows only
@@ -40,6 +54,9 @@ def test_copying_scatter_reads_lists_and_maps(shape, bs, bst, bo, M):
     mis = flat[1:].view(base_d.shape)                # aligned to 4 bytes only
     mis.copy_(base_d)
     overlap = bs[0] > bst[0] or bs[1] > bst[1]
+    assert route(shape, bs, bst, bo, M, False, not overlap)[:2] == (STRIPS, M <= 1536)
+    planar = route(shape, bs, bst, bo, M, True, not overlap)   # (tiles beside strips by the map: in a test of their own)
+    assert planar[:2] in ((STRIPS, M <= 1536), (CELLS, M <= 1536), (REST, 1), (NONE, 0)) and (planar[0] != NONE or M >= 1536)
     for transpose in (False, True):
         stack = rng.standard_normal((M, C, *bs) if transpose else (M, *bs, C)).astype(np.float32)
         stack_d = dev(stack)
@@ -70,6 +87,39 @@ def test_long_lists_that_name_blocks_several_times(shape, bs, bo):
             np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="transpose %s add %s" % (transpose, add))
 
 
+@pytest.mark.parametrize("shape,bs,bst,bo,M", [
+    ((4, 134, 140, 128), (6, 7), (4, 5), (-1, -2), 1600),   # overlap in both directions
+    ((4, 150, 150, 126), (8, 5), (5, 5), (-1, 0), 1600),    # in rows only; 8-byte vectors
+    ((4, 150, 150, 96), (5, 8), (5, 6), (-2, -3), 2048),    # in columns only
+    ((4, 150, 153, 115), (5, 6), (6, 7), (-1, -1), 1900),   # gaps; floats
+    ((1, 120, 120, 512), (5, 4), (4, 4), (-1, 0), 600),     # many tiles: a map for a list of few rows
+    ((1, 125, 127, 512), (4, 4), (5, 5), (0, -1), 610),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_tiles_and_strips_by_the_map(shape, bs, bst, bo, M):
+    N, H, W, C = shape
+    rng = np.random.default_rng(C)
+    bc = [1 + (H - bo[0] - 1) // bst[0], 1 + (W - bo[1] - 1) // bst[1]]
+    cells = np.array([(n, i, j) for n in range(N) for i in range(-1, bc[0] + 1) for j in range(-1, bc[1])], np.int16)
+    idx = cells[rng.permutation(len(cells))[:M]]
+    assert len(idx) == M
+    idx_d, base = dev(idx), rng.standard_normal(shape).astype(np.float32)
+    base_d = dev(base)
+    mis = torch.empty(base_d.numel() + 1, device=DEV)[1:].view(base_d.shape)   # aligned to 4 bytes only
+    mis.copy_(base_d)
+    stack = rng.standard_normal((M, C, *bs)).astype(np.float32)
+    stack_d = dev(stack)
+    overlap = bs[0] > bst[0] or bs[1] > bst[1]
+    for add in ((False,) if overlap else (False, True)):
+        widths = [route(shape, bs, bst, bo, M, True, add, a) for a in (0, 4)]
+        assert widths == [(REST, 0, 4 if C % 4 == 0 else 2 if C % 2 == 0 else 1), (REST, 0, 1)]
+        for count in (M, M - 3):
+            cnt = torch.tensor([count], dtype=torch.int32, device="cpu" if count == M else DEV)
+            want = orc.sparse_scatter(stack, [count], idx, base, bs, bst, bo, add=add, transpose=True)
+            for b in (base_d, mis):
+                y = sbnet_amd.sparse_scatter(stack_d, cnt, idx_d, b, bs, bst, bo, add=add, transpose=True)
+                np.testing.assert_array_equal(y.cpu().numpy(), want, err_msg="add %s count %d" % (add, count))
+
+
 @pytest.mark.parametrize("shape,bs,bst,bo", [
     ((3, 41, 38, 32), (5, 6), (6, 7), (-1, -2)),       # 16-byte vectors; a list that the workgroups read
     ((3, 41, 38, 6), (5, 6), (5, 7), (-1, 0)),
@@ -94,6 +144,7 @@ def test_repeated_rows_of_planar_blocks_with_gaps(shape, bs, bst, bo):
     mis = flat[1:].view(base.shape)
     mis.copy_(dev(base))
     for add in (False, True):
+        assert route(shape, bs, bst, bo, M, True, add)[:2] == route(shape, bs, bst, bo, M, True, add, 4)[:2] == (REST, not long)
         for count in (M, M - 3):
             cnt = torch.tensor([count], dtype=torch.int32, device="cpu" if count == M else DEV)
             want = orc.sparse_scatter(stack, [count], idx, base, bs, bst, bo, add=add, transpose=True)
