@@ -7,6 +7,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 
 import sbnet_amd
 from sbnet_amd import SparseGatherFunction, SparseScatterFunction, ops
+from sbnet_amd import sparse_conv as sc
 
 DEV = "cuda:0"
 BS, BT, BO = [6, 6], [4, 5], [-1, -2]
@@ -216,3 +217,127 @@ def test_relu_is_the_librarys(n):
     assert fn(x.data_ptr(), n, ops._stream()) == 0
     assert torch.equal(x.view(torch.int32), want.view(torch.int32))
     assert fn(x.data_ptr() + 4, 1, ops._stream()) == _lib.SBNET_EINVAL_ARG
+
+
+# ---- the residual function ----------------------------------------------------------------------------------------
+
+class LooksOn(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def residual_native(p, params):
+    q = sc._residual_in_training(p, params)
+    assert "ResidualFunction" in q.grad_fn.name() and "InTraining" not in q.grad_fn.name()
+    return q
+
+
+def residual_python(p, params):
+    with LooksOn():     # which the native function leaves to the one in Python
+        q = sc._residual_in_training(p, params)
+    assert "_ResidualInTraining" in q.grad_fn.name()
+    return q
+
+
+def make_residual(stats=True, seed=3):
+    params = sc.BottleneckParams([(1, 1, 16, 8), (3, 3, 8, 8), (1, 1, 8, 16)], DEV, seed=seed)
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    if not stats:
+        params.bn = [sc.BatchNormParams(b.gamma, b.beta, None, None) for b in params.bn]
+    return params, torch.randn(6, 16, 9, 9, device=DEV, generator=g).requires_grad_()
+
+
+def same(got, want):
+    """The same kernels on the same values, but for the order of the batch norms' sums, which are added up in double: a unit in
+    the last place of a coefficient, 2^-24 of each term, and what the later layers make of it."""
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and torch.linalg.vector_norm(a - b) <= 1e-6 * torch.linalg.vector_norm(b) + 1e-9
+
+
+def leaves_of(p, params):
+    return [p] + params.parameters()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wanted", ["all", "input", "kernels", "norms"])
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_residual_function_is_the_one_in_python(wanted, create_graph):
+    results = []
+    for op in (residual_native, residual_python):
+        params, p = make_residual()
+        for i, t in enumerate(leaves_of(p, params)):
+            t.requires_grad_(wanted == "all" or (wanted == "input") == (i == 0) and (wanted == "kernels") == (1 <= i <= 3))
+        leaves = [t for t in leaves_of(p, params) if t.requires_grad]
+        q = op(p, params)
+        dq = torch.linspace(-1, 1, q.numel(), device=DEV).view(q.shape)
+        grads = torch.autograd.grad(q, leaves, dq, create_graph=create_graph)
+        stats = [t for b in params.bn for t in (b.moving_mean, b.moving_var)]
+        if create_graph:
+            grads += torch.autograd.grad(sum((g * g).sum() for g in grads), leaves)
+        results.append([q.detach(), *stats, *(g.detach() for g in grads)])
+    same(*results)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [residual_native, residual_python])
+def test_residual_function_under_hooks_of_saved_tensors(op):
+    params, p = make_residual()
+    want = torch.autograd.grad(op(p, params).square().sum(), leaves_of(p, params))
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t.shape) or t.cpu(), lambda t: t.to(DEV)):
+        q = op(p, params)
+    assert len(kept) == 18
+    same(torch.autograd.grad(q.square().sum(), leaves_of(p, params)), want)
+    # what comes back in another order of memory goes through the layers: other kernels' sums, of up to 486 pixels and 144 taps
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.to(memory_format=torch.channels_last) if t.dim() == 4 else t):
+        q = op(p, params)
+    for a, b in zip(torch.autograd.grad(q.square().sum(), leaves_of(p, params)), want):
+        assert torch.linalg.vector_norm(a - b) <= 1e-4 * torch.linalg.vector_norm(b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [residual_native, residual_python])
+def test_residual_function_in_a_checkpoint(op):
+    from torch.utils.checkpoint import checkpoint
+    params, p = make_residual(stats=False)
+    want = torch.autograd.grad(op(p, params).square().sum(), leaves_of(p, params))
+    q = checkpoint(lambda t: op(t, params), p, use_reentrant=False)
+    same(torch.autograd.grad(q.square().sum(), leaves_of(p, params)), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", [residual_native, residual_python])
+def test_residual_function_takes_a_batch_of_gradients(op):
+    """Through the layers, one by one: sums of up to 486 pixels and 144 taps in another order."""
+    params, p = make_residual(stats=False)
+    q = op(p, params)
+    dq = torch.randn(3, *q.shape, device=DEV)
+    got = torch.autograd.grad(q, leaves_of(p, params), dq, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for a, b in zip(got, torch.autograd.grad(q, leaves_of(p, params), dq[i], retain_graph=True)):
+            assert torch.linalg.vector_norm(a[i] - b) <= 1e-4 * torch.linalg.vector_norm(b)
+
+
+@pytest.mark.gpu
+def test_residual_functions_of_two_threads():
+    """The forward pass runs without the interpreter's lock."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def job(seed):
+        params, p = make_residual(seed=seed)
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            out = []
+            for _ in range(5):
+                q = residual_native(p, params)
+                out = [q.detach(), *torch.autograd.grad(q.square().sum(), leaves_of(p, params))]
+            stream.synchronize()
+        return [t.cpu() for t in out]
+
+    want = [job(seed) for seed in (1, 2)]
+    with ThreadPoolExecutor(2) as pool:
+        got = list(pool.map(job, (1, 2)))
+    for a, b in zip(got, want):
+        same(a, b)
