@@ -774,25 +774,22 @@ struct ScatterFunction : torch::autograd::Function<ScatterFunction> {
         const int32_t M = (int32_t)v[0];
         const Pair bs = pair_at(v, 1), bt = pair_at(v, 3), bo = pair_at(v, 5);
         const bool transpose = v[11] & 1, add = v[11] & 2;
-        const bool blocks = ctx->needs_input_grad(0), base = ctx->needs_input_grad(1);
+        variable_list out(3);
+        bool todo[2] = {ctx->needs_input_grad(0), ctx->needs_input_grad(1)};   // of the blocks, of the base
         if (plain_list(idx, M, grad) && grad.sizes() == at::IntArrayRef(v.data() + 7, 4)) {
-            at::Tensor dbase;
-            if (base && add) dbase = grad;
-            else if (base && !(at::GradMode::is_enabled() && grad.requires_grad())) dbase = run_base_grad(grad, idx, M, bs, bt, bo);
-            if (!base || dbase.defined()) {
-                at::Tensor dblocks;
-                if (blocks) dblocks = run_gather({&grad, {&idx, M, nullptr}, bs, bt, bo, transpose}, nullptr);
-                return {dblocks, dbase, at::Tensor()};
-            }
+            if (todo[0]) out[0] = run_gather({&grad, {&idx, M, nullptr}, bs, bt, bo, transpose}, nullptr);
+            if (todo[1] && add) out[1] = grad;
+            else if (todo[1] && !(at::GradMode::is_enabled() && grad.requires_grad())) out[1] = run_base_grad(grad, idx, M, bs, bt, bo);
+            for (int i = 0; i < 2; ++i) todo[i] = todo[i] && !out[i].defined();
         }
+        if (!todo[0] && !todo[1]) return out;
         // besides: a graph of the gradients is asked for, or a geometry that the one pass does not take
         THPObjectPtr g(THPVariable_Wrap(grad)), list(THPVariable_Wrap(idx)), sizes(tuple_of(v));
         if (!g || !list) raise_pending();
-        THPObjectPtr got(PyObject_CallFunctionObjArgs(g_scatter_gradients, g.get(), list.get(), sizes.get(), blocks ? Py_True : Py_False,
-                                                      base ? Py_True : Py_False, nullptr));
+        THPObjectPtr got(PyObject_CallFunctionObjArgs(g_scatter_gradients, g.get(), list.get(), sizes.get(), todo[0] ? Py_True : Py_False,
+                                                      todo[1] ? Py_True : Py_False, nullptr));
         if (!got) raise_pending();
         TORCH_CHECK(PyTuple_CheckExact(got.get()) && PyTuple_GET_SIZE(got.get()) == 2, "gradients of two inputs");
-        variable_list out(3);
         for (int i = 0; i < 2; ++i) {
             PyObject* const o = PyTuple_GET_ITEM(got.get(), i);
             if (o != Py_None) out[i] = THPVariable_Unpack(o);
