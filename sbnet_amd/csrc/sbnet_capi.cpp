@@ -103,8 +103,8 @@ inline void cpu_relax()
 
 // Reads of the word before the stream is asked.  The question is no mere look: the runtime answers it by enqueueing a
 // barrier packet behind the kernels, which costs host time and holds up the launch that follows the count.  Asked every 256
-// reads, one came into nearly every wait: a step of mask, gather and scatter on a [1,64,64,16] map took 38.9 us (31.4 now),
-// on [3,301,203,15] 46.6 us (31.5).  After 2^14 reads, most of them behind a yield, some milliseconds have passed.
+// reads, one came into nearly every wait: a step of mask, gather and scatter on a [1,64,64,16] map took 38.9 us,
+// 31.4 without it, on [3,301,203,15] 46.6 and 31.5.  After 2^14 reads, most of them behind a yield, some milliseconds have passed.
 constexpr uint32_t SPINS_PER_QUERY = 1u << 14;
 
 // Waits until the word carries `seq` and returns the count; gives up (false) as soon as the stream has

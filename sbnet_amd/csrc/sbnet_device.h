@@ -370,6 +370,8 @@ struct NeighbourPos {
     int32_t pos[9];
 };
 
+// MARKED: the map marks blocks that several rows name (CELL_REPEATED), this block's own cell included.
+template <bool MARKED>
 __device__ __forceinline__ NeighbourPos neighbour_positions(const ColorArgs& col, const BlockOrigin& o, uint32_t ib)
 {
     typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
@@ -379,12 +381,12 @@ __device__ __forceinline__ NeighbourPos neighbour_positions(const ColorArgs& col
     for (int q = 0; q < 9; ++q) {  // (independent loads; a neighbour beyond the map reads the first entry and is masked)
         const int dh = q / 3 - 1, dw = q % 3 - 1;
         const int ih = o.bh + dh - col.bhMin, iw = o.bw + dw - col.bwMin;
-        in[q] = (unsigned)ih < (unsigned)col.nBH && (unsigned)iw < (unsigned)col.nBW;
+        in[q] = (MARKED || q != 4) && (unsigned)ih < (unsigned)col.nBH && (unsigned)iw < (unsigned)col.nBW;
         const int64_t slot = in[q] ? ((int64_t)o.n * col.nBH + ih) * col.nBW + iw : 0;
         other[q] = *(const_i32_ptr)(reinterpret_cast<uintptr_t>(col.map + slot));
     }
     NeighbourPos nb;
-    nb.later = in[4] && other[4] == CELL_REPEATED ? 0x1ffu : 0u;
+    nb.later = MARKED && in[4] && other[4] == CELL_REPEATED ? 0x1ffu : 0u;
     nb.pos[4] = -1;
 #pragma unroll
     for (int q = 0; q < 9; ++q) {

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256) void k_scatter_nhwc(const float* __restrict__ 
     NeighbourPos nb;
     nb.later = 0u;
     const bool repeats = MODE == SCATTER_SUM && list_has_repeats(col);
-    if (MODE == SCATTER_SUM && !repeats) nb = neighbour_positions(col, o, ib);
+    if (MODE == SCATTER_SUM && !repeats) nb = neighbour_positions<false>(col, o, ib);
     const rsrc_t wr = make_rsrc(MODE == SCATTER_OWNED ? col.owner + (int64_t)o.n * a.g.H * a.g.W : nullptr,
                                 MODE == SCATTER_OWNED ? (uint32_t)(a.g.H * a.g.W) * 4u : 0u);
     // SCATTER_RANKED_INLINE: the block is ranked against the rows listed after it inside the kernel.  The rows are
@@ -317,7 +317,7 @@ __device__ __forceinline__ void scatter_planar_tile(const float* __restrict__ x,
         const BlockOrigin o = origin_of(raw, a.g);
         atomics = MODE == SCATTER_SUM && list_has_repeats(col);
         if (!o.valid || atomics) return;
-        nb = neighbour_positions(col, o, t.ib);
+        nb = neighbour_positions<MODE == SCATTER_SUM_MARKED>(col, o, t.ib);
         summed = true;
         const rsrc_t sr2 = make_rsrc(x, (uint32_t)a.blocks * G::C(a) * RS * 4u);  // the whole stack
         const int S = (int)G::S(a);
@@ -1781,7 +1781,7 @@ __device__ __forceinline__ void strip_cells_of_map(const StripArgs& a, const int
 // STRIP_MASK: y = base * (0 where a block covers the pixel, 1 elsewhere), the gradient of plain writes with respect to their
 // base.  A product, so that infinities and NaN under a block become NaN, as they do in the product with a stamped-out mask that
 // this replaces (fill with ones, fill a stack with zeros, scatter it, multiply: 125 us at 300x480x256 with 30 % of the 18x18
-// blocks, 443 MB of them the product's).  This pass moves 295 MB: 46 us there, 6.4 TB/s.
+// blocks, 443 MB of them the product's).  This pass moves 295 MB: 42 us alone, 47 inside a training step.
 // STRIP_SUM: y = 0 + the blocks over a pixel, in list order, without a base: the gradient of the gather (NHWC stack).
 // STRIP_ZERO: zeros where no block lies, and sums in list order where one lies that several rows name (planar stack); the
 // tiles of the same launch sum up the rest.
